@@ -5,15 +5,21 @@
 
 namespace flue {
 
-// exp(X) by scaling and squaring a Taylor polynomial of degree <= 16 (Horner form).
+// exp(X) of a traceless anti-Hermitian X, by scaling and squaring a Taylor polynomial reduced
+// with the Cayley-Hamilton theorem.  For Y = X / 2^s (|Y| <= 1/8) and traceless Y,
+//   Y^3 = t Y + i u I,   t = Tr Y^2 / 2 (real, <= 0),   i u = det Y,
+// so every power of Y, and the polynomial, is a0 + a1 Y + a2 Y^2 with scalar coefficients.
+// Horner's rule on the coefficients (I + Y E / k) costs 10 flops a term, against one 3x3
+// product (216) a term on the matrices: one product in all, for Y^2, which is Hermitian.
+// Degree 11 always: the first dropped term, |Y|^12 / 12!, is below 4e-20.
 __device__ __forceinline__ Mat<double> su3_exp(const Mat<double>& X) {
     double nrm = 0.0;
 #pragma unroll
     for (int e = 0; e < 9; ++e) nrm += X.r[e] * X.r[e] + X.i[e] * X.i[e];
-    nrm = sqrt(nrm);
+    // 2^-s by halving the squared norm by 4 until it is at most 1/64
     int s = 0;
-    while (nrm > 0.125 && s < 60) {
-        nrm *= 0.5;
+    while (nrm > 0.015625 && s < 60) {
+        nrm *= 0.25;
         ++s;
     }
     const double scale = ldexp(1.0, -s);
@@ -23,24 +29,59 @@ __device__ __forceinline__ Mat<double> su3_exp(const Mat<double>& X) {
         Y.r[e] = X.r[e] * scale;
         Y.i[e] = X.i[e] * scale;
     }
-    // Taylor degree: the smallest K <= 16 whose first dropped term, |Y|^(K+1)/(K+1)!, is
-    // below 1e-17 (|Y| <= 0.125 after the scaling, so K <= 11; small flow steps need ~8)
-    int K = 1;
-    double term = 0.5 * nrm * nrm;  // |Y|^2 / 2!, the first term a degree-1 polynomial drops
-    while (K < 16 && term > 1e-17) {
-        ++K;
-        term *= nrm / (double)(K + 1);
-    }
-    Mat<double> E = identity<double>();
-    for (int k = K; k >= 1; --k) {
-        Mat<double> T = mul(Y, E);
-        const double inv = 1.0 / (double)k;
+    // Q = Y^2: (Y^2)_ab = -sum_k Y_ak conj(Y_bk), a <= b (Hermitian)
+    Mat<double> Q;
 #pragma unroll
-        for (int e = 0; e < 9; ++e) {
-            E.r[e] = T.r[e] * inv + ((e % 4 == 0) ? 1.0 : 0.0);
-            E.i[e] = T.i[e] * inv;
+    for (int a = 0; a < 3; ++a) {
+#pragma unroll
+        for (int b = a; b < 3; ++b) {
+            double qr = 0.0, qi = 0.0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                qr = fmad(-Y.r[a * 3 + k], Y.r[b * 3 + k], qr);
+                qr = fmad(-Y.i[a * 3 + k], Y.i[b * 3 + k], qr);
+                if (a == b) continue;
+                qi = fmad(-Y.i[a * 3 + k], Y.r[b * 3 + k], qi);
+                qi = fmad(Y.r[a * 3 + k], Y.i[b * 3 + k], qi);
+            }
+            Q.r[a * 3 + b] = Q.r[b * 3 + a] = qr;
+            Q.i[a * 3 + b] = qi;
+            Q.i[b * 3 + a] = -qi;
         }
     }
+    const double t = 0.5 * (Q.r[0] + Q.r[4] + Q.r[8]);
+    // i u = det Y = Tr(Y Q) / 3; Im Tr(Y Q) = sum_ab (Im Y_ab Re Q_ab - Re Y_ab Im Q_ab)
+    double u = 0.0;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {
+        u = fmad(Y.i[e], Q.r[e], u);
+        u = fmad(-Y.r[e], Q.i[e], u);
+    }
+    u *= 1.0 / 3.0;
+    // E <- I + Y E / k for k = 11 .. 1 on the coefficients:
+    //   (a0, a1, a2) <- (1 + i u a2 / k, (a0 + t a2) / k, a1 / k)
+    double a0r = 1.0, a0i = 0.0, a1r = 0.0, a1i = 0.0, a2r = 0.0, a2i = 0.0;
+#pragma unroll
+    for (int k = 11; k >= 1; --k) {
+        const double inv = 1.0 / (double)k;
+        const double n1r = fmad(t, a2r, a0r) * inv, n1i = fmad(t, a2i, a0i) * inv;
+        a0r = fmad(-u * inv, a2i, 1.0);
+        a0i = u * inv * a2r;
+        a2r = a1r * inv;
+        a2i = a1i * inv;
+        a1r = n1r;
+        a1i = n1i;
+    }
+    Mat<double> E;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {
+        double er = e % 4 == 0 ? a0r : 0.0, ei = e % 4 == 0 ? a0i : 0.0;
+        cmac(er, ei, a1r, a1i, Y.r[e], Y.i[e]);
+        cmac(er, ei, a2r, a2i, Q.r[e], Q.i[e]);
+        E.r[e] = er;
+        E.i[e] = ei;
+    }
+#pragma unroll 1
     for (int k = 0; k < s; ++k) E = mul(E, E);
     return E;
 }
