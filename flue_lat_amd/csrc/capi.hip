@@ -806,7 +806,7 @@ int flue_wilson_grad_ex(const int32_t dims[4], const void* U, int32_t prec, doub
     if (!U || !grad) return FLUE_ENULL;
     if (check_prec(prec) || !std::isfinite(beta) || variant < 0 || variant > kFlowVariants) return FLUE_EINVAL;
     const Lat L = make_lat(dims);
-    if (variant == 0) variant = variant_or(FLUE_OP_FLOW, dims, prec, kFlowDefault);
+    if (variant == 0) variant = variant_or(FLUE_OP_FLOW, dims, prec, grad_default(L));
     // the plaquette-first form needs unitary links (FP32 and declared-SU(3) fields) and a
     // workspace; otherwise the staple form in the same visit order
     void* T = nullptr;
@@ -856,8 +856,9 @@ int flue_flow_stage(const int32_t dims[4], const void* Win, int32_t prec, void* 
     if (check_prec(prec) || stage < 0 || stage > 2 || !std::isfinite(eps)) return FLUE_EINVAL;
     // Luescher RK3: acc <- ca acc + cb Z, (ca, cb) = (0, 1/4), (-17/9, 8/9), (-1, 3/4)
     // a single stage has no workspace for the plaquette-first form: staple sums
-    const int variant = staple_order_of(variant_or(FLUE_OP_FLOW, dims, prec, kFlowDefault));
-    return flow_stage_run(make_lat(dims), Win, prec, Wout, acc, eps, stage, variant, nullptr, S(stream));
+    const Lat L = make_lat(dims);
+    const int variant = staple_order_of(variant_or(FLUE_OP_FLOW, dims, prec, grad_default(L)));
+    return flow_stage_run(L, Win, prec, Wout, acc, eps, stage, variant, nullptr, S(stream));
 }
 
 int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, int32_t nsteps, int32_t use_graph,
@@ -872,7 +873,7 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
     void* W2 = w;
     double* acc = (double*)((char*)w + flow_acc_offset(L, prec));
     void* T = (char*)acc + (size_t)L.V * 32 * 8;
-    const int variant = variant_or(FLUE_OP_FLOW, dims, prec, kFlowDefault);
+    const int variant = variant_or(FLUE_OP_FLOW, dims, prec, flow_default(L));
     hipStream_t st = S(stream);
     // three stages per step alternate between U and W2, so two steps return the field to U
     auto two_steps = [&]() -> int {
@@ -1208,7 +1209,7 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
 
     int32_t key[4];
     ens_key(p, n, key);
-    const int variant = variant_or(FLUE_OP_ENSEMBLE_FLOW, key, prec, kEnsembleDefault);
+    const int variant = variant_or(FLUE_OP_ENSEMBLE_FLOW, key, prec, ensemble_default(p.field_reals / kPlanes));
     uint32_t grid = 0;
     if ((rc = ens_grid(p, variant, &grid))) return rc;
     void* T = variant > 4 ? ew.T : nullptr;  // the plaquette-first variants

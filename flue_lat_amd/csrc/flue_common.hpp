@@ -91,6 +91,68 @@ struct FieldView {
     }
 };
 
+// n planes of V reals each (or of V pairs, with E = the pair type's reals) at a uniform base,
+// element k of plane j at [j * V + k].  BUF: one buffer resource for the planes, so an access
+// is one 32-bit vector offset and a scalar plane offset (n * V * E * sizeof(R) < 2^32, which
+// fits_buffer's 18 planes imply for n * E <= 18); stream accesses are non-temporal.
+template <typename R, bool BUF>
+struct Planes {
+    R* p;
+    uint32_t V;
+    int n;
+    static constexpr int kNT = 2;  // aux bits of a buffer access: non-temporal
+
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int E) const {
+        const uint32_t bytes = (uint32_t)(n * E) * V * (uint32_t)sizeof(R);
+        return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, __builtin_bit_cast(int, bytes), 0x00020000);
+    }
+    template <bool NT>
+    __device__ __forceinline__ R ld(int j, uint32_t k) const {
+        if constexpr (BUF) {
+            const uint32_t so = (uint32_t)j * V * (uint32_t)sizeof(R), vo = k * (uint32_t)sizeof(R);
+            if constexpr (sizeof(R) == 4)
+                return __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b32(rsrc(1), vo, so, NT ? kNT : 0));
+            else
+                return __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b64(rsrc(1), vo, so, NT ? kNT : 0));
+        } else {
+            const R* q = p + (size_t)j * V + k;
+            return NT ? __builtin_nontemporal_load(q) : *q;
+        }
+    }
+    __device__ __forceinline__ void st(int j, uint32_t k, R v) const {
+        if constexpr (BUF) {
+            const uint32_t so = (uint32_t)j * V * (uint32_t)sizeof(R), vo = k * (uint32_t)sizeof(R);
+            if constexpr (sizeof(R) == 4) {
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc(1), vo, so, kNT);
+            } else {
+                typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), rsrc(1), vo, so, kNT);
+            }
+        } else {
+            __builtin_nontemporal_store(v, p + (size_t)j * V + k);
+        }
+    }
+    // the pair (re, im) of plane j (planes of V pairs)
+    __device__ __forceinline__ void st2(int j, uint32_t k, R re, R im) const {
+        typedef R r2 __attribute__((ext_vector_type(2)));
+        r2 v;
+        v.x = re;
+        v.y = im;
+        if constexpr (BUF) {
+            const uint32_t so = (uint32_t)j * V * 2u * (uint32_t)sizeof(R), vo = k * 2u * (uint32_t)sizeof(R);
+            if constexpr (sizeof(R) == 4) {
+                typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), rsrc(2), vo, so, kNT);
+            } else {
+                typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc(2), vo, so, kNT);
+            }
+        } else {
+            __builtin_nontemporal_store(v, reinterpret_cast<r2*>(p) + (size_t)j * V + k);
+        }
+    }
+};
+
 template <typename R>
 struct Pair2;
 template <>
@@ -193,17 +255,23 @@ __device__ __forceinline__ T ld_stream(const T* p) {
 #endif
 }
 
-// store_link with streaming stores
-template <typename R>
-__device__ __forceinline__ void store_link_stream(R* __restrict__ p, uint32_t V, int mu, uint32_t s, const Mat<R>& m) {
+// the first ROWS rows of a link with streaming stores
+template <int ROWS, typename R>
+__device__ __forceinline__ void store_rows_stream(R* __restrict__ p, uint32_t V, int mu, uint32_t s, const Mat<R>& m) {
     typedef R r2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int e = 0; e < 9; ++e) {
+    for (int e = 0; e < 3 * ROWS; ++e) {
         r2 v;
         v.x = m.r[e];
         v.y = m.i[e];
         st_stream(reinterpret_cast<r2*>(p + (size_t)(mu * 9 + e) * 2 * V) + s, v);
     }
+}
+
+// store_link with streaming stores
+template <typename R>
+__device__ __forceinline__ void store_link_stream(R* __restrict__ p, uint32_t V, int mu, uint32_t s, const Mat<R>& m) {
+    store_rows_stream<3>(p, V, mu, s, m);
 }
 
 // ---------------------------------------------------------------- SU(3) algebra
@@ -341,6 +409,37 @@ __device__ __forceinline__ void fill_row2(Mat<R>& M) {
         M.r[6 + c] = xr;
         M.i[6 + c] = -xi;
     }
+}
+
+// The first two rows of a link (row 2 left zero)
+template <typename R, bool BUF>
+__device__ __forceinline__ Mat<R> load_rows2(const FieldView<R, BUF>& f, int mu, uint32_t s) {
+    Mat<R> m;
+    if constexpr (BUF) {
+        const __amdgpu_buffer_rsrc_t r = f.dir_rsrc(mu);
+        const uint32_t vo = s * 2u * (uint32_t)sizeof(R), pb = f.V * 2u * (uint32_t)sizeof(R);
+#pragma unroll
+        for (int e = 0; e < 6; ++e) f.bld2(r, vo, e * pb, m.r[e], m.i[e]);
+    } else {
+        using P = typename Pair2<R>::type;
+#pragma unroll
+        for (int e = 0; e < 6; ++e) {
+            const P v = reinterpret_cast<const P*>(f.cplane(mu, e))[s];
+            m.r[e] = v.x;
+            m.i[e] = v.y;
+        }
+    }
+#pragma unroll
+    for (int e = 6; e < 9; ++e) m.r[e] = m.i[e] = R(0);
+    return m;
+}
+
+// An SU(3) link from its first two rows: two thirds of load_link's bytes for 24 multiply-adds
+template <typename R, bool BUF>
+__device__ __forceinline__ Mat<R> load_su3(const FieldView<R, BUF>& f, int mu, uint32_t s) {
+    Mat<R> m = load_rows2(f, mu, s);
+    fill_row2(m);
+    return m;
 }
 
 // C = A^dagger * B

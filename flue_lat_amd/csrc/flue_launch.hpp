@@ -90,22 +90,22 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
 
 // gradients and flow (k_grad.hip, k_b2grad.hip); grad / Wout / Abuf are SoA in the field
 // precision, and so is acc (8 su(3) coordinates x 4 directions x V)
-uint32_t grad_blocks(const Lat& L);
-// stencil variants (k_grad.hip): 1 = staple sums in storage order, 2..6 = staple sums in
-// (z, t) brick orders, 7 = plaquette-first (the six plaquette parts of every site into T,
-// plaq_ta_bytes, then each link from 3 links and 6 stored parts; unitary links only),
-// 8 = plaquette-first with both passes walking along t, 9..13 = plaquette-first in the (z, t)
-// brick orders of 2..6
+// stencil variants (k_grad.hip): 1 = staple sums in storage order, 2..6 = staple sums in boxes
+// swept along t, 7 = plaquette-first (the six plaquette parts of every site into T, plaq_ta_bytes,
+// then each link from 3 links and 6 stored parts; unitary links only) in storage order, 8 and
+// 9..13 = plaquette-first in boxes (8 the largest, 9..13 those of 2..6)
 constexpr int kFlowVariants = 13;
 constexpr int kFlowPF = 7;
-constexpr int kFlowPFWalk = 8;
-constexpr int kFlowDefault = 1;
+constexpr int kFlowPFWide = 8;
 // whether a flow/gradient variant is a plaquette-first form (needs plaq_ta_bytes of workspace)
 constexpr bool flow_is_pf(int variant) { return variant >= kFlowPF && variant <= kFlowVariants; }
-// the staple-sum variant with the visit order of `variant` (storage order for 7 and 8)
+// the staple-sum variant with the visit order of `variant`
 constexpr int staple_order_of(int variant) {
-    return variant > kFlowPFWalk ? variant - kFlowPF : (flow_is_pf(variant) ? kFlowDefault : variant);
+    return variant == kFlowPFWide ? 6 : (variant == kFlowPF ? 1 : (variant > kFlowPF ? variant - kFlowPF : variant));
 }
+// the untuned variant of the flow and of the Wilson gradient
+int flow_default(const Lat& L);
+int grad_default(const Lat& L);
 size_t plaq_ta_bytes(const Lat& L, int is_f32);
 hipError_t launch_wilson_grad(const Lat& L, const void* U, int is_f32, double beta, void* grad, hipStream_t st,
                               int variant, void* T);
@@ -152,6 +152,9 @@ hipError_t launch_copy(size_t n_reals, int is_f32, const void* src, void* dst, h
 // ensemble flow variants: persistent grid of 1, 2, 4 or 8 workgroups per CU with the staple
 // stencil (1..4) or the plaquette-first stencil (5..8)
 constexpr int kEnsembleVariants = 8;
-constexpr int kEnsembleDefault = 3;
+// the untuned variant for a number of sites: below 32768 the staple stencil on 4 workgroups per
+// CU (25,000 sites in three fields, ms a stage: 0.056 against 0.063 FP32), else plaquette-first
+// (2.6 M sites in 16 fields: 1.76 -> 1.20 FP32, 3.77 -> 2.00 FP64)
+constexpr int ensemble_default(uint64_t sites) { return sites < 32768 ? 3 : 7; }
 
 }  // namespace flue

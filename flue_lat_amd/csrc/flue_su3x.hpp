@@ -5,32 +5,17 @@
 
 namespace flue {
 
-// exp(X) of a traceless anti-Hermitian X, by scaling and squaring a Taylor polynomial reduced
-// with the Cayley-Hamilton theorem.  For Y = X / 2^s (|Y| <= 1/8) and traceless Y,
-//   Y^3 = t Y + i u I,   t = Tr Y^2 / 2 (real, <= 0),   i u = det Y,
+// Rows 0 and 1 of exp(X), X traceless anti-Hermitian (row 2 left zero; exp(X) is SU(3), so
+// fill_row2 gives it), by scaling and squaring a Taylor polynomial reduced with the
+// Cayley-Hamilton theorem.  For Y = X / 2^s (|Y|^2 <= 1/64) and traceless Y,
+//   Y^3 = t Y + i u I,   t = Tr Y^2 / 2 = -|Y|^2 / 2,   i u = det Y,
 // so every power of Y, and the polynomial, is a0 + a1 Y + a2 Y^2 with scalar coefficients.
-// Horner's rule on the coefficients (I + Y E / k) costs 10 flops a term, against one 3x3
-// product (216) a term on the matrices: one product in all, for Y^2, which is Hermitian.
+// Horner's rule on the coefficients (E <- 1/k! + Y E) costs 4 flops-with-add a term, against
+// one 3x3 product a term on the matrices; the one product left, Y^2, is Hermitian.
 // Degree 11 always: the first dropped term, |Y|^12 / 12!, is below 4e-20.
-__device__ __forceinline__ Mat<double> su3_exp(const Mat<double>& X) {
-    double nrm = 0.0;
-#pragma unroll
-    for (int e = 0; e < 9; ++e) nrm += X.r[e] * X.r[e] + X.i[e] * X.i[e];
-    // 2^-s by halving the squared norm by 4 until it is at most 1/64
-    int s = 0;
-    while (nrm > 0.015625 && s < 60) {
-        nrm *= 0.25;
-        ++s;
-    }
-    const double scale = ldexp(1.0, -s);
-    Mat<double> Y;
-#pragma unroll
-    for (int e = 0; e < 9; ++e) {
-        Y.r[e] = X.r[e] * scale;
-        Y.i[e] = X.i[e] * scale;
-    }
+__device__ __forceinline__ Mat<double> su3_exp_rows2(const Mat<double>& X) {
+    Mat<double> Y = X, Q;
     // Q = Y^2: (Y^2)_ab = -sum_k Y_ak conj(Y_bk), a <= b (Hermitian)
-    Mat<double> Q;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
 #pragma unroll
@@ -49,7 +34,7 @@ __device__ __forceinline__ Mat<double> su3_exp(const Mat<double>& X) {
             Q.i[b * 3 + a] = -qi;
         }
     }
-    const double t = 0.5 * (Q.r[0] + Q.r[4] + Q.r[8]);
+    double t = 0.5 * (Q.r[0] + Q.r[4] + Q.r[8]);
     // i u = det Y = Tr(Y Q) / 3; Im Tr(Y Q) = sum_ab (Im Y_ab Re Q_ab - Re Y_ab Im Q_ab)
     double u = 0.0;
 #pragma unroll
@@ -58,31 +43,58 @@ __device__ __forceinline__ Mat<double> su3_exp(const Mat<double>& X) {
         u = fmad(-Y.r[e], Q.i[e], u);
     }
     u *= 1.0 / 3.0;
-    // E <- I + Y E / k for k = 11 .. 1 on the coefficients:
-    //   (a0, a1, a2) <- (1 + i u a2 / k, (a0 + t a2) / k, a1 / k)
-    double a0r = 1.0, a0i = 0.0, a1r = 0.0, a1i = 0.0, a2r = 0.0, a2i = 0.0;
+    // |X|^2 = -2 t; flow steps rarely scale
+    int s = 0;
+    for (double n = -2.0 * t; n > 0.015625 && s < 60; n *= 0.25) ++s;
+    if (s > 0) {
+        const double h = ldexp(1.0, -s), h2 = h * h;
 #pragma unroll
-    for (int k = 11; k >= 1; --k) {
-        const double inv = 1.0 / (double)k;
-        const double n1r = fmad(t, a2r, a0r) * inv, n1i = fmad(t, a2i, a0i) * inv;
-        a0r = fmad(-u * inv, a2i, 1.0);
-        a0i = u * inv * a2r;
-        a2r = a1r * inv;
-        a2i = a1i * inv;
+        for (int e = 0; e < 9; ++e) {
+            Y.r[e] *= h;
+            Y.i[e] *= h;
+            Q.r[e] *= h2;
+            Q.i[e] *= h2;
+        }
+        t *= h2;
+        u *= h * h2;
+    }
+    // E <- 1/k! + Y E for k = 10 .. 0 from 1/11!:  (a0, a1, a2) <- (1/k! + i u a2, a0 + t a2, a1)
+    constexpr double inv_fact[12] = {1.0,        1.0,         1.0 / 2,      1.0 / 6,       1.0 / 24,       1.0 / 120,
+                                     1.0 / 720,  1.0 / 5040,  1.0 / 40320,  1.0 / 362880,  1.0 / 3628800,  1.0 / 39916800};
+    double a0r = inv_fact[11], a0i = 0.0, a1r = 0.0, a1i = 0.0, a2r = 0.0, a2i = 0.0;
+#pragma unroll
+    for (int k = 10; k >= 0; --k) {
+        const double n1r = fmad(t, a2r, a0r), n1i = fmad(t, a2i, a0i);
+        a0r = fmad(-u, a2i, inv_fact[k]);
+        a0i = u * a2r;
+        a2r = a1r;
+        a2i = a1i;
         a1r = n1r;
         a1i = n1i;
     }
     Mat<double> E;
 #pragma unroll
-    for (int e = 0; e < 9; ++e) {
+    for (int e = 0; e < 6; ++e) {
         double er = e % 4 == 0 ? a0r : 0.0, ei = e % 4 == 0 ? a0i : 0.0;
         cmac(er, ei, a1r, a1i, Y.r[e], Y.i[e]);
         cmac(er, ei, a2r, a2i, Q.r[e], Q.i[e]);
         E.r[e] = er;
         E.i[e] = ei;
     }
+#pragma unroll
+    for (int e = 6; e < 9; ++e) E.r[e] = E.i[e] = 0.0;
 #pragma unroll 1
-    for (int k = 0; k < s; ++k) E = mul(E, E);
+    for (int k = 0; k < s; ++k) {
+        Mat<double> F = E;
+        fill_row2(F);
+        E = mul2(E, F);
+    }
+    return E;
+}
+
+__device__ __forceinline__ Mat<double> su3_exp(const Mat<double>& X) {
+    Mat<double> E = su3_exp_rows2(X);
+    fill_row2(E);
     return E;
 }
 
@@ -223,8 +235,8 @@ __device__ __forceinline__ Mat<double> random_link(uint64_t seed, uint64_t link,
     X.i[5] = h * g[5];
     X.r[7] = -h * g[6];
     X.i[7] = h * g[5];
-    Mat<double> U = su3_exp(X);
-    fix_su3(U);
+    Mat<double> U = su3_exp_rows2(X);
+    fix_su3(U);  // reads rows 0 and 1
     return U;
 }
 

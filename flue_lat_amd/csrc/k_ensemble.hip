@@ -76,7 +76,8 @@ __global__ void __launch_bounds__(kBS) ens_flow_kernel(const EnsEntry* __restric
 }
 
 // Plaquette-first stencil over the ensemble: the six plaquette parts of every site of every
-// field (48 reals per site, config c's block at 2/3 of its field offset), then the links.
+// field (48 reals per site, config c's block at 2/3 of its field offset), then the links, the
+// four waves of a workgroup on the four directions of 64 sites.
 template <typename R, bool BUF>
 __global__ void __launch_bounds__(kBS) ens_plaq_ta_kernel(const EnsEntry* __restrict__ tab, int n, uint32_t total,
                                                           uint32_t chunk, const R* __restrict__ win, R* __restrict__ T) {
@@ -87,7 +88,9 @@ __global__ void __launch_bounds__(kBS) ens_plaq_ta_kernel(const EnsEntry* __rest
         const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
         if (s < e.L.V) {
             const FieldView<R, BUF> f{win + e.off, e.L.V};
-            plaquette_ta_site(e.L, f, s, T + e.off / 72 * 48);
+            int c[4];
+            site_coords(e.L, s, c);
+            plaquette_ta_site<true>(e.L, f, s, c, T + e.off / 72 * 48);
         }
     }
 }
@@ -98,13 +101,13 @@ __global__ void __launch_bounds__(kBS) ens_flow_pf_kernel(const EnsEntry* __rest
                                                           const R* __restrict__ T, R* __restrict__ wout,
                                                           R* __restrict__ acc, double eps, double ca, double cb,
                                                           int reunit) {
+    const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     uint32_t lo, hi;
     my_range(4u * total, chunk, lo, hi);
     for (uint32_t lu = lo; lu < hi; ++lu) {
         const uint32_t lb = lu >> 2;
-        const int mu = (int)(lu & 3u);
         const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
-        const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
+        const uint32_t s = (lb - e.blk0) * kBS + (lu & 3u) * 64u + (threadIdx.x & 63u);
         if (s < e.L.V) {
             const FieldView<R, BUF> f{win + e.off, e.L.V};
             int c[4];

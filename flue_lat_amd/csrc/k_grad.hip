@@ -15,25 +15,39 @@ namespace {
 
 constexpr int kBS = 256;
 
-// Visit orders of the 256-site blocks (the autotuner's variants of the flow and gradient
-// stencils).  Every order runs the same per-link code, so results are bit-identical.
-//   bz = 0:  storage order (x, y, z, t).
-//   bz > 0:  bricks of bz z-planes x bt t-slices (whole (x, y) planes of 256k sites):
-//            within a brick t runs fastest, then z, then the blocks of a plane, so the
-//            blocks in flight on an XCD hold the z and t neighbours of what they read.
+// Visit orders of the sites (the autotuner's variants of the flow and gradient stencils).
+// Every order runs the same per-link code, so results are bit-identical.
+//   yt = 0:  storage order (x, y, z, t), 256-site blocks.
+//   yt > 0:  boxes of yt x zt rows along x, each box swept along t: the blocks of a box at t
+//            are followed by its blocks at t + 1, so the lines that the z and t neighbours
+//            share are read while they are still in the XCD's L2.
 struct BlockOrder {
-    uint32_t bz, bt;    // brick extents (0 = storage order)
-    uint32_t nbp;       // 256-site blocks per (z, t) plane
-    uint32_t ntb;       // bricks along t
+    uint32_t yt, zt;    // box extents along y and z (0 = storage order)
+    uint32_t nty;       // boxes along y
+    uint32_t nbt;       // 256-site blocks per box and slice
+    uint32_t nb;        // blocks in all
 };
 
-__device__ __forceinline__ uint32_t site_block(const Lat& L, const BlockOrder& bo, uint32_t lb) {
-    if (bo.bz == 0) return lb;
-    const uint32_t k = lb % bo.nbp, q = lb / bo.nbp;
-    const uint32_t per = bo.bz * bo.bt, pib = q % per, b = q / per;
-    const uint32_t t = (b % bo.ntb) * bo.bt + pib % bo.bt;
-    const uint32_t z = (b / bo.ntb) * bo.bz + pib / bo.bt;
-    return (t * (uint32_t)L.n[3] + z) * bo.nbp + k;
+// the site i of block lb of the order (0 <= i < 256), with its coordinates; false past the end
+__device__ __forceinline__ bool order_site(const Lat& L, const BlockOrder& bo, uint32_t lb, uint32_t i, uint32_t& s,
+                                           int c[4]) {
+    if (bo.yt == 0) {
+        s = lb * kBS + i;
+        if (s >= L.V) return false;
+        site_coords(L, s, c);
+        return true;
+    }
+    const uint32_t q = lb / bo.nbt, k = lb - q * bo.nbt;
+    const uint32_t box = q / (uint32_t)L.n[0], t = q - box * (uint32_t)L.n[0];
+    const uint32_t bz = box / bo.nty, by = box - bz * bo.nty;
+    const uint32_t j = k * kBS + i;
+    const uint32_t r = j / (uint32_t)L.n[1], z = r / bo.yt;
+    c[0] = (int)t;
+    c[1] = (int)(j - r * (uint32_t)L.n[1]);
+    c[2] = (int)(by * bo.yt + r - z * bo.yt);
+    c[3] = (int)(bz * bo.zt + z);
+    s = (uint32_t)c[1] + L.st[2] * (uint32_t)c[2] + L.st[3] * (uint32_t)c[3] + L.st[0] * t;
+    return z < bo.zt && c[2] < L.n[2] && c[3] < L.n[3];
 }
 
 // One thread per link.  The direction is the fastest block index: the four blocks of the
@@ -45,10 +59,9 @@ __global__ void __launch_bounds__(kBS) wilson_grad_kernel(Lat L, FV f, BlockOrde
     using R = typename FV::real;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const int mu = (int)(blk & 3u);
-    const uint32_t s = site_block(L, bo, blk >> 2) * kBS + threadIdx.x;
-    if (s >= L.V) return;
+    uint32_t s;
     int c[4];
-    site_coords(L, s, c);
+    if (!order_site(L, bo, blk >> 2, threadIdx.x, s, c)) return;
     {
         const Mat<R> M = mul(load_link(f, mu, s), staple_sum(L, f, s, c, mu));
         Mat<R> G = proj_ta(M);
@@ -68,19 +81,23 @@ __global__ void __launch_bounds__(kBS) flow_stage_kernel(Lat L, FV f, BlockOrder
                                                          double cb, int reunit) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const int mu = (int)(blk & 3u);
-    const uint32_t s = site_block(L, bo, blk >> 2) * kBS + threadIdx.x;
-    if (s >= L.V) return;
+    uint32_t s;
     int c[4];
-    site_coords(L, s, c);
+    if (!order_site(L, bo, blk >> 2, threadIdx.x, s, c)) return;
     flow_link(L, f, wout, acc, s, c, mu, eps, ca, cb, reunit);
 }
 
-// plaquette-first stencil (kFlowPF): the plaquette parts of every site, then per link
-template <typename FV>
+// Plaquette-first stencil (kFlowPF): the plaquette parts of every site, then per link with the
+// four waves of a workgroup on the four directions of 64 sites.  ROWS2: the flow.
+// At 48^3x96 the first pass takes 1.15 ms (FP32) and 2.11 ms (FP64) with ROWS2, at 4.0 and 4.4
+// TB/s beyond L2; taking two of the six planes per wave instead, with 21 link reads a site
+// instead of 16, took 1.33 and 2.34 ms and gained nothing on a lattice of 162,000 sites.
+template <bool ROWS2, typename FV>
 __global__ void __launch_bounds__(kBS) plaq_ta_kernel(Lat L, FV f, BlockOrder bo, typename FV::real* __restrict__ T) {
-    const uint32_t s = site_block(L, bo, xcd_block(blockIdx.x, gridDim.x)) * kBS + threadIdx.x;
-    if (s >= L.V) return;
-    plaquette_ta_site(L, f, s, T);
+    uint32_t s;
+    int c[4];
+    if (!order_site(L, bo, xcd_block(blockIdx.x, gridDim.x), threadIdx.x, s, c)) return;
+    plaquette_ta_site<ROWS2>(L, f, s, c, T);
 }
 
 template <typename FV>
@@ -89,11 +106,10 @@ __global__ void __launch_bounds__(kBS) wilson_grad_pf_kernel(Lat L, FV f, BlockO
                                                              typename FV::real* __restrict__ grad) {
     using R = typename FV::real;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const int mu = (int)(blk & 3u);
-    const uint32_t s = site_block(L, bo, blk >> 2) * kBS + threadIdx.x;
-    if (s >= L.V) return;
+    const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    uint32_t s;
     int c[4];
-    site_coords(L, s, c);
+    if (!order_site(L, bo, blk >> 2, (blk & 3u) * 64u + (threadIdx.x & 63u), s, c)) return;
     Mat<R> G = ta_force(L, f, T, s, c, mu);
     const R sc = (R)(beta / 6.0);
 #pragma unroll
@@ -111,142 +127,79 @@ __global__ void __launch_bounds__(kBS) flow_stage_pf_kernel(Lat L, FV f, BlockOr
                                                             typename FV::real* __restrict__ acc, double eps, double ca,
                                                             double cb, int reunit) {
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const int mu = (int)(blk & 3u);
-    const uint32_t s = site_block(L, bo, blk >> 2) * kBS + threadIdx.x;
-    if (s >= L.V) return;
+    const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    uint32_t s;
     int c[4];
-    site_coords(L, s, c);
+    if (!order_site(L, bo, blk >> 2, (blk & 3u) * 64u + (threadIdx.x & 63u), s, c)) return;
     flow_link_pf(L, f, T, wout, acc, s, c, mu, eps, ca, cb, reunit);
-}
-
-// Plaquette-first with walks along t (kFlowPFWalk).  Pass 1: one thread per spatial site walks
-// kPFWalk slices, keeping the spatial links at x + t in registers as the next slice's own
-// links (13 link loads per site and slice, none from another slice).  Pass 2: one thread per
-// (spatial site, direction) walks the same slices, carrying the previous slice's T_{0 mu} and
-// U_0 for the t term of a spatial link, so no thread reads another slice after its first.
-constexpr int kPFWalk = 6;
-
-template <typename FV>
-__global__ void __launch_bounds__(kBS) plaq_ta_walk_kernel(Lat L, FV f, uint32_t nbs, typename FV::real* __restrict__ T) {
-    using R = typename FV::real;
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const uint32_t tc = blk / nbs, pb = blk - tc * nbs;
-    const uint32_t p = pb * kBS + threadIdx.x;
-    if (p >= L.Vs) return;
-    const int NT = L.n[0];
-    const int t0 = (int)tc * kPFWalk, t1 = min(t0 + kPFWalk, NT);
-    int c[4];
-    site_coords(L, p, c);
-    uint32_t sf[4];  // forward spatial neighbours within a slice
-#pragma unroll
-    for (int d = 1; d < 4; ++d) sf[d] = c[d] == L.n[d] - 1 ? p - (uint32_t)(L.n[d] - 1) * L.st[d] : p + L.st[d];
-    Mat<R> Us[3];
-#pragma unroll
-    for (int b = 1; b < 4; ++b) Us[b - 1] = load_link(f, b, p + L.Vs * (uint32_t)t0);
-    for (int t = t0; t < t1; ++t) {
-        const uint32_t ts = L.Vs * (uint32_t)t, s = p + ts;
-        const uint32_t sn = t == NT - 1 ? p : s + L.Vs;  // x + t
-        const Mat<R> Ut = load_link(f, 0, s);
-        Mat<R> N[3];
-#pragma unroll
-        for (int b = 1; b < 4; ++b) {
-            N[b - 1] = load_link(f, b, sn);
-            store_plaq_ta(T, L.V, plaq_index(0, b), s, mul(Ut, N[b - 1]), mul(Us[b - 1], load_link(f, 0, sf[b] + ts)));
-        }
-#pragma unroll
-        for (int a = 1; a < 3; ++a)
-#pragma unroll
-            for (int b = a + 1; b < 4; ++b)
-                store_plaq_ta(T, L.V, plaq_index(a, b), s, mul(Us[a - 1], load_link(f, b, sf[a] + ts)),
-                              mul(Us[b - 1], load_link(f, a, sf[b] + ts)));
-#pragma unroll
-        for (int b = 0; b < 3; ++b) Us[b] = N[b];
-    }
-}
-
-// pass 2 of kFlowPFWalk for the flow (GRAD = false) or the Wilson gradient (GRAD = true)
-template <bool GRAD, typename FV>
-__global__ void __launch_bounds__(kBS) pf_walk_kernel(Lat L, FV f, const typename FV::real* __restrict__ T,
-                                                      uint32_t nbs, typename FV::real* __restrict__ out,
-                                                      typename FV::real* __restrict__ acc, double eps, double ca,
-                                                      double cb, int reunit, double beta) {
-    using R = typename FV::real;
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const int mu = (int)(blk & 3u);
-    const uint32_t rest = blk >> 2, tc = rest / nbs, pb = rest - tc * nbs;
-    const uint32_t p = pb * kBS + threadIdx.x;
-    if (p >= L.Vs) return;
-    const int NT = L.n[0];
-    const int t0 = (int)tc * kPFWalk, t1 = min(t0 + kPFWalk, NT);
-    int c[4];
-    site_coords(L, p, c);
-    Mat<R> Tprev, U0prev;
-    if (mu != 0) {
-        const uint32_t sp = p + L.Vs * (uint32_t)(t0 == 0 ? NT - 1 : t0 - 1);
-        Tprev = load_ta(T, L.V, plaq_index(0, mu), sp);
-        U0prev = load_link(f, 0, sp);
-    }
-    for (int t = t0; t < t1; ++t) {
-        const uint32_t s = p + L.Vs * (uint32_t)t;
-        c[0] = t;
-        Mat<R> Z = ta_force_walk(L, f, T, s, c, mu, Tprev, U0prev);
-        if constexpr (GRAD) {
-            const R sc = (R)(beta / 6.0);
-#pragma unroll
-            for (int e = 0; e < 9; ++e) {
-                Z.r[e] *= sc;
-                Z.i[e] *= sc;
-            }
-            store_link_stream(out, L.V, mu, s, Z);
-        } else {
-            flow_update(L, f, out, acc, s, mu, eps, ca, cb, reunit, Z);
-        }
-    }
 }
 
 }  // namespace
 
-// brick extents (z-planes, t-slices) of the staple-form variants; variant 1 is the storage order
-constexpr uint32_t kBrickZ[kFlowPF - 1] = {0, 1, 2, 1, 2, 4};  // variants 1..6
-constexpr uint32_t kBrickT[kFlowPF - 1] = {0, 2, 2, 4, 4, 4};
+// Sites of a box slice for variants 1..6 (0 = storage order).  At 48^3x96 (one RK3 step, ms):
+//   sites          storage   1024    2048    3072    4096    6144
+//   staple  FP32     16.1    14.9    14.9    14.4    14.4    14.5
+//           FP64     27.3    24.4    24.8    24.3    24.3    24.4
+//   plaq.   FP32     10.9    10.7    10.7    10.5    10.5    10.5
+//   first   FP64     20.9    19.8    20.0    19.6    19.6    19.7
+constexpr uint32_t kBoxSites[kFlowPF - 1] = {0, 1024, 2048, 3072, 4096, 6144};
 
-// the order of a variant, or the storage order where the bricks do not tile the lattice
-// (planes of a whole number of blocks, extents divisible by the brick).  Plaquette-first
-// variant kFlowPF + k (k = 2..6) takes the order of staple variant k; kFlowPF and the walks
-// (which order their own blocks) take the storage order.
+// The order of a variant: plaquette-first variant kFlowPF + k (k = 2..6) takes the boxes of
+// staple variant k, kFlowPFWide the largest.  Of the boxes with at most the variant's sites, the one
+// with the fewest blocks (a box's last block is padded) times lines read again by the boxes beside it.
 static BlockOrder block_order(const Lat& L, int variant) {
-    BlockOrder bo{0, 0, 1, 1};
-    if (variant > kFlowPFWalk && variant <= kFlowVariants) variant -= kFlowPF;
-    if (variant < 1 || variant >= kFlowPF) variant = kFlowDefault;
-    const uint32_t bz = kBrickZ[variant - 1], bt = kBrickT[variant - 1];
-    const uint32_t plane = (uint32_t)L.n[1] * (uint32_t)L.n[2];
-    if (bz == 0 || plane % kBS != 0 || L.n[3] % bz != 0 || L.n[0] % bt != 0) return bo;
-    return BlockOrder{bz, bt, plane / kBS, (uint32_t)L.n[0] / bt};
+    const uint32_t plain = (L.V + kBS - 1) / kBS, NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
+    const int k = variant == kFlowPFWide ? 6 : (variant > kFlowPF ? variant - kFlowPF : variant);
+    const uint32_t want = k >= 1 && k < kFlowPF ? kBoxSites[k - 1] : 0;
+    uint32_t yt = 0, zt = 0;
+    double cost = 0.0;
+    for (uint32_t y = 1; y <= NY; ++y)
+        for (uint32_t z = 1; z <= NZ && (uint64_t)L.n[1] * y * z <= want; ++z) {
+            const double n = (NY + y - 1) / y * (double)((NZ + z - 1) / z) * (((uint32_t)L.n[1] * y * z + kBS - 1) / kBS);
+            const double c = n * (1.0 + (y < NY ? 1.0 / y : 0.0) + (z < NZ ? 1.0 / z : 0.0));
+            if (yt == 0 || c < cost) {
+                cost = c;
+                yt = y;
+                zt = z;
+            }
+        }
+    if (yt == 0) return BlockOrder{0, 0, 1, 1, plain};  // storage order, or no row fits
+    const uint32_t nty = (NY + yt - 1) / yt, nbt = ((uint32_t)L.n[1] * yt * zt + kBS - 1) / kBS;
+    return BlockOrder{yt, zt, nty, nbt, nty * ((NZ + zt - 1) / zt) * nbt * (uint32_t)L.n[0]};
 }
 
-// four blocks (one per direction) per 256 sites
-uint32_t grad_blocks(const Lat& L) { return 4u * ((L.V + kBS - 1) / kBS); }
+// Untuned choices, ms per RK3 step as measured (FP32 / FP64):
+//                     staple sums        plaquette-first    its boxes of 3072
+//   8^3x16          0.034 / 0.038       0.044 / 0.047      0.045 / 0.049
+//   12^3x24         0.070 / 0.092       0.065 / 0.091      0.065 / 0.093
+//   16^3x32         0.150 / 0.242       0.138 / 0.239      0.141 / 0.252
+//   20^3x40         0.347 / 0.703       0.305 / 0.574      0.379 / 0.630
+//   24^3x48         0.904 / 1.53        0.629 / 1.24       0.628 / 1.21
+//   48^3x96         16.0  / 27.1        10.4  / 20.3       10.0  / 19.1
+// The flow, whose links are SU(3), takes the plaquette-first stencil from 32768 sites (below,
+// its second launch costs more than it saves).  Boxes pay once a slice's links and plaquette
+// parts outgrow an XCD's 4 MB L2 several times.
+constexpr uint32_t kPFSites = 32768, kBoxSlice = 32768;
+int flow_default(const Lat& L) {
+    if (L.V < kPFSites) return grad_default(L);
+    return L.Vs >= kBoxSlice ? kFlowPF + 4 : kFlowPF;
+}
+int grad_default(const Lat& L) { return L.Vs >= kBoxSlice ? 4 : 1; }
 
 size_t plaq_ta_bytes(const Lat& L, int is_f32) { return (size_t)48 * L.V * (is_f32 ? 4 : 8); }
 
 hipError_t launch_wilson_grad(const Lat& L, const void* U, int is_f32, double beta, void* grad, hipStream_t st,
                               int variant, void* T) {
-    const uint32_t g = grad_blocks(L);
     if (flow_is_pf(variant) && !T) return hipErrorInvalidValue;
     const BlockOrder bo = block_order(L, variant);
-    const uint32_t nbs = (L.Vs + kBS - 1) / kBS, ntc = ((uint32_t)L.n[0] + kPFWalk - 1) / kPFWalk;
     with_view(L.V, U, is_f32, [&](auto f) {
         using F = decltype(f);
         using R = typename F::real;
-        if (variant == kFlowPFWalk) {
-            plaq_ta_walk_kernel<F><<<nbs * ntc, kBS, 0, st>>>(L, f, nbs, (R*)T);
-            pf_walk_kernel<true, F><<<4 * nbs * ntc, kBS, 0, st>>>(L, f, (const R*)T, nbs, (R*)grad, nullptr, 0.0, 0.0,
-                                                                  0.0, 0, beta);
-        } else if (flow_is_pf(variant)) {
-            plaq_ta_kernel<F><<<(L.V + kBS - 1) / kBS, kBS, 0, st>>>(L, f, bo, (R*)T);
-            wilson_grad_pf_kernel<F><<<g, kBS, 0, st>>>(L, f, bo, (const R*)T, beta, (R*)grad);
+        if (flow_is_pf(variant)) {
+            plaq_ta_kernel<false, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T);
+            wilson_grad_pf_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (const R*)T, beta, (R*)grad);
         } else {
-            wilson_grad_kernel<F><<<g, kBS, 0, st>>>(L, f, bo, beta, (R*)grad);
+            wilson_grad_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, beta, (R*)grad);
         }
     });
     return hipGetLastError();
@@ -254,23 +207,17 @@ hipError_t launch_wilson_grad(const Lat& L, const void* U, int is_f32, double be
 
 hipError_t launch_flow_stage(const Lat& L, const void* Win, int is_f32, void* Wout, void* acc_, double eps,
                              double ca, double cb, int reunit, hipStream_t st, int variant, void* T) {
-    const uint32_t g = grad_blocks(L);
     if (flow_is_pf(variant) && !T) return hipErrorInvalidValue;
     const BlockOrder bo = block_order(L, variant);
-    const uint32_t nbs = (L.Vs + kBS - 1) / kBS, ntc = ((uint32_t)L.n[0] + kPFWalk - 1) / kPFWalk;
     with_view(L.V, Win, is_f32, [&](auto f) {
         using F = decltype(f);
         using R = typename F::real;
         R* acc = (R*)acc_;
-        if (variant == kFlowPFWalk) {
-            plaq_ta_walk_kernel<F><<<nbs * ntc, kBS, 0, st>>>(L, f, nbs, (R*)T);
-            pf_walk_kernel<false, F><<<4 * nbs * ntc, kBS, 0, st>>>(L, f, (const R*)T, nbs, (R*)Wout, acc, eps, ca, cb,
-                                                                   reunit, 0.0);
-        } else if (flow_is_pf(variant)) {
-            plaq_ta_kernel<F><<<(L.V + kBS - 1) / kBS, kBS, 0, st>>>(L, f, bo, (R*)T);
-            flow_stage_pf_kernel<F><<<g, kBS, 0, st>>>(L, f, bo, (const R*)T, (R*)Wout, acc, eps, ca, cb, reunit);
+        if (flow_is_pf(variant)) {
+            plaq_ta_kernel<true, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T);
+            flow_stage_pf_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (const R*)T, (R*)Wout, acc, eps, ca, cb, reunit);
         } else {
-            flow_stage_kernel<F><<<g, kBS, 0, st>>>(L, f, bo, (R*)Wout, acc, eps, ca, cb, reunit);
+            flow_stage_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (R*)Wout, acc, eps, ca, cb, reunit);
         }
     });
     return hipGetLastError();
