@@ -72,7 +72,7 @@ hipError_t launch_scalar_gluon(const Lat& L, const void* U, int is_f32, int NS, 
 constexpr uint32_t kFinalChunk = 2048;
 
 // number of magnetic kernel variants the autotuner chooses from: 1..6 forms x occupancy
-// targets (k_clover.hip), 7 rectangle-first (k_rect.hip; NX, NY, NZ multiples of 16 and a
+// targets (k_clover.hip), 7 rectangle-first (k_rect.hip; where rect_fits, and a
 // footprint buffer)
 constexpr int kMagneticVariants = 7;
 constexpr int kMagneticRect = 7;
@@ -83,7 +83,8 @@ constexpr size_t kMagneticScratchBytes = (size_t)8 << 20;
 hipError_t launch_magnetic(const Lat& L, const void* U, int is_f32, int su3, double* partials, hipStream_t st,
                            int variant, uint32_t* npart, void* fpbuf = nullptr);
 bool rect_fits(const Lat& L);
-uint32_t rect_tiles(const Lat& L);
+// partials of variant 7: one per tile of its three planes
+uint32_t rect_partials(const Lat& L, int is_f32);
 size_t rect_fp_bytes(const Lat& L, int is_f32);
 hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3, double* partials, void* fpbuf,
                                 hipStream_t st, uint32_t* npart, void* Abuf = nullptr);

@@ -1,65 +1,87 @@
 // k_rect.hip -- the magnetic B with rectangle-first clover sums (magnetic variant 7).
 //
-// Planes (x, y) and (x, z): one wavefront per 16 x 16 tile of base sites in one plane slice,
-// x along the lanes (16 consecutive sites, so link loads coalesce) and four rows of the second
-// direction per loop iteration.  Every base site forms its seven rectangles once (rect_base) and adds
-// the AH parts of the leaves at the four corners of each into the tile's footprint, 19 x 19
-// cells in LDS (the tile plus the three rows and columns its rectangles reach beyond it).
-// The footprint has one wavefront, whose LDS additions execute in program order, so each
-// cell's sum is formed in a fixed order.  The footprints go to memory; the gather adds to
-// each site of a tile the overlapping cells of the tiles before it along x, along the second
-// direction and diagonally (in that fixed order), and sums |F|^2.  Plane (z, y) has no x
-// direction to coalesce along: its z and y links are first copied with z fastest (an LDS-tiled
-// transpose), which makes it plane (x', y') of the lattice with extents (NT, NZ, NY, NX), and
-// the same two kernels run there.  The gather can also store each site's AH parts instead of
-// summing |F|^2: the clover sums of the B^2 adjoint.
-#include "flue_rect.hpp"
+// Planes (x, y) and (x, z): one wavefront per tile of base sites in one plane slice, the tile's
+// sites numbered x fastest and taken 64 at a time (rows of consecutive sites, so link loads
+// coalesce).  Every base site forms its seven rectangles once (rect_base) and adds the AH parts
+// of the leaves at the four corners of each into the tile's footprint in LDS (the tile plus the
+// three rows and columns its rectangles reach beyond it).  The footprint has one wavefront, whose
+// LDS additions execute in program order, so each cell's sum is formed in a fixed order.  The
+// footprints go to memory; the gather adds to each site of a tile the overlapping cells of the
+// tiles before it along x, along the second direction and diagonally (in that fixed order), and
+// sums |F|^2.  Plane (z, y) has no x direction to coalesce along: its z and y links are first
+// copied with z fastest (an LDS-tiled transpose), which makes it plane (x', y') of the lattice
+// with extents (NT, NZ, NY, NX), and the same two kernels run there.  The gather can also store
+// each site's AH parts instead of summing |F|^2: the clover sums of the B^2 adjoint.
+#include <algorithm>
+#include <cmath>
+
 #include "flue_launch.hpp"
+#include "flue_rect.hpp"
 
 namespace flue {
 
 namespace {
 
-constexpr int kRT = 16;             // tile edge (base sites)
-constexpr int kFP = kRT + 3;        // footprint edge
-constexpr int kFC = kFP * kFP;      // footprint cells
-constexpr int kRW = 64;             // one wavefront per tile
+constexpr int kRW = 64;  // one wavefront per tile
 
-// the second direction and the spectator spatial direction of rectangle plane rp (0: (x, y),
-// 1: (x, z))
-__device__ __forceinline__ int rect_d2(int rp) { return rp == 0 ? 2 : 3; }
+// LDS reals per footprint cell: 9 parts, padded to 12 in FP32 (16-byte accesses)
+template <typename R>
+constexpr int kCellReals = sizeof(R) == 4 ? 12 : 9;
+// cells of the largest footprint: eight wavefronts (FP32, two per SIMD) or four (FP64, one per
+// SIMD) share a CU's 160 KB of LDS
+template <typename R>
+constexpr int kMaxCells = sizeof(R) == 4 ? 420 : 560;
 
-struct TileIdx {
-    uint32_t tx, t2, cs, ct;  // tile along x, tile along d2, spectator coordinate, t
+// One plane's tiling.  Direction 1 (x) has n1 tiles, the first r1 of q1 + 1 sites and the others
+// of q1; direction 2 likewise.  Footprints have rows of f cells, fc cells in all, and start at
+// real 9 * cell0 of the buffer.
+struct PlaneTiles {
+    uint32_t n1, q1, r1, n2, q2, r2;
+    uint32_t f, fc, tiles;
+    uint64_t cell0;
+    bool square() const { return q1 == 16 && r1 == 0 && q2 == 16 && r2 == 0; }
+};
+struct RectTiles {
+    PlaneTiles p[3];  // planes (x,y), (x,z), (z,y) (the last as plane (x,y) of the copy)
 };
 
-__device__ __forceinline__ TileIdx tile_idx(const Lat& L, int rp, uint32_t tile) {
-    const uint32_t ntx = (uint32_t)L.n[1] / kRT, nt2 = (uint32_t)L.n[rect_d2(rp)] / kRT;
+// the second direction of rectangle plane rp (0: (x, y), 1: (x, z))
+__device__ __forceinline__ int rect_d2(int rp) { return rp == 0 ? 2 : 3; }
+
+struct Tile {
+    uint32_t t1, t2, cs, ct;  // tile along x, tile along d2, spectator coordinate, t
+    uint32_t o1, o2, l1, l2;  // first site and extent along x and d2
+};
+
+__device__ __forceinline__ Tile tile_at(const Lat& L, int rp, const PlaneTiles& g, uint32_t tile) {
     const uint32_t ns = (uint32_t)L.n[rp == 0 ? 3 : 2];
-    TileIdx t;
-    t.tx = tile % ntx;
-    uint32_t q = tile / ntx;
-    t.t2 = q % nt2;
-    q /= nt2;
+    Tile t;
+    t.t1 = tile % g.n1;
+    uint32_t q = tile / g.n1;
+    t.t2 = q % g.n2;
+    q /= g.n2;
     t.cs = q % ns;
     t.ct = q / ns;
+    t.o1 = t.t1 * g.q1 + min(t.t1, g.r1);
+    t.o2 = t.t2 * g.q2 + min(t.t2, g.r2);
+    t.l1 = g.q1 + (t.t1 < g.r1 ? 1u : 0u);
+    t.l2 = g.q2 + (t.t2 < g.r2 ? 1u : 0u);
     return t;
 }
 
-__device__ __forceinline__ uint32_t tile_of(const Lat& L, int rp, uint32_t tx, uint32_t t2, uint32_t cs,
-                                            uint32_t ct) {
-    const uint32_t ntx = (uint32_t)L.n[1] / kRT, nt2 = (uint32_t)L.n[rect_d2(rp)] / kRT;
-    const uint32_t ns = (uint32_t)L.n[rp == 0 ? 3 : 2];
-    return ((ct * ns + cs) * nt2 + t2) * ntx + tx;
+// rectangle plane blockIdx.y of a kernel over the three planes
+__device__ __forceinline__ PlaneTiles plane_tiles(const RectTiles& g) {
+    return blockIdx.y == 0 ? g.p[0] : (blockIdx.y == 1 ? g.p[1] : g.p[2]);
 }
 
-// Footprint accumulation.  FP64 fields: LDS atomic adds, element e of cell c at [e * kFC + c].
+// Footprint accumulation.  FP64 fields: LDS atomic adds, element e of cell c at
+// [e * FS + c] (a fixed stride, so the elements are offsets of one address).
 // FP32 fields: the cell's 9 values padded to 12 floats at [c * 12], read, added and written
 // back as three 16-byte LDS accesses, volatile so they stay in program order.  That is safe
 // because the footprint belongs to one wavefront: its LDS operations execute in order and the
 // lanes of one access address distinct cells.  (FP32 LDS atomic adds kept the waves waiting to
 // issue LDS instructions for two thirds of their cycles; FP64 ones do not.)
-template <typename R>
+template <int FS, typename R>
 __device__ __forceinline__ void fp_add(R* fp, int cell, const AH<R>& p) {
     if constexpr (sizeof(R) == 4) {
         typedef float f4 __attribute__((ext_vector_type(4)));
@@ -81,79 +103,77 @@ __device__ __forceinline__ void fp_add(R* fp, int cell, const AH<R>& p) {
     } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            __hip_atomic_fetch_add(fp + k * kFC + cell, p.d[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(fp + (3 + k) * kFC + cell, p.or_[k], __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(fp + k * FS + cell, p.d[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(fp + (3 + k) * FS + cell, p.or_[k], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(fp + (6 + k) * kFC + cell, p.oi[k], __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(fp + (6 + k) * FS + cell, p.oi[k], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         }
     }
 }
 
-// LDS reals per footprint cell
-template <typename R>
-constexpr int kCellReals = sizeof(R) == 4 ? 12 : 9;
-
 // WPE == 1 (FP64) takes the chains with a one-link lookahead (rect_base); at two waves per
-// SIMD (FP32) the other wave covers the load latency
-template <typename FV, bool C2, int WPE>
+// SIMD (FP32) the other wave covers the load latency.  W > 0: every tile is W x W, so its rows and
+// footprint strides are constants (48^3x96: 5.44 -> 5.35 ms in FP32, 10.2 -> 9.9 ms in FP64).
+template <typename FV, bool C2, int WPE, int W>
 __global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, uint32_t ntiles, typename FV::real* __restrict__ fpout) {
+rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, typename FV::real* __restrict__ fpout) {
     using R = typename FV::real;
     constexpr int CR = kCellReals<R>;
-    __shared__ __align__(16) R fp[CR * kFC];
+    constexpr int FS = W ? (W + 3) * (W + 3) : kMaxCells<R>;  // FP64: reals between a cell's elements
+    __shared__ __align__(16) R fp[CR * FS];
     // blockIdx.y: 0 plane (x,y), 1 plane (x,z), 2 plane (z,y) as plane (x,y) of the copy
     const bool zy = blockIdx.y == 2;
+    const PlaneTiles g = plane_tiles(rt);
+    if (blockIdx.x >= g.tiles) return;
     const Lat L = zy ? Lzy : L0;
     const FV f = zy ? fzy : f0;
     const int rp = zy ? 0 : (int)blockIdx.y;
     const int d2 = rect_d2(rp);
-    const uint32_t tile = xcd_block(blockIdx.x, ntiles);
-    const TileIdx ti = tile_idx(L, rp, tile);
-    for (int k = threadIdx.x; k < CR * kFC; k += kRW) fp[k] = R(0);
+    const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
+    const Tile t = tile_at(L, rp, g, tile);
+    const int fc = W ? FS : (int)g.fc, f1 = W ? W + 3 : (int)g.f;
+    const uint32_t w = W ? (uint32_t)W : t.l1, h = W ? (uint32_t)W : t.l2;
+    for (int k = threadIdx.x; k < (CR == 12 ? CR * fc : CR * FS); k += kRW) fp[k] = R(0);
     __syncthreads();
-    const int lx = (int)threadIdx.x & 15;
 #pragma unroll 1
-    for (int r = 0; r < kRT / 4; ++r) {
-        const int ly = ((int)threadIdx.x >> 4) + 4 * r;
-        const int cx = (int)ti.tx * kRT + lx, c2 = (int)ti.t2 * kRT + ly;
-        const int cy = rp == 0 ? c2 : (int)ti.cs, cz = rp == 0 ? (int)ti.cs : c2;
-        const uint32_t s = (uint32_t)cx + L.st[2] * (uint32_t)cy + L.st[3] * (uint32_t)cz + L.st[0] * ti.ct;
-        const PlaneGeom<FV> g = plane_geom(L, f, s, cx, c2, 1, d2);
-        rect_base<C2, WPE == 1>(make_quad<1, 1, true>(g), [&](int da, int db, const AH<R>& p) {
-            fp_add(fp, (ly + db) * kFP + lx + da, p);
+    for (uint32_t j0 = 0; j0 < w * h; j0 += kRW) {
+        const uint32_t j = j0 + threadIdx.x;
+        if (!W && j >= w * h) break;
+        // (with W the column is the same in every turn, and its offsets are formed once)
+        const int ly = W ? (int)(j0 / w + threadIdx.x / w) : (int)(j / w);
+        const int lx = W ? (int)(threadIdx.x % w) : (int)(j - (uint32_t)ly * w);
+        const int cx = (int)t.o1 + lx, c2 = (int)t.o2 + ly;
+        const int cy = rp == 0 ? c2 : (int)t.cs, cz = rp == 0 ? (int)t.cs : c2;
+        const uint32_t s = (uint32_t)cx + L.st[2] * (uint32_t)cy + L.st[3] * (uint32_t)cz + L.st[0] * t.ct;
+        const PlaneGeom<FV> pg = plane_geom(L, f, s, cx, c2, 1, d2);
+        const int cell = ly * f1 + lx;
+        rect_base<C2, WPE == 1>(make_quad<1, 1, true>(pg), [&](int da, int db, const AH<R>& p) {
+            fp_add<FS>(fp, cell + db * f1 + da, p);
         });
     }
     __syncthreads();
-    // to memory as [e * kFC + c] in both precisions
-    R* out = fpout + ((size_t)blockIdx.y * ntiles + tile) * (9 * kFC);
-    if constexpr (CR == 12) {
-        for (int c = threadIdx.x; c < kFC; c += kRW)
+    // to memory as [e * fc + c] in both precisions
+    R* out = fpout + 9 * (g.cell0 + (uint64_t)tile * g.fc);
+    for (int c = threadIdx.x; c < fc; c += kRW)
 #pragma unroll
-            for (int e = 0; e < 9; ++e) out[e * kFC + c] = fp[c * 12 + e];
-    } else {
-        for (int k = threadIdx.x; k < 9 * kFC; k += kRW) out[k] = fp[k];
-    }
+        for (int e = 0; e < 9; ++e) out[e * fc + c] = fp[CR == 12 ? c * 12 + e : e * FS + c];
 }
 
-// per tile: the 256 sites' clover AH parts from the four footprints that cover them, then
-// sum |F|^2 into one compensated partial per tile
-// gather block: one wavefront, four sites per thread (measured faster than a thread per site)
-constexpr int kGB = 64;
-
 // the clover AH parts of tile cell (cx, cy): its own footprint's cell, then the overlapping
-// cells of the tiles before it along x, along d2 and diagonally, in that order
+// cells of the tiles before it along x, along d2 and diagonally, in that order (shift1 and
+// shift2 are those tiles' extents along x and d2, in cells)
 template <typename R>
-__device__ __forceinline__ AH<R> cell_sum(const R* own, const R* left, const R* below, const R* diag, int cx,
-                                          int cy) {
-    const int c = cy * kFP + cx;
+__device__ __forceinline__ AH<R> cell_sum(const R* own, const R* left, const R* below, const R* diag, int fc, int f,
+                                          int cx, int cy, int shift1, int shift2) {
+    const int c = cy * f + cx;
     R v[9];
 #pragma unroll
     for (int e = 0; e < 9; ++e) {
-        R x = own[e * kFC + c];
-        if (cx < 3) x += left[e * kFC + c + kRT];
-        if (cy < 3) x += below[e * kFC + c + kRT * kFP];
-        if (cx < 3 && cy < 3) x += diag[e * kFC + c + kRT * kFP + kRT];
+        R x = own[e * fc + c];
+        if (cx < 3) x += left[e * fc + c + shift1];
+        if (cy < 3) x += below[e * fc + c + shift2 * f];
+        if (cx < 3 && cy < 3) x += diag[e * fc + c + shift2 * f + shift1];
         v[e] = x;
     }
     AH<R> h;
@@ -166,41 +186,49 @@ __device__ __forceinline__ AH<R> cell_sum(const R* own, const R* left, const R* 
     return h;
 }
 
-// STORE = false: sum |F|^2 over the tile into one compensated partial per tile.  STORE = true:
-// write each site's AH parts into Abuf in the B^2 adjoint's layout (9 planes of V values per
-// magnetic plane (y,x), (x,z), (z,y): d0 d1 d2, o01r o02r o12r, o01i o02i o12i).
-template <typename R, bool STORE>
-__global__ void __launch_bounds__(kGB) rect_gather_kernel(Lat L0, Lat Lzy, const R* __restrict__ fpin,
-                                                         uint32_t ntiles, double* __restrict__ partials,
-                                                         R* __restrict__ Abuf) {
+// Per tile: its sites' clover AH parts from the four footprints that cover them.  One wavefront
+// (measured faster than a thread per site).  STORE = false: sum |F|^2 over the tile into one
+// compensated partial per tile.  STORE = true: write each site's AH parts into Abuf in the B^2
+// adjoint's layout (9 planes of V values per magnetic plane (y,x), (x,z), (z,y): d0 d1 d2,
+// o01r o02r o12r, o01i o02i o12i).
+template <typename R, bool STORE, int W>
+__global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectTiles rt, const R* __restrict__ fpin,
+                                                         double* __restrict__ partials, R* __restrict__ Abuf) {
     const bool zy = blockIdx.y == 2;
+    const PlaneTiles g = plane_tiles(rt);
+    if (blockIdx.x >= g.tiles) return;
     const Lat L = zy ? Lzy : L0;
     const int rp = zy ? 0 : (int)blockIdx.y;
-    const uint32_t tile = xcd_block(blockIdx.x, ntiles);
-    const TileIdx ti = tile_idx(L, rp, tile);
-    const uint32_t ntx = (uint32_t)L.n[1] / kRT, nt2 = (uint32_t)L.n[rect_d2(rp)] / kRT;
-    const uint32_t txl = (ti.tx + ntx - 1) % ntx, t2b = (ti.t2 + nt2 - 1) % nt2;
-    const R* base = fpin + (size_t)blockIdx.y * ntiles * (9 * kFC);
-    const R* own = base + (size_t)tile * (9 * kFC);
-    const R* left = base + (size_t)tile_of(L, rp, txl, ti.t2, ti.cs, ti.ct) * (9 * kFC);
-    const R* below = base + (size_t)tile_of(L, rp, ti.tx, t2b, ti.cs, ti.ct) * (9 * kFC);
-    const R* diag = base + (size_t)tile_of(L, rp, txl, t2b, ti.cs, ti.ct) * (9 * kFC);
-    const int cx = (int)threadIdx.x & 15;
+    const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
+    const Tile t = tile_at(L, rp, g, tile);
+    // the tiles before this one along x and d2 (periodic)
+    const uint32_t tl = t.t1 ? t.t1 - 1 : g.n1 - 1, tb = t.t2 ? t.t2 - 1 : g.n2 - 1;
+    const int dl = (int)tl - (int)t.t1, db = ((int)tb - (int)t.t2) * (int)g.n1;
+    const int shift1 = W ? W : (int)(g.q1 + (tl < g.r1 ? 1u : 0u)), shift2 = W ? W : (int)(g.q2 + (tb < g.r2 ? 1u : 0u));
+    const int fc = W ? (W + 3) * (W + 3) : (int)g.fc, f1 = W ? W + 3 : (int)g.f;
+    const uint32_t w = W ? (uint32_t)W : t.l1, h = W ? (uint32_t)W : t.l2;
+    const R* own = fpin + 9 * (g.cell0 + (uint64_t)tile * g.fc);
+    const R* left = own + 9 * (int64_t)fc * dl;
+    const R* below = own + 9 * (int64_t)fc * db;
+    const R* diag = own + 9 * (int64_t)fc * (dl + db);
     double acc = 0.0;
 #pragma unroll
-    for (int r = 0; r < kRT * kRT / kGB; ++r) {
-        const int cy = ((int)threadIdx.x >> 4) + r * (kGB / kRT);
+    for (uint32_t j0 = 0; j0 < w * h; j0 += kRW) {
+        const uint32_t j = j0 + threadIdx.x;
+        if (!W && j >= w * h) break;
+        const int cy = W ? (int)(j0 / w + threadIdx.x / w) : (int)(j / w);
+        const int cx = W ? (int)(threadIdx.x % w) : (int)(j - (uint32_t)cy * w);
+        const AH<R> h = cell_sum(own, left, below, diag, fc, f1, cx, cy, shift1, shift2);
         if constexpr (STORE) {
-            const AH<R> h = cell_sum(own, left, below, diag, cx, cy);
             // the site in the field's own lattice: for plane 2, the copy's x', y', z' are z, y, x
-            const uint32_t c2 = ti.t2 * kRT + (uint32_t)cy, c1 = ti.tx * kRT + (uint32_t)cx;
+            const uint32_t c2 = t.o2 + (uint32_t)cy, c1 = t.o1 + (uint32_t)cx;
             uint32_t s;
             if (zy)
-                s = ti.cs + L0.st[2] * c2 + L0.st[3] * c1 + L0.st[0] * ti.ct;
+                s = t.cs + L0.st[2] * c2 + L0.st[3] * c1 + L0.st[0] * t.ct;
             else if (rp == 0)
-                s = c1 + L0.st[2] * c2 + L0.st[3] * ti.cs + L0.st[0] * ti.ct;
+                s = c1 + L0.st[2] * c2 + L0.st[3] * t.cs + L0.st[0] * t.ct;
             else
-                s = c1 + L0.st[2] * ti.cs + L0.st[3] * c2 + L0.st[0] * ti.ct;
+                s = c1 + L0.st[2] * t.cs + L0.st[3] * c2 + L0.st[0] * t.ct;
             // the adjoint's planes are (y,x), (x,z), (z,y): the first is the tiles' (x,y) reversed
             const R sg = blockIdx.y == 0 ? R(-1) : R(1);
             R* o = Abuf + (size_t)blockIdx.y * 9 * L0.V + s;
@@ -211,13 +239,13 @@ __global__ void __launch_bounds__(kGB) rect_gather_kernel(Lat L0, Lat Lzy, const
                 o[(size_t)(6 + k) * L0.V] = sg * h.oi[k];
             }
         } else {
-            acc += f_norm2(cell_sum(own, left, below, diag, cx, cy));
+            acc += f_norm2(h);
         }
     }
     if constexpr (!STORE) {
-        const DD s = block_sum<kGB>(DD{acc, 0.0});
+        const DD s = block_sum<kRW>(DD{acc, 0.0});
         if (threadIdx.x == 0) {
-            const uint32_t i = blockIdx.y * ntiles + tile;
+            const uint32_t i = (blockIdx.y > 0 ? rt.p[0].tiles : 0u) + (blockIdx.y > 1 ? rt.p[1].tiles : 0u) + tile;
             partials[2 * i] = s.hi;
             partials[2 * i + 1] = s.lo;
         }
@@ -233,15 +261,17 @@ __global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __rest
     using P2 = typename Pair2<R>::type;
     __shared__ P2 tile[16][17];
     const uint32_t NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
+    const uint32_t bxs = (NX + 15) / 16, bzs = (NZ + 15) / 16;
     uint32_t q = blockIdx.x;
-    const uint32_t bx = q % (NX / 16);
-    q /= NX / 16;
-    const uint32_t bz = q % (NZ / 16);
-    q /= NZ / 16;
+    const uint32_t bx = q % bxs;
+    q /= bxs;
+    const uint32_t bz = q % bzs;
+    q /= bzs;
     const uint32_t y = q % NY, t = q / NY;
     const uint32_t i = threadIdx.x >> 4, j = threadIdx.x & 15;
     const uint32_t s = bx * 16 + j + NX * (y + NY * (bz * 16 + i + NZ * t));
     const uint32_t s2 = bz * 16 + j + NZ * (y + NY * (bx * 16 + i + NX * t));
+    const bool rd = bx * 16 + j < NX && bz * 16 + i < NZ, wr = bz * 16 + j < NZ && bx * 16 + i < NX;
     const P2* src = reinterpret_cast<const P2*>(U);
     P2* dst = reinterpret_cast<P2*>(P);
 #pragma unroll 1
@@ -249,9 +279,9 @@ __global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __rest
         const int mu = k == 0 ? 3 : 2;
 #pragma unroll 1
         for (int e = 0; e < 9; ++e) {
-            tile[i][j] = src[(size_t)(mu * 9 + e) * L.V + s];
+            if (rd) tile[i][j] = src[(size_t)(mu * 9 + e) * L.V + s];
             __syncthreads();
-            {
+            if (wr) {
                 typedef R r2 __attribute__((ext_vector_type(2)));
                 const P2 v = tile[j][i];
                 r2 w;
@@ -270,52 +300,126 @@ Lat zy_lattice(const Lat& L) {
     return make_lat(d);
 }
 
-}  // namespace
-
-bool rect_fits(const Lat& L) { return L.n[1] % kRT == 0 && L.n[2] % kRT == 0 && L.n[3] % kRT == 0; }
-
-uint32_t rect_tiles(const Lat& L) { return L.V / (kRT * kRT); }
-
-// the three planes' footprints, then the z-fastest copy of U_z and U_y
-size_t rect_fp_bytes(const Lat& L, int is_f32) {
-    const size_t sz = is_f32 ? 4 : 8;
-    return (size_t)3 * rect_tiles(L) * 9 * kFC * sz + (size_t)36 * L.V * sz;
+// Tiles of one plane with extents N1 x N2 and `slices` plane slices: of the splits into nearly
+// equal tiles whose footprint fits the LDS, the one that keeps the chip busy shortest -- 64-site
+// turns of a tile times the rounds in which the three planes' tiles run on `slots` wavefronts
+// (whole rounds while there are few of them) -- then the one with the fewest footprint cells.
+// The rounds are counted for kNominalNT time slices whatever the lattice has: the split sets the
+// order in which a site's rectangles are added, and a field repeated along t gives the same B.
+// Every tile is at least 4 sites wide (rect_fits), so a footprint's three extra rows and columns
+// reach into one further tile only.
+constexpr uint32_t kNominalNT = 32;
+PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint32_t max_cells, uint32_t slots) {
+    PlaneTiles best{};
+    double time = 0.0;
+    uint64_t cells = 0;
+    for (uint32_t n1 = 1; N1 / n1 >= 4; ++n1)
+        for (uint32_t n2 = 1; N2 / n2 >= 4; ++n2) {
+            const uint32_t l1 = (N1 + n1 - 1) / n1, l2 = (N2 + n2 - 1) / n2, fc = (l1 + 3) * (l2 + 3);
+            if (fc > max_cells) continue;
+            // (16 x 16 tiles have kernels of their own: they win ties)
+            const bool sq = N1 == 16 * n1 && N2 == 16 * n2;
+            const uint64_t cn = sq ? 0 : (uint64_t)n1 * n2 * fc;
+            const double rounds = 3.0 * n1 * n2 * (double)N3 * kNominalNT / slots;
+            const double tm = (double)((l1 * l2 + 63) / 64) * (rounds < 8.0 ? std::ceil(rounds) : rounds);
+            if (time == 0.0 || tm < time || (tm == time && cn < cells)) {
+                time = tm;
+                cells = cn;
+                best = PlaneTiles{n1, N1 / n1, N1 % n1, n2, N2 / n2, N2 % n2, l1 + 3, fc,
+                                  n1 * n2 * N3 * NT, 0};
+            }
+        }
+    return best;
 }
 
-// partials: rect_tiles for each of the planes (x, y), (x, z), (z, y).  With Abuf, the per-site
-// AH parts go there instead (the B^2 adjoint's clover sums) and no partials are written.
+RectTiles rect_tiles_of(const Lat& L, int is_f32) {
+    const uint32_t m = is_f32 ? kMaxCells<float> : kMaxCells<double>;
+    const uint32_t w = is_f32 ? 2048 : 1024;  // wavefronts resident on 256 CUs
+    const uint32_t NT = (uint32_t)L.n[0], NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
+    RectTiles r;
+    r.p[0] = plane_split(NX, NY, NZ, NT, m, w);
+    r.p[1] = plane_split(NX, NZ, NY, NT, m, w);
+    r.p[2] = plane_split(NZ, NY, NX, NT, m, w);
+    r.p[1].cell0 = r.p[0].cell0 + (uint64_t)r.p[0].tiles * r.p[0].fc;
+    r.p[2].cell0 = r.p[1].cell0 + (uint64_t)r.p[1].tiles * r.p[1].fc;
+    return r;
+}
+
+uint64_t rect_cells(const RectTiles& r) { return r.p[2].cell0 + (uint64_t)r.p[2].tiles * r.p[2].fc; }
+
+}  // namespace
+
+// Where the rectangle-first form runs: spatial extents of 12 or more (below, a tile is mostly
+// halo), and either all multiples of 16, which tile without idle lanes, or 90000 sites.  As
+// measured, quadrant form against this one, ms (FP32 / FP64 / FP64 declared SU(3)):
+//   12^3x24     41,472 sites   0.051 / 0.079 / 0.070   ->   0.063 / 0.078 / 0.075
+//   18x15x20x8  43,200         0.055 / 0.082 / 0.075   ->   0.063 / 0.083 / 0.080
+//   18x15x20x16 86,400         0.103 / 0.162 / 0.145   ->   0.091 / 0.160 / 0.152
+//   20^3x12     96,000         0.116 / 0.185 / 0.166   ->   0.087 / 0.144 / 0.137
+//   24^3x48                    0.663 / 1.15  / 1.02    ->   0.433 / 0.770 / 0.734
+//   33x34x32x27                0.983 / 1.75  / 1.58    ->   0.631 / 1.11  / 1.07
+//   16^3x8      32,768         0.049 / 0.072 / 0.062   ->   0.036 / 0.059 / 0.057
+//   48^3x96                    10.6  / 18.8  / 16.8    ->   6.26  / 11.4  / 11.0
+constexpr uint32_t kRectSites = 90000;
+bool rect_fits(const Lat& L) {
+    if (L.n[1] % 16 == 0 && L.n[2] % 16 == 0 && L.n[3] % 16 == 0) return true;
+    return std::min({L.n[1], L.n[2], L.n[3]}) >= 12 && L.V >= kRectSites;
+}
+
+uint32_t rect_partials(const Lat& L, int is_f32) {
+    const RectTiles r = rect_tiles_of(L, is_f32);
+    return r.p[0].tiles + r.p[1].tiles + r.p[2].tiles;
+}
+
+// the three planes' footprints, then the z-fastest copy of U_z and U_y
+static size_t rect_copy_offset(const RectTiles& r, size_t sz) { return ((size_t)rect_cells(r) * 9 * sz + 255) & ~(size_t)255; }
+size_t rect_fp_bytes(const Lat& L, int is_f32) {
+    const size_t sz = is_f32 ? 4 : 8;
+    return rect_copy_offset(rect_tiles_of(L, is_f32), sz) + (size_t)36 * L.V * sz;
+}
+
+// partials: rect_partials, the tiles of the planes (x, y), (x, z), (z, y) in turn.  With Abuf, the
+// per-site AH parts go there instead (the B^2 adjoint's clover sums) and no partials are written.
 hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3, double* partials, void* fpbuf,
                                 hipStream_t st, uint32_t* npart, void* Abuf) {
     if (!rect_fits(L) || !fits_buffer(L.V, is_f32)) return hipErrorInvalidValue;
-    const uint32_t nt = rect_tiles(L);
+    const RectTiles rt = rect_tiles_of(L, is_f32);
     const Lat Lzy = zy_lattice(L);
     with_view(L.V, U, is_f32, [&](auto f) {
         using F = decltype(f);
         using R = typename F::real;
         if constexpr (F::buffered) {
             R* fp = (R*)fpbuf;
-            R* P = fp + (size_t)3 * nt * 9 * kFC;
-            zy_relayout_kernel<R><<<L.V / 256, 256, 0, st>>>(L, f.p, P);
+            R* P = (R*)((char*)fpbuf + rect_copy_offset(rt, sizeof(R)));
+            const uint32_t nxz = (uint32_t)((L.n[1] + 15) / 16) * (uint32_t)((L.n[3] + 15) / 16);
+            zy_relayout_kernel<R><<<nxz * (uint32_t)L.n[2] * (uint32_t)L.n[0], 256, 0, st>>>(L, f.p, P);
             // the copy read as a field of Lzy whose directions 1 and 2 are its two blocks (the
             // view's base is one direction block before P; directions 0 and 3 are never read)
             const F fzy{(const R*)((uintptr_t)P - (uintptr_t)18 * L.V * sizeof(R)), L.V};
-            const dim3 g(nt, 3);
+            const dim3 g(std::max({rt.p[0].tiles, rt.p[1].tiles, rt.p[2].tiles}), 3);
             // FP32 and declared-SU(3) FP64 links: two-row chains; plain FP64: full products
-            if constexpr (sizeof(R) == 4) {
-                rect_kernel<F, true, 2><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, nt, fp);
-            } else {
-                if (su3)
-                    rect_kernel<F, true, 1><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, nt, fp);
+            auto rect = [&](auto w) {
+                constexpr int W = decltype(w)::value;
+                if constexpr (sizeof(R) == 4) {
+                    rect_kernel<F, true, 2, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
+                } else {
+                    if (su3)
+                        rect_kernel<F, true, 1, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
+                    else
+                        rect_kernel<F, false, 1, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
+                }
+                if (Abuf)
+                    rect_gather_kernel<R, true, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
                 else
-                    rect_kernel<F, false, 1><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, nt, fp);
-            }
-            if (Abuf)
-                rect_gather_kernel<R, true><<<g, kGB, 0, st>>>(L, Lzy, fp, nt, nullptr, (R*)Abuf);
+                    rect_gather_kernel<R, false, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, partials, nullptr);
+            };
+            if (rt.p[0].square() && rt.p[1].square() && rt.p[2].square())
+                rect(std::integral_constant<int, 16>());
             else
-                rect_gather_kernel<R, false><<<g, kGB, 0, st>>>(L, Lzy, fp, nt, partials, nullptr);
+                rect(std::integral_constant<int, 0>());
         }
     });
-    if (npart) *npart = 3 * nt;
+    if (npart) *npart = rect_partials(L, is_f32);
     return hipGetLastError();
 }
 

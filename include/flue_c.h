@@ -277,7 +277,8 @@ int flue_magnetic(const int32_t dims[4], const void* U, int32_t prec, double* d_
  *         orders), 1..3 waves per SIMD;
  *   7     rectangle-first: each rectangle of the clover is formed once and its leaves at
  *         the other three corners follow by conjugation (plane (z,y) from a z-fastest copy
- *         of its links).  It needs NX, NY, NZ divisible by 16 and a workspace of
+ *         of its links).  It needs NX, NY, NZ divisible by 16, or of 12 or more on a
+ *         lattice of 90,000 sites or more, and a workspace of
  *         flue_magnetic_work_bytes (about 300 bytes per site in FP32, 600 in FP64);
  *         otherwise the call runs the default form instead.
  * Every variant is deterministic; they agree to rounding (their summation orders differ). */
@@ -344,7 +345,7 @@ int flue_b2_grad_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t 
 
 /* gradient of the magnetic B (flue_magnetic); temporal links get 0.  `work` holds the
  * per-site anti-Hermitian parts of the three spatial-plane leaf sums, then the reverse form's
- * slots (and, on extents divisible by 16, the rectangle-first tiles that form those sums)
+ * slots (and, where variant 7 of flue_magnetic_ex applies, the tiles that form those sums)
  * (flue_b2_work_bytes; NULL = library buffer).  Precondition in every precision: SU(3)
  * links, since the gather takes the product from a leaf corner to the walk's end as
  * X^+ F.  The call first runs flue_check_field's scan with the precision's bound (waiting

@@ -1,0 +1,47 @@
+"""Rectangle-first forms on extents that the tiles do not divide, against the oracle.
+
+The tiles split an extent into nearly equal parts, so odd and prime extents leave tiles of two
+widths, lanes idle in a tile's last turn, and transposes past an edge of 16.  Tolerances as for
+the tileable lattices (tests/test_gpu_rect.py): FP64 sums 1e-12, FP32 links 1e-6; adjoint 1e-12
+and 1e-5 of the largest entry.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+# every extent below 16, none a multiple of it, primes, one row wider than a footprint
+DIMS = [(39, 13, 14, 15), (5, 29, 27, 25), (3, 47, 17, 41), (2, 400, 12, 19)]
+
+
+@pytest.fixture(scope="module")
+def FL():
+    import flue_lat_amd as FL
+    return FL
+
+
+@pytest.mark.parametrize("dims", DIMS)
+def test_rect_uneven_extents(FL, dims):
+    print(f"[tiles] {dims}", flush=True)
+    U = O.random_field(dims, 8100 + dims[1], 0.3)
+    want = O.magnetic(U)
+    f = FL.GaugeField.from_complex(U)
+    assert abs(f.magnetic(variant=7) - want) < 1e-12 * want
+    assert f.magnetic() == f.magnetic(variant=7) == f.magnetic(variant=7)
+    assert abs(f.astype("fp64-su3").magnetic(variant=7) - want) < 1e-12 * want
+    assert abs(f.astype("fp32").magnetic(variant=7) - want) < 1e-6 * want
+
+
+@pytest.mark.parametrize("dims", DIMS[:2])
+def test_adjoint_uneven_extents(FL, dims):
+    print(f"[tiles] adjoint {dims}", flush=True)
+    U = O.random_field(dims, 8200 + dims[1], 0.3)
+    Go = O.b2_grad(U)
+    scale = np.abs(Go).max()
+    f = FL.GaugeField.from_complex(U)
+    for g, tol in ((f, 1e-12), (f.astype("fp32"), 1e-5)):
+        for v in (1, 2):
+            assert np.abs(g.magnetic_grad(variant=v).to_complex().cpu().numpy() - Go).max() < tol * scale, v
