@@ -120,25 +120,34 @@ size_t b2_ah_bytes(const Lat& L, int32_t prec) {
     return ((size_t)27 * L.V * (prec == FLUE_F32 ? 4 : 8) + 255) & ~(size_t)255;
 }
 
-// the region after the clover sums: the reverse form's slot buffer, and before it, where the
-// rectangle-first magnetic form applies, that form's footprints and link copy
+// Where the rectangle-first magnetic form applies, the region after the clover sums holds that
+// form's footprints, over them the footprints of the tiled adjoint, and behind both the z-fastest
+// copy, which the two share.  Elsewhere it holds the slots of the reverse form.
+size_t b2_copy_at(const Lat& L, int32_t prec) {
+    const int f32 = prec == FLUE_F32;
+    return align256(std::max(rect_footprint_bytes(L, f32), b2_tile_bytes(L, f32)));
+}
 size_t b2_region_bytes(const Lat& L, int32_t prec) {
-    const size_t slots = b2_slot_bytes(L, prec == FLUE_F32);
-    return magnetic_rect_ok(L, prec) ? std::max(slots, rect_fp_bytes(L, prec == FLUE_F32)) : slots;
+    const int f32 = prec == FLUE_F32;
+    if (!magnetic_rect_ok(L, prec)) return b2_slot_bytes(L, f32);
+    return b2_copy_at(L, prec) + (size_t)36 * L.V * (f32 ? 4 : 8);
 }
 
 // the B^2 adjoint after the SU(3) check: clover sums into the start of `work` (rectangle-first
 // where it applies, with two-row chains in both precisions since the links are SU(3)), then
-// variant 1 (per-link gather) or 2 (reverse mode with the slot buffer after the clover sums)
+// variant 1 (per-link gather) or 2 (reverse mode: on tiles, or with slots after the clover sums)
 int b2_grad_run(const Lat& L, const void* U, int32_t prec, int variant, void* work, void* grad, hipStream_t st) {
-    const int f32 = prec == FLUE_F32;
-    void* region = (char*)work + b2_ah_bytes(L, prec);
-    if (magnetic_rect_ok(L, prec))
-        FLUE_TRY(launch_magnetic_rect(L, U, f32, 1, nullptr, region, st, nullptr, work));
+    const int f32 = prec == FLUE_F32, rect = magnetic_rect_ok(L, prec), tiled = rect && variant != 1;
+    char* region = (char*)work + b2_ah_bytes(L, prec);
+    const size_t copy_at = rect ? b2_copy_at(L, prec) : 0;
+    if (rect)
+        FLUE_TRY(launch_magnetic_rect(L, U, f32, 1, nullptr, region, st, nullptr, work, tiled, copy_at));
     else
         FLUE_TRY(launch_magnetic_ah(L, U, f32, work, st));
     if (variant == 1)
         FLUE_TRY(launch_b2_grad(L, U, f32, work, grad, st));
+    else if (tiled)
+        FLUE_TRY(launch_b2_grad_tile(L, U, f32, region + copy_at, work, region, grad, st));
     else
         FLUE_TRY(launch_b2_grad_rev(L, U, f32, work, region, grad, st));
     return FLUE_OK;

@@ -87,7 +87,10 @@ bool rect_fits(const Lat& L);
 uint32_t rect_partials(const Lat& L, int is_f32);
 size_t rect_fp_bytes(const Lat& L, int is_f32);
 hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3, double* partials, void* fpbuf,
-                                hipStream_t st, uint32_t* npart, void* Abuf = nullptr);
+                                hipStream_t st, uint32_t* npart, void* Abuf = nullptr, int tiled = 0,
+                                size_t copy_at = 0);
+// the footprints of variant 7 alone (the z-fastest copy follows them in rect_fp_bytes)
+size_t rect_footprint_bytes(const Lat& L, int is_f32);
 
 // gradients and flow (k_grad.hip, k_b2grad.hip); grad / Wout / Abuf are SoA in the field
 // precision, and so is acc (8 su(3) coordinates x 4 directions x V)
@@ -126,6 +129,12 @@ uint32_t b2_slab_slices(const Lat& L, int is_f32);
 size_t b2_slot_bytes(const Lat& L, int is_f32);
 hipError_t launch_b2_grad_rev(const Lat& L, const void* U, int is_f32, const void* Abuf, void* slots, void* grad,
                               hipStream_t st);
+// the reverse form where the rectangle-first magnetic form applies (k_b2tile.hip): the terms of each
+// tile into footprints (b2_tile_bytes, slabs of time slices), from clover sums stored for it by
+// launch_magnetic_rect and that call's z-fastest copy
+size_t b2_tile_bytes(const Lat& L, int is_f32);
+hipError_t launch_b2_grad_tile(const Lat& L, const void* U, int is_f32, const void* zycopy, const void* Abuf, void* fpbuf,
+                               void* grad, hipStream_t st);
 hipError_t launch_finalize_affine(const double* partials, uint32_t n, double* out, double scale, double offset,
                                   hipStream_t st);
 

@@ -1,0 +1,109 @@
+// flue_tiles.hpp -- how the rectangle-first kernels split the plane slices of a lattice into tiles
+// of base sites, one wavefront each, and where a tile's footprint lies.
+#pragma once
+#include <cmath>
+
+#include "flue_common.hpp"
+
+namespace flue {
+namespace {
+
+// One plane's tiling.  Direction 1 (x) has n1 tiles, the first r1 of q1 + 1 sites and the others
+// of q1; direction 2 likewise.  Footprints (the tile plus three rows and columns) have rows of f
+// cells and fc cells in all; the plane's first one is cell cell0 of the buffer.
+struct PlaneTiles {
+    uint32_t n1, q1, r1, n2, q2, r2;
+    uint32_t f, fc, tiles;
+    uint64_t cell0;
+    bool square() const { return q1 == 16 && r1 == 0 && q2 == 16 && r2 == 0; }
+};
+struct RectTiles {
+    PlaneTiles p[3];  // planes (x,y), (x,z), (z,y) (the last as plane (x,y) of the copy)
+};
+
+// the second direction of rectangle plane rp (0: (x, y), 1: (x, z))
+__device__ __forceinline__ int rect_d2(int rp) { return rp == 0 ? 2 : 3; }
+
+struct Tile {
+    uint32_t t1, t2, cs, ct;  // tile along x, tile along d2, spectator coordinate, t
+    uint32_t o1, o2, l1, l2;  // first site and extent along x and d2
+};
+
+__device__ __forceinline__ Tile tile_at(const Lat& L, int rp, const PlaneTiles& g, uint32_t tile) {
+    const uint32_t ns = (uint32_t)L.n[rp == 0 ? 3 : 2];
+    Tile t;
+    t.t1 = tile % g.n1;
+    uint32_t q = tile / g.n1;
+    t.t2 = q % g.n2;
+    q /= g.n2;
+    t.cs = q % ns;
+    t.ct = q / ns;
+    t.o1 = t.t1 * g.q1 + min(t.t1, g.r1);
+    t.o2 = t.t2 * g.q2 + min(t.t2, g.r2);
+    t.l1 = g.q1 + (t.t1 < g.r1 ? 1u : 0u);
+    t.l2 = g.q2 + (t.t2 < g.r2 ? 1u : 0u);
+    return t;
+}
+
+// rectangle plane blockIdx.y of a kernel over the three planes
+__device__ __forceinline__ PlaneTiles plane_tiles(const RectTiles& g) {
+    return blockIdx.y == 0 ? g.p[0] : (blockIdx.y == 1 ? g.p[1] : g.p[2]);
+}
+
+// lattice whose x, y, z are the z, y, x of L: its plane (x, y) is L's plane (z, y)
+Lat zy_lattice(const Lat& L) {
+    const int32_t d[4] = {L.n[0], L.n[3], L.n[2], L.n[1]};
+    return make_lat(d);
+}
+
+// Tiles of one plane with extents N1 x N2 and `slices` plane slices: of the splits into nearly
+// equal tiles whose footprint fits the LDS, the one that keeps the chip busy shortest -- 64-site
+// turns of a tile times the rounds in which the three planes' tiles run on `slots` wavefronts
+// (whole rounds while there are few of them) -- then the one with the fewest footprint cells.
+// The rounds are counted for kNominalNT time slices whatever the lattice has: the split sets the
+// order in which a site's rectangles are added, and a field repeated along t gives the same B.
+// Every tile is at least 4 sites wide (rect_fits), so a footprint's three extra rows and columns
+// reach into one further tile only.
+constexpr uint32_t kNominalNT = 32, kMaxTileEdge = 32;
+PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint32_t max_cells, uint32_t slots) {
+    PlaneTiles best{};
+    double time = 0.0;
+    uint64_t cells = 0;
+    // tile counts along a direction of N sites, from the fewest, each with a smaller widest tile
+    auto widest = [](uint32_t N, uint32_t n) { return (N + n - 1) / n; };
+    auto next = [&](uint32_t N, uint32_t n) { return widest(N, widest(N, n) - 1); };
+    for (uint32_t n1 = widest(N1, kMaxTileEdge); N1 / n1 >= 4; n1 = next(N1, n1))
+        for (uint32_t n2 = widest(N2, kMaxTileEdge); N2 / n2 >= 4; n2 = next(N2, n2)) {
+            const uint32_t l1 = widest(N1, n1), l2 = widest(N2, n2), fc = (l1 + 3) * (l2 + 3);
+            if (fc > max_cells) continue;
+            // (16 x 16 tiles have kernels of their own: they win ties)
+            const bool sq = N1 == 16 * n1 && N2 == 16 * n2;
+            const uint64_t cn = sq ? 0 : (uint64_t)n1 * n2 * fc;
+            const double rounds = 3.0 * n1 * n2 * (double)N3 * kNominalNT / slots;
+            const double tm = (double)((l1 * l2 + 63) / 64) * (rounds < 8.0 ? std::ceil(rounds) : rounds);
+            if (time == 0.0 || tm < time || (tm == time && cn < cells)) {
+                time = tm;
+                cells = cn;
+                best = PlaneTiles{n1, N1 / n1, N1 % n1, n2, N2 / n2, N2 % n2, l1 + 3, fc,
+                                  n1 * n2 * N3 * NT, 0};
+            }
+        }
+    return best;
+}
+
+// the three planes of a lattice; `slots` wavefronts are resident on the chip
+RectTiles rect_split(const Lat& L, uint32_t max_cells, uint32_t slots) {
+    const uint32_t NT = (uint32_t)L.n[0], NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
+    RectTiles r;
+    r.p[0] = plane_split(NX, NY, NZ, NT, max_cells, slots);
+    r.p[1] = plane_split(NX, NZ, NY, NT, max_cells, slots);
+    r.p[2] = plane_split(NZ, NY, NX, NT, max_cells, slots);
+    r.p[1].cell0 = r.p[0].cell0 + (uint64_t)r.p[0].tiles * r.p[0].fc;
+    r.p[2].cell0 = r.p[1].cell0 + (uint64_t)r.p[1].tiles * r.p[1].fc;
+    return r;
+}
+
+uint64_t rect_cells(const RectTiles& r) { return r.p[2].cell0 + (uint64_t)r.p[2].tiles * r.p[2].fc; }
+
+}  // namespace
+}  // namespace flue

@@ -13,10 +13,10 @@
 // with extents (NT, NZ, NY, NX), and the same two kernels run there.  The gather can also store
 // each site's AH parts instead of summing |F|^2: the clover sums of the B^2 adjoint.
 #include <algorithm>
-#include <cmath>
 
 #include "flue_launch.hpp"
 #include "flue_rect.hpp"
+#include "flue_tiles.hpp"
 
 namespace flue {
 
@@ -31,48 +31,6 @@ constexpr int kCellReals = sizeof(R) == 4 ? 12 : 9;
 // SIMD) share a CU's 160 KB of LDS
 template <typename R>
 constexpr int kMaxCells = sizeof(R) == 4 ? 420 : 560;
-
-// One plane's tiling.  Direction 1 (x) has n1 tiles, the first r1 of q1 + 1 sites and the others
-// of q1; direction 2 likewise.  Footprints have rows of f cells, fc cells in all, and start at
-// real 9 * cell0 of the buffer.
-struct PlaneTiles {
-    uint32_t n1, q1, r1, n2, q2, r2;
-    uint32_t f, fc, tiles;
-    uint64_t cell0;
-    bool square() const { return q1 == 16 && r1 == 0 && q2 == 16 && r2 == 0; }
-};
-struct RectTiles {
-    PlaneTiles p[3];  // planes (x,y), (x,z), (z,y) (the last as plane (x,y) of the copy)
-};
-
-// the second direction of rectangle plane rp (0: (x, y), 1: (x, z))
-__device__ __forceinline__ int rect_d2(int rp) { return rp == 0 ? 2 : 3; }
-
-struct Tile {
-    uint32_t t1, t2, cs, ct;  // tile along x, tile along d2, spectator coordinate, t
-    uint32_t o1, o2, l1, l2;  // first site and extent along x and d2
-};
-
-__device__ __forceinline__ Tile tile_at(const Lat& L, int rp, const PlaneTiles& g, uint32_t tile) {
-    const uint32_t ns = (uint32_t)L.n[rp == 0 ? 3 : 2];
-    Tile t;
-    t.t1 = tile % g.n1;
-    uint32_t q = tile / g.n1;
-    t.t2 = q % g.n2;
-    q /= g.n2;
-    t.cs = q % ns;
-    t.ct = q / ns;
-    t.o1 = t.t1 * g.q1 + min(t.t1, g.r1);
-    t.o2 = t.t2 * g.q2 + min(t.t2, g.r2);
-    t.l1 = g.q1 + (t.t1 < g.r1 ? 1u : 0u);
-    t.l2 = g.q2 + (t.t2 < g.r2 ? 1u : 0u);
-    return t;
-}
-
-// rectangle plane blockIdx.y of a kernel over the three planes
-__device__ __forceinline__ PlaneTiles plane_tiles(const RectTiles& g) {
-    return blockIdx.y == 0 ? g.p[0] : (blockIdx.y == 1 ? g.p[1] : g.p[2]);
-}
 
 // Footprint accumulation.  FP64 fields: LDS atomic adds, element e of cell c at
 // [e * FS + c] (a fixed stride, so the elements are offsets of one address).
@@ -188,10 +146,14 @@ __device__ __forceinline__ AH<R> cell_sum(const R* own, const R* left, const R* 
 
 // Per tile: its sites' clover AH parts from the four footprints that cover them.  One wavefront
 // (measured faster than a thread per site).  STORE = false: sum |F|^2 over the tile into one
-// compensated partial per tile.  STORE = true: write each site's AH parts into Abuf in the B^2
-// adjoint's layout (9 planes of V values per magnetic plane (y,x), (x,z), (z,y): d0 d1 d2,
-// o01r o02r o12r, o01i o02i o12i).
-template <typename R, bool STORE, int W>
+// compensated partial per tile.  Otherwise write each site's AH parts into Abuf, 9 planes of V
+// values per plane, d0 d1 d2, o01r o02r o12r, o01i o02i o12i, for a form of the B^2 adjoint:
+// kTiles (k_b2tile.hip) takes the rectangle planes (x,y), (x,z), (z,y), the last with its sites
+// numbered as in the copy (z fastest); kSites (k_b2grad.hip) the magnetic planes (y,x), (x,z), (z,y)
+// with sites in the field's order (its plane (z,y) is written at strided sites: 1.8 ms at 48^3x96
+// in FP32, against 0.6 ms for kTiles).
+enum class Store { kNone, kTiles, kSites };
+template <typename R, Store STORE, int W>
 __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectTiles rt, const R* __restrict__ fpin,
                                                          double* __restrict__ partials, R* __restrict__ Abuf) {
     const bool zy = blockIdx.y == 2;
@@ -219,30 +181,27 @@ __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectT
         const int cy = W ? (int)(j0 / w + threadIdx.x / w) : (int)(j / w);
         const int cx = W ? (int)(threadIdx.x % w) : (int)(j - (uint32_t)cy * w);
         const AH<R> h = cell_sum(own, left, below, diag, fc, f1, cx, cy, shift1, shift2);
-        if constexpr (STORE) {
-            // the site in the field's own lattice: for plane 2, the copy's x', y', z' are z, y, x
+        if constexpr (STORE != Store::kNone) {
             const uint32_t c2 = t.o2 + (uint32_t)cy, c1 = t.o1 + (uint32_t)cx;
-            uint32_t s;
-            if (zy)
-                s = t.cs + L0.st[2] * c2 + L0.st[3] * c1 + L0.st[0] * t.ct;
-            else if (rp == 0)
-                s = c1 + L0.st[2] * c2 + L0.st[3] * t.cs + L0.st[0] * t.ct;
-            else
-                s = c1 + L0.st[2] * t.cs + L0.st[3] * c2 + L0.st[0] * t.ct;
-            // the adjoint's planes are (y,x), (x,z), (z,y): the first is the tiles' (x,y) reversed
-            const R sg = blockIdx.y == 0 ? R(-1) : R(1);
-            R* o = Abuf + (size_t)blockIdx.y * 9 * L0.V + s;
+            uint32_t s = c1 + L.st[2] * (rp == 0 ? c2 : t.cs) + L.st[3] * (rp == 0 ? t.cs : c2) + L.st[0] * t.ct;
+            R sg = R(1);
+            if constexpr (STORE == Store::kSites) {
+                // the copy's x', y', z' are z, y, x; plane (y,x) is (x,y) reversed
+                if (zy) s = t.cs + L0.st[2] * c2 + L0.st[3] * c1 + L0.st[0] * t.ct;
+                if (blockIdx.y == 0) sg = R(-1);
+            }
+            R* o = Abuf + (size_t)blockIdx.y * 9 * L.V + s;
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                o[(size_t)k * L0.V] = sg * h.d[k];
-                o[(size_t)(3 + k) * L0.V] = sg * h.or_[k];
-                o[(size_t)(6 + k) * L0.V] = sg * h.oi[k];
+                o[(size_t)k * L.V] = sg * h.d[k];
+                o[(size_t)(3 + k) * L.V] = sg * h.or_[k];
+                o[(size_t)(6 + k) * L.V] = sg * h.oi[k];
             }
         } else {
             acc += f_norm2(h);
         }
     }
-    if constexpr (!STORE) {
+    if constexpr (STORE == Store::kNone) {
         const DD s = block_sum<kRW>(DD{acc, 0.0});
         if (threadIdx.x == 0) {
             const uint32_t i = (blockIdx.y > 0 ? rt.p[0].tiles : 0u) + (blockIdx.y > 1 ? rt.p[1].tiles : 0u) + tile;
@@ -294,58 +253,9 @@ __global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __rest
     }
 }
 
-// lattice whose x, y, z are the z, y, x of L: its plane (x, y) is L's plane (z, y)
-Lat zy_lattice(const Lat& L) {
-    const int32_t d[4] = {L.n[0], L.n[3], L.n[2], L.n[1]};
-    return make_lat(d);
-}
-
-// Tiles of one plane with extents N1 x N2 and `slices` plane slices: of the splits into nearly
-// equal tiles whose footprint fits the LDS, the one that keeps the chip busy shortest -- 64-site
-// turns of a tile times the rounds in which the three planes' tiles run on `slots` wavefronts
-// (whole rounds while there are few of them) -- then the one with the fewest footprint cells.
-// The rounds are counted for kNominalNT time slices whatever the lattice has: the split sets the
-// order in which a site's rectangles are added, and a field repeated along t gives the same B.
-// Every tile is at least 4 sites wide (rect_fits), so a footprint's three extra rows and columns
-// reach into one further tile only.
-constexpr uint32_t kNominalNT = 32;
-PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint32_t max_cells, uint32_t slots) {
-    PlaneTiles best{};
-    double time = 0.0;
-    uint64_t cells = 0;
-    for (uint32_t n1 = 1; N1 / n1 >= 4; ++n1)
-        for (uint32_t n2 = 1; N2 / n2 >= 4; ++n2) {
-            const uint32_t l1 = (N1 + n1 - 1) / n1, l2 = (N2 + n2 - 1) / n2, fc = (l1 + 3) * (l2 + 3);
-            if (fc > max_cells) continue;
-            // (16 x 16 tiles have kernels of their own: they win ties)
-            const bool sq = N1 == 16 * n1 && N2 == 16 * n2;
-            const uint64_t cn = sq ? 0 : (uint64_t)n1 * n2 * fc;
-            const double rounds = 3.0 * n1 * n2 * (double)N3 * kNominalNT / slots;
-            const double tm = (double)((l1 * l2 + 63) / 64) * (rounds < 8.0 ? std::ceil(rounds) : rounds);
-            if (time == 0.0 || tm < time || (tm == time && cn < cells)) {
-                time = tm;
-                cells = cn;
-                best = PlaneTiles{n1, N1 / n1, N1 % n1, n2, N2 / n2, N2 % n2, l1 + 3, fc,
-                                  n1 * n2 * N3 * NT, 0};
-            }
-        }
-    return best;
-}
-
 RectTiles rect_tiles_of(const Lat& L, int is_f32) {
-    const uint32_t m = is_f32 ? kMaxCells<float> : kMaxCells<double>;
-    const uint32_t w = is_f32 ? 2048 : 1024;  // wavefronts resident on 256 CUs
-    const uint32_t NT = (uint32_t)L.n[0], NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
-    RectTiles r;
-    r.p[0] = plane_split(NX, NY, NZ, NT, m, w);
-    r.p[1] = plane_split(NX, NZ, NY, NT, m, w);
-    r.p[2] = plane_split(NZ, NY, NX, NT, m, w);
-    r.p[1].cell0 = r.p[0].cell0 + (uint64_t)r.p[0].tiles * r.p[0].fc;
-    r.p[2].cell0 = r.p[1].cell0 + (uint64_t)r.p[1].tiles * r.p[1].fc;
-    return r;
+    return rect_split(L, is_f32 ? kMaxCells<float> : kMaxCells<double>, is_f32 ? 2048 : 1024);
 }
-
-uint64_t rect_cells(const RectTiles& r) { return r.p[2].cell0 + (uint64_t)r.p[2].tiles * r.p[2].fc; }
 
 }  // namespace
 
@@ -378,10 +288,13 @@ size_t rect_fp_bytes(const Lat& L, int is_f32) {
     return rect_copy_offset(rect_tiles_of(L, is_f32), sz) + (size_t)36 * L.V * sz;
 }
 
+size_t rect_footprint_bytes(const Lat& L, int is_f32) { return rect_copy_offset(rect_tiles_of(L, is_f32), is_f32 ? 4 : 8); }
+
 // partials: rect_partials, the tiles of the planes (x, y), (x, z), (z, y) in turn.  With Abuf, the
-// per-site AH parts go there instead (the B^2 adjoint's clover sums) and no partials are written.
+// per-site AH parts go there instead, for the tiled B^2 adjoint or for the others (tiled == 0), and
+// no partials are written.  copy_at > 0 places the z-fastest copy there in fpbuf.
 hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3, double* partials, void* fpbuf,
-                                hipStream_t st, uint32_t* npart, void* Abuf) {
+                                hipStream_t st, uint32_t* npart, void* Abuf, int tiled, size_t copy_at) {
     if (!rect_fits(L) || !fits_buffer(L.V, is_f32)) return hipErrorInvalidValue;
     const RectTiles rt = rect_tiles_of(L, is_f32);
     const Lat Lzy = zy_lattice(L);
@@ -390,7 +303,7 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
         using R = typename F::real;
         if constexpr (F::buffered) {
             R* fp = (R*)fpbuf;
-            R* P = (R*)((char*)fpbuf + rect_copy_offset(rt, sizeof(R)));
+            R* P = (R*)((char*)fpbuf + (copy_at ? copy_at : rect_copy_offset(rt, sizeof(R))));
             const uint32_t nxz = (uint32_t)((L.n[1] + 15) / 16) * (uint32_t)((L.n[3] + 15) / 16);
             zy_relayout_kernel<R><<<nxz * (uint32_t)L.n[2] * (uint32_t)L.n[0], 256, 0, st>>>(L, f.p, P);
             // the copy read as a field of Lzy whose directions 1 and 2 are its two blocks (the
@@ -408,10 +321,12 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
                     else
                         rect_kernel<F, false, 1, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
                 }
-                if (Abuf)
-                    rect_gather_kernel<R, true, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
+                if (Abuf && tiled)
+                    rect_gather_kernel<R, Store::kTiles, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
+                else if (Abuf)
+                    rect_gather_kernel<R, Store::kSites, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
                 else
-                    rect_gather_kernel<R, false, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, partials, nullptr);
+                    rect_gather_kernel<R, Store::kNone, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, partials, nullptr);
             };
             if (rt.p[0].square() && rt.p[1].square() && rt.p[2].square())
                 rect(std::integral_constant<int, 16>());

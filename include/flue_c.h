@@ -345,7 +345,7 @@ int flue_b2_grad_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t 
 
 /* gradient of the magnetic B (flue_magnetic); temporal links get 0.  `work` holds the
  * per-site anti-Hermitian parts of the three spatial-plane leaf sums, then the reverse form's
- * slots (and, where variant 7 of flue_magnetic_ex applies, the tiles that form those sums)
+ * slots (or, where variant 7 of flue_magnetic_ex applies, the tiles of both passes)
  * (flue_b2_work_bytes; NULL = library buffer).  Precondition in every precision: SU(3)
  * links, since the gather takes the product from a leaf corner to the walk's end as
  * X^+ F.  The call first runs flue_check_field's scan with the precision's bound (waiting
