@@ -67,6 +67,7 @@ SIGNATURES = {
     "flue_workspace_bytes": [_P],
     "flue_import_field": [_P, _P, _I, _P, _P, _I, _P],
     "flue_export_field": [_P, _P, _I, _P, _I, _P, _P],
+    "flue_tangent_field": [_P, _P, _I, _P, _P, _P],
     "flue_convert_field": [_P, _P, _I, _P, _I, _P],
     "flue_random_field": [_P, ctypes.c_uint64, _D, _P, _I, _P],
     "flue_check_field": [_P, _P, _I, _D, _P, _P, _SZ, _P],

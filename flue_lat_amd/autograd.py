@@ -14,13 +14,22 @@ group are therefore exact; the components of E normal to SU(3) are zero.
 import numpy as np
 import torch
 
-from .field import GaugeField
+from . import _lib
+from ._lib import check
+from .field import GaugeField, _ptr, _stream
 
 SQRT3 = float(np.sqrt(3.0))
 
 
-def _grad_complex(g: GaugeField):
-    return g.to_complex()
+def _tangent(G: GaugeField, U, g: GaugeField):
+    """2 G U as a C-ordered complex128 tensor, for the Lie gradient G and the links U (a complex
+    tensor), of which g is the imported field: an FP64 one holds U itself, an FP32 one U rounded."""
+    links = g if g.dtype == torch.float64 else GaugeField.from_complex(U, "fp64", G.device)
+    out = torch.empty(G.dims + (4, 3, 3), dtype=torch.complex128, device=G.device)
+    with torch.cuda.device(G.device):
+        check(_lib.lib().flue_tangent_field(G._cdims, _ptr(G.data), G.prec, _ptr(links.data), _ptr(out), _stream()),
+              "flue_tangent_field")
+    return out.to(U.device)
 
 
 def tangent_from_lie(G, U):
@@ -71,8 +80,7 @@ class _Magnetic(torch.autograd.Function):
     def backward(ctx, grad_out):
         (U,) = ctx.saved_tensors
         g = GaugeField.from_complex(U.detach(), ctx.precision)
-        G = _grad_complex(g.magnetic_grad()).to(U.device)
-        E = tangent_from_lie(G, U.detach().to(torch.complex128))
+        E = _tangent(g.magnetic_grad(), U.detach(), g)
         return (grad_out.to(torch.float64) * E).to(U.dtype), None
 
 
@@ -89,8 +97,7 @@ class _WilsonAction(torch.autograd.Function):
     def backward(ctx, grad_out):
         (U,) = ctx.saved_tensors
         g = GaugeField.from_complex(U.detach(), ctx.precision)
-        G = _grad_complex(g.wilson_grad(ctx.beta)).to(U.device)
-        E = tangent_from_lie(G, U.detach().to(torch.complex128))
+        E = _tangent(g.wilson_grad(ctx.beta), U.detach(), g)
         return (grad_out.to(torch.float64) * E).to(U.dtype), None, None
 
 

@@ -514,6 +514,15 @@ int flue_export_field(const int32_t dims[4], const void* src, int32_t prec, void
     return hip_status(launch_export(make_lat(dims), src, prec == FLUE_F32, dst, dst_type == FLUE_C64, strides, S(stream)));
 }
 
+int flue_tangent_field(const int32_t dims[4], const void* G, int32_t prec, const void* U, void* out, void* stream) {
+    int rc = check_dims(dims);
+    if (rc) return rc;
+    if (!G || !U || !out) return FLUE_ENULL;
+    if (check_prec(prec)) return FLUE_EINVAL;
+    if ((uintptr_t)out % 16 || (uintptr_t)U % 16 || (uintptr_t)G % (prec == FLUE_F32 ? 8 : 16)) return FLUE_EINVAL;
+    return hip_status(launch_tangent(make_lat(dims), G, prec == FLUE_F32, U, out, S(stream)));
+}
+
 int flue_convert_field(const int32_t dims[4], const void* src, int32_t src_prec, void* dst, int32_t dst_prec,
                        void* stream) {
     int rc = check_dims(dims);

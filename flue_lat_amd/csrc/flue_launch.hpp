@@ -15,6 +15,8 @@ hipError_t launch_import(const Lat& L, const void* src, int src_is_f32, const in
                          int dst_is_f32, hipStream_t st);
 hipError_t launch_export(const Lat& L, const void* src, int src_is_f32, void* dst, int dst_is_f32,
                          const int64_t strides[7], hipStream_t st);
+// out = 2 G U, out a C-ordered complex128 array, G in the given precision, U FP64 planes
+hipError_t launch_tangent(const Lat& L, const void* G, int is_f32, const void* U, void* out, hipStream_t st);
 hipError_t launch_random_field(const Lat& L, uint64_t seed, double eps, void* dst, int is_f32, hipStream_t st);
 hipError_t launch_convert(const Lat& L, const void* src, int src_is_f32, void* dst, int dst_is_f32, hipStream_t st);
 // SU(3) check of every link: part holds 3 doubles per block (check_blocks), out3 receives

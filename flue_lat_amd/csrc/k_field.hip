@@ -118,6 +118,52 @@ __global__ void __launch_bounds__(256) site_block_kernel(Lat L, ArrayLayout l, P
     }
 }
 
+// out = 2 G U for a C-ordered complex128 array out (NT, NX, NY, NZ, 4, 3, 3): the gradient field G and
+// the links U from their planes, the four waves on the four directions of 16 x 4 sites along x and
+// z, the products handed over through LDS and written as whole sites.
+template <typename R>
+__global__ void __launch_bounds__(256) tangent_kernel(Lat L, ArrayLayout l, const Pair<R>* __restrict__ G,
+                                                      const Pair<double>* __restrict__ U, Pair<double>* __restrict__ out) {
+    __shared__ Pair<double> sh[64 * 37];
+    int c0[4];
+    block_corner(L, l, 16, 4, 3, c0);
+    const int nx = L.n[1] - c0[1], nz = L.n[3] - c0[3];
+    {
+        const int lane = (int)threadIdx.x & 63, mu = (int)threadIdx.x >> 6, x = lane & 15, z = lane >> 4;
+        if (x < nx && z < nz) {
+            const int c[4] = {c0[0], c0[1] + x, c0[2], c0[3] + z};
+            const uint32_t s = field_site(L, c);
+            Mat<double> A, B;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) {
+                const Pair<R> g = G[(size_t)(mu * 9 + e) * L.V + s];
+                const Pair<double> u = U[(size_t)(mu * 9 + e) * L.V + s];
+                A.r[e] = 2.0 * (double)g.x;
+                A.i[e] = 2.0 * (double)g.y;
+                B.r[e] = u.x;
+                B.i[e] = u.y;
+            }
+            const Mat<double> E = mul(A, B);
+#pragma unroll
+            for (int e = 0; e < 9; ++e) {
+                Pair<double> v;
+                v.x = E.r[e];
+                v.y = E.i[e];
+                sh[(x * 4 + z) * 37 + mu * 9 + e] = v;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const int k = (int)threadIdx.x + 256 * i, site = k / 36, e = k - site * 36, x = site >> 2, z = site & 3;
+        if (x < nx && z < nz) {
+            const int c[4] = {c0[0], c0[1] + x, c0[2], c0[3] + z};
+            out[array_site(l, c) + e] = sh[site * 37 + e];
+        }
+    }
+}
+
 // kArrayPlanes: a 32 x 32 tile of (f, x); blockIdx.y is the link direction
 template <bool IN, typename Ra, typename Rf>
 __global__ void __launch_bounds__(256) plane_tile_kernel(Lat L, ArrayLayout l, Pair<Ra>* __restrict__ arr,
@@ -485,6 +531,21 @@ hipError_t launch_export(const Lat& L, const void* src, int src_is_f32, void* ds
     else
         export_kernel<double, double><<<g, 256, 0, st>>>(L, (const double*)src, (double*)dst, s[0], s[1], s[2], s[3],
                                                          s[4], s[5], s[6]);
+    return hipGetLastError();
+}
+
+hipError_t launch_tangent(const Lat& L, const void* G, int is_f32, const void* U, void* out, hipStream_t st) {
+    ArrayLayout l;
+    const int64_t z = 36, y = z * L.n[3], x = y * L.n[2], s[7] = {x * L.n[1], x, y, z, 9, 3, 1};
+    for (int k = 0; k < 7; ++k) l.st[k] = s[k];
+    l.f = 3;
+    l.o1 = 2;
+    l.o2 = 0;
+    const uint32_t g = ((uint32_t)L.n[1] + 15) / 16 * (((uint32_t)L.n[3] + 3) / 4) * (uint32_t)L.n[2] * (uint32_t)L.n[0];
+    if (is_f32)
+        tangent_kernel<float><<<g, 256, 0, st>>>(L, l, (const Pair<float>*)G, (const Pair<double>*)U, (Pair<double>*)out);
+    else
+        tangent_kernel<double><<<g, 256, 0, st>>>(L, l, (const Pair<double>*)G, (const Pair<double>*)U, (Pair<double>*)out);
     return hipGetLastError();
 }
 

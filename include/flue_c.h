@@ -192,6 +192,12 @@ int flue_export_field(const int32_t dims[4], const void* src, int32_t prec, void
 int flue_convert_field(const int32_t dims[4], const void* src, int32_t src_prec, void* dst, int32_t dst_prec,
                        void* stream);
 
+/* out = 2 G U per link, the tangent vector of a Lie gradient G (section 3) as a C-ordered
+ * complex128 device array (NT, NX, NY, NZ, 4, 3, 3): G is a SoA field in prec, U the links as
+ * a SoA field in FP64.  Computed in FP64.  out and the fields must be aligned to their
+ * complex elements.  No reference counterpart (torch.autograd's gradient of a real function). */
+int flue_tangent_field(const int32_t dims[4], const void* G, int32_t prec, const void* U, void* out, void* stream);
+
 /* SU(3) check of every link, computed in FP64 (no reference counterpart; the reference
  * readers reunitarise every link instead, src/gaugeIO/ILDG_bin.f90:138-151): stats[0] = the
  * number of links with a non-finite entry, stats[1] = max over links and entries of

@@ -75,3 +75,19 @@ def test_expanded_and_unaligned_sources(FL):
     buf.zero_()
     assert _lib.lib().flue_export_field(f._cdims, ctypes.c_void_p(f.data.data_ptr()), 0, ptr, _lib.FLUE_C128, cs, st) == 0
     assert torch.equal(buf[1:], torch.view_as_real(U).reshape(-1)) and buf[0] == 0
+
+
+@pytest.mark.parametrize("dims", [(3, 5, 7, 6), (1, 17, 2, 4), (2, 16, 3, 9), (4, 1, 1, 1)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_tangent_field(FL, dims, prec):
+    # 2 G U against the product of the exported arrays: one rounding per product and sum of three
+    # (6 eps relative to the row norms)
+    from flue_lat_amd.autograd import _tangent, tangent_from_lie
+    g = FL.GaugeField.random(dims, 31, 0.3, "fp64")
+    U = g.to_complex()
+    f = g.astype(prec)
+    G = f.wilson_grad(6.0)
+    E = _tangent(G, U, f)
+    assert E.is_contiguous() and E.shape == dims + (4, 3, 3)
+    want = tangent_from_lie(G.to_complex(), U)
+    assert float((E - want).abs().max()) <= 6 * 2.3e-16 * 2 * float(want.abs().max())
