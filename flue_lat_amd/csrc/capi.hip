@@ -1147,10 +1147,11 @@ int ens_grid(const EnsPlan& p, int variant, uint32_t* grid) {
     return FLUE_OK;
 }
 
-// the ensemble work buffer: table, second link buffer, accumulators (room for FP64), partial sums, and
+// the ensemble work buffer: tables, second link buffer, accumulators (room for FP64), partial sums, and
 // the plaquette parts of the plaquette-first stencil
 struct EnsWork {
     EnsEntry* tab;
+    EnsRect* rect;
     void* W2;
     double* acc;
     double* partials;
@@ -1162,6 +1163,8 @@ EnsWork ens_work(void* w, int32_t n, const EnsPlan& p, size_t sz) {
     EnsWork r;
     r.tab = (EnsEntry*)base;
     base += align256(sizeof(EnsEntry) * n);
+    r.rect = (EnsRect*)base;
+    base += align256(sizeof(EnsRect) * n);
     r.W2 = base;
     base += align256((size_t)p.field_reals * sz);
     r.acc = (double*)base;
@@ -1183,9 +1186,9 @@ size_t flue_ensemble_field_bytes(int32_t n, const int32_t* dims, int32_t prec) {
 size_t flue_ensemble_work_bytes(int32_t n, const int32_t* dims, int32_t prec) {
     EnsPlan p;
     if (ens_plan(n, dims, p) || check_prec(prec)) return 0;
-    // table, second link buffer, accumulators (room for FP64), per-block partial sums, plaquette parts
+    // tables, second link buffer, accumulators (room for FP64), per-block partial sums, plaquette parts
     const size_t sz = prec == FLUE_F32 ? 4 : 8;
-    return align256(sizeof(EnsEntry) * n) + align256((size_t)p.field_reals * sz) + align256((size_t)p.acc_doubles * 8) +
+    return align256(sizeof(EnsEntry) * n) + align256(sizeof(EnsRect) * n) + align256((size_t)p.field_reals * sz) + align256((size_t)p.acc_doubles * 8) +
            align256((size_t)p.total_blocks * 16) + align256((size_t)p.field_reals / 72 * 48 * sz);
 }
 
@@ -1223,7 +1226,12 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
     double* partials = ew.partials;
     hipStream_t st = S(stream);
     FLUE_TRY(hipMemcpyAsync(d_tab, p.tab.data(), sizeof(EnsEntry) * n, hipMemcpyHostToDevice, st));
-    FLUE_TRY(hipStreamSynchronize(st));  // the host table goes out of scope with this call
+    const int nmeas = measure_every > 0 ? nsteps / measure_every + 1 : 0;
+    std::vector<EnsRect> rect(nmeas > 0 ? n : 0);
+    EnsRectGrid rect_grid;
+    const bool tiled = nmeas > 0 && ens_rect_plan(p.tab.data(), n, is_f32, p.maxV, rect.data(), &rect_grid);
+    if (tiled) FLUE_TRY(hipMemcpyAsync(ew.rect, rect.data(), sizeof(EnsRect) * n, hipMemcpyHostToDevice, st));
+    FLUE_TRY(hipStreamSynchronize(st));  // the host tables go out of scope with this call
 
     int32_t key[4];
     ens_key(p, n, key);
@@ -1232,21 +1240,30 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
     if ((rc = ens_grid(p, variant, &grid))) return rc;
     void* T = variant > 4 ? ew.T : nullptr;  // the plaquette-first variants
 
-    const int nmeas = measure_every > 0 ? nsteps / measure_every + 1 : 0;
     static const double ca[3] = {0.0, -17.0 / 9.0, -1.0};
     static const double cb[3] = {0.25, 8.0 / 9.0, 0.75};
     void* bufs[2] = {fields, W2};
-    auto measure = [&](const void* fld, int m) -> hipError_t {
+    // Measurements fall between RK3 steps, when the other link buffer, the accumulators (a step's
+    // first stage only writes them) and the plaquette parts hold nothing: the tiled B keeps its
+    // copies, partials (2 doubles for 4 x 4 sites at least, of 32 a site) and footprints there.
+    auto measure = [&](int b, int m) -> hipError_t {
+        const void* fld = bufs[b];
         hipError_t e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 0, partials, grid, st);
-        if (e == hipSuccess) e = launch_ens_finalize(d_tab, n, partials, d_plaq + (size_t)m * n, 1, 0, st);
-        if (e == hipSuccess) e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 1, partials, grid, st);
-        if (e == hipSuccess) e = launch_ens_finalize(d_tab, n, partials, d_B + (size_t)m * n, 1, 1, st);
+        if (e == hipSuccess) e = launch_ens_finalize(d_tab, nullptr, n, partials, d_plaq + (size_t)m * n, 1, 0, st);
+        if (e != hipSuccess) return e;
+        if (tiled)
+            e = launch_ens_rect(d_tab, ew.rect, n, rect_grid, fld, is_f32, bufs[b ^ 1], ew.T, acc, st);
+        else
+            e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 1, partials, grid, st);
+        if (e == hipSuccess)
+            e = launch_ens_finalize(d_tab, tiled ? ew.rect : nullptr, n, tiled ? acc : partials, d_B + (size_t)m * n, 1,
+                                    1, st);
         return e;
     };
     // the whole run: measurement at step 0 and after every measure_every steps
     auto run = [&]() -> hipError_t {
         hipError_t e = hipSuccess;
-        if (nmeas > 0) e = measure(fields, 0);
+        if (nmeas > 0) e = measure(0, 0);
         for (int32_t j = 0; j < nsteps && e == hipSuccess; ++j) {
             for (int k = 0; k < 3 && e == hipSuccess; ++k) {
                 const int q = 3 * j + k;
@@ -1254,7 +1271,7 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
                                           eps, ca[k], cb[k], k == 2, grid, T, st);
             }
             if (e == hipSuccess && nmeas > 0 && (j + 1) % measure_every == 0)
-                e = measure(bufs[(j + 1) & 1], (j + 1) / measure_every);
+                e = measure((j + 1) & 1, (j + 1) / measure_every);
         }
         if (e == hipSuccess && (nsteps & 1)) e = launch_copy((size_t)p.field_reals, is_f32, W2, fields, st);
         return e;

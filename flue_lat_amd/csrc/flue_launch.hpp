@@ -84,6 +84,19 @@ constexpr size_t kMagneticScratchBytes = (size_t)8 << 20;
 // fpbuf: the footprint buffer of variant 7 (rect_fp_bytes), unused by the others
 hipError_t launch_magnetic(const Lat& L, const void* U, int is_f32, int su3, double* partials, hipStream_t st,
                            int variant, uint32_t* npart, void* fpbuf = nullptr);
+// One plane's tiling.  Direction 1 (x) has n1 tiles, the first r1 of q1 + 1 sites and the others
+// of q1; direction 2 likewise.  Footprints (the tile plus three rows and columns) have rows of f
+// cells and fc cells in all; the plane's first one is cell cell0 of the buffer.
+struct PlaneTiles {
+    uint32_t n1, q1, r1, n2, q2, r2;
+    uint32_t f, fc, tiles;
+    uint64_t cell0;
+    bool square() const { return q1 == 16 && r1 == 0 && q2 == 16 && r2 == 0; }
+};
+struct RectTiles {
+    PlaneTiles p[3];  // planes (x,y), (x,z), (z,y) (the last as plane (x,y) of the copy)
+};
+
 bool rect_fits(const Lat& L);
 // partials of variant 7: one per tile of its three planes
 uint32_t rect_partials(const Lat& L, int is_f32);
@@ -151,6 +164,13 @@ struct EnsEntry {
     uint32_t blk0;
     uint32_t nblk;
 };
+// configuration c in the rectangle-first magnetic: its tiles [tile0, tile0 + tiles) (the three planes'
+// in turn) and the blocks from copy0 that make its z-fastest copy
+struct EnsRect {
+    RectTiles rt;
+    Lat Lzy;
+    uint32_t tile0, tiles, copy0;
+};
 // T != nullptr: the plaquette-first stencil with the plaquette parts of every field in T
 // (48 reals per site, field c's at 2/3 of its field offset); T == nullptr: staple sums
 hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* win,
@@ -158,8 +178,20 @@ hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uin
                                  uint32_t grid, void* T, hipStream_t st);
 hipError_t launch_ens_sum(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* fld, int is_f32,
                           int obs, double* partials, uint32_t grid, hipStream_t st);
-hipError_t launch_ens_finalize(const EnsEntry* tab, int n, const double* partials, double* out, int stride,
-                               int per_volume, hipStream_t st);
+// the partials of configuration c: its logical blocks', or its tiles' with rect
+hipError_t launch_ens_finalize(const EnsEntry* tab, const EnsRect* rect, int n, const double* partials, double* out,
+                               int stride, int per_volume, hipStream_t st);
+// the magnetic B of every configuration on rectangle-first tiles (k_rect.hip).  ens_rect_plan fills
+// the table where the ensemble takes that form, and is false where it keeps launch_ens_sum; field c's
+// copy lies at its field offset in `copy` (a buffer of the ensemble's size), its footprints at 2/3 of
+// that in `fp` (48 reals a site); one partial per tile (EnsRectGrid::tiles).
+struct EnsRectGrid {
+    uint32_t tiles, copies;
+    bool square;
+};
+bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRect* rect, EnsRectGrid* g);
+hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, const EnsRectGrid& g, const void* fld,
+                           int is_f32, void* copy, void* fp, double* partials, hipStream_t st);
 hipError_t launch_copy(size_t n_reals, int is_f32, const void* src, void* dst, hipStream_t st);
 // ensemble flow variants: persistent grid of 1, 2, 4 or 8 workgroups per CU with the staple
 // stencil (1..4) or the plaquette-first stencil (5..8)

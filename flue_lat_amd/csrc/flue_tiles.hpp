@@ -3,23 +3,10 @@
 #pragma once
 #include <cmath>
 
-#include "flue_common.hpp"
+#include "flue_launch.hpp"
 
 namespace flue {
 namespace {
-
-// One plane's tiling.  Direction 1 (x) has n1 tiles, the first r1 of q1 + 1 sites and the others
-// of q1; direction 2 likewise.  Footprints (the tile plus three rows and columns) have rows of f
-// cells and fc cells in all; the plane's first one is cell cell0 of the buffer.
-struct PlaneTiles {
-    uint32_t n1, q1, r1, n2, q2, r2;
-    uint32_t f, fc, tiles;
-    uint64_t cell0;
-    bool square() const { return q1 == 16 && r1 == 0 && q2 == 16 && r2 == 0; }
-};
-struct RectTiles {
-    PlaneTiles p[3];  // planes (x,y), (x,z), (z,y) (the last as plane (x,y) of the copy)
-};
 
 // the second direction of rectangle plane rp (0: (x, y), 1: (x, z))
 __device__ __forceinline__ int rect_d2(int rp) { return rp == 0 ? 2 : 3; }
@@ -45,9 +32,9 @@ __device__ __forceinline__ Tile tile_at(const Lat& L, int rp, const PlaneTiles& 
     return t;
 }
 
-// rectangle plane blockIdx.y of a kernel over the three planes
-__device__ __forceinline__ PlaneTiles plane_tiles(const RectTiles& g) {
-    return blockIdx.y == 0 ? g.p[0] : (blockIdx.y == 1 ? g.p[1] : g.p[2]);
+// rectangle plane y of a lattice's three
+__device__ __forceinline__ PlaneTiles plane_tiles(const RectTiles& g, uint32_t y = blockIdx.y) {
+    return y == 0 ? g.p[0] : (y == 1 ? g.p[1] : g.p[2]);
 }
 
 // lattice whose x, y, z are the z, y, x of L: its plane (x, y) is L's plane (z, y)
@@ -91,7 +78,8 @@ PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint3
     return best;
 }
 
-// the three planes of a lattice; `slots` wavefronts are resident on the chip
+// the three planes of a lattice; `slots` wavefronts are resident on the chip (1: whatever the launch
+// holds besides, the chip is full)
 RectTiles rect_split(const Lat& L, uint32_t max_cells, uint32_t slots) {
     const uint32_t NT = (uint32_t)L.n[0], NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
     RectTiles r;

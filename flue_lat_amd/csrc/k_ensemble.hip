@@ -7,7 +7,8 @@
 // adjacent), finds the configuration of a logical block by binary search in a table
 // kept in device memory, and runs the same per-site (flow: per-link) code as the
 // single-field kernels.
-// Sums are reduced per logical block and then per configuration in a fixed order.
+// Sums are reduced per logical block and then per configuration in a fixed order.  (B takes the
+// rectangle-first tiles of k_rect.hip where they apply, one launch for every tile of the ensemble.)
 #include "flue_clover.hpp"
 #include "flue_flow.hpp"
 #include "flue_launch.hpp"
@@ -140,13 +141,15 @@ __global__ void __launch_bounds__(kBS) ens_sum_kernel(const EnsEntry* __restrict
     }
 }
 
-// one workgroup per configuration: out[c * stride] = scale_c * sum of its block partials
+// one workgroup per configuration: out[c * stride] = scale_c * sum of its block or tile partials
 __global__ void __launch_bounds__(kBS) ens_finalize_kernel(const EnsEntry* __restrict__ tab,
+                                                           const EnsRect* __restrict__ rect,
                                                            const double* __restrict__ partials,
                                                            double* __restrict__ out, int stride, int per_volume) {
     const EnsEntry e = tab[blockIdx.x];
-    const uint32_t lo = e.blk0 + (uint32_t)(((uint64_t)e.nblk * threadIdx.x) / kBS);
-    const uint32_t hi = e.blk0 + (uint32_t)(((uint64_t)e.nblk * (threadIdx.x + 1)) / kBS);
+    const uint32_t first = rect ? rect[blockIdx.x].tile0 : e.blk0, count = rect ? rect[blockIdx.x].tiles : e.nblk;
+    const uint32_t lo = first + (uint32_t)(((uint64_t)count * threadIdx.x) / kBS);
+    const uint32_t hi = first + (uint32_t)(((uint64_t)count * (threadIdx.x + 1)) / kBS);
     DD acc = {0.0, 0.0};
     for (uint32_t i = lo; i < hi; ++i) acc = dd_add(acc, DD{partials[2 * i], partials[2 * i + 1]});
     const DD r = block_sum<kBS>(acc);
@@ -211,9 +214,9 @@ hipError_t launch_ens_sum(const EnsEntry* tab, int n, uint32_t total, uint32_t m
     return hipGetLastError();
 }
 
-hipError_t launch_ens_finalize(const EnsEntry* tab, int n, const double* partials, double* out, int stride,
-                               int per_volume, hipStream_t st) {
-    ens_finalize_kernel<<<n, kBS, 0, st>>>(tab, partials, out, stride, per_volume);
+hipError_t launch_ens_finalize(const EnsEntry* tab, const EnsRect* rect, int n, const double* partials, double* out,
+                               int stride, int per_volume, hipStream_t st) {
+    ens_finalize_kernel<<<n, kBS, 0, st>>>(tab, rect, partials, out, stride, per_volume);
     return hipGetLastError();
 }
 

@@ -70,25 +70,22 @@ __device__ __forceinline__ void fp_add(R* fp, int cell, const AH<R>& p) {
     }
 }
 
+// LDS reals of a tile's footprint, and of the stride between a cell's elements (FP64)
+template <typename R, int W>
+constexpr int kTileStride = W ? (W + 3) * (W + 3) : kMaxCells<R>;
+
+// One wavefront, one tile of rectangle plane rp of f: its footprint in LDS (fp), then in memory at
+// out as [e * fc + c] in both precisions.
 // WPE == 1 (FP64) takes the chains with a one-link lookahead (rect_base); at two waves per
 // SIMD (FP32) the other wave covers the load latency.  W > 0: every tile is W x W, so its rows and
 // footprint strides are constants (48^3x96: 5.44 -> 5.35 ms in FP32, 10.2 -> 9.9 ms in FP64).
-template <typename FV, bool C2, int WPE, int W>
-__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, typename FV::real* __restrict__ fpout) {
+template <bool C2, int WPE, int W, typename FV>
+__device__ __forceinline__ void rect_tile(const Lat L, const FV f, int rp, const PlaneTiles g, uint32_t tile,
+                                          typename FV::real* fp, typename FV::real* __restrict__ out) {
     using R = typename FV::real;
     constexpr int CR = kCellReals<R>;
-    constexpr int FS = W ? (W + 3) * (W + 3) : kMaxCells<R>;  // FP64: reals between a cell's elements
-    __shared__ __align__(16) R fp[CR * FS];
-    // blockIdx.y: 0 plane (x,y), 1 plane (x,z), 2 plane (z,y) as plane (x,y) of the copy
-    const bool zy = blockIdx.y == 2;
-    const PlaneTiles g = plane_tiles(rt);
-    if (blockIdx.x >= g.tiles) return;
-    const Lat L = zy ? Lzy : L0;
-    const FV f = zy ? fzy : f0;
-    const int rp = zy ? 0 : (int)blockIdx.y;
+    constexpr int FS = kTileStride<R, W>;
     const int d2 = rect_d2(rp);
-    const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
     const Tile t = tile_at(L, rp, g, tile);
     const int fc = W ? FS : (int)g.fc, f1 = W ? W + 3 : (int)g.f;
     const uint32_t w = W ? (uint32_t)W : t.l1, h = W ? (uint32_t)W : t.l2;
@@ -111,11 +108,23 @@ rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, typename FV::real* __r
         });
     }
     __syncthreads();
-    // to memory as [e * fc + c] in both precisions
-    R* out = fpout + 9 * (g.cell0 + (uint64_t)tile * g.fc);
     for (int c = threadIdx.x; c < fc; c += kRW)
 #pragma unroll
         for (int e = 0; e < 9; ++e) out[e * fc + c] = fp[CR == 12 ? c * 12 + e : e * FS + c];
+}
+
+template <typename FV, bool C2, int WPE, int W>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, typename FV::real* __restrict__ fpout) {
+    using R = typename FV::real;
+    __shared__ __align__(16) R fp[kCellReals<R> * kTileStride<R, W>];
+    // blockIdx.y: 0 plane (x,y), 1 plane (x,z), 2 plane (z,y) as plane (x,y) of the copy
+    const bool zy = blockIdx.y == 2;
+    const PlaneTiles g = plane_tiles(rt);
+    if (blockIdx.x >= g.tiles) return;
+    const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
+    rect_tile<C2, WPE, W>(zy ? Lzy : L0, zy ? fzy : f0, zy ? 0 : (int)blockIdx.y, g, tile, fp,
+                          fpout + 9 * (g.cell0 + (uint64_t)tile * g.fc));
 }
 
 // the clover AH parts of tile cell (cx, cy): its own footprint's cell, then the overlapping
@@ -144,6 +153,41 @@ __device__ __forceinline__ AH<R> cell_sum(const R* own, const R* left, const R* 
     return h;
 }
 
+// The four footprints that cover a tile's sites: its own and those of the tiles before it along x
+// and d2 (periodic), and the geometry of the overlaps.  fp is the plane's first footprint.
+template <typename R, int W>
+struct Cover {
+    const R *own, *left, *below, *diag;
+    int fc, f1, shift1, shift2;
+    uint32_t w, h;
+    __device__ __forceinline__ Cover(const PlaneTiles& g, const Tile& t, uint32_t tile, const R* fp) {
+        const uint32_t tl = t.t1 ? t.t1 - 1 : g.n1 - 1, tb = t.t2 ? t.t2 - 1 : g.n2 - 1;
+        const int dl = (int)tl - (int)t.t1, db = ((int)tb - (int)t.t2) * (int)g.n1;
+        shift1 = W ? W : (int)(g.q1 + (tl < g.r1 ? 1u : 0u));
+        shift2 = W ? W : (int)(g.q2 + (tb < g.r2 ? 1u : 0u));
+        fc = W ? (W + 3) * (W + 3) : (int)g.fc;
+        f1 = W ? W + 3 : (int)g.f;
+        w = W ? (uint32_t)W : t.l1;
+        h = W ? (uint32_t)W : t.l2;
+        own = fp + 9 * (uint64_t)tile * g.fc;
+        left = own + 9 * (int64_t)fc * dl;
+        below = own + 9 * (int64_t)fc * db;
+        diag = own + 9 * (int64_t)fc * (dl + db);
+    }
+    // body(cx, cy, AH parts of the site) for this wavefront's share of the tile's sites
+    template <typename Body>
+    __device__ __forceinline__ void sites(Body&& body) const {
+#pragma unroll
+        for (uint32_t j0 = 0; j0 < w * h; j0 += kRW) {
+            const uint32_t j = j0 + threadIdx.x;
+            if (!W && j >= w * h) break;
+            const int cy = W ? (int)(j0 / w + threadIdx.x / w) : (int)(j / w);
+            const int cx = W ? (int)(threadIdx.x % w) : (int)(j - (uint32_t)cy * w);
+            body(cx, cy, cell_sum(own, left, below, diag, fc, f1, cx, cy, shift1, shift2));
+        }
+    }
+};
+
 // Per tile: its sites' clover AH parts from the four footprints that cover them.  One wavefront
 // (measured faster than a thread per site).  STORE = false: sum |F|^2 over the tile into one
 // compensated partial per tile.  Otherwise write each site's AH parts into Abuf, 9 planes of V
@@ -163,24 +207,9 @@ __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectT
     const int rp = zy ? 0 : (int)blockIdx.y;
     const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
     const Tile t = tile_at(L, rp, g, tile);
-    // the tiles before this one along x and d2 (periodic)
-    const uint32_t tl = t.t1 ? t.t1 - 1 : g.n1 - 1, tb = t.t2 ? t.t2 - 1 : g.n2 - 1;
-    const int dl = (int)tl - (int)t.t1, db = ((int)tb - (int)t.t2) * (int)g.n1;
-    const int shift1 = W ? W : (int)(g.q1 + (tl < g.r1 ? 1u : 0u)), shift2 = W ? W : (int)(g.q2 + (tb < g.r2 ? 1u : 0u));
-    const int fc = W ? (W + 3) * (W + 3) : (int)g.fc, f1 = W ? W + 3 : (int)g.f;
-    const uint32_t w = W ? (uint32_t)W : t.l1, h = W ? (uint32_t)W : t.l2;
-    const R* own = fpin + 9 * (g.cell0 + (uint64_t)tile * g.fc);
-    const R* left = own + 9 * (int64_t)fc * dl;
-    const R* below = own + 9 * (int64_t)fc * db;
-    const R* diag = own + 9 * (int64_t)fc * (dl + db);
+    const Cover<R, W> cover(g, t, tile, fpin + 9 * g.cell0);
     double acc = 0.0;
-#pragma unroll
-    for (uint32_t j0 = 0; j0 < w * h; j0 += kRW) {
-        const uint32_t j = j0 + threadIdx.x;
-        if (!W && j >= w * h) break;
-        const int cy = W ? (int)(j0 / w + threadIdx.x / w) : (int)(j / w);
-        const int cx = W ? (int)(threadIdx.x % w) : (int)(j - (uint32_t)cy * w);
-        const AH<R> h = cell_sum(own, left, below, diag, fc, f1, cx, cy, shift1, shift2);
+    cover.sites([&](int cx, int cy, const AH<R>& h) {
         if constexpr (STORE != Store::kNone) {
             const uint32_t c2 = t.o2 + (uint32_t)cy, c1 = t.o1 + (uint32_t)cx;
             uint32_t s = c1 + L.st[2] * (rp == 0 ? c2 : t.cs) + L.st[3] * (rp == 0 ? t.cs : c2) + L.st[0] * t.ct;
@@ -200,7 +229,7 @@ __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectT
         } else {
             acc += f_norm2(h);
         }
-    }
+    });
     if constexpr (STORE == Store::kNone) {
         const DD s = block_sum<kRW>(DD{acc, 0.0});
         if (threadIdx.x == 0) {
@@ -213,15 +242,14 @@ __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectT
 
 // U_z and U_y of the field (lattice L) into P, z fastest: P holds two direction blocks of
 // 9 complex planes, [k][e][s'] with s' = z + NZ (y + NY (x + NX t)), k = 0 for U_z, 1 for
-// U_y.  One block per 16 x 16 (x, z) tile at fixed (y, t), through a padded LDS tile so that
+// U_y.  Block q of one per 16 x 16 (x, z) tile at fixed (y, t), through a padded LDS tile so that
 // both the reads (along x) and the writes (along z) coalesce.
 template <typename R>
-__global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __restrict__ U, R* __restrict__ P) {
+__device__ __forceinline__ void zy_relayout(const Lat& L, uint32_t q, const R* __restrict__ U, R* __restrict__ P) {
     using P2 = typename Pair2<R>::type;
     __shared__ P2 tile[16][17];
     const uint32_t NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
     const uint32_t bxs = (NX + 15) / 16, bzs = (NZ + 15) / 16;
-    uint32_t q = blockIdx.x;
     const uint32_t bx = q % bxs;
     q /= bxs;
     const uint32_t bz = q % bzs;
@@ -250,6 +278,100 @@ __global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __rest
             }
             __syncthreads();
         }
+    }
+}
+
+uint32_t zy_blocks(const Lat& L) {
+    return (uint32_t)((L.n[1] + 15) / 16) * (uint32_t)((L.n[3] + 15) / 16) * (uint32_t)L.n[2] * (uint32_t)L.n[0];
+}
+
+template <typename R>
+__global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __restrict__ U, R* __restrict__ P) {
+    zy_relayout(L, blockIdx.x, U, P);
+}
+
+// the copy read as a field of Lzy whose directions 1 and 2 are its two blocks (the view's base is one
+// direction block before P; directions 0 and 3 are never read)
+template <typename R>
+__host__ __device__ __forceinline__ const R* zy_view(const R* P, uint32_t V) {
+    return (const R*)((uintptr_t)P - (uintptr_t)18 * V * sizeof(R));
+}
+
+// ---- ensembles: the same tiles, those of every configuration and plane in one launch.  16 fields of
+// 16^3 with 644 time slices in all, FP32, one B of each: 3.72 ms by quadrants, 1.65 ms so.
+
+// the configuration of a tile or of a block of the copies; table reads are uniform (scalar loads)
+using CEnsRect = const __attribute__((address_space(4))) EnsRect;
+using CEnsEntry = const __attribute__((address_space(4))) EnsEntry;
+template <uint32_t EnsRect::*First>
+__device__ __forceinline__ int rect_cfg(const EnsRect* rect, int n, uint32_t b) {
+    const EnsRect* tab = (const EnsRect*)(CEnsRect*)rect;
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (tab[mid].*First <= b)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
+}
+
+// tile b of the ensemble: its plane (0 .. 2), leaving b its number in the plane
+__device__ __forceinline__ uint32_t rect_plane(const EnsRect& r, uint32_t& b) {
+    b -= r.tile0;
+    if (b < r.rt.p[0].tiles) return 0;
+    b -= r.rt.p[0].tiles;
+    if (b < r.rt.p[1].tiles) return 1;
+    b -= r.rt.p[1].tiles;
+    return 2;
+}
+
+template <typename R>
+__global__ void __launch_bounds__(256) ens_relayout_kernel(const EnsEntry* __restrict__ tab,
+                                                           const EnsRect* __restrict__ rect, int n,
+                                                           const R* __restrict__ U, R* __restrict__ P) {
+    const int c = rect_cfg<&EnsRect::copy0>(rect, n, blockIdx.x);
+    const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
+    zy_relayout(e.L, blockIdx.x - rect[c].copy0, U + e.off, P + e.off);
+}
+
+template <typename R, bool C2, int WPE, int W>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+ens_rect_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ rect, int n, const R* __restrict__ U,
+                const R* __restrict__ P, R* __restrict__ fpout) {
+    __shared__ __align__(16) R fp[kCellReals<R> * kTileStride<R, W>];
+    uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
+    const int c = rect_cfg<&EnsRect::tile0>(rect, n, tile);
+    const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
+    const EnsRect& r = *(const EnsRect*)((CEnsRect*)rect + c);
+    const uint32_t y = rect_plane(r, tile);
+    const PlaneTiles g = plane_tiles(r.rt, y);
+    const FieldView<R, true> f{y == 2 ? zy_view(P + e.off, e.L.V) : U + e.off, e.L.V};
+    rect_tile<C2, WPE, W>(y == 2 ? r.Lzy : e.L, f, y == 1 ? 1 : 0, g, tile, fp,
+                          fpout + e.off / 72 * 48 + 9 * (g.cell0 + (uint64_t)tile * g.fc));
+}
+
+template <typename R, int W>
+__global__ void __launch_bounds__(kRW) ens_gather_kernel(const EnsEntry* __restrict__ tab,
+                                                         const EnsRect* __restrict__ rect, int n,
+                                                         const R* __restrict__ fpin, double* __restrict__ partials) {
+    const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
+    const int c = rect_cfg<&EnsRect::tile0>(rect, n, b);
+    const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
+    const EnsRect& r = *(const EnsRect*)((CEnsRect*)rect + c);
+    uint32_t tile = b;
+    const uint32_t y = rect_plane(r, tile);
+    const PlaneTiles g = plane_tiles(r.rt, y);
+    const Tile t = tile_at(y == 2 ? r.Lzy : e.L, y == 1 ? 1 : 0, g, tile);
+    double acc = 0.0;
+    Cover<R, W>(g, t, tile, fpin + e.off / 72 * 48 + 9 * g.cell0).sites([&](int, int, const AH<R>& h) {
+        acc += f_norm2(h);
+    });
+    const DD s = block_sum<kRW>(DD{acc, 0.0});
+    if (threadIdx.x == 0) {
+        partials[2 * b] = s.hi;
+        partials[2 * b + 1] = s.lo;
     }
 }
 
@@ -304,11 +426,8 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
         if constexpr (F::buffered) {
             R* fp = (R*)fpbuf;
             R* P = (R*)((char*)fpbuf + (copy_at ? copy_at : rect_copy_offset(rt, sizeof(R))));
-            const uint32_t nxz = (uint32_t)((L.n[1] + 15) / 16) * (uint32_t)((L.n[3] + 15) / 16);
-            zy_relayout_kernel<R><<<nxz * (uint32_t)L.n[2] * (uint32_t)L.n[0], 256, 0, st>>>(L, f.p, P);
-            // the copy read as a field of Lzy whose directions 1 and 2 are its two blocks (the
-            // view's base is one direction block before P; directions 0 and 3 are never read)
-            const F fzy{(const R*)((uintptr_t)P - (uintptr_t)18 * L.V * sizeof(R)), L.V};
+            zy_relayout_kernel<R><<<zy_blocks(L), 256, 0, st>>>(L, f.p, P);
+            const F fzy{zy_view<R>(P, L.V), L.V};
             const dim3 g(std::max({rt.p[0].tiles, rt.p[1].tiles, rt.p[2].tiles}), 3);
             // FP32 and declared-SU(3) FP64 links: two-row chains; plain FP64: full products
             auto rect = [&](auto w) {
@@ -335,6 +454,62 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
         }
     });
     if (npart) *npart = rect_partials(L, is_f32);
+    return hipGetLastError();
+}
+
+// Every configuration has to suit the tiles (extents as in rect_fits) and its footprints to fit the
+// plaquette parts' 48 reals a site; the sites are counted over the ensemble, since it runs as one launch,
+// and the tiles are those that cost least on a full chip.  A measurement (B and the plaquettes), ms by
+// quadrants -> by tiles, FP32 and FP64:
+//   2 x 16^3x12         98,304 sites   0.156 -> 0.115   0.272 -> 0.194
+//   5 x 12^3x13        112,320         0.167 -> 0.155   0.277 -> 0.241
+//   8 x 12x13x14x10    174,720         0.247 -> 0.166   0.392 -> 0.304
+//   8 x 16^4           524,288         0.665 -> 0.365   1.191 -> 0.677
+bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRect* rect, EnsRectGrid* g) {
+    if (!fits_buffer(maxV, is_f32)) return false;
+    uint64_t sites = 0, tiles = 0, copies = 0;
+    g->square = true;
+    for (int c = 0; c < n; ++c) {
+        const Lat& L = tab[c].L;
+        if (std::min({L.n[1], L.n[2], L.n[3]}) < 12) return false;
+        EnsRect& r = rect[c];
+        r.rt = rect_split(L, is_f32 ? kMaxCells<float> : kMaxCells<double>, 1);
+        if (rect_cells(r.rt) * 9 > (uint64_t)48 * L.V) return false;
+        r.Lzy = zy_lattice(L);
+        r.tile0 = (uint32_t)tiles;
+        r.tiles = r.rt.p[0].tiles + r.rt.p[1].tiles + r.rt.p[2].tiles;
+        r.copy0 = (uint32_t)copies;
+        for (const PlaneTiles& p : r.rt.p) g->square = g->square && p.square();
+        sites += L.V;
+        tiles += r.tiles;
+        copies += zy_blocks(L);
+    }
+    g->tiles = (uint32_t)tiles;
+    g->copies = (uint32_t)copies;
+    return sites >= kRectSites && tiles < 0x80000000ull && copies < 0x80000000ull;
+}
+
+hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, const EnsRectGrid& g, const void* fld,
+                           int is_f32, void* copy, void* fp, double* partials, hipStream_t st) {
+    auto run = [&](auto real, auto w) {
+        using R = decltype(real);
+        constexpr int W = decltype(w)::value;
+        constexpr bool F32 = sizeof(R) == 4;  // FP32: two-row chains, two waves per SIMD
+        ens_relayout_kernel<R><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy);
+        ens_rect_kernel<R, F32, F32 ? 2 : 1, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fld, (const R*)copy,
+                                                                         (R*)fp);
+        ens_gather_kernel<R, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fp, partials);
+    };
+    auto sized = [&](auto real) {
+        if (g.square)
+            run(real, std::integral_constant<int, 16>());
+        else
+            run(real, std::integral_constant<int, 0>());
+    };
+    if (is_f32)
+        sized(float(0));
+    else
+        sized(double(0));
     return hipGetLastError();
 }
 

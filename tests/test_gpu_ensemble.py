@@ -112,3 +112,27 @@ def test_ensemble_c4_member_against_oracle_fp64(FL):
         assert np.abs(e.field(c).to_complex().cpu().numpy() - W).max() < 1e-12, c
         assert abs(B[1, c] - O.magnetic(W)) < 1e-12 * O.magnetic(W), c
         assert abs(plaq[1, c] - O.plaquette(W, 1, 4, 4)[0]) < 1e-12 * abs(plaq[1, c]), c
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 2e-7)])
+@pytest.mark.parametrize("dims", [
+    [(11, 16, 16, 32), (1, 32, 16, 16)],                                 # 16 x 16 tiles
+    [(9, 17, 13, 21), (14, 12, 15, 12), (2, 33, 12, 18), (5, 20, 20, 20)],  # uneven tiles, fields of several shapes
+    [(16, 16, 16, 16), (7, 11, 16, 16)],                                 # one extent too small: quadrants
+])
+def test_ensemble_magnetic_tiles(FL, dims, prec, tol):
+    # B of an ensemble on rectangle-first tiles, before, between and after an odd number of steps (the
+    # links lie in either buffer), against the quadrant form of each field.  FP32: the forms round the
+    # products of a leaf differently, 2^-24 each and averaged over the sites; 2e-7 is three roundings.
+    from flue_lat_amd.ensemble import Ensemble
+    seeds = [50 + c for c in range(len(dims))]
+    e = Ensemble.random(dims, seeds, 0.3, prec)
+    singles = [e.field(c).clone() for c in range(len(dims))]
+    _, B = e.flow(0.01, 3, measure_every=1)
+    for c, g in enumerate(singles):
+        for m in range(4):
+            b = g.magnetic(variant=1)
+            assert abs(B[m, c] - b) < tol * b, (dims[c], m)
+            if m < 3:
+                g.wilson_flow(0.01, 1, use_graph=False)
+        assert torch.allclose(e.field(c).data, g.data, rtol=0, atol=1e-12 if prec == "fp64" else 2e-5)
