@@ -130,7 +130,7 @@ size_t b2_copy_at(const Lat& L, int32_t prec) {
 size_t b2_region_bytes(const Lat& L, int32_t prec) {
     const int f32 = prec == FLUE_F32;
     if (!magnetic_rect_ok(L, prec)) return b2_slot_bytes(L, f32);
-    return b2_copy_at(L, prec) + (size_t)36 * L.V * (f32 ? 4 : 8);
+    return b2_copy_at(L, prec) + (size_t)36 * L.V * (f32 ? 4 : 8) + 256;  // (and its flag)
 }
 
 // the B^2 adjoint after the SU(3) check: clover sums into the start of `work` (rectangle-first

@@ -184,7 +184,8 @@ hipError_t launch_ens_finalize(const EnsEntry* tab, const EnsRect* rect, int n, 
 // the magnetic B of every configuration on rectangle-first tiles (k_rect.hip).  ens_rect_plan fills
 // the table where the ensemble takes that form, and is false where it keeps launch_ens_sum; field c's
 // copy lies at its field offset in `copy` (a buffer of the ensemble's size), its footprints at 2/3 of
-// that in `fp` (48 reals a site); one partial per tile (EnsRectGrid::tiles).
+// that in `fp` (48 reals a site); one partial per tile (EnsRectGrid::tiles)
+// and the word behind them.
 struct EnsRectGrid {
     uint32_t tiles, copies;
     bool square;

@@ -14,6 +14,9 @@
 // chain products, 14 AH closings and 6 conjugations, against 74 products and 28 closings for
 // the four quadrants of quadrant() with shared lines.  (Reversing the orientation of a plane
 // negates every F, so B, a sum of |F|^2, may use either.)
+//
+// The leaves at x + a d1 and x + b d2 take V^+ for V^-1, so they are exact for unitary links only.
+// Links that nobody declared unitary are tested on the way: every link is V1 or V3 of some site.
 #pragma once
 #include "flue_clover.hpp"
 
@@ -68,6 +71,36 @@ __device__ __forceinline__ void ah_add(AH<R>& h, const AH<R>& g) {
     }
 }
 
+// whether M M^+ = 1 to 1e-13, in the sum of the entries' deviations (rounded SU(3) links are at
+// some 1e-15, and a leaf moved along three links that pass is right to 1e-12; NaN does not pass)
+template <typename R>
+__device__ __forceinline__ bool unitary(const Mat<R>& M) {
+    R dev = R(0);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        R n = R(-1);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            n = fmad(M.r[a * 3 + k], M.r[a * 3 + k], n);
+            n = fmad(M.i[a * 3 + k], M.i[a * 3 + k], n);
+        }
+        dev += n < R(0) ? -n : n;
+#pragma unroll
+        for (int b = 0; b < a; ++b) {
+            R xr = R(0), xi = R(0);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                xr = fmad(M.r[a * 3 + k], M.r[b * 3 + k], xr);
+                xr = fmad(M.i[a * 3 + k], M.i[b * 3 + k], xr);
+                xi = fmad(M.i[a * 3 + k], M.r[b * 3 + k], xi);
+                xi = fmad(-M.r[a * 3 + k], M.i[b * 3 + k], xi);
+            }
+            dev += (xr < R(0) ? -xr : xr) + (xi < R(0) ? -xi : xi);
+        }
+    }
+    return dev <= R(1e-13);
+}
+
 // One rectangle closed at both ends of its diagonal: the weighted AH part of the leaf at x
 // (W = CA CB^+) goes to h0 and to the two groups it belongs to; the weighted leaf at the
 // opposite corner (CB^+ CA) is returned.
@@ -90,9 +123,10 @@ __device__ __forceinline__ AH<R> rect_close(R w, const Mat<R>& CA, const Mat<R>&
 // The seven rectangles with lower-left corner x in quadrant q = (+d1, +d2).  emit(da, db, p)
 // adds the AH parts p to the site x + da d1 + db d2; the calls come in a fixed order.  With
 // LA each group of products also loads the link of the next group's first product (P), so
-// that product starts on a link in registers (for forms at one wave per SIMD).
-template <bool C2, bool LA, typename FV, typename Emit>
-__device__ __forceinline__ void rect_base(const Quad<FV>& q, Emit&& emit) {
+// that product starts on a link in registers (for forms at one wave per SIMD).  seen(l1, l2) is
+// given the links at x along d1 and d2.
+template <bool C2, bool LA, typename FV, typename Emit, typename Seen>
+__device__ __forceinline__ void rect_base(const Quad<FV>& q, Emit&& emit, Seen&& seen) {
     using R = typename FV::real;
     const R w11 = R(kK1), w22 = R(kK2), w33 = R(kK5), w12 = R(0.5 * kK3), w13 = R(0.5 * kK4);
     AH<R> h0, ga, gb1, gb2, gb3;  // leaves at x; current row a; columns b = 1, 2, 3
@@ -107,6 +141,7 @@ __device__ __forceinline__ void rect_base(const Quad<FV>& q, Emit&& emit) {
     Mat<R> CA = ext<1, 2, 1, 0, C2>(q, L1);            // CA(1,1)
     const Mat<R> Ld1 = first_link<1, 2, 0, 0>(q);  // Line(x,d2,1)
     Mat<R> CB1 = ext<1, 1, 0, 1, C2>(q, Ld1);          // CB(1,1)
+    seen(L1, Ld1);
     if constexpr (LA) P = ext_link<1, 2, 1, 1>(q);
     emit(1, 1, rect_close<C2>(w11, CA, CB1, h0, ga, gb1));
     FLUE_SCHED_FENCE();

@@ -79,9 +79,13 @@ constexpr int kTileStride = W ? (W + 3) * (W + 3) : kMaxCells<R>;
 // WPE == 1 (FP64) takes the chains with a one-link lookahead (rect_base); at two waves per
 // SIMD (FP32) the other wave covers the load latency.  W > 0: every tile is W x W, so its rows and
 // footprint strides are constants (48^3x96: 5.44 -> 5.35 ms in FP32, 10.2 -> 9.9 ms in FP64).
-template <bool C2, int WPE, int W, typename FV>
+// CHECK: sets *bad where a link is not unitary, testing the one along d2 of every site, and with
+// both_dirs the one along d1 (plane (x,y) tests x and y, plane (x,z) z).  The test costs 2% on 24^3x48
+// (0.73 -> 0.75 ms) and nothing that shows on 48^3x96 (11.4 ms).
+template <bool C2, int WPE, int W, bool CHECK, typename FV>
 __device__ __forceinline__ void rect_tile(const Lat L, const FV f, int rp, const PlaneTiles g, uint32_t tile,
-                                          typename FV::real* fp, typename FV::real* __restrict__ out) {
+                                          typename FV::real* fp, typename FV::real* __restrict__ out,
+                                          bool both_dirs, uint32_t* bad) {
     using R = typename FV::real;
     constexpr int CR = kCellReals<R>;
     constexpr int FS = kTileStride<R, W>;
@@ -89,6 +93,7 @@ __device__ __forceinline__ void rect_tile(const Lat L, const FV f, int rp, const
     const Tile t = tile_at(L, rp, g, tile);
     const int fc = W ? FS : (int)g.fc, f1 = W ? W + 3 : (int)g.f;
     const uint32_t w = W ? (uint32_t)W : t.l1, h = W ? (uint32_t)W : t.l2;
+    bool ok = true;
     for (int k = threadIdx.x; k < (CR == 12 ? CR * fc : CR * FS); k += kRW) fp[k] = R(0);
     __syncthreads();
 #pragma unroll 1
@@ -105,26 +110,39 @@ __device__ __forceinline__ void rect_tile(const Lat L, const FV f, int rp, const
         const int cell = ly * f1 + lx;
         rect_base<C2, WPE == 1>(make_quad<1, 1, true>(pg), [&](int da, int db, const AH<R>& p) {
             fp_add<FS>(fp, cell + db * f1 + da, p);
+        }, [&](const Mat<R>& l1, const Mat<R>& l2) {
+            if constexpr (CHECK) {
+                ok = ok && unitary(l2);
+                if (both_dirs) ok = ok && unitary(l1);
+            }
         });
     }
+    if (CHECK && !ok) __hip_atomic_store(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     for (int c = threadIdx.x; c < fc; c += kRW)
 #pragma unroll
         for (int e = 0; e < 9; ++e) out[e * fc + c] = fp[CR == 12 ? c * 12 + e : e * FS + c];
 }
 
-template <typename FV, bool C2, int WPE, int W>
+// what an earlier tile found; read for speed alone, so a stale value is as good
+template <bool CHECK>
+__device__ __forceinline__ bool given_up(const uint32_t* bad) {
+    return CHECK && __builtin_amdgcn_readfirstlane(__hip_atomic_load(bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+
+template <typename FV, bool C2, int WPE, int W, bool CHECK>
 __global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, typename FV::real* __restrict__ fpout) {
+rect_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, typename FV::real* __restrict__ fpout,
+            uint32_t* __restrict__ bad) {
     using R = typename FV::real;
     __shared__ __align__(16) R fp[kCellReals<R> * kTileStride<R, W>];
     // blockIdx.y: 0 plane (x,y), 1 plane (x,z), 2 plane (z,y) as plane (x,y) of the copy
     const bool zy = blockIdx.y == 2;
     const PlaneTiles g = plane_tiles(rt);
-    if (blockIdx.x >= g.tiles) return;
+    if (blockIdx.x >= g.tiles || given_up<CHECK>(bad)) return;
     const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
-    rect_tile<C2, WPE, W>(zy ? Lzy : L0, zy ? fzy : f0, zy ? 0 : (int)blockIdx.y, g, tile, fp,
-                          fpout + 9 * (g.cell0 + (uint64_t)tile * g.fc));
+    rect_tile<C2, WPE, W, CHECK>(zy ? Lzy : L0, zy ? fzy : f0, zy ? 0 : (int)blockIdx.y, g, tile, fp,
+                                 fpout + 9 * (g.cell0 + (uint64_t)tile * g.fc), blockIdx.y == 0, bad);
 }
 
 // the clover AH parts of tile cell (cx, cy): its own footprint's cell, then the overlapping
@@ -286,8 +304,43 @@ uint32_t zy_blocks(const Lat& L) {
 }
 
 template <typename R>
-__global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __restrict__ U, R* __restrict__ P) {
+__global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __restrict__ U, R* __restrict__ P,
+                                                          uint32_t* __restrict__ bad) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
     zy_relayout(L, blockIdx.x, U, P);
+}
+
+// B of links that turned out not unitary: partials[i] of `tiles`, by quadrants, i the share of the
+// lattice's sites that starts at V i / tiles.  (Full products in the order of magnetic variant 4.)
+template <typename FV>
+__device__ __forceinline__ void general_share(const Lat& L, const FV& f, uint32_t i, uint32_t tiles,
+                                              double* __restrict__ partial) {
+    const uint32_t lo = (uint32_t)((uint64_t)L.V * i / tiles), hi = (uint32_t)((uint64_t)L.V * (i + 1) / tiles);
+    double acc = 0.0;
+    for (uint32_t s = lo + threadIdx.x; s < hi; s += kRW) {
+        int c[4];
+        site_coords(L, s, c);
+#pragma unroll 1
+        for (int p = 0; p < 3; ++p) {
+            const int mu = p == 0 ? 2 : (p == 1 ? 1 : 3), nu = p == 0 ? 1 : (p == 1 ? 3 : 2);
+            acc += f_norm2(plane_ah<false, true, false, true>(plane_geom(L, f, s, c[mu], c[nu], mu, nu)));
+        }
+    }
+    const DD r = block_sum<kRW>(DD{acc, 0.0});
+    if (threadIdx.x == 0) {
+        partial[0] = r.hi;
+        partial[1] = r.lo;
+    }
+    __syncthreads();  // block_sum's shared slots serve the next share
+}
+
+// workgroups that look whether there is anything to do: those resident at once
+constexpr uint32_t kGeneralGrid = 1024;
+template <typename FV>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
+general_kernel(Lat L, FV f, uint32_t tiles, const uint32_t* __restrict__ bad, double* __restrict__ partials) {
+    if (!*bad) return;
+    for (uint32_t i = blockIdx.x; i < tiles; i += gridDim.x) general_share(L, f, i, tiles, partials + 2 * i);
 }
 
 // the copy read as a field of Lzy whose directions 1 and 2 are its two blocks (the view's base is one
@@ -330,16 +383,19 @@ __device__ __forceinline__ uint32_t rect_plane(const EnsRect& r, uint32_t& b) {
 template <typename R>
 __global__ void __launch_bounds__(256) ens_relayout_kernel(const EnsEntry* __restrict__ tab,
                                                            const EnsRect* __restrict__ rect, int n,
-                                                           const R* __restrict__ U, R* __restrict__ P) {
+                                                           const R* __restrict__ U, R* __restrict__ P,
+                                                           uint32_t* __restrict__ bad) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
     const int c = rect_cfg<&EnsRect::copy0>(rect, n, blockIdx.x);
     const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
     zy_relayout(e.L, blockIdx.x - rect[c].copy0, U + e.off, P + e.off);
 }
 
-template <typename R, bool C2, int WPE, int W>
+template <typename R, bool C2, int WPE, int W, bool CHECK>
 __global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 ens_rect_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ rect, int n, const R* __restrict__ U,
-                const R* __restrict__ P, R* __restrict__ fpout) {
+                const R* __restrict__ P, R* __restrict__ fpout, uint32_t* __restrict__ bad) {
+    if (given_up<CHECK>(bad)) return;
     __shared__ __align__(16) R fp[kCellReals<R> * kTileStride<R, W>];
     uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
     const int c = rect_cfg<&EnsRect::tile0>(rect, n, tile);
@@ -348,8 +404,21 @@ ens_rect_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ re
     const uint32_t y = rect_plane(r, tile);
     const PlaneTiles g = plane_tiles(r.rt, y);
     const FieldView<R, true> f{y == 2 ? zy_view(P + e.off, e.L.V) : U + e.off, e.L.V};
-    rect_tile<C2, WPE, W>(y == 2 ? r.Lzy : e.L, f, y == 1 ? 1 : 0, g, tile, fp,
-                          fpout + e.off / 72 * 48 + 9 * (g.cell0 + (uint64_t)tile * g.fc));
+    rect_tile<C2, WPE, W, CHECK>(y == 2 ? r.Lzy : e.L, f, y == 1 ? 1 : 0, g, tile, fp,
+                                 fpout + e.off / 72 * 48 + 9 * (g.cell0 + (uint64_t)tile * g.fc), y == 0, bad);
+}
+
+template <typename R>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
+ens_general_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ rect, int n, uint32_t tiles,
+                   const R* __restrict__ U, const uint32_t* __restrict__ bad, double* __restrict__ partials) {
+    if (!*bad) return;
+    for (uint32_t i = blockIdx.x; i < tiles; i += gridDim.x) {
+        const int c = rect_cfg<&EnsRect::tile0>(rect, n, i);
+        const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
+        const FieldView<R, true> f{U + e.off, e.L.V};
+        general_share(e.L, f, i - rect[c].tile0, rect[c].tiles, partials + 2 * i);
+    }
 }
 
 template <typename R, int W>
@@ -403,11 +472,12 @@ uint32_t rect_partials(const Lat& L, int is_f32) {
     return r.p[0].tiles + r.p[1].tiles + r.p[2].tiles;
 }
 
-// the three planes' footprints, then the z-fastest copy of U_z and U_y
+// the three planes' footprints, then the z-fastest copy of U_z and U_y and the flag of links that are
+// not unitary
 static size_t rect_copy_offset(const RectTiles& r, size_t sz) { return ((size_t)rect_cells(r) * 9 * sz + 255) & ~(size_t)255; }
 size_t rect_fp_bytes(const Lat& L, int is_f32) {
     const size_t sz = is_f32 ? 4 : 8;
-    return rect_copy_offset(rect_tiles_of(L, is_f32), sz) + (size_t)36 * L.V * sz;
+    return rect_copy_offset(rect_tiles_of(L, is_f32), sz) + (size_t)36 * L.V * sz + 256;
 }
 
 size_t rect_footprint_bytes(const Lat& L, int is_f32) { return rect_copy_offset(rect_tiles_of(L, is_f32), is_f32 ? 4 : 8); }
@@ -426,19 +496,22 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
         if constexpr (F::buffered) {
             R* fp = (R*)fpbuf;
             R* P = (R*)((char*)fpbuf + (copy_at ? copy_at : rect_copy_offset(rt, sizeof(R))));
-            zy_relayout_kernel<R><<<zy_blocks(L), 256, 0, st>>>(L, f.p, P);
+            uint32_t* bad = (uint32_t*)(P + (size_t)36 * L.V);
+            zy_relayout_kernel<R><<<zy_blocks(L), 256, 0, st>>>(L, f.p, P, bad);
             const F fzy{zy_view<R>(P, L.V), L.V};
             const dim3 g(std::max({rt.p[0].tiles, rt.p[1].tiles, rt.p[2].tiles}), 3);
-            // FP32 and declared-SU(3) FP64 links: two-row chains; plain FP64: full products
+            // FP32 and declared-SU(3) FP64 links: two-row chains; plain FP64: full products, and the
+            // quadrant sums for links that are not unitary
+            const bool check = sizeof(R) == 8 && !su3;
             auto rect = [&](auto w) {
                 constexpr int W = decltype(w)::value;
                 if constexpr (sizeof(R) == 4) {
-                    rect_kernel<F, true, 2, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
+                    rect_kernel<F, true, 2, W, false><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp, bad);
                 } else {
                     if (su3)
-                        rect_kernel<F, true, 1, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
+                        rect_kernel<F, true, 1, W, false><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp, bad);
                     else
-                        rect_kernel<F, false, 1, W><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp);
+                        rect_kernel<F, false, 1, W, true><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp, bad);
                 }
                 if (Abuf && tiled)
                     rect_gather_kernel<R, Store::kTiles, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
@@ -451,6 +524,10 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
                 rect(std::integral_constant<int, 16>());
             else
                 rect(std::integral_constant<int, 0>());
+            if constexpr (sizeof(R) == 8)
+                if (check && !Abuf)
+                    general_kernel<<<std::min(kGeneralGrid, rect_partials(L, is_f32)), kRW, 0, st>>>(
+                        L, f, rect_partials(L, is_f32), bad, partials);
         }
     });
     if (npart) *npart = rect_partials(L, is_f32);
@@ -491,14 +568,18 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
 
 hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, const EnsRectGrid& g, const void* fld,
                            int is_f32, void* copy, void* fp, double* partials, hipStream_t st) {
+    uint32_t* bad = (uint32_t*)(partials + 2 * (size_t)g.tiles);
     auto run = [&](auto real, auto w) {
         using R = decltype(real);
         constexpr int W = decltype(w)::value;
         constexpr bool F32 = sizeof(R) == 4;  // FP32: two-row chains, two waves per SIMD
-        ens_relayout_kernel<R><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy);
-        ens_rect_kernel<R, F32, F32 ? 2 : 1, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fld, (const R*)copy,
-                                                                         (R*)fp);
+        ens_relayout_kernel<R><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy, bad);
+        ens_rect_kernel<R, F32, F32 ? 2 : 1, W, !F32>
+            <<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fld, (const R*)copy, (R*)fp, bad);
         ens_gather_kernel<R, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fp, partials);
+        if constexpr (!F32)  // links that are not unitary
+            ens_general_kernel<R><<<std::min(kGeneralGrid, g.tiles), kRW, 0, st>>>(tab, rect, n, g.tiles, (const R*)fld,
+                                                                                   bad, partials);
     };
     auto sized = [&](auto real) {
         if (g.square)

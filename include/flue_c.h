@@ -283,7 +283,9 @@ int flue_magnetic(const int32_t dims[4], const void* U, int32_t prec, double* d_
  *         orders), 1..3 waves per SIMD;
  *   7     rectangle-first: each rectangle of the clover is formed once and its leaves at
  *         the other three corners follow by conjugation (plane (z,y) from a z-fastest copy
- *         of its links).  It needs NX, NY, NZ divisible by 16, or of 12 or more on a
+ *         of its links).  That holds for unitary links: those of a FLUE_F64 field are
+ *         tested on the way, and B comes from the quadrants if one is not unitary to 1e-13.
+ *         It needs NX, NY, NZ divisible by 16, or of 12 or more on a
  *         lattice of 90,000 sites or more, and a workspace of
  *         flue_magnetic_work_bytes (about 300 bytes per site in FP32, 600 in FP64);
  *         otherwise the call runs the default form instead.

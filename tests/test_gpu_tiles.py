@@ -45,3 +45,37 @@ def test_adjoint_uneven_extents(FL, dims):
     for g, tol in ((f, 1e-12), (f.astype("fp32"), 1e-5)):
         for v in (1, 2):
             assert np.abs(g.magnetic_grad(variant=v).to_complex().cpu().numpy() - Go).max() < tol * scale, v
+
+
+@pytest.mark.parametrize("mu", [1, 2, 3])
+@pytest.mark.parametrize("kind", ["scaled", "sheared"])
+@pytest.mark.parametrize("dims", [(3, 16, 16, 32), (11, 20, 21, 23)])
+def test_magnetic_of_links_that_are_not_unitary(FL, dims, kind, mu):
+    # FP64 makes no assumption on the links: one link of one direction that is not unitary, in the last
+    # tile, and B is that of the quadrant form.  (Both forms add the same leaves: 1e-12.)
+    f = FL.GaugeField.random(dims, 5, 0.3, "fp64")
+    U = f.to_complex()
+    if kind == "scaled":
+        U[-1, -1, -1, -1, mu] *= 1.5
+    else:
+        U[-1, -1, -1, -1, mu, 0] += 0.5 * U[-1, -1, -1, -1, mu, 1]
+    g = FL.GaugeField.from_complex(U)
+    ref = g.magnetic(variant=1)
+    assert abs(ref - f.magnetic(variant=1)) > 1e-9 * ref
+    for v in (0, 7):
+        assert abs(g.magnetic(variant=v) - ref) < 1e-12 * ref
+    assert abs(f.magnetic() - f.magnetic(variant=1)) < 1e-12 * ref   # (the workspace again, clean links)
+
+
+@pytest.mark.parametrize("mu", [1, 2, 3])
+def test_ensemble_of_links_that_are_not_unitary(FL, mu):
+    from flue_lat_amd.ensemble import Ensemble
+    dims = [(4, 16, 16, 32), (11, 17, 13, 21), (5, 20, 20, 20)]
+    e = Ensemble.random(dims, [1, 2, 3], 0.3, "fp64")
+    U = e.field(1).to_complex()
+    U[-1, -1, -1, -1, mu] *= 1.5
+    e.field(1).data.copy_(FL.GaugeField.from_complex(U).data)
+    ref = [e.field(c).magnetic(variant=1) for c in range(3)]
+    _, B = e.flow(0.01, 0, measure_every=1)
+    for c in range(3):
+        assert abs(B[0, c] - ref[c]) < 1e-12 * ref[c]
