@@ -147,7 +147,8 @@ fmunu_kernel(Lat L, FV f, int mu, int nu, void* __restrict__ out, int layout, Ou
     }
     int c[4];
     site_coords(L, s, c);
-    const AH<R> h = plane_ah<CLOVER, sizeof(R) == 4, sizeof(R) == 4>(plane_geom(L, f, s, c[mu], c[nu], mu, nu));
+    // FP32 carries two rows, FP64 (one wave per SIMD) loads a link ahead
+    const AH<R> h = plane_ah<CLOVER, true, sizeof(R) == 4, sizeof(R) == 8>(plane_geom(L, f, s, c[mu], c[nu], mu, nu));
     // F = A^T / 4: F_aa = i d_a / 4, F_ab = -conj(o_ab)/8, F_ba = o_ab/8 (a < b)
     R fr[9], fi[9];
     constexpr int pa[3] = {0, 0, 1}, pb[3] = {1, 2, 2};
