@@ -77,6 +77,8 @@ SIGNATURES = {
     "flue_generic_path": [_P, _P, _I, _P, _P, _I, _P, _P],
     "flue_wilson_loops": [_P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _SZ, _P],
     "flue_wilson_loops_slices": [_P, _P, _I, _I, _I, _I, _I, _P, _P, _SZ, _P],
+    "flue_fmunu_work_bytes": [_P, _I, _I, _I],
+    "flue_fmunu_ex": [_P, _P, _I, _I, _I, _I, _P, _I, _P, _P, _SZ, _P],
     "flue_fmunu": [_P, _P, _I, _I, _I, _I, _P, _I, _P, _P],
     "flue_gluon_prop_mom": [_P, _P, _I, _P, _I, _D, _P, _P, _P, _P],
     "flue_scalar_gluon_prop": [_P, _P, _I, _P, _P],
@@ -108,7 +110,8 @@ SIGNATURES = {
 _RESTYPE = {"flue_strerror": ctypes.c_char_p, "flue_field_bytes": _SZ, "flue_workspace_bytes": _SZ,
             "flue_b2_work_bytes": _SZ, "flue_flow_work_bytes": _SZ, "flue_ensemble_field_bytes": _SZ,
             "flue_ensemble_work_bytes": _SZ, "flue_autotune_work_bytes": _SZ,
-            "flue_pf_work_bytes": _SZ, "flue_magnetic_work_bytes": _SZ}
+            "flue_pf_work_bytes": _SZ, "flue_magnetic_work_bytes": _SZ,
+            "flue_fmunu_work_bytes": _SZ}
 
 
 def lib():

@@ -642,6 +642,16 @@ int flue_generic_path(const int32_t dims[4], const void* U, int32_t prec, const 
 
 int flue_fmunu(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, int32_t nu, int32_t variant, void* out,
                int32_t layout, const int64_t strides[6], void* stream) {
+    return flue_fmunu_ex(dims, U, prec, mu, nu, variant, out, layout, strides, nullptr, 0, stream);
+}
+
+size_t flue_fmunu_work_bytes(const int32_t dims[4], int32_t prec, int32_t mu, int32_t nu) {
+    if (check_dims(dims) || check_prec(prec) || mu < 1 || mu > 4 || nu < 1 || nu > 4) return 0;
+    return fmunu_rect_bytes(make_lat(dims), prec == FLUE_F32, mu - 1, nu - 1);
+}
+
+int flue_fmunu_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, int32_t nu, int32_t variant, void* out,
+                  int32_t layout, const int64_t strides[6], void* ws, size_t ws_bytes, void* stream) {
     int rc = check_dims(dims);
     if (rc) return rc;
     if (!U || !out) return FLUE_ENULL;
@@ -649,8 +659,14 @@ int flue_fmunu(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, i
         return FLUE_EINVAL;
     if (layout != FLUE_OUT_STRIDED && layout != FLUE_OUT_SOA) return FLUE_EINVAL;
     if (layout == FLUE_OUT_STRIDED && !strides) return FLUE_ENULL;
-    return hip_status(launch_fmunu(make_lat(dims), U, prec == FLUE_F32, mu - 1, nu - 1, variant, out,
-                                   layout == FLUE_OUT_SOA, strides, S(stream)));
+    const Lat L = make_lat(dims);
+    const int f32 = prec == FLUE_F32;
+    const size_t need = ws && variant == 0 && layout == FLUE_OUT_STRIDED && strides[0] == 1
+                            ? fmunu_rect_bytes(L, f32, mu - 1, nu - 1)
+                            : 0;
+    if (need && ws_bytes >= need)
+        return hip_status(launch_fmunu_rect(L, U, f32, mu - 1, nu - 1, out, strides, ws, S(stream)));
+    return hip_status(launch_fmunu(L, U, f32, mu - 1, nu - 1, variant, out, layout == FLUE_OUT_SOA, strides, S(stream)));
 }
 
 int flue_gluon_prop_mom(const int32_t dims[4], const void* Uq, int32_t prec, const int64_t qstrides[4],

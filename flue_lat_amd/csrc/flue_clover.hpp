@@ -570,6 +570,44 @@ __device__ __forceinline__ AH<typename FV::real> plane_ah(const PlaneGeom<FV>& g
     return h;
 }
 
+// F = A^T / 4 of the accumulated anti-Hermitian part: F_aa = i d_a / 4, F_ab = -conj(o_ab)/8,
+// F_ba = o_ab/8 (a < b); element (a, b) at a * 3 + b
+template <typename R>
+__device__ __forceinline__ void f_entries(const AH<R>& h, R fr[9], R fi[9]) {
+    constexpr int pa[3] = {0, 0, 1}, pb[3] = {1, 2, 2};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        fr[k * 4] = R(0);
+        fi[k * 4] = h.d[k] * R(0.25);
+        const int a = pa[k], b = pb[k];
+        fr[a * 3 + b] = -h.or_[k] * R(0.125);
+        fi[a * 3 + b] = h.oi[k] * R(0.125);
+        fr[b * 3 + a] = h.or_[k] * R(0.125);
+        fi[b * 3 + a] = h.oi[k] * R(0.125);
+    }
+}
+
+// strides of a complex128 array (NT, NX, NY, NZ, 3, 3), in complex elements
+struct OutStrides {
+    int64_t t, x, y, z, a, b;
+};
+
+// F of the site at coordinates c into such an array
+template <typename R>
+__device__ __forceinline__ void store_f(const AH<R>& h, const int c[4], double* __restrict__ o, const OutStrides& os) {
+    R fr[9], fi[9];
+    f_entries(h, fr, fi);
+    const int64_t base = c[0] * os.t + c[1] * os.x + c[2] * os.y + c[3] * os.z;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const int64_t off = 2 * (base + a * os.a + b * os.b);
+            o[off] = (double)fr[a * 3 + b];
+            o[off + 1] = (double)fi[a * 3 + b];
+        }
+}
+
 // sum_ab |F_ab|^2 = -ReTr(F F) for F = A^T/4 with A the accumulated anti-Hermitian part
 // (FP64): |F_aa|^2 = d_a^2/16 and |F_ab|^2 + |F_ba|^2 = |o_ab|^2/32
 template <typename R>

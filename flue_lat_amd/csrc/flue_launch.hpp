@@ -52,6 +52,11 @@ hipError_t launch_finalize(const double* partials, uint32_t n, double* out, doub
 // field precision
 hipError_t launch_fmunu(const Lat& L, const void* U, int is_f32, int mu, int nu, int clover_only, void* out,
                         int out_layout, const int64_t strides[6], hipStream_t st);
+// the 5-loop F of a plane on rectangle-first tiles (k_rect.hip), into an array with stride 1 along t;
+// fmunu_rect_bytes of workspace, 0 where the plane does not take them
+size_t fmunu_rect_bytes(const Lat& L, int is_f32, int mu, int nu);
+hipError_t launch_fmunu_rect(const Lat& L, const void* U, int is_f32, int mu, int nu, void* out, const int64_t strides[6],
+                             void* ws, hipStream_t st);
 uint32_t magnetic_blocks(const Lat& L, int is_f32);
 int magnetic_default_variant(int is_f32);
 // rectangular Wilson-loop table (k_wloops.hip): R, T up to kMaxLoopRT
@@ -188,6 +193,7 @@ hipError_t launch_ens_finalize(const EnsEntry* tab, const EnsRect* rect, int n, 
 // and the word behind them.
 struct EnsRectGrid {
     uint32_t tiles, copies;
+    int copy_edge;
     bool square;
 };
 bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRect* rect, EnsRectGrid* g);

@@ -8,16 +8,20 @@
 namespace flue {
 namespace {
 
-// the second direction of rectangle plane rp (0: (x, y), 1: (x, z))
-__device__ __forceinline__ int rect_d2(int rp) { return rp == 0 ? 2 : 3; }
+// the second direction of rectangle plane rp (0: (x, y), 1: (x, z); with TIME (x, t))
+template <bool TIME = false>
+__device__ __forceinline__ int rect_d2(int rp) {
+    return TIME ? 0 : (rp == 0 ? 2 : 3);
+}
 
 struct Tile {
-    uint32_t t1, t2, cs, ct;  // tile along x, tile along d2, spectator coordinate, t
+    uint32_t t1, t2, cs, ct;  // tile along x, tile along d2, spectator coordinates (z or y and t; TIME: y and z)
     uint32_t o1, o2, l1, l2;  // first site and extent along x and d2
 };
 
+template <bool TIME = false>
 __device__ __forceinline__ Tile tile_at(const Lat& L, int rp, const PlaneTiles& g, uint32_t tile) {
-    const uint32_t ns = (uint32_t)L.n[rp == 0 ? 3 : 2];
+    const uint32_t ns = (uint32_t)L.n[!TIME && rp == 0 ? 3 : 2];
     Tile t;
     t.t1 = tile % g.n1;
     uint32_t q = tile / g.n1;
@@ -29,6 +33,21 @@ __device__ __forceinline__ Tile tile_at(const Lat& L, int rp, const PlaneTiles& 
     t.o2 = t.t2 * g.q2 + min(t.t2, g.r2);
     t.l1 = g.q1 + (t.t1 < g.r1 ? 1u : 0u);
     t.l2 = g.q2 + (t.t2 < g.r2 ? 1u : 0u);
+    return t;
+}
+
+// the site at x, second-direction coordinate c2 and the spectators of a tile
+template <bool TIME = false>
+__device__ __forceinline__ uint32_t tile_site(const Lat& L, int rp, uint32_t x, uint32_t c2, const Tile& t) {
+    if (TIME) return x + L.st[2] * t.cs + L.st[3] * t.ct + L.st[0] * c2;
+    return x + L.st[2] * (rp == 0 ? c2 : t.cs) + L.st[3] * (rp == 0 ? t.cs : c2) + L.st[0] * t.ct;
+}
+
+// the tile of N sites split as (q, r) that holds site c, and its first site
+__device__ __forceinline__ uint32_t tile_of(uint32_t c, uint32_t q, uint32_t r, uint32_t* first) {
+    const uint32_t wide = r * (q + 1);
+    const uint32_t t = c < wide ? c / (q + 1) : r + (c - wide) / q;
+    *first = t * q + min(t, r);
     return t;
 }
 
@@ -50,9 +69,10 @@ Lat zy_lattice(const Lat& L) {
 // The rounds are counted for kNominalNT time slices whatever the lattice has: the split sets the
 // order in which a site's rectangles are added, and a field repeated along t gives the same B.
 // Every tile is at least 4 sites wide (rect_fits), so a footprint's three extra rows and columns
-// reach into one further tile only.
+// reach into one further tile only.  (A launch over one plane counts its own slices.)
 constexpr uint32_t kNominalNT = 32, kMaxTileEdge = 32;
-PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint32_t max_cells, uint32_t slots) {
+PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint32_t max_cells, uint32_t slots,
+                       double slices = 3.0 * kNominalNT) {
     PlaneTiles best{};
     double time = 0.0;
     uint64_t cells = 0;
@@ -66,7 +86,7 @@ PlaneTiles plane_split(uint32_t N1, uint32_t N2, uint32_t N3, uint32_t NT, uint3
             // (16 x 16 tiles have kernels of their own: they win ties)
             const bool sq = N1 == 16 * n1 && N2 == 16 * n2;
             const uint64_t cn = sq ? 0 : (uint64_t)n1 * n2 * fc;
-            const double rounds = 3.0 * n1 * n2 * (double)N3 * kNominalNT / slots;
+            const double rounds = slices * n1 * n2 * (double)N3 / slots;
             const double tm = (double)((l1 * l2 + 63) / 64) * (rounds < 8.0 ? std::ceil(rounds) : rounds);
             if (time == 0.0 || tm < time || (tm == time && cn < cells)) {
                 time = tm;

@@ -117,10 +117,6 @@ magnetic_kernel(Lat L, FV f, PlaneOrder po, uint32_t nb, double* __restrict__ pa
     }
 }
 
-struct OutStrides {
-    int64_t t, x, y, z, a, b;
-};
-
 // per-site F for one plane.  layout 0: complex128 at the given strides; layout 1: SoA
 // planes (element e = a*3+b, re/im) in the field precision.
 template <typename FV, bool CLOVER>
@@ -149,31 +145,11 @@ fmunu_kernel(Lat L, FV f, int mu, int nu, void* __restrict__ out, int layout, Ou
     site_coords(L, s, c);
     // FP32 carries two rows, FP64 (one wave per SIMD) loads a link ahead
     const AH<R> h = plane_ah<CLOVER, true, sizeof(R) == 4, sizeof(R) == 8>(plane_geom(L, f, s, c[mu], c[nu], mu, nu));
-    // F = A^T / 4: F_aa = i d_a / 4, F_ab = -conj(o_ab)/8, F_ba = o_ab/8 (a < b)
-    R fr[9], fi[9];
-    constexpr int pa[3] = {0, 0, 1}, pb[3] = {1, 2, 2};
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        fr[k * 4] = R(0);
-        fi[k * 4] = h.d[k] * R(0.25);
-        const int a = pa[k], b = pb[k];
-        fr[a * 3 + b] = -h.or_[k] * R(0.125);
-        fi[a * 3 + b] = h.oi[k] * R(0.125);
-        fr[b * 3 + a] = h.or_[k] * R(0.125);
-        fi[b * 3 + a] = h.oi[k] * R(0.125);
-    }
     if (layout == 0) {
-        double* o = (double*)out;
-        const int64_t base = c[0] * os.t + c[1] * os.x + c[2] * os.y + c[3] * os.z;
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int b = 0; b < 3; ++b) {
-                const int64_t off = 2 * (base + a * os.a + b * os.b);
-                o[off] = (double)fr[a * 3 + b];
-                o[off + 1] = (double)fi[a * 3 + b];
-            }
+        store_f(h, c, (double*)out, os);
     } else {
+        R fr[9], fi[9];
+        f_entries(h, fr, fi);
         R* o = (R*)out;
 #pragma unroll
         for (int e = 0; e < 9; ++e) {

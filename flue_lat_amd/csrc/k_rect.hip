@@ -82,15 +82,15 @@ constexpr int kTileStride = W ? (W + 3) * (W + 3) : kMaxCells<R>;
 // CHECK: sets *bad where a link is not unitary, testing the one along d2 of every site, and with
 // both_dirs the one along d1 (plane (x,y) tests x and y, plane (x,z) z).  The test costs 2% on 24^3x48
 // (0.73 -> 0.75 ms) and nothing that shows on 48^3x96 (11.4 ms).
-template <bool C2, int WPE, int W, bool CHECK, typename FV>
+template <bool C2, int WPE, int W, bool CHECK, bool TIME = false, typename FV>
 __device__ __forceinline__ void rect_tile(const Lat L, const FV f, int rp, const PlaneTiles g, uint32_t tile,
                                           typename FV::real* fp, typename FV::real* __restrict__ out,
                                           bool both_dirs, uint32_t* bad) {
     using R = typename FV::real;
     constexpr int CR = kCellReals<R>;
     constexpr int FS = kTileStride<R, W>;
-    const int d2 = rect_d2(rp);
-    const Tile t = tile_at(L, rp, g, tile);
+    const int d2 = rect_d2<TIME>(rp);
+    const Tile t = tile_at<TIME>(L, rp, g, tile);
     const int fc = W ? FS : (int)g.fc, f1 = W ? W + 3 : (int)g.f;
     const uint32_t w = W ? (uint32_t)W : t.l1, h = W ? (uint32_t)W : t.l2;
     bool ok = true;
@@ -104,8 +104,7 @@ __device__ __forceinline__ void rect_tile(const Lat L, const FV f, int rp, const
         const int ly = W ? (int)(j0 / w + threadIdx.x / w) : (int)(j / w);
         const int lx = W ? (int)(threadIdx.x % w) : (int)(j - (uint32_t)ly * w);
         const int cx = (int)t.o1 + lx, c2 = (int)t.o2 + ly;
-        const int cy = rp == 0 ? c2 : (int)t.cs, cz = rp == 0 ? (int)t.cs : c2;
-        const uint32_t s = (uint32_t)cx + L.st[2] * (uint32_t)cy + L.st[3] * (uint32_t)cz + L.st[0] * t.ct;
+        const uint32_t s = tile_site<TIME>(L, rp, (uint32_t)cx, (uint32_t)c2, t);
         const PlaneGeom<FV> pg = plane_geom(L, f, s, cx, c2, 1, d2);
         const int cell = ly * f1 + lx;
         rect_base<C2, WPE == 1>(make_quad<1, 1, true>(pg), [&](int da, int db, const AH<R>& p) {
@@ -230,7 +229,7 @@ __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectT
     cover.sites([&](int cx, int cy, const AH<R>& h) {
         if constexpr (STORE != Store::kNone) {
             const uint32_t c2 = t.o2 + (uint32_t)cy, c1 = t.o1 + (uint32_t)cx;
-            uint32_t s = c1 + L.st[2] * (rp == 0 ? c2 : t.cs) + L.st[3] * (rp == 0 ? t.cs : c2) + L.st[0] * t.ct;
+            uint32_t s = tile_site(L, rp, c1, c2, t);
             R sg = R(1);
             if constexpr (STORE == Store::kSites) {
                 // the copy's x', y', z' are z, y, x; plane (y,x) is (x,y) reversed
@@ -258,56 +257,76 @@ __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectT
     }
 }
 
-// U_z and U_y of the field (lattice L) into P, z fastest: P holds two direction blocks of
-// 9 complex planes, [k][e][s'] with s' = z + NZ (y + NY (x + NX t)), k = 0 for U_z, 1 for
-// U_y.  Block q of one per 16 x 16 (x, z) tile at fixed (y, t), through a padded LDS tile so that
-// both the reads (along x) and the writes (along z) coalesce.
-template <typename R>
-__device__ __forceinline__ void zy_relayout(const Lat& L, uint32_t q, const R* __restrict__ U, R* __restrict__ P) {
+// U_mu0 and U_mu1 of the field (lattice L) into P with direction a (y or z) fastest: P holds two
+// blocks of 9 complex planes, [k][e][s'] with k = 0 for U_mu0, 1 for U_mu1, and s' as in L with a and x
+// exchanged.  Blocks of 256 threads take T x T (x, a) tiles at fixed other coordinates, through LDS so
+// that both the reads (along x) and the writes (along a) coalesce, nine planes in flight: one 16 x 16
+// tile, or four 8 x 8 ones where those cover the extents with less padding.
+template <typename R, int T>
+__device__ __forceinline__ void relayout(const Lat& L, int a, int mu0, int mu1, uint32_t blk, const R* __restrict__ U,
+                                         R* __restrict__ P) {
     using P2 = typename Pair2<R>::type;
-    __shared__ P2 tile[16][17];
-    const uint32_t NX = (uint32_t)L.n[1], NY = (uint32_t)L.n[2], NZ = (uint32_t)L.n[3];
-    const uint32_t bxs = (NX + 15) / 16, bzs = (NZ + 15) / 16;
+    constexpr int NT2 = 256 / (T * T);  // tiles per block
+    __shared__ P2 tile[NT2][9][T][T + 1];
+    const uint32_t NX = (uint32_t)L.n[1], NA = (uint32_t)L.n[a], NO = (uint32_t)L.n[5 - a];
+    const uint32_t bxs = (NX + T - 1) / T, bas = (NA + T - 1) / T;
+    const uint32_t n = threadIdx.x / (T * T), i = threadIdx.x / T % T, j = threadIdx.x % T;
+    uint32_t q = blk * NT2 + n;
+    const bool any = q < bxs * bas * NO * (uint32_t)L.n[0];
     const uint32_t bx = q % bxs;
     q /= bxs;
-    const uint32_t bz = q % bzs;
-    q /= bzs;
-    const uint32_t y = q % NY, t = q / NY;
-    const uint32_t i = threadIdx.x >> 4, j = threadIdx.x & 15;
-    const uint32_t s = bx * 16 + j + NX * (y + NY * (bz * 16 + i + NZ * t));
-    const uint32_t s2 = bz * 16 + j + NZ * (y + NY * (bx * 16 + i + NX * t));
-    const bool rd = bx * 16 + j < NX && bz * 16 + i < NZ, wr = bz * 16 + j < NZ && bx * 16 + i < NX;
+    const uint32_t ba = q % bas;
+    q /= bas;
+    const uint32_t o = q % NO, t = q / NO;
+    const uint32_t s = bx * T + j + L.st[a] * (ba * T + i) + L.st[5 - a] * o + L.st[0] * t;
+    // (with a and x exchanged: x has the stride of a, the other direction that of the exchanged extents)
+    const uint32_t dx = a == 3 ? NA * NO : NA, d_o = a == 3 ? NA : NA * NX;
+    const uint32_t s2 = ba * T + j + dx * (bx * T + i) + d_o * o + L.st[0] * t;
+    const bool rd = any && bx * T + j < NX && ba * T + i < NA, wr = any && ba * T + j < NA && bx * T + i < NX;
     const P2* src = reinterpret_cast<const P2*>(U);
-    P2* dst = reinterpret_cast<P2*>(P);
+    typedef R r2 __attribute__((ext_vector_type(2)));
+    r2* dst = reinterpret_cast<r2*>(P);
 #pragma unroll 1
     for (int k = 0; k < 2; ++k) {
-        const int mu = k == 0 ? 3 : 2;
-#pragma unroll 1
-        for (int e = 0; e < 9; ++e) {
-            if (rd) tile[i][j] = src[(size_t)(mu * 9 + e) * L.V + s];
-            __syncthreads();
-            if (wr) {
-                typedef R r2 __attribute__((ext_vector_type(2)));
-                const P2 v = tile[j][i];
+        const int mu = k == 0 ? mu0 : mu1;
+        if (rd) {
+            P2 v[9];
+#pragma unroll
+            for (int e = 0; e < 9; ++e) v[e] = src[(size_t)(mu * 9 + e) * L.V + s];
+#pragma unroll
+            for (int e = 0; e < 9; ++e) tile[n][e][i][j] = v[e];
+        }
+        __syncthreads();
+        if (wr) {
+#pragma unroll
+            for (int e = 0; e < 9; ++e) {
+                const P2 v = tile[n][e][j][i];
                 r2 w;
                 w.x = v.x;
                 w.y = v.y;
-                st_stream(reinterpret_cast<r2*>(dst) + (size_t)(k * 9 + e) * L.V + s2, w);
+                st_stream(dst + (size_t)(k * 9 + e) * L.V + s2, w);
             }
-            __syncthreads();
         }
+        __syncthreads();
     }
 }
 
-uint32_t zy_blocks(const Lat& L) {
-    return (uint32_t)((L.n[1] + 15) / 16) * (uint32_t)((L.n[3] + 15) / 16) * (uint32_t)L.n[2] * (uint32_t)L.n[0];
+// the tile edge for (x, a): 8 where its tiles cover a tenth less than those of 16
+int relayout_edge(const Lat& L, int a) {
+    auto covered = [&](uint64_t T) { return ((L.n[1] + T - 1) / T) * ((L.n[a] + T - 1) / T) * T * T; };
+    return 10 * covered(8) <= 9 * covered(16) ? 8 : 16;
+}
+uint32_t relayout_blocks(const Lat& L, int a, int T) {
+    const uint64_t n = (uint64_t)((L.n[1] + T - 1) / T) * (uint64_t)((L.n[a] + T - 1) / T) * (uint64_t)L.n[5 - a] *
+                       (uint64_t)L.n[0];
+    return (uint32_t)(T == 8 ? (n + 3) / 4 : n);
 }
 
-template <typename R>
+template <typename R, int T>
 __global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __restrict__ U, R* __restrict__ P,
                                                           uint32_t* __restrict__ bad) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
-    zy_relayout(L, blockIdx.x, U, P);
+    relayout<R, T>(L, 3, 3, 2, blockIdx.x, U, P);
 }
 
 // B of links that turned out not unitary: partials[i] of `tiles`, by quadrants, i the share of the
@@ -380,7 +399,7 @@ __device__ __forceinline__ uint32_t rect_plane(const EnsRect& r, uint32_t& b) {
     return 2;
 }
 
-template <typename R>
+template <typename R, int T>
 __global__ void __launch_bounds__(256) ens_relayout_kernel(const EnsEntry* __restrict__ tab,
                                                            const EnsRect* __restrict__ rect, int n,
                                                            const R* __restrict__ U, R* __restrict__ P,
@@ -388,7 +407,7 @@ __global__ void __launch_bounds__(256) ens_relayout_kernel(const EnsEntry* __res
     if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
     const int c = rect_cfg<&EnsRect::copy0>(rect, n, blockIdx.x);
     const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
-    zy_relayout(e.L, blockIdx.x - rect[c].copy0, U + e.off, P + e.off);
+    relayout<R, T>(e.L, 3, 3, 2, blockIdx.x - rect[c].copy0, U + e.off, P + e.off);
 }
 
 template <typename R, bool C2, int WPE, int W, bool CHECK>
@@ -444,6 +463,107 @@ __global__ void __launch_bounds__(kRW) ens_gather_kernel(const EnsEntry* __restr
     }
 }
 
+// ---- one plane's field strength, per site.  A plane with x runs on the field; (z, y), (z, t) and
+// (y, t) on a copy of their two links with z or y fastest, whose lattice has that extent as its x.
+// 24^3x48 in FP64, us by quadrants -> by tiles (tiles 255, gather 40 to 50, copy 80): (x,y) 512 -> 287,
+// (x,z) 447 -> 272, (x,t) 512 -> 297, (z,y) 469 -> 355, (z,t), (y,t) 452 -> 350.  The tiles run at the
+// FP64 rate of the whole form (matrix products, one wave per SIMD); one plane alone ends in a partly
+// filled last round.  FP32 carries whole rows here: 138 us against 132 with two, and an error of F of
+// 1.64e-7 (rms, of F's) against 1.86e-7 with two and 1.81e-7 by quadrants.
+
+// the links of the copy, and the flag of links that are not unitary cleared (the copy's or, alone,
+// block 0's work)
+template <typename R, int T>
+__global__ void __launch_bounds__(256) plane_copy_kernel(Lat L, int a, int mu0, int mu1, const R* __restrict__ U,
+                                                         R* __restrict__ P, uint32_t* __restrict__ bad) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
+    if (P) relayout<R, T>(L, a, mu0, mu1, blockIdx.x, U, P);
+}
+
+template <typename FV, bool C2, int WPE, bool CHECK, bool TIME>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+plane_kernel(Lat L, FV f, int rp, PlaneTiles g, typename FV::real* __restrict__ fpout, uint32_t* __restrict__ bad) {
+    using R = typename FV::real;
+    __shared__ __align__(16) R fp[kCellReals<R> * kTileStride<R, 0>];
+    if (given_up<CHECK>(bad)) return;
+    const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
+    rect_tile<C2, WPE, 0, CHECK, TIME>(L, f, rp, g, tile, fp, fpout + 9 * (uint64_t)tile * g.fc, true, bad);
+}
+
+// F of every site from the footprints, in an array whose t is dense: a block has 16 x and 16 t at fixed
+// y and z, reads the footprints along x and writes along t, through LDS.  sign: that of the plane's
+// orientation; os: strides in the directions of L (its x may be the field's z or y).
+constexpr int kFT = 16;
+template <typename R, bool TIME>
+__global__ void __launch_bounds__(kFT * kFT) plane_gather_kernel(Lat L, int rp, PlaneTiles g,
+                                                               const R* __restrict__ fpin, R sign,
+                                                               double* __restrict__ out, OutStrides os) {
+    __shared__ R parts[9][kFT][kFT + 1];
+    const uint32_t nx = (uint32_t)L.n[1], nt = (uint32_t)L.n[0], ny = (uint32_t)L.n[2];
+    const uint32_t bts = (nt + kFT - 1) / kFT, bxs = (nx + kFT - 1) / kFT;
+    uint32_t q = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t t0 = (q % bts) * kFT;
+    q /= bts;
+    const uint32_t x0 = (q % bxs) * kFT;
+    q /= bxs;
+    const uint32_t y = q % ny, z = q / ny;
+    const uint32_t i = threadIdx.x % kFT, j = threadIdx.x / kFT;
+    if (x0 + i < nx && t0 + j < nt) {
+        const uint32_t c2 = TIME ? t0 + j : (rp == 0 ? y : z);
+        uint32_t o1, o2;
+        Tile t;
+        t.t1 = tile_of(x0 + i, g.q1, g.r1, &o1);
+        t.t2 = tile_of(c2, g.q2, g.r2, &o2);
+        const uint32_t cs = TIME || rp == 1 ? y : z, ct = TIME ? z : t0 + j;
+        const uint32_t ns = (uint32_t)L.n[TIME || rp == 1 ? 2 : 3];
+        const Cover<R, 0> cover(g, t, t.t1 + g.n1 * (t.t2 + g.n2 * (cs + ns * ct)), fpin);
+        const AH<R> h = cell_sum(cover.own, cover.left, cover.below, cover.diag, cover.fc, cover.f1,
+                                 (int)(x0 + i - o1), (int)(c2 - o2), cover.shift1, cover.shift2);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            parts[k][i][j] = sign * h.d[k];
+            parts[3 + k][i][j] = sign * h.or_[k];
+            parts[6 + k][i][j] = sign * h.oi[k];
+        }
+    }
+    __syncthreads();
+    // i along t, j along x
+    if (x0 + j < nx && t0 + i < nt) {
+        AH<R> h;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            h.d[k] = parts[k][j][i];
+            h.or_[k] = parts[3 + k][j][i];
+            h.oi[k] = parts[6 + k][j][i];
+        }
+        const int c[4] = {(int)(t0 + i), (int)(x0 + j), (int)y, (int)z};
+        store_f(h, c, out, os);
+    }
+}
+
+// F by quadrants, where a link turned out not unitary
+template <typename FV>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
+plane_general_kernel(Lat L, FV f, int mu, int nu, const uint32_t* __restrict__ bad, double* __restrict__ out,
+                     OutStrides os) {
+    if (!*bad) return;
+    for (uint32_t s = blockIdx.x * kRW + threadIdx.x; s < L.V; s += gridDim.x * kRW) {
+        int c[4];
+        site_coords(L, s, c);
+        store_f(plane_ah<false, true, false, true>(plane_geom(L, f, s, c[mu], c[nu], mu, nu)), c, out, os);
+    }
+}
+
+// How plane (mu, nu) is tiled: L and the plane of it, the field's directions along its x (d1) and its
+// second direction (d2), and the directions whose links are copied (mu0 < 0: none).
+struct FPlane {
+    Lat L;
+    int rp, d1, d2, mu0, mu1;
+    PlaneTiles g;
+    size_t copy_at, bytes;  // (the flag lies in front of `bytes`)
+    bool first_is_zero;     // the copy's first block is its lattice's direction 0, else 1
+};
+
 RectTiles rect_tiles_of(const Lat& L, int is_f32) {
     return rect_split(L, is_f32 ? kMaxCells<float> : kMaxCells<double>, is_f32 ? 2048 : 1024);
 }
@@ -497,7 +617,10 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
             R* fp = (R*)fpbuf;
             R* P = (R*)((char*)fpbuf + (copy_at ? copy_at : rect_copy_offset(rt, sizeof(R))));
             uint32_t* bad = (uint32_t*)(P + (size_t)36 * L.V);
-            zy_relayout_kernel<R><<<zy_blocks(L), 256, 0, st>>>(L, f.p, P, bad);
+            if (relayout_edge(L, 3) == 8)
+                zy_relayout_kernel<R, 8><<<relayout_blocks(L, 3, 8), 256, 0, st>>>(L, f.p, P, bad);
+            else
+                zy_relayout_kernel<R, 16><<<relayout_blocks(L, 3, 16), 256, 0, st>>>(L, f.p, P, bad);
             const F fzy{zy_view<R>(P, L.V), L.V};
             const dim3 g(std::max({rt.p[0].tiles, rt.p[1].tiles, rt.p[2].tiles}), 3);
             // FP32 and declared-SU(3) FP64 links: two-row chains; plain FP64: full products, and the
@@ -546,6 +669,9 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
     if (!fits_buffer(maxV, is_f32)) return false;
     uint64_t sites = 0, tiles = 0, copies = 0;
     g->square = true;
+    g->copy_edge = 16;
+    for (int c = 0; c < n; ++c)
+        if (relayout_edge(tab[c].L, 3) == 8) g->copy_edge = 8;
     for (int c = 0; c < n; ++c) {
         const Lat& L = tab[c].L;
         if (std::min({L.n[1], L.n[2], L.n[3]}) < 12) return false;
@@ -559,7 +685,7 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
         for (const PlaneTiles& p : r.rt.p) g->square = g->square && p.square();
         sites += L.V;
         tiles += r.tiles;
-        copies += zy_blocks(L);
+        copies += relayout_blocks(L, 3, g->copy_edge);
     }
     g->tiles = (uint32_t)tiles;
     g->copies = (uint32_t)copies;
@@ -573,7 +699,10 @@ hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, cons
         using R = decltype(real);
         constexpr int W = decltype(w)::value;
         constexpr bool F32 = sizeof(R) == 4;  // FP32: two-row chains, two waves per SIMD
-        ens_relayout_kernel<R><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy, bad);
+        if (g.copy_edge == 8)
+            ens_relayout_kernel<R, 8><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy, bad);
+        else
+            ens_relayout_kernel<R, 16><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy, bad);
         ens_rect_kernel<R, F32, F32 ? 2 : 1, W, !F32>
             <<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fld, (const R*)copy, (R*)fp, bad);
         ens_gather_kernel<R, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fp, partials);
@@ -591,6 +720,91 @@ hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, cons
         sized(float(0));
     else
         sized(double(0));
+    return hipGetLastError();
+}
+
+// Planes with both extents of 12 or more on lattices of 90000 sites or more, as measured (us by quadrants
+// -> by tiles): 20^3x12 FP64 82 -> 57 and, on a copy, 78 -> 73, FP32 54 -> 38 and 53 -> 47; 16^3x24 FP64
+// 81 -> 54 and 75 -> 66, FP32 54 -> 35 and 50 -> 45.  Below, two and a half thousand tiles do not fill the
+// chip's slots, and the three or four launches outweigh the products saved.
+static bool f_plane(const Lat& L, int is_f32, int mu, int nu, FPlane* p) {
+    if (mu == nu || !fits_buffer(L.V, is_f32) || L.V < kRectSites || std::min(L.n[mu], L.n[nu]) < 12) return false;
+    auto has = [&](int d) { return mu == d || nu == d; };
+    const int32_t yfast[4] = {L.n[0], L.n[2], L.n[1], L.n[3]};
+    p->first_is_zero = has(0);
+    p->mu0 = p->mu1 = -1;
+    p->L = L;
+    if (has(1)) {
+        p->d1 = 1;
+        p->d2 = mu + nu - 1;
+    } else if (has(3)) {
+        p->L = zy_lattice(L);
+        p->d1 = 3;
+        p->d2 = mu + nu - 3;
+        p->mu0 = has(0) ? 0 : 3;
+        p->mu1 = has(0) ? 3 : 2;
+    } else {
+        p->L = make_lat(yfast);
+        p->d1 = p->mu1 = 2;
+        p->d2 = p->mu0 = 0;
+    }
+    p->rp = p->d2 == 0 ? 2 : (p->d1 == 1 && p->d2 == 3 ? 1 : 0);
+    const uint32_t NX = (uint32_t)p->L.n[1], NY = (uint32_t)p->L.n[2], NZ = (uint32_t)p->L.n[3], NT = (uint32_t)L.n[0];
+    const uint32_t n2 = p->rp == 0 ? NY : (p->rp == 1 ? NZ : NT), s1 = p->rp == 0 ? NZ : NY, s2 = p->rp == 2 ? NZ : NT;
+    p->g = plane_split(NX, n2, s1, s2, is_f32 ? kMaxCells<float> : kMaxCells<double>, is_f32 ? 2048 : 1024, s2);
+    const size_t sz = is_f32 ? 4 : 8;
+    p->copy_at = ((size_t)p->g.tiles * p->g.fc * 9 * sz + 255) & ~(size_t)255;
+    p->bytes = p->copy_at + (p->mu0 >= 0 ? (size_t)36 * L.V * sz : 0) + 256;
+    return true;
+}
+
+size_t fmunu_rect_bytes(const Lat& L, int is_f32, int mu, int nu) {
+    FPlane p;
+    return f_plane(L, is_f32, mu, nu, &p) ? p.bytes : 0;
+}
+
+hipError_t launch_fmunu_rect(const Lat& L, const void* U, int is_f32, int mu, int nu, void* out, const int64_t s6[6],
+                             void* ws, hipStream_t st) {
+    FPlane p;
+    if (!f_plane(L, is_f32, mu, nu, &p) || s6[0] != 1) return hipErrorInvalidValue;
+    const OutStrides os{s6[0], s6[1], s6[2], s6[3], s6[4], s6[5]};
+    // the strides along the directions of p.L
+    OutStrides osl = os;
+    if (p.d1 != 1) {
+        osl.x = p.d1 == 3 ? os.z : os.y;
+        (p.d1 == 3 ? osl.z : osl.y) = os.x;
+    }
+    with_view(L.V, U, is_f32, [&](auto f) {
+        using F = decltype(f);
+        using R = typename F::real;
+        if constexpr (F::buffered) {
+            R* fp = (R*)ws;
+            R* P = p.mu0 >= 0 ? (R*)((char*)ws + p.copy_at) : nullptr;
+            uint32_t* bad = (uint32_t*)((char*)ws + p.bytes - 256);
+            const int a = p.d1 == 1 ? 2 : p.d1;
+            if (P && relayout_edge(L, a) == 16)
+                plane_copy_kernel<R, 16><<<relayout_blocks(L, a, 16), 256, 0, st>>>(L, a, p.mu0, p.mu1, f.p, P, bad);
+            else
+                plane_copy_kernel<R, 8>
+                    <<<P ? relayout_blocks(L, a, 8) : 1, 256, 0, st>>>(L, a, p.mu0, p.mu1, f.p, P, bad);
+            // the copy's two blocks are directions 0 and 1 of its lattice, or 1 and 2
+            const F fl{P ? (p.first_is_zero ? P : zy_view<R>(P, L.V)) : f.p, L.V};
+            constexpr bool F32 = sizeof(R) == 4;
+            const R sign = mu == p.d1 ? R(1) : R(-1);
+            auto run = [&](auto time) {
+                constexpr bool TIME = decltype(time)::value;
+                plane_kernel<F, false, F32 ? 2 : 1, !F32, TIME><<<p.g.tiles, kRW, 0, st>>>(p.L, fl, p.rp, p.g, fp, bad);
+                const uint32_t nb = (uint32_t)((p.L.n[0] + kFT - 1) / kFT) * (uint32_t)((p.L.n[1] + kFT - 1) / kFT) *
+                                    (uint32_t)p.L.n[2] * (uint32_t)p.L.n[3];
+                plane_gather_kernel<R, TIME><<<nb, kFT * kFT, 0, st>>>(p.L, p.rp, p.g, fp, sign, (double*)out, osl);
+            };
+            if (p.rp == 2)
+                run(std::true_type());
+            else
+                run(std::false_type());
+            if constexpr (!F32) plane_general_kernel<<<kGeneralGrid, kRW, 0, st>>>(L, f, mu, nu, bad, (double*)out, os);
+        }
+    });
     return hipGetLastError();
 }
 

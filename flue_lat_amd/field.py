@@ -259,9 +259,14 @@ class GaugeField:
         NT, NX, NY, NZ = self.dims
         buf = torch.empty((3, 3, NZ, NY, NX, NT), dtype=torch.complex128, device=self.device)
         out = buf.permute(5, 4, 3, 2, 1, 0)
+        n = 0 if clover else _lib.lib().flue_fmunu_work_bytes(self._cdims, self.prec, int(mu), int(nu))
+        try:
+            ws = torch.empty(n, dtype=torch.uint8, device=self.device) if n else None
+        except torch.cuda.OutOfMemoryError:   # the form without a workspace
+            ws, n = None, 0
         with torch.cuda.device(self.device):
-            check_status(_lib.lib().flue_fmunu(self._cdims, _ptr(self.data), self.prec, int(mu), int(nu), 1 if clover else 0,
-                                        _ptr(out), FLUE_OUT_STRIDED, _i64(out.stride()), _stream()), "flue_fmunu")
+            check_status(_lib.lib().flue_fmunu_ex(self._cdims, _ptr(self.data), self.prec, int(mu), int(nu), 1 if clover else 0,
+                                        _ptr(out), FLUE_OUT_STRIDED, _i64(out.stride()), _ptr(ws) if n else None, n, _stream()), "flue_fmunu")
         return out
 
     def momentum_field(self):

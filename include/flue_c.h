@@ -253,6 +253,15 @@ int flue_generic_path(const int32_t dims[4], const void* U, int32_t prec, const 
 int flue_fmunu(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, int32_t nu, int32_t variant,
                void* out, int32_t layout, const int64_t strides[6], void* stream);
 
+/* the same given a workspace of flue_fmunu_work_bytes: where both extents of the plane are 12
+ * or more on a lattice of 90,000 sites or more, variant 0 into a strided array with stride 1
+ * along t forms each rectangle once, as variant 7 of flue_magnetic_ex does (FLUE_F64 links
+ * that are not unitary are found on the way and take the quadrants); the two forms agree to
+ * rounding.  Elsewhere work_bytes is 0 and ws is not used. */
+size_t flue_fmunu_work_bytes(const int32_t dims[4], int32_t prec, int32_t mu, int32_t nu);
+int flue_fmunu_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, int32_t nu, int32_t variant,
+                  void* out, int32_t layout, const int64_t strides[6], void* ws, size_t ws_bytes, void* stream);
+
 /* calc_mom_space_scalarD (src/gluonCalc/gluonProp.f90:112-250) on a Fourier-transformed
  * field Uq held like a SoA field over its extents dims (36 complex planes of V elements,
  * the momenta q in place of the sites): within a plane, momentum q sits at

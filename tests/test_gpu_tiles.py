@@ -5,6 +5,8 @@ widths, lanes idle in a tile's last turn, and transposes past an edge of 16.  To
 the tileable lattices (tests/test_gpu_rect.py): FP64 sums 1e-12, FP32 links 1e-6; adjoint 1e-12
 and 1e-5 of the largest entry.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -79,3 +81,41 @@ def test_ensemble_of_links_that_are_not_unitary(FL, mu):
     _, B = e.flow(0.01, 0, measure_every=1)
     for c in range(3):
         assert abs(B[0, c] - ref[c]) < 1e-12 * ref[c]
+
+
+def quadrant_f(f, mu, nu):
+    """F by quadrants: the form without a workspace."""
+    from flue_lat_amd import _lib
+    out = torch.empty((3, 3) + tuple(reversed(f.dims)), dtype=torch.complex128, device=f.device)
+    out = out.permute(5, 4, 3, 2, 1, 0)
+    st = (ctypes.c_int64 * 6)(*out.stride())
+    assert _lib.lib().flue_fmunu(f._cdims, ctypes.c_void_p(f.data.data_ptr()), f.prec, mu, nu, 0,
+                                 ctypes.c_void_p(out.data_ptr()), _lib.FLUE_OUT_STRIDED, st,
+                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    return out
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 2e-6)])
+@pytest.mark.parametrize("dims", [(12, 13, 31, 20), (37, 12, 14, 17), (16, 32, 16, 16)])
+def test_fmunu_tiles(FL, dims, prec, tol):
+    # every plane in both orientations.  The forms add the same 28 leaves of at most 12 links, of size
+    # O(1) each with weights of sum 2.2 or so: FP64 100 eps of the largest entry; FP32 30 eps.
+    f = FL.GaugeField.random(dims, 9, 0.3, prec)
+    for mu in range(1, 5):
+        for nu in range(1, 5):
+            if mu == nu:
+                continue
+            want, got = quadrant_f(f, mu, nu), f.fmunu(mu, nu)
+            scale = want.abs().max()
+            assert (got - want).abs().max() < tol * scale, (mu, nu)
+
+
+@pytest.mark.parametrize("mu,nu,d", [(2, 1, 2), (1, 4, 4), (3, 4, 3), (3, 1, 1), (2, 3, 3), (4, 2, 2)])
+def test_fmunu_of_links_that_are_not_unitary(FL, mu, nu, d):
+    f = FL.GaugeField.random((12, 13, 31, 20), 9, 0.3, "fp64")
+    U = f.to_complex()
+    U[-1, -1, -1, -1, d - 1] *= 1.5
+    g = FL.GaugeField.from_complex(U)
+    want = quadrant_f(g, mu, nu)
+    assert (quadrant_f(f, mu, nu) - want).abs().max() > 1e-3 * want.abs().max()
+    assert torch.equal(g.fmunu(mu, nu), want)
