@@ -119,3 +119,26 @@ def test_fmunu_of_links_that_are_not_unitary(FL, mu, nu, d):
     want = quadrant_f(g, mu, nu)
     assert (quadrant_f(f, mu, nu) - want).abs().max() > 1e-3 * want.abs().max()
     assert torch.equal(g.fmunu(mu, nu), want)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 1e-6)])
+@pytest.mark.parametrize("R,T", [(6, 6), (1, 3), (4, 5), (6, 2)])
+@pytest.mark.parametrize("dims", [(5, 16, 16, 3), (4, 33, 31, 2), (2, 300, 7, 3), (31, 8, 5, 4), (3, 2, 128, 2)])
+def test_wilson_loop_tiles(FL, dims, R, T, prec, tol):
+    # planes with x, which take tiles, against the same loops where they do not: with x and the third
+    # direction exchanged, and, time in the plane, slice by slice.  Both form the same products (FP64
+    # 1e-13; FP32 traces round at 2^-24 of 3, averaged over the sites).
+    f = FL.GaugeField.random(dims, 4, 0.3, prec)
+    U = f.to_complex()
+    for o, s in ((3, 4), (4, 3)):                      # plane (x, o); s the direction outside
+        perm = {1: 1, 2: s, s: 2, o: o}                # x and s exchanged
+        ax = [perm[d] - 1 for d in (1, 2, 3, 4)]
+        V = U.permute(*ax, 4, 5, 6)[..., ax, :, :]
+        g = FL.GaugeField.from_complex(V.contiguous(), precision=prec)
+        assert np.abs(f.wilson_loops(2, o, R, T) - g.wilson_loops(s, o, R, T)).max() < 3 * tol
+        assert np.abs(f.wilson_loops(o, 2, R, T) - g.wilson_loops(o, s, R, T)).max() < 3 * tol
+        assert np.abs(f.wilson_loops_slices(2, o, R, T) - g.wilson_loops_slices(s, o, R, T)).max() < 3 * tol
+        assert np.abs(f.wilson_loops(2, o, R, T, tau=2) - g.wilson_loops(s, o, R, T, tau=2)).max() < 3 * tol
+    for mu, nu in ((1, 2), (2, 1)):
+        table = f.wilson_loops(mu, nu, R, T)
+        assert np.abs(table - f.wilson_loops_slices(mu, nu, R, T).mean(axis=2)).max() < 3 * tol
