@@ -11,8 +11,10 @@ namespace flue {
 
 // field layout conversion: complex input/output with element strides (in complex
 // elements) for the index order (t, x, y, z, mu, a, b)
+// (ndir < 4, where imports_by_direction and both are aligned to their elements: of `ndir` directions)
+bool imports_by_direction(const Lat& L, const int64_t strides[7]);
 hipError_t launch_import(const Lat& L, const void* src, int src_is_f32, const int64_t strides[7], void* dst,
-                         int dst_is_f32, hipStream_t st);
+                         int dst_is_f32, hipStream_t st, int ndir = 4);
 hipError_t launch_export(const Lat& L, const void* src, int src_is_f32, void* dst, int dst_is_f32,
                          const int64_t strides[7], hipStream_t st);
 // out = 2 G U, out a C-ordered complex128 array, G in the given precision, U FP64 planes

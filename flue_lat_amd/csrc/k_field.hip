@@ -460,7 +460,7 @@ static int array_order(const Lat& L, const int64_t s[7], bool written, ArrayLayo
 
 template <bool IN, typename Ra, typename Rf>
 static hipError_t convert_layout(const Lat& L, int order, const ArrayLayout& l, const void* arr, const void* fld,
-                                 hipStream_t st) {
+                                 hipStream_t st, int ndir = 4) {
     Pair<Ra>* a = (Pair<Ra>*)arr;
     Pair<Rf>* p = (Pair<Rf>*)fld;
     const uint32_t rest = (uint32_t)L.ext(l.o1) * (uint32_t)L.ext(l.o2);
@@ -471,25 +471,33 @@ static hipError_t convert_layout(const Lat& L, int order, const ArrayLayout& l, 
         site_block_kernel<IN, Ra, Rf><<<g, 256, 0, st>>>(L, l, a, p);
     } else if (order == kArrayPlanes) {
         const uint32_t g = ((uint32_t)L.n[1] + 31) / 32 * (((uint32_t)L.ext(l.f) + 31) / 32) * rest;
-        plane_tile_kernel<IN, Ra, Rf><<<dim3(g, 4), 256, 0, st>>>(L, l, a, p);
+        plane_tile_kernel<IN, Ra, Rf><<<dim3(g, ndir), 256, 0, st>>>(L, l, a, p);
     } else {
-        row_kernel<IN, Ra, Rf><<<dim3(grid_for(L.V), 4), 256, 0, st>>>(L, l, a, p);
+        row_kernel<IN, Ra, Rf><<<dim3(grid_for(L.V), ndir), 256, 0, st>>>(L, l, a, p);
     }
     return hipGetLastError();
 }
 
 static bool pair_aligned(const void* p, int is_f32) { return (uintptr_t)p % (is_f32 ? 8 : 16) == 0; }
 
-hipError_t launch_import(const Lat& L, const void* src, int src_is_f32, const int64_t s[7], void* dst,
-                         int dst_is_f32, hipStream_t st) {
+bool imports_by_direction(const Lat& L, const int64_t s[7]) {
     ArrayLayout l;
     const int order = array_order(L, s, false, l);
+    return order == kArrayPlanes || order == kArrayRows;
+}
+
+hipError_t launch_import(const Lat& L, const void* src, int src_is_f32, const int64_t s[7], void* dst,
+                         int dst_is_f32, hipStream_t st, int ndir) {
+    ArrayLayout l;
+    const int order = array_order(L, s, false, l);
+    if (ndir < 4 && (!imports_by_direction(L, s) || !pair_aligned(src, src_is_f32) || !pair_aligned(dst, dst_is_f32)))
+        return hipErrorInvalidValue;
     if (order >= 0 && pair_aligned(src, src_is_f32) && pair_aligned(dst, dst_is_f32)) {
         if (src_is_f32)
-            return dst_is_f32 ? convert_layout<true, float, float>(L, order, l, src, dst, st)
-                              : convert_layout<true, float, double>(L, order, l, src, dst, st);
-        return dst_is_f32 ? convert_layout<true, double, float>(L, order, l, src, dst, st)
-                          : convert_layout<true, double, double>(L, order, l, src, dst, st);
+            return dst_is_f32 ? convert_layout<true, float, float>(L, order, l, src, dst, st, ndir)
+                              : convert_layout<true, float, double>(L, order, l, src, dst, st, ndir);
+        return dst_is_f32 ? convert_layout<true, double, float>(L, order, l, src, dst, st, ndir)
+                          : convert_layout<true, double, double>(L, order, l, src, dst, st, ndir);
     }
     const uint32_t g = grid_for((uint64_t)L.V * 4);
     if (src_is_f32 && dst_is_f32)

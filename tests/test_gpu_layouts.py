@@ -6,7 +6,9 @@ tile's edge, expanded (zero-stride) sources and a pointer that is not aligned to
 conversion moves values, so results are compared exactly (FP32: the rounded value).
 """
 import ctypes
+import itertools
 
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -91,3 +93,21 @@ def test_tangent_field(FL, dims, prec):
     assert E.is_contiguous() and E.shape == dims + (4, 3, 3)
     want = tangent_from_lie(G.to_complex(), U)
     assert float((E - want).abs().max()) <= 6 * 2.3e-16 * 2 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("dims", [(3, 1, 1, 1), (4, 1, 3, 1), (3, 4, 1, 2), (5, 7, 3, 4), (1, 1, 1, 2), (33, 34, 3, 2)])
+def test_host_functions_copy_what_they_read(FL, dims):
+    # the host functions bring the directions they read to the device; the same kernels on a resident
+    # field of all of them give the same numbers
+    fc = FL.compiled.flue_c
+    U = np.asfortranarray(FL.GaugeField.random(dims, 17, 0.4).to_complex().cpu().numpy())
+    f = FL.GaugeField.from_complex(U)
+    for args in itertools.product(range(1, 5), range(1, 5), range(1, 5)):
+        assert fc.plaquette_c(U, *args)[:2] == f.plaquette(*args), args
+    if dims[0] >= 3:
+        assert fc.polyakov_c(U)[:2] == f.polyakov()
+    assert fc.magnetic_c(U) == f.magnetic()
+    for mu, nu in itertools.product(range(1, 5), range(1, 5)):
+        assert np.array_equal(fc.loop5munucoord_c(U, mu, nu), f.fmunu(mu, nu).cpu().numpy())
+        assert fc.wmunu_c(U, mu, nu, 2, 1) == f.wilson_loop(mu, nu, 2, 1)
+        assert fc.wmunutau_c(U, 1, mu, nu, 1, 2) == f.wilson_loop(mu, nu, 1, 2, tau=1)
