@@ -21,9 +21,8 @@
 // moved 25 GB from L2 for 32^3x64 (1.5 ms, three times the products' time).  Planes with x take
 // tiles of up to 256 sites in the plane, whose links (the tile and six more rows and columns, up to
 // 155 KB in FP64) are read into LDS once: 1.9 links of either direction per site for 16 x 16 tiles.
-// Then the vector unit issues 61% of the cycles in FP64 (of 13,600 instructions a wave 9,500 are the
-// products' and traces'; the chains beyond 256 registers are moved by the rest) and a fifth goes into
-// waiting for the tile's loads.
+// Then the vector unit issues 73% of the cycles in FP64 (of 13,800 instructions a wave 9,500 are the
+// products and traces; most others move the chains beyond 256 registers), and 15% wait for a tile's loads.
 #include "flue_common.hpp"
 #include "flue_launch.hpp"
 #include "flue_tiles.hpp"
@@ -134,7 +133,7 @@ wloop_table_kernel(Lat L, FV f, int mu, int nu, int Rmax, int tslice, uint32_t n
             v = live ? v : 0.0;
             v += quad_swap<0xB1>(v);
             v += quad_swap<0x4E>(v);
-            if ((threadIdx.x & 3) == 0) mine[(T - 1) * (kBS / 4)] = v;
+            mine[(T - 1) * (kBS / 4)] = v;  // (the four lanes' one value: a branch here spills the chains, 1.61 for 1.27 ms)
             __builtin_amdgcn_sched_barrier(0);
         }
         mine += TM * (kBS / 4);
@@ -272,7 +271,7 @@ wloop_tile_kernel(Lat L, FV f, int mu, int nu, int Rmax, PlaneTiles g, int tslic
             }
             double v = (double)retr_nd(CA, CB[T - 1]);
             v = row_sum(live ? v : 0.0);
-            if ((threadIdx.x & 15) == 0) mine[(T - 1) * (kBS / 16)] = v;
+            mine[(T - 1) * (kBS / 16)] = v;
             __builtin_amdgcn_sched_barrier(0);
         }
         mine += TM * (kBS / 16);
@@ -318,17 +317,19 @@ PlaneTiles loop_split(uint32_t n1, uint32_t n2, uint32_t halo1, uint32_t halo2, 
     return best;
 }
 
-// block (k, j) of the grid sums table entry k of slice
+// block (k, j) of the grid sums table entry k (of rows of `cols`) of slice
 // group j (of gridDim.y) over its nb block partials in a fixed order and writes
-// out[k * gridDim.y + j] = scale * sum
+// out[k' * gridDim.y + j] = scale * sum, k' = k or the transposed table's entry
 __global__ void __launch_bounds__(kBS) wloop_finalize_kernel(const double* __restrict__ partials, uint32_t nb,
-                                                             double* __restrict__ out, double scale) {
+                                                             int cols, int transposed, double* __restrict__ out,
+                                                             double scale) {
     const int k = blockIdx.x;
+    const int to = transposed ? (k % cols) * ((int)gridDim.x / cols) + k / cols : k;
     const double* p = partials + 2 * (((size_t)k * gridDim.y + blockIdx.y) * nb);
     DD acc = {0.0, 0.0};
     for (uint32_t i = threadIdx.x; i < nb; i += kBS) acc = dd_add(acc, DD{p[2 * i], p[2 * i + 1]});
     const DD r = block_sum<kBS>(acc);
-    if (threadIdx.x == 0) out[(size_t)k * gridDim.y + blockIdx.y] = (r.hi + r.lo) * scale;
+    if (threadIdx.x == 0) out[(size_t)to * gridDim.y + blockIdx.y] = (r.hi + r.lo) * scale;
 }
 
 }  // namespace
@@ -341,11 +342,11 @@ uint32_t wloop_blocks(const Lat& L, int tslice, int mu, int nu) {
     return (mu == 0 || nu == 0) ? (uint32_t)L.n[0] * per_slice : (L.V + kBS - 1) / kBS;
 }
 
-// Whether n tiles beat nb blocks of 256 sites.  Table by 6 x 6, us by blocks -> by tiles, planes (x,t)
-// and (x,y): 32^3x64 FP64 1543 -> 1283 and 1476 -> 1273, FP32 951 -> 603 and 920 -> 590; 24^3x48 FP64
-// 511 -> 457 and, a quarter of the lanes idle, 504 -> 522, FP32 322 -> 212 and 316 -> 239; 16^4 FP64
-// 55 -> 47, FP32 40 -> 32.  In FP64 a block holds a CU's LDS, so its loads are not hidden, and few
-// chains (T = 2, 32^3x64: 253 -> 287; T = 4: 650 -> 584; T = 3 and 6 rows: 695 -> 598) do not repay that.
+// Whether n tiles beat nb blocks of 256 sites.  us by blocks -> by tiles, plane (x,t) of 32^3x64, 6 x 6:
+// FP64 1270 -> 1076, FP32 755 -> 525; 6 x 3: FP64 693 -> 595, FP32 416 -> 304; 18x15x20x30, a seventh of
+// the lanes idle, FP32 79 -> 68.  In FP64 a block holds a CU's LDS, so its loads are not hidden: one or two
+// chains (253 -> 287 before the rows were straight) and idle lanes (24^3x48, a quarter: 504 -> 522) do
+// not repay that.
 static bool tiles_pay(int is_f32, int Tmax, uint64_t n, uint64_t nb) {
     return is_f32 ? n * 2 <= nb * 3 : Tmax >= 3 && n * 4 <= nb * 5;
 }
@@ -359,6 +360,14 @@ size_t wloop_partial_bytes(const Lat& L, int tslice) {
 
 hipError_t launch_wloop_table(const Lat& L, const void* U, int is_f32, int mu, int nu, int Rmax, int Tmax,
                               int tslice, double* partials, double* out, double scale, hipStream_t st) {
+    // A loop of the plane (nu, mu) is the same loop walked the other way round, its chains and its trace the
+    // same products: the longer side makes the rows, since rows are cheaper than chains (24^3x14 FP64,
+    // 1 x 6 against 6 x 1: 75 and 36 us).
+    const bool swapped = Tmax > Rmax;
+    if (swapped) {
+        std::swap(mu, nu);
+        std::swap(Rmax, Tmax);
+    }
     uint32_t nb = wloop_blocks(L, tslice, mu, nu);
     const uint32_t groups = tslice == kEverySlice ? (uint32_t)L.n[0] : 1u;
     PlaneTiles tiles{};
@@ -394,7 +403,7 @@ hipError_t launch_wloop_table(const Lat& L, const void* U, int is_f32, int mu, i
     });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    wloop_finalize_kernel<<<dim3(Rmax * Tmax, groups), kBS, 0, st>>>(partials, nb, out, scale);
+    wloop_finalize_kernel<<<dim3(Rmax * Tmax, groups), kBS, 0, st>>>(partials, nb, Tmax, swapped, out, scale);
     return hipGetLastError();
 }
 
