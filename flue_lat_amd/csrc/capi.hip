@@ -566,7 +566,7 @@ int flue_plaquette(const int32_t dims[4], const void* U, int32_t prec, int32_t m
     if (!U || !d_sum) return FLUE_ENULL;
     if (check_prec(prec) || check_plaq_args(muStart, muEnd, nuEnd)) return FLUE_EINVAL;
     const Lat L = make_lat(dims);
-    const int variant = variant_or(FLUE_OP_PLAQUETTE, dims, prec, kPlaquetteDefault);
+    const int variant = variant_or(FLUE_OP_PLAQUETTE, dims, prec, plaquette_default(L, prec == FLUE_F32));
     uint32_t nb = plaquette_blocks(L, variant);
     void* w;
     if ((rc = get_ws(ws, ws_bytes, partial_bytes(nb), &w))) return rc;
@@ -833,7 +833,7 @@ int flue_wilson_action(const int32_t dims[4], const void* U, int32_t prec, doubl
     if (!U || !d_S) return FLUE_ENULL;
     if (check_prec(prec) || !std::isfinite(beta)) return FLUE_EINVAL;
     const Lat L = make_lat(dims);
-    const int variant = variant_or(FLUE_OP_PLAQUETTE, dims, prec, kPlaquetteDefault);
+    const int variant = variant_or(FLUE_OP_PLAQUETTE, dims, prec, plaquette_default(L, prec == FLUE_F32));
     uint32_t nb = plaquette_blocks(L, variant);
     void* w;
     if ((rc = get_ws(ws, ws_bytes, partial_bytes(nb), &w))) return rc;

@@ -28,11 +28,14 @@ hipError_t launch_check_field(const Lat& L, const void* U, int is_f32, double* p
 
 // reductions: each writes one compensated partial (hi, lo) per block to `partials`,
 // then launch_finalize sums them in a fixed order into out[0] (double, device)
-// plaquette walk lengths (time slices per thread), one per variant; variant 0 = the default
+// plaquette walk lengths (time slices per thread), one per variant, and the form with a thread per
+// site and plane, which small lattices take untuned
 constexpr int kPlaquetteVariants = 6;
 constexpr int kPlaqWalks[kPlaquetteVariants] = {2, 3, 4, 6, 8, 12};
-constexpr int kPlaquetteDefault = 4;  // walks of 6 slices
-int plaquette_walk(int variant);
+constexpr int kPlaquetteLongest = 4;  // the longest untuned walk: 6 slices
+constexpr int kPlaquettePlanes = kPlaquetteVariants + 1;
+constexpr uint32_t kPlaqPlaneSites = 65536;  // its most sites (FP32; a quarter in FP64)
+int plaquette_default(const Lat& L, int is_f32);
 uint32_t plaquette_blocks(const Lat& L, int variant);
 uint32_t plaquette_max_blocks(const Lat& L);
 // *npart (optional) receives the number of partials written

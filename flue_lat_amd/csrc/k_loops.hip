@@ -94,6 +94,25 @@ __global__ void __launch_bounds__(kBS) plaquette_kernel(Lat L, FV f, int mu0, in
     write_partial(partials, blk, block_sum<kBS>(DD{acc, 0.0}));
 }
 
+// The same sum with one thread per site and plane (blockIdx.y: the plane, two bits each for mu and nu in
+// `planes`), for lattices whose walks would leave most of the chip idle.
+template <typename FV>
+__global__ void __launch_bounds__(kBS) plaquette_plane_kernel(Lat L, FV f, uint32_t planes, double* __restrict__ partials) {
+    const int mu = (int)(planes >> 4 * blockIdx.y & 3u), nu = (int)(planes >> (4 * blockIdx.y + 2) & 3u);
+    const uint32_t s = blockIdx.x * kBS + threadIdx.x;
+    double acc = 0.0;
+    if (s < L.V) {
+        int c[4];
+        site_coords(L, s, c);
+        auto next = [&](int d, int cd) { return cd == L.ext(d) - 1 ? s - (uint32_t)cd * L.stride(d) : s + L.stride(d); };
+        const uint32_t smu = next(mu, c[mu]), snu = next(nu, c[nu]);
+        const auto Umu = load_link(f, mu, s), Unu = load_link(f, nu, s);
+        const auto Vnu = load_link(f, nu, smu), Vmu = load_link(f, mu, snu);
+        acc = (double)retr_nd(mul(Umu, Vnu), mul(Unu, Vmu));
+    }
+    write_partial(partials, blockIdx.y * gridDim.x + blockIdx.x, block_sum<kBS>(DD{acc, 0.0}));
+}
+
 // Polyakov loop: ordered product of the time links over t = 0..NT-1 at each spatial
 // site (src/wloops.F90:1043-1063).  A block holds 64 spatial sites x 4 time segments;
 // segment products are combined left to right in shared memory.
@@ -245,11 +264,28 @@ PathArg make_path(const int32_t* path, int npath) {
 // blocks per time chunk (the spatial sites of one slice), times the time chunks
 static uint32_t plaquette_slice_blocks(const Lat& L) { return (L.Vs + kBS - 1) / kBS; }
 
-int plaquette_walk(int variant) {
-    return (variant >= 1 && variant <= kPlaquetteVariants) ? kPlaqWalks[variant - 1] : kPlaqWalks[kPlaquetteDefault - 1];
+// The untuned variant: a thread per site and plane on the smallest lattices, else the shortest walk
+// whose threads are resident at once (one wave per SIMD in FP64, two in FP32), up to 6 slices.  As
+// measured, us with the finalize pass, per plane / walks of 2, 3, 4, 6:
+//   8^3x16          8,192 sites  FP64   9 /  14  18  22  30   FP32   8 /  14  18  21  29
+//   12^3x24        41,472               22 /  17  20  27  39           12 /  14  18  22  30
+//   16^4           65,536               21 /  18  23  29  40           13 /  15  20  25  35
+//   16^3x32       131,072               55 /  24  26  29  41           24 /  16  21  24  35
+//   20x22x18x26   205,920               98 /  40  51  36  43           48 /  24  30  27  36
+//   24^4          331,776              152 /  59  54  66  50           66 /  37  32  38  38
+//   24^3x48       663,552              295 / 119 120 119 117          124 /  63  61  64  56
+int plaquette_default(const Lat& L, int is_f32) {
+    if (L.V <= (is_f32 ? kPlaqPlaneSites : kPlaqPlaneSites / 4)) return kPlaquettePlanes;
+    const uint32_t resident = (is_f32 ? 2u : 1u) * 65536;
+    int v = 1;
+    while (v < kPlaquetteLongest && L.V / (uint32_t)kPlaqWalks[v - 1] > resident) ++v;
+    return v;
 }
 
+static int plaquette_walk(int variant) { return kPlaqWalks[variant - 1]; }
+
 uint32_t plaquette_blocks(const Lat& L, int variant) {
+    if (variant == kPlaquettePlanes) return 6 * ((L.V + kBS - 1) / kBS);
     const int lt = plaquette_walk(variant);
     return plaquette_slice_blocks(L) * (uint32_t)((L.n[0] + lt - 1) / lt);
 }
@@ -257,11 +293,24 @@ uint32_t plaquette_blocks(const Lat& L, int variant) {
 uint32_t plaquette_max_blocks(const Lat& L) {
     uint32_t m = 0;
     for (int v = 1; v <= kPlaquetteVariants; ++v) m = std::max(m, plaquette_blocks(L, v));
+    if (L.V <= kPlaqPlaneSites) m = std::max(m, plaquette_blocks(L, kPlaquettePlanes));
     return m;
 }
 
 hipError_t launch_plaquette(const Lat& L, const void* U, int is_f32, int mu0, int mu1, int nu1, double* partials,
                             hipStream_t st, int variant, uint32_t* npart) {
+    if (variant == kPlaquettePlanes) {
+        uint32_t planes = 0, n = 0;
+        for (int mu = mu0; mu <= mu1; ++mu)
+            for (int nu = mu + 1; nu <= nu1; ++nu) planes |= (uint32_t)(mu | nu << 2) << 4 * n++;
+        const uint32_t nb = (L.V + kBS - 1) / kBS;
+        if (n)
+            with_view(L.V, U, is_f32, [&](auto f) {
+                plaquette_plane_kernel<decltype(f)><<<dim3(nb, n), kBS, 0, st>>>(L, f, planes, partials);
+            });
+        if (npart) *npart = n * nb;
+        return hipGetLastError();
+    }
     const int lt = plaquette_walk(variant);
     const uint32_t g = plaquette_blocks(L, variant), nbs = plaquette_slice_blocks(L);
     with_view(L.V, U, is_f32, [&](auto f) {
