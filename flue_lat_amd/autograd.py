@@ -11,6 +11,8 @@ df = Re sum conj(E) dU; restricted to the group (dU = X U, X in su(3)) the match
 tangent vector is E = 2 G U, which is what backward returns.  Derivatives along the
 group are therefore exact; the components of E normal to SU(3) are zero.
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -30,6 +32,17 @@ def _tangent(G: GaugeField, U, g: GaugeField):
         check(_lib.lib().flue_tangent_field(G._cdims, _ptr(G.data), G.prec, _ptr(links.data), _ptr(out), _stream()),
               "flue_tangent_field")
     return out.to(U.device)
+
+
+def _b2_variant(g: GaugeField):
+    """The form of the B adjoint: the default's for FP64.  FP32 keeps the reverse form with slots: the
+    gradient is handed out in FP64, and the tiled form's FP32 sums round apart from those by 2e-7."""
+    if g.dtype == torch.float64:
+        return 0
+    v = ctypes.c_int32()
+    with torch.cuda.device(g.device):
+        check(_lib.lib().flue_tuned_variant(_lib.OPS["b2_grad"], g._cdims, g.prec, ctypes.byref(v)), "flue_tuned_variant")
+    return v.value or 2
 
 
 def tangent_from_lie(G, U):
@@ -80,7 +93,7 @@ class _Magnetic(torch.autograd.Function):
     def backward(ctx, grad_out):
         (U,) = ctx.saved_tensors
         g = GaugeField.from_complex(U.detach(), ctx.precision)
-        E = _tangent(g.magnetic_grad(), U.detach(), g)
+        E = _tangent(g.magnetic_grad(_b2_variant(g)), U.detach(), g)
         return (grad_out.to(torch.float64) * E).to(U.dtype), None
 
 

@@ -99,14 +99,18 @@ size_t magnetic_rect_partials(const Lat& L, int32_t prec) {
 size_t magnetic_ws_bytes(const Lat& L, int32_t prec, int variant) {
     if (variant == kMagneticRect && magnetic_rect_ok(L, prec))
         return magnetic_rect_partials(L, prec) + rect_fp_bytes(L, prec == FLUE_F32);
+    if (variant == kMagneticQuad) return partial_bytes(quad_blocks(L));
     return partial_bytes(magnetic_blocks(L, prec == FLUE_F32));
 }
 
-// runs magnetic `variant` (1..7) on workspace w and finalizes B into d_B
+// runs magnetic `variant` (1..7, or that of small lattices) on workspace w and finalizes B into d_B
 int magnetic_run(const Lat& L, const void* U, int32_t prec, int variant, void* w, double* d_B, hipStream_t st) {
     uint32_t np = 0;
     void* fp = variant == kMagneticRect ? (char*)w + magnetic_rect_partials(L, prec) : nullptr;
-    FLUE_TRY(launch_magnetic(L, U, prec == FLUE_F32, prec == FLUE_F64_SU3, (double*)w, st, variant, &np, fp));
+    if (variant == kMagneticQuad)
+        FLUE_TRY(launch_magnetic_quad(L, U, prec == FLUE_F64_SU3, (double*)w, st, &np));
+    else
+        FLUE_TRY(launch_magnetic(L, U, prec == FLUE_F32, prec == FLUE_F64_SU3, (double*)w, st, variant, &np, fp));
     if (d_B) FLUE_TRY(launch_finalize((double*)w, np, d_B, 1.0 / (double)L.V, st));
     return FLUE_OK;
 }
@@ -130,14 +134,20 @@ size_t b2_copy_at(const Lat& L, int32_t prec) {
 size_t b2_region_bytes(const Lat& L, int32_t prec) {
     const int f32 = prec == FLUE_F32;
     if (!magnetic_rect_ok(L, prec)) return b2_slot_bytes(L, f32);
-    return b2_copy_at(L, prec) + (size_t)36 * L.V * (f32 ? 4 : 8) + 256;  // (and its flag)
+    const size_t tiles = b2_copy_at(L, prec) + (size_t)36 * L.V * (f32 ? 4 : 8) + 256;  // (and its flag)
+    return std::max(tiles, b2_slot_bytes(L, f32));
+}
+
+// the form that a tuned or untuned variant runs as
+int b2_form(const Lat& L, int32_t prec, int variant) {
+    return variant == kB2DefaultVariant && magnetic_rect_ok(L, prec) ? kB2Tiled : variant;
 }
 
 // the B^2 adjoint after the SU(3) check: clover sums into the start of `work` (rectangle-first
 // where it applies, with two-row chains in both precisions since the links are SU(3)), then
-// variant 1 (per-link gather) or 2 (reverse mode: on tiles, or with slots after the clover sums)
+// variant 1 (per-link gather), 2 (reverse mode with slots) or kB2Tiled
 int b2_grad_run(const Lat& L, const void* U, int32_t prec, int variant, void* work, void* grad, hipStream_t st) {
-    const int f32 = prec == FLUE_F32, rect = magnetic_rect_ok(L, prec), tiled = rect && variant != 1;
+    const int f32 = prec == FLUE_F32, rect = magnetic_rect_ok(L, prec), tiled = variant == kB2Tiled;
     char* region = (char*)work + b2_ah_bytes(L, prec);
     const size_t copy_at = rect ? b2_copy_at(L, prec) : 0;
     if (rect)
@@ -290,7 +300,8 @@ int load_host_field(const int32_t* NT, const int32_t* NX, const int32_t* NY, con
     h.L = make_lat(h.dims);
     int64_t st[7];
     fortran_strides(h.dims, st);
-    if (!imports_by_direction(h.L, st)) {
+    // (nine pieces cost 0.1 ms more than one: not for less than 2 MB)
+    if (!imports_by_direction(h.L, st) || (uint64_t)h.L.V * (3 - (hi - lo)) * 9 * sizeof(flue_c128) < 2000000) {
         lo = 0;
         hi = 3;
     }
@@ -499,6 +510,7 @@ size_t flue_workspace_bytes(const int32_t dims[4]) {
     nb = std::max(nb, path_blocks(L, -1, nullptr, 0));
     nb = std::max(nb, magnetic_blocks(L, 0));
     nb = std::max(nb, magnetic_blocks(L, 1));
+    if (quad_fits(L, 0)) nb = std::max(nb, quad_blocks(L));
     return std::max({partial_bytes(nb), wloop_partial_bytes(L, -1) + 256, wloop_partial_bytes(L, kEverySlice) + 256,
                      check_bytes(L)});
 }
@@ -666,7 +678,7 @@ int flue_fmunu(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, i
 
 size_t flue_fmunu_work_bytes(const int32_t dims[4], int32_t prec, int32_t mu, int32_t nu) {
     if (check_dims(dims) || check_prec(prec) || mu < 1 || mu > 4 || nu < 1 || nu > 4) return 0;
-    return fmunu_rect_bytes(make_lat(dims), prec == FLUE_F32, mu - 1, nu - 1);
+    return prec == FLUE_F32 ? 0 : fmunu_rect_bytes(make_lat(dims), mu - 1, nu - 1);
 }
 
 int flue_fmunu_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, int32_t nu, int32_t variant, void* out,
@@ -680,11 +692,11 @@ int flue_fmunu_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t mu
     if (layout == FLUE_OUT_STRIDED && !strides) return FLUE_ENULL;
     const Lat L = make_lat(dims);
     const int f32 = prec == FLUE_F32;
-    const size_t need = ws && variant == 0 && layout == FLUE_OUT_STRIDED && strides[0] == 1
-                            ? fmunu_rect_bytes(L, f32, mu - 1, nu - 1)
+    const size_t need = ws && !f32 && variant == 0 && layout == FLUE_OUT_STRIDED && strides[0] == 1
+                            ? fmunu_rect_bytes(L, mu - 1, nu - 1)
                             : 0;
     if (need && ws_bytes >= need)
-        return hip_status(launch_fmunu_rect(L, U, f32, mu - 1, nu - 1, out, strides, ws, S(stream)));
+        return hip_status(launch_fmunu_rect(L, U, mu - 1, nu - 1, out, strides, ws, S(stream)));
     return hip_status(launch_fmunu(L, U, f32, mu - 1, nu - 1, variant, out, layout == FLUE_OUT_SOA, strides, S(stream)));
 }
 
@@ -732,7 +744,8 @@ int flue_magnetic(const int32_t dims[4], const void* U, int32_t prec, double* d_
 size_t flue_magnetic_work_bytes(const int32_t dims[4], int32_t prec) {
     if (check_dims(dims) || check_prec(prec)) return 0;
     const Lat L = make_lat(dims);
-    return std::max(magnetic_ws_bytes(L, prec, kMagneticRect), magnetic_ws_bytes(L, prec, 1));
+    return std::max({magnetic_ws_bytes(L, prec, kMagneticRect), magnetic_ws_bytes(L, prec, 1),
+                     quad_fits(L, prec == FLUE_F32) ? magnetic_ws_bytes(L, prec, kMagneticQuad) : 0});
 }
 
 int flue_magnetic_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t variant, double* d_B, void* ws,
@@ -742,9 +755,12 @@ int flue_magnetic_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t
     if (!U || !d_B) return FLUE_ENULL;
     if (check_prec(prec) || variant < 0 || variant > kMagneticVariants) return FLUE_EINVAL;
     const Lat L = make_lat(dims);
-    // untuned: the rectangle-first form where it applies, else the precision's quadrant form
+    // untuned: a wave per quadrant on small lattices, the rectangle-first form where it applies, else the
+    // precision's quadrant form
     if (variant == 0) variant = tuned_variant(FLUE_OP_MAGNETIC, dims, prec);
-    if (variant == 0) variant = magnetic_rect_ok(L, prec) ? kMagneticRect : magnetic_default_variant(prec == FLUE_F32);
+    if (variant == 0 && quad_fits(L, prec == FLUE_F32) && (!ws || ws_bytes >= magnetic_ws_bytes(L, prec, kMagneticQuad)))
+        variant = kMagneticQuad;
+    if (variant == 0) variant = magnetic_rect_ok(L, prec) && rect_untuned(L, prec == FLUE_F32) ? kMagneticRect : magnetic_default_variant(prec == FLUE_F32);
     // the rectangle-first form needs tileable extents and room for its footprints; otherwise
     // the precision's default form
     if (variant == kMagneticRect &&
@@ -883,7 +899,8 @@ int flue_b2_grad(const int32_t dims[4], const void* U, int32_t prec, void* grad,
     // the gather takes the product from a corner to the walk's end as X_c^+ F, which holds
     // for unitary links only: refuse fields that are not SU(3) to the precision's bound
     if ((rc = run_su3_check(L, U, prec, 0.0, nullptr, A, S(stream)))) return rc;
-    return b2_grad_run(L, U, prec, variant_or(FLUE_OP_B2_GRAD, dims, prec, kB2DefaultVariant), A, grad, S(stream));
+    return b2_grad_run(L, U, prec, b2_form(L, prec, variant_or(FLUE_OP_B2_GRAD, dims, prec, kB2DefaultVariant)), A, grad,
+                       S(stream));
 }
 
 int flue_b2_grad_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t variant, void* grad, void* work,
@@ -896,7 +913,7 @@ int flue_b2_grad_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t 
     void* A;
     if ((rc = get_ws(work, work_bytes, flue_b2_work_bytes(dims, prec), &A))) return rc;
     if ((rc = run_su3_check(L, U, prec, 0.0, nullptr, A, S(stream)))) return rc;
-    if (variant == 0) variant = variant_or(FLUE_OP_B2_GRAD, dims, prec, kB2DefaultVariant);
+    if (variant == 0) variant = b2_form(L, prec, variant_or(FLUE_OP_B2_GRAD, dims, prec, kB2DefaultVariant));
     return b2_grad_run(L, U, prec, variant, A, grad, S(stream));
 }
 
@@ -1064,7 +1081,7 @@ int flue_autotune(int32_t op, const int32_t dims[4], const void* U, int32_t prec
         switch (op) {
         case FLUE_OP_MAGNETIC: return magnetic_run(L, U, prec, v, w, nullptr, st);
         case FLUE_OP_PLAQUETTE: return hip_status(launch_plaquette(L, U, is_f32, 0, 3, 3, (double*)w, st, v, nullptr));
-        case FLUE_OP_B2_GRAD: return b2_grad_run(L, U, prec, v, w, (char*)w + flue_b2_work_bytes(dims, prec), st);
+        case FLUE_OP_B2_GRAD: return b2_grad_run(L, U, prec, b2_form(L, prec, v), w, (char*)w + flue_b2_work_bytes(dims, prec), st);
         default: {  // FLUE_OP_FLOW: one RK3 step, U -> w -> w2 -> w.  Stage 0 sets the
                     // accumulator afresh, so every timed step sees the same values (stages 1
                     // and 2 alone would scale it on every call and slow each variant more).

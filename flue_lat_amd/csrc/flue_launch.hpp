@@ -57,11 +57,11 @@ hipError_t launch_finalize(const double* partials, uint32_t n, double* out, doub
 // field precision
 hipError_t launch_fmunu(const Lat& L, const void* U, int is_f32, int mu, int nu, int clover_only, void* out,
                         int out_layout, const int64_t strides[6], hipStream_t st);
-// the 5-loop F of a plane on rectangle-first tiles (k_rect.hip), into an array with stride 1 along t;
-// fmunu_rect_bytes of workspace, 0 where the plane does not take them
-size_t fmunu_rect_bytes(const Lat& L, int is_f32, int mu, int nu);
-hipError_t launch_fmunu_rect(const Lat& L, const void* U, int is_f32, int mu, int nu, void* out, const int64_t strides[6],
-                             void* ws, hipStream_t st);
+// the 5-loop F of a plane of an FP64 field on rectangle-first tiles (k_rect.hip), into an array with
+// stride 1 along t; fmunu_rect_bytes of workspace, 0 where the plane does not take them
+size_t fmunu_rect_bytes(const Lat& L, int mu, int nu);
+hipError_t launch_fmunu_rect(const Lat& L, const void* U, int mu, int nu, void* out, const int64_t strides[6], void* ws,
+                             hipStream_t st);
 uint32_t magnetic_blocks(const Lat& L, int is_f32);
 int magnetic_default_variant(int is_f32);
 // rectangular Wilson-loop table (k_wloops.hip): R, T up to kMaxLoopRT
@@ -107,7 +107,14 @@ struct RectTiles {
     PlaneTiles p[3];  // planes (x,y), (x,z), (z,y) (the last as plane (x,y) of the copy)
 };
 
+// the untuned form of small lattices (k_quad.hip), a wave per quadrant: quad_blocks partials
+constexpr int kMagneticQuad = kMagneticVariants + 1;
+bool quad_fits(const Lat& L, int is_f32);
+uint32_t quad_blocks(const Lat& L);
+hipError_t launch_magnetic_quad(const Lat& L, const void* U, int su3, double* partials, hipStream_t st, uint32_t* npart);
 bool rect_fits(const Lat& L);
+// whether it is the untuned form
+bool rect_untuned(const Lat& L, int is_f32);
 // partials of variant 7: one per tile of its three planes
 uint32_t rect_partials(const Lat& L, int is_f32);
 size_t rect_fp_bytes(const Lat& L, int is_f32);
@@ -147,7 +154,9 @@ hipError_t launch_b2_grad(const Lat& L, const void* U, int is_f32, const void* A
 // at most kB2SlotReals reals (4 GiB in FP64, 2 GiB in FP32; at least one slice).  At 48^3
 // that is 3 slices in both precisions, which ran faster than 1, 7 or 14.
 constexpr uint64_t kB2SlotReals = (uint64_t)1 << 29;
-// B^2 adjoint forms: 1 = per-link gather, 2 = reverse mode (default)
+// B^2 adjoint forms: 1 = per-link gather, 2 = reverse mode (default), on tiles (kB2Tiled) where the
+// rectangle-first magnetic form applies, unless asked for by its number
+constexpr int kB2Tiled = 3;
 constexpr int kB2Variants = 2;
 constexpr int kB2DefaultVariant = 2;
 uint32_t b2_slab_slices(const Lat& L, int is_f32);

@@ -464,12 +464,11 @@ __global__ void __launch_bounds__(kRW) ens_gather_kernel(const EnsEntry* __restr
 }
 
 // ---- one plane's field strength, per site.  A plane with x runs on the field; (z, y), (z, t) and
-// (y, t) on a copy of their two links with z or y fastest, whose lattice has that extent as its x.
-// 24^3x48 in FP64, us by quadrants -> by tiles (tiles 255, gather 40 to 50, copy 80): (x,y) 512 -> 287,
+// (y, t) on a copy of their two links with z or y fastest, whose lattice has that extent as its x.  FP64
+// fields: F of an FP32 field, handed out in FP64, keeps the rounding of the quadrants.  24^3x48, us by quadrants -> by tiles (tiles 255, gather 40 to 50, copy 80): (x,y) 512 -> 287,
 // (x,z) 447 -> 272, (x,t) 512 -> 297, (z,y) 469 -> 355, (z,t), (y,t) 452 -> 350.  The tiles run at the
 // FP64 rate of the whole form (matrix products, one wave per SIMD); one plane alone ends in a partly
-// filled last round.  FP32 carries whole rows here: 138 us against 132 with two, and an error of F of
-// 1.64e-7 (rms, of F's) against 1.86e-7 with two and 1.81e-7 by quadrants.
+// filled last round.
 
 // the links of the copy, and the flag of links that are not unitary cleared (the copy's or, alone,
 // block 0's work)
@@ -480,14 +479,14 @@ __global__ void __launch_bounds__(256) plane_copy_kernel(Lat L, int a, int mu0, 
     if (P) relayout<R, T>(L, a, mu0, mu1, blockIdx.x, U, P);
 }
 
-template <typename FV, bool C2, int WPE, bool CHECK, bool TIME>
-__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+template <typename FV, bool TIME>
+__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
 plane_kernel(Lat L, FV f, int rp, PlaneTiles g, typename FV::real* __restrict__ fpout, uint32_t* __restrict__ bad) {
     using R = typename FV::real;
     __shared__ __align__(16) R fp[kCellReals<R> * kTileStride<R, 0>];
-    if (given_up<CHECK>(bad)) return;
+    if (given_up<true>(bad)) return;
     const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
-    rect_tile<C2, WPE, 0, CHECK, TIME>(L, f, rp, g, tile, fp, fpout + 9 * (uint64_t)tile * g.fc, true, bad);
+    rect_tile<false, 1, 0, true, TIME>(L, f, rp, g, tile, fp, fpout + 9 * (uint64_t)tile * g.fc, true, bad);
 }
 
 // F of every site from the footprints, in an array whose t is dense: a block has 16 x and 16 t at fixed
@@ -564,7 +563,12 @@ struct FPlane {
     bool first_is_zero;     // the copy's first block is its lattice's direction 0, else 1
 };
 
+bool rect_by16(const Lat& L) { return L.n[1] % 16 == 0 && L.n[2] % 16 == 0 && L.n[3] % 16 == 0; }
+
+// (FP32 keeps 16 x 16 tiles on extents that they divide: the order of a site's FP32 sum, with it 1e-9 of B
+// of few sites, goes with the tiles)
 RectTiles rect_tiles_of(const Lat& L, int is_f32) {
+    if (is_f32 && rect_by16(L)) return rect_split(L, 19 * 19, 1);
     return rect_split(L, is_f32 ? kMaxCells<float> : kMaxCells<double>, is_f32 ? 2048 : 1024);
 }
 
@@ -583,9 +587,14 @@ RectTiles rect_tiles_of(const Lat& L, int is_f32) {
 //   48^3x96                    10.6  / 18.8  / 16.8    ->   6.26  / 11.4  / 11.0
 constexpr uint32_t kRectSites = 90000;
 bool rect_fits(const Lat& L) {
-    if (L.n[1] % 16 == 0 && L.n[2] % 16 == 0 && L.n[3] % 16 == 0) return true;
+    if (rect_by16(L)) return true;
     return std::min({L.n[1], L.n[2], L.n[3]}) >= 12 && L.V >= kRectSites;
 }
+
+// Untuned, FP32 lattices of other extents take it from 200,000 sites on: the two forms round B apart by
+// 3e-10 and 1e-7 over the root of the sites.
+constexpr uint32_t kRectSitesF32 = 200000;
+bool rect_untuned(const Lat& L, int is_f32) { return !is_f32 || rect_by16(L) || L.V >= kRectSitesF32; }
 
 uint32_t rect_partials(const Lat& L, int is_f32) {
     const RectTiles r = rect_tiles_of(L, is_f32);
@@ -689,7 +698,7 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
     }
     g->tiles = (uint32_t)tiles;
     g->copies = (uint32_t)copies;
-    return sites >= kRectSites && tiles < 0x80000000ull && copies < 0x80000000ull;
+    return sites >= (is_f32 ? kRectSitesF32 : kRectSites) && tiles < 0x80000000ull && copies < 0x80000000ull;
 }
 
 hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, const EnsRectGrid& g, const void* fld,
@@ -724,11 +733,10 @@ hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, cons
 }
 
 // Planes with both extents of 12 or more on lattices of 90000 sites or more, as measured (us by quadrants
-// -> by tiles): 20^3x12 FP64 82 -> 57 and, on a copy, 78 -> 73, FP32 54 -> 38 and 53 -> 47; 16^3x24 FP64
-// 81 -> 54 and 75 -> 66, FP32 54 -> 35 and 50 -> 45.  Below, two and a half thousand tiles do not fill the
+// -> by tiles): 20^3x12 82 -> 57 and, on a copy, 78 -> 73; 16^3x24 81 -> 54 and 75 -> 66.  Below, two and a half thousand tiles do not fill the
 // chip's slots, and the three or four launches outweigh the products saved.
-static bool f_plane(const Lat& L, int is_f32, int mu, int nu, FPlane* p) {
-    if (mu == nu || !fits_buffer(L.V, is_f32) || L.V < kRectSites || std::min(L.n[mu], L.n[nu]) < 12) return false;
+static bool f_plane(const Lat& L, int mu, int nu, FPlane* p) {
+    if (mu == nu || !fits_buffer(L.V, 0) || L.V < kRectSites || std::min(L.n[mu], L.n[nu]) < 12) return false;
     auto has = [&](int d) { return mu == d || nu == d; };
     const int32_t yfast[4] = {L.n[0], L.n[2], L.n[1], L.n[3]};
     p->first_is_zero = has(0);
@@ -751,22 +759,22 @@ static bool f_plane(const Lat& L, int is_f32, int mu, int nu, FPlane* p) {
     p->rp = p->d2 == 0 ? 2 : (p->d1 == 1 && p->d2 == 3 ? 1 : 0);
     const uint32_t NX = (uint32_t)p->L.n[1], NY = (uint32_t)p->L.n[2], NZ = (uint32_t)p->L.n[3], NT = (uint32_t)L.n[0];
     const uint32_t n2 = p->rp == 0 ? NY : (p->rp == 1 ? NZ : NT), s1 = p->rp == 0 ? NZ : NY, s2 = p->rp == 2 ? NZ : NT;
-    p->g = plane_split(NX, n2, s1, s2, is_f32 ? kMaxCells<float> : kMaxCells<double>, is_f32 ? 2048 : 1024, s2);
-    const size_t sz = is_f32 ? 4 : 8;
+    p->g = plane_split(NX, n2, s1, s2, kMaxCells<double>, 1024, s2);
+    const size_t sz = sizeof(double);
     p->copy_at = ((size_t)p->g.tiles * p->g.fc * 9 * sz + 255) & ~(size_t)255;
     p->bytes = p->copy_at + (p->mu0 >= 0 ? (size_t)36 * L.V * sz : 0) + 256;
     return true;
 }
 
-size_t fmunu_rect_bytes(const Lat& L, int is_f32, int mu, int nu) {
+size_t fmunu_rect_bytes(const Lat& L, int mu, int nu) {
     FPlane p;
-    return f_plane(L, is_f32, mu, nu, &p) ? p.bytes : 0;
+    return f_plane(L, mu, nu, &p) ? p.bytes : 0;
 }
 
-hipError_t launch_fmunu_rect(const Lat& L, const void* U, int is_f32, int mu, int nu, void* out, const int64_t s6[6],
-                             void* ws, hipStream_t st) {
+hipError_t launch_fmunu_rect(const Lat& L, const void* U, int mu, int nu, void* out, const int64_t s6[6], void* ws,
+                             hipStream_t st) {
     FPlane p;
-    if (!f_plane(L, is_f32, mu, nu, &p) || s6[0] != 1) return hipErrorInvalidValue;
+    if (!f_plane(L, mu, nu, &p) || s6[0] != 1) return hipErrorInvalidValue;
     const OutStrides os{s6[0], s6[1], s6[2], s6[3], s6[4], s6[5]};
     // the strides along the directions of p.L
     OutStrides osl = os;
@@ -774,37 +782,32 @@ hipError_t launch_fmunu_rect(const Lat& L, const void* U, int is_f32, int mu, in
         osl.x = p.d1 == 3 ? os.z : os.y;
         (p.d1 == 3 ? osl.z : osl.y) = os.x;
     }
-    with_view(L.V, U, is_f32, [&](auto f) {
-        using F = decltype(f);
-        using R = typename F::real;
-        if constexpr (F::buffered) {
-            R* fp = (R*)ws;
-            R* P = p.mu0 >= 0 ? (R*)((char*)ws + p.copy_at) : nullptr;
-            uint32_t* bad = (uint32_t*)((char*)ws + p.bytes - 256);
-            const int a = p.d1 == 1 ? 2 : p.d1;
-            if (P && relayout_edge(L, a) == 16)
-                plane_copy_kernel<R, 16><<<relayout_blocks(L, a, 16), 256, 0, st>>>(L, a, p.mu0, p.mu1, f.p, P, bad);
-            else
-                plane_copy_kernel<R, 8>
-                    <<<P ? relayout_blocks(L, a, 8) : 1, 256, 0, st>>>(L, a, p.mu0, p.mu1, f.p, P, bad);
-            // the copy's two blocks are directions 0 and 1 of its lattice, or 1 and 2
-            const F fl{P ? (p.first_is_zero ? P : zy_view<R>(P, L.V)) : f.p, L.V};
-            constexpr bool F32 = sizeof(R) == 4;
-            const R sign = mu == p.d1 ? R(1) : R(-1);
-            auto run = [&](auto time) {
-                constexpr bool TIME = decltype(time)::value;
-                plane_kernel<F, false, F32 ? 2 : 1, !F32, TIME><<<p.g.tiles, kRW, 0, st>>>(p.L, fl, p.rp, p.g, fp, bad);
-                const uint32_t nb = (uint32_t)((p.L.n[0] + kFT - 1) / kFT) * (uint32_t)((p.L.n[1] + kFT - 1) / kFT) *
-                                    (uint32_t)p.L.n[2] * (uint32_t)p.L.n[3];
-                plane_gather_kernel<R, TIME><<<nb, kFT * kFT, 0, st>>>(p.L, p.rp, p.g, fp, sign, (double*)out, osl);
-            };
-            if (p.rp == 2)
-                run(std::true_type());
-            else
-                run(std::false_type());
-            if constexpr (!F32) plane_general_kernel<<<kGeneralGrid, kRW, 0, st>>>(L, f, mu, nu, bad, (double*)out, os);
-        }
-    });
+    using F = FieldView<double, true>;
+    const F f{(const double*)U, L.V};
+    double* fp = (double*)ws;
+    double* P = p.mu0 >= 0 ? (double*)((char*)ws + p.copy_at) : nullptr;
+    uint32_t* bad = (uint32_t*)((char*)ws + p.bytes - 256);
+    const int a = p.d1 == 1 ? 2 : p.d1;
+    if (P && relayout_edge(L, a) == 16)
+        plane_copy_kernel<double, 16><<<relayout_blocks(L, a, 16), 256, 0, st>>>(L, a, p.mu0, p.mu1, f.p, P, bad);
+    else
+        plane_copy_kernel<double, 8>
+            <<<P ? relayout_blocks(L, a, 8) : 1, 256, 0, st>>>(L, a, p.mu0, p.mu1, f.p, P, bad);
+    // the copy's two blocks are directions 0 and 1 of its lattice, or 1 and 2
+    const F fl{P ? (p.first_is_zero ? P : zy_view<double>(P, L.V)) : f.p, L.V};
+    const double sign = mu == p.d1 ? 1.0 : -1.0;
+    auto run = [&](auto time) {
+        constexpr bool TIME = decltype(time)::value;
+        plane_kernel<F, TIME><<<p.g.tiles, kRW, 0, st>>>(p.L, fl, p.rp, p.g, fp, bad);
+        const uint32_t nb = (uint32_t)((p.L.n[0] + kFT - 1) / kFT) * (uint32_t)((p.L.n[1] + kFT - 1) / kFT) *
+                            (uint32_t)p.L.n[2] * (uint32_t)p.L.n[3];
+        plane_gather_kernel<double, TIME><<<nb, kFT * kFT, 0, st>>>(p.L, p.rp, p.g, fp, sign, (double*)out, osl);
+    };
+    if (p.rp == 2)
+        run(std::true_type());
+    else
+        run(std::false_type());
+    plane_general_kernel<<<kGeneralGrid, kRW, 0, st>>>(L, f, mu, nu, bad, (double*)out, os);
     return hipGetLastError();
 }
 

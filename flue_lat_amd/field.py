@@ -370,8 +370,8 @@ class GaugeField:
     def magnetic_grad(self, variant=0):
         """Lie gradient of the magnetic B (temporal links get 0).  Needs SU(3) links in every
         precision: the library checks them first and FlueError (FLUE_ESU3) is raised for a
-        field that fails the check.  variant: 1 = per-link gather, 2 = reverse mode,
-        0 = tuned or reverse mode."""
+        field that fails the check.  variant: 1 = per-link gather, 2 = reverse mode
+        with slots, 0 = tuned or reverse mode (on tiles where they apply)."""
         g = self._like()
         n = _lib.lib().flue_b2_work_bytes(self._cdims, self.prec)
         work = torch.empty(n, dtype=torch.uint8, device=self.device)

@@ -254,8 +254,8 @@ int flue_fmunu(const int32_t dims[4], const void* U, int32_t prec, int32_t mu, i
                void* out, int32_t layout, const int64_t strides[6], void* stream);
 
 /* the same given a workspace of flue_fmunu_work_bytes: where both extents of the plane are 12
- * or more on a lattice of 90,000 sites or more, variant 0 into a strided array with stride 1
- * along t forms each rectangle once, as variant 7 of flue_magnetic_ex does (FLUE_F64 links
+ * or more on a lattice of 90,000 sites or more, variant 0 of an FP64 field into a strided array
+ * with stride 1 along t forms each rectangle once, as variant 7 of flue_magnetic_ex does (links
  * that are not unitary are found on the way and take the quadrants); the two forms agree to
  * rounding.  Elsewhere work_bytes is 0 and ws is not used. */
 size_t flue_fmunu_work_bytes(const int32_t dims[4], int32_t prec, int32_t mu, int32_t nu);
@@ -356,7 +356,9 @@ int flue_wilson_grad_ex(const int32_t dims[4], const void* U, int32_t prec, doub
                         void* ws, size_t ws_bytes, void* stream);
 
 /* flue_b2_grad with an explicit form: 1 = per-link gather, 2 = reverse mode (each leaf
- * rectangle walked once, its terms summed per link from fixed slots); 0 = tuned or 2 */
+ * rectangle walked once, its terms summed per link from fixed slots); 0 = tuned or 2.  As the
+ * tuned or untuned form, reverse mode sums the terms on tiles where variant 7 of
+ * flue_magnetic_ex applies */
 int flue_b2_grad_ex(const int32_t dims[4], const void* U, int32_t prec, int32_t variant, void* grad, void* work,
                     size_t work_bytes, void* stream);
 
@@ -403,7 +405,7 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
 /* bit-identical results, the others agree to rounding (their summation orders differ).    */
 /*   FLUE_OP_MAGNETIC       1..7  kernel form x waves per SIMD, or rectangle-first (7, timed  */
 /*                                only where it applies) (flue_magnetic_ex)                 */
-/*   FLUE_OP_B2_GRAD        1..2  per-link gather / reverse mode with slots (flue_b2_grad_ex) */
+/*   FLUE_OP_B2_GRAD        1..2  per-link gather / reverse mode (flue_b2_grad_ex)            */
 /*   FLUE_OP_PLAQUETTE      1..6  time slices per thread 2, 3, 4, 6, 8, 12 (flue_plaquette,   */
 /*                                flue_wilson_action)                                        */
 /*   FLUE_OP_FLOW          1..13  stencil of the flow and the Wilson gradient: staple sums   */

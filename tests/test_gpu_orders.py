@@ -7,6 +7,7 @@ is compared with the staple sums: both are FP64-accurate per stage, and links di
 rounding of the force times the step, far below 1e-12 (FP64) and 2e-6 (FP32 links: a few
 roundings of a unit entry, the bound the flow's other tests use).
 """
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,29 @@ def test_untuned_flow_matches_staple_sums(FL, tmp_path, dims, prec, tol):
     untuned = flowed(f, 3)
     force(FL, tmp_path, dims, prec, 1)
     assert float((untuned - flowed(f, 3)).abs().max()) < tol
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 1e-6)])
+@pytest.mark.parametrize("dims", [(1, 1, 1, 1), (2, 3, 1, 5), (16, 8, 8, 8), (5, 13, 16, 16), (9, 29, 31, 33), (64, 16, 16, 17)])
+def test_untuned_plaquette(FL, dims, prec, tol):
+    # the untuned forms by size (a thread per site and plane, walks of 2 to 6 slices), for every range
+    # of planes, against the loops walked link by link
+    f = FL.GaugeField.random(dims, 6, 0.3, prec)
+    loop = {(mu, nu): f.wilson_loop(mu, nu, 1, 1) for mu in range(1, 5) for nu in range(mu + 1, 5)}
+    V = np.prod(dims)
+    for mu0 in range(1, 5):
+        for mu1 in range(1, 5):
+            for nu1 in range(1, 5):
+                want = V * sum(v for (mu, nu), v in loop.items() if mu0 <= mu <= mu1 and nu <= nu1)
+                assert abs(f.plaquette(mu0, mu1, nu1)[0] - want) <= tol * 18 * V, (mu0, mu1, nu1)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp64-su3", 1e-13), ("fp32", 1e-7)])
+@pytest.mark.parametrize("dims", [(1, 1, 1, 1), (1, 2, 3, 4), (3, 3, 7, 1), (4, 4, 4, 4), (13, 5, 5, 13), (16, 10, 8, 8),
+                                  (4, 16, 16, 16), (5, 16, 16, 16)])
+def test_untuned_magnetic_of_small_lattices(FL, dims, prec, tol):
+    # a wave per quadrant, partial blocks of 64 sites and the sizes at which other forms take over,
+    # against a thread per site.  FP32: the four parts of a site round at 2^-24 once more each.
+    f = FL.GaugeField.random(dims, 8, 0.3, "fp64").astype(prec)
+    want = f.magnetic(variant=1)
+    assert abs(f.magnetic() - want) <= tol * abs(want)
