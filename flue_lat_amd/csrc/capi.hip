@@ -147,7 +147,10 @@ int b2_form(const Lat& L, int32_t prec, int variant) {
 // where it applies, with two-row chains in both precisions since the links are SU(3)), then
 // variant 1 (per-link gather), 2 (reverse mode with slots) or kB2Tiled
 int b2_grad_run(const Lat& L, const void* U, int32_t prec, int variant, void* work, void* grad, hipStream_t st) {
-    const int f32 = prec == FLUE_F32, rect = magnetic_rect_ok(L, prec), tiled = variant == kB2Tiled;
+    // (FP32, beside the tiled form, keeps the quadrants where the tiles are not 16 x 16: their order of
+    // summation)
+    const int f32 = prec == FLUE_F32, tiled = variant == kB2Tiled;
+    const bool rect = tiled || (magnetic_rect_ok(L, prec) && (!f32 || rect_by16(L)));
     char* region = (char*)work + b2_ah_bytes(L, prec);
     const size_t copy_at = rect ? b2_copy_at(L, prec) : 0;
     if (rect)
@@ -305,9 +308,11 @@ int load_host_field(const int32_t* NT, const int32_t* NX, const int32_t* NY, con
         lo = 0;
         hi = 3;
     }
-    // in the array, the directions of an (a, b) follow each other
+    // In the array, the directions of an (a, b) follow each other.  (Room for all four whatever is copied: the
+    // runtime keeps a released allocation for the next of its size, and a program's calls on one lattice,
+    // each of another size, took 0.3 ms more.)
     const size_t n = (size_t)(hi - lo + 1), dir = (size_t)h.L.V * sizeof(flue_c128);
-    const size_t soa = align256(flue_field_bytes(h.dims, FLUE_F64)), raw = align256(9 * n * dir);
+    const size_t soa = align256(flue_field_bytes(h.dims, FLUE_F64)), raw = align256(36 * dir);
     FLUE_TRY(hipMalloc(&h.mem.p, soa + raw + 256));
     h.soa = h.mem.p;
     char* array = (char*)h.mem.p + soa;

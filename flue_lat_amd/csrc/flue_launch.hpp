@@ -113,6 +113,7 @@ bool quad_fits(const Lat& L, int is_f32);
 uint32_t quad_blocks(const Lat& L);
 hipError_t launch_magnetic_quad(const Lat& L, const void* U, int su3, double* partials, hipStream_t st, uint32_t* npart);
 bool rect_fits(const Lat& L);
+bool rect_by16(const Lat& L);  // spatial extents multiples of 16
 // whether it is the untuned form
 bool rect_untuned(const Lat& L, int is_f32);
 // partials of variant 7: one per tile of its three planes

@@ -563,7 +563,11 @@ struct FPlane {
     bool first_is_zero;     // the copy's first block is its lattice's direction 0, else 1
 };
 
+}  // namespace
+
 bool rect_by16(const Lat& L) { return L.n[1] % 16 == 0 && L.n[2] % 16 == 0 && L.n[3] % 16 == 0; }
+
+namespace {
 
 // (FP32 keeps 16 x 16 tiles on extents that they divide: the order of a site's FP32 sum, with it 1e-9 of B
 // of few sites, goes with the tiles)
@@ -591,9 +595,9 @@ bool rect_fits(const Lat& L) {
     return std::min({L.n[1], L.n[2], L.n[3]}) >= 12 && L.V >= kRectSites;
 }
 
-// Untuned, FP32 lattices of other extents take it from 200,000 sites on: the two forms round B apart by
+// Untuned, FP32 lattices of other extents take it from 300,000 sites on: the two forms round B apart by
 // 3e-10 and 1e-7 over the root of the sites.
-constexpr uint32_t kRectSitesF32 = 200000;
+constexpr uint32_t kRectSitesF32 = 300000;
 bool rect_untuned(const Lat& L, int is_f32) { return !is_f32 || rect_by16(L) || L.V >= kRectSitesF32; }
 
 uint32_t rect_partials(const Lat& L, int is_f32) {
