@@ -158,7 +158,7 @@ def ensemble_leg(FL, torch):
            "measure_every": 10}
     for prec in ("fp32", "fp64"):
         e = Ensemble.random(dims, seeds, 0.4, prec)
-        grid_variant = e.autotune(reps=2)[0]   # persistent grid, chosen on this ensemble
+        grid_variant = e.autotune(reps=2)[0]   # stencil, chosen on this ensemble
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         plaq, B = e.flow(0.01, 100, measure_every=10, use_graph=True)

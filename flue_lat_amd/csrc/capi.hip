@@ -1193,17 +1193,6 @@ void ens_key(const EnsPlan& p, int32_t n, int32_t key[4]) {
     key[3] = 0;
 }
 
-// persistent grid of the ensemble kernels: 1, 2, 4 or 8 workgroups per CU (variant 1..4, and
-// 5..8 with the plaquette-first stencil)
-int ens_grid(const EnsPlan& p, int variant, uint32_t* grid) {
-    int dev = 0, cus = 0;
-    FLUE_TRY(hipGetDevice(&dev));
-    FLUE_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const uint32_t per_cu = 1u << ((variant - 1) % 4);
-    *grid = std::max<uint32_t>(1, std::min<uint32_t>(p.total_blocks, (uint32_t)std::max(cus, 1) * per_cu));
-    return FLUE_OK;
-}
-
 // the ensemble work buffer: tables, second link buffer, accumulators (room for FP64), partial sums, and
 // the plaquette parts of the plaquette-first stencil
 struct EnsWork {
@@ -1293,8 +1282,6 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
     int32_t key[4];
     ens_key(p, n, key);
     const int variant = variant_or(FLUE_OP_ENSEMBLE_FLOW, key, prec, ensemble_default(p.field_reals / kPlanes));
-    uint32_t grid = 0;
-    if ((rc = ens_grid(p, variant, &grid))) return rc;
     void* T = variant > 4 ? ew.T : nullptr;  // the plaquette-first variants
 
     static const double ca[3] = {0.0, -17.0 / 9.0, -1.0};
@@ -1305,13 +1292,13 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
     // copies, partials (2 doubles for 4 x 4 sites at least, of 32 a site) and footprints there.
     auto measure = [&](int b, int m) -> hipError_t {
         const void* fld = bufs[b];
-        hipError_t e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 0, partials, grid, st);
+        hipError_t e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 0, partials, st);
         if (e == hipSuccess) e = launch_ens_finalize(d_tab, nullptr, n, partials, d_plaq + (size_t)m * n, 1, 0, st);
         if (e != hipSuccess) return e;
         if (tiled)
             e = launch_ens_rect(d_tab, ew.rect, n, rect_grid, fld, is_f32, bufs[b ^ 1], ew.T, acc, st);
         else
-            e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 1, partials, grid, st);
+            e = launch_ens_sum(d_tab, n, p.total_blocks, p.maxV, fld, is_f32, 1, partials, st);
         if (e == hipSuccess)
             e = launch_ens_finalize(d_tab, tiled ? ew.rect : nullptr, n, tiled ? acc : partials, d_B + (size_t)m * n, 1,
                                     1, st);
@@ -1325,7 +1312,7 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
             for (int k = 0; k < 3 && e == hipSuccess; ++k) {
                 const int q = 3 * j + k;
                 e = launch_ens_flow_stage(d_tab, n, p.total_blocks, p.maxV, bufs[q & 1], is_f32, bufs[(q + 1) & 1], acc,
-                                          eps, ca[k], cb[k], k == 2, grid, T, st);
+                                          eps, ca[k], cb[k], k == 2, T, st);
             }
             if (e == hipSuccess && nmeas > 0 && (j + 1) % measure_every == 0)
                 e = measure((j + 1) & 1, (j + 1) / measure_every);
@@ -1377,11 +1364,8 @@ int flue_ensemble_autotune(int32_t n, const int32_t* dims, const void* fields, i
     // the first RK3 stage of every field into the second buffer (the fields are not changed;
     // it only writes the accumulator, so repeated calls do not drift, as flue_autotune)
     auto launch = [&](int v) -> int {
-        uint32_t grid = 0;
-        int r = ens_grid(p, v, &grid);
-        if (r) return r;
         return hip_status(launch_ens_flow_stage(ew.tab, n, p.total_blocks, p.maxV, fields, is_f32, ew.W2, ew.acc, 0.01,
-                                                0.0, 0.25, 0, grid, v > 4 ? ew.T : nullptr, st));
+                                                0.0, 0.25, 0, v > 4 ? ew.T : nullptr, st));
     };
     int bv = 0;
     double bms = 0.0;

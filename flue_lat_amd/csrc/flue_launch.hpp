@@ -195,9 +195,9 @@ struct EnsRect {
 // (48 reals per site, field c's at 2/3 of its field offset); T == nullptr: staple sums
 hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* win,
                                  int is_f32, void* wout, void* acc, double eps, double ca, double cb, int reunit,
-                                 uint32_t grid, void* T, hipStream_t st);
+                                 void* T, hipStream_t st);
 hipError_t launch_ens_sum(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* fld, int is_f32,
-                          int obs, double* partials, uint32_t grid, hipStream_t st);
+                          int obs, double* partials, hipStream_t st);
 // the partials of configuration c: its logical blocks', or its tiles' with rect
 hipError_t launch_ens_finalize(const EnsEntry* tab, const EnsRect* rect, int n, const double* partials, double* out,
                                int stride, int per_volume, hipStream_t st);
@@ -215,12 +215,11 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
 hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, const EnsRectGrid& g, const void* fld,
                            int is_f32, void* copy, void* fp, double* partials, hipStream_t st);
 hipError_t launch_copy(size_t n_reals, int is_f32, const void* src, void* dst, hipStream_t st);
-// ensemble flow variants: persistent grid of 1, 2, 4 or 8 workgroups per CU with the staple
-// stencil (1..4) or the plaquette-first stencil (5..8)
+// ensemble flow variants: the staple stencil (1..4) or the plaquette-first one (5..8), each a single form
 constexpr int kEnsembleVariants = 8;
-// the untuned variant for a number of sites: below 32768 the staple stencil on 4 workgroups per
-// CU (25,000 sites in three fields, ms a stage: 0.056 against 0.063 FP32), else plaquette-first
-// (2.6 M sites in 16 fields: 1.76 -> 1.20 FP32, 3.77 -> 2.00 FP64)
+// the untuned variant for a number of sites: below 32768 the staple stencil (ms a stage, staple sums
+// against plaquette-first: 2,048 sites 0.0095 and 0.0139, 16,384 0.0125 and 0.0156, 24,576 0.0193 and
+// 0.0182 FP64), else plaquette-first (2.6 M sites in 16 fields: 1.39 and 0.92 FP32, 1.99 and 1.67 FP64)
 constexpr int ensemble_default(uint64_t sites) { return sites < 32768 ? 3 : 7; }
 
 }  // namespace flue

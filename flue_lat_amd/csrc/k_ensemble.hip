@@ -2,11 +2,14 @@
 // launch per operation: the RK3 flow stage, the plaquette sum and the magnetic B.
 //
 // The fields lie back to back, each in the SoA layout of its own lattice.  Every
-// configuration owns a contiguous range of logical blocks (256 sites each); a persistent
-// grid walks the logical blocks in contiguous chunks per workgroup (chunks of one XCD
-// adjacent), finds the configuration of a logical block by binary search in a table
-// kept in device memory, and runs the same per-site (flow: per-link) code as the
-// single-field kernels.
+// configuration owns a contiguous range of logical blocks (256 sites each).  A workgroup takes a logical
+// block (or a quarter or a direction of one), finds its configuration by binary search in a table kept in
+// device memory, and runs the same per-site (flow: per-link) code as the single-field kernels.  The
+// logical blocks of an XCD are contiguous, so those running together share
+// their links in L2, and one block per workgroup leaves the registers to the stencil: 16 fields of 16^3
+// with 644 time slices, FP32, a plaquette-first flow stage 1.32 -> 0.97 ms and a plaquette sum
+// 0.51 -> 0.36 ms against a persistent grid of contiguous chunks (86 registers and 5 waves per SIMD, now 72
+// and 7).
 // Sums are reduced per logical block and then per configuration in a fixed order.  (B takes the
 // rectangle-first tiles of k_rect.hip where they apply, one launch for every tile of the ensemble.)
 #include "flue_clover.hpp"
@@ -42,102 +45,72 @@ __device__ __forceinline__ int find_cfg(const EnsEntry* __restrict__ tab, int n,
     return lo;
 }
 
-// logical blocks [lo, hi) of this workgroup: chunks of `chunk` blocks (chunk = total /
-// gridDim rounded up, from the host).  No division here: a division would be lowered to
-// vector instructions, and every value derived from it -- the configuration entry and
-// each buffer descriptor -- would then leave scalar registers.
-__device__ __forceinline__ void my_range(uint32_t total, uint32_t chunk, uint32_t& lo, uint32_t& hi) {
-    const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
-    const uint64_t l = (uint64_t)b * chunk;
-    lo = l < total ? (uint32_t)l : total;
-    hi = total - lo > chunk ? lo + chunk : total;
-}
-
+// Workgroups are (logical block, direction), direction fastest: one thread per link, and the four of a
+// block, which read the same neighbour links, run close together.
 template <typename R, bool BUF>
-__global__ void __launch_bounds__(kBS) ens_flow_kernel(const EnsEntry* __restrict__ tab, int n, uint32_t total,
-                                                       uint32_t chunk, const R* __restrict__ win, R* __restrict__ wout,
+__global__ void __launch_bounds__(kBS) ens_flow_kernel(const EnsEntry* __restrict__ tab, int n,
+                                                       const R* __restrict__ win, R* __restrict__ wout,
                                                        R* __restrict__ acc, double eps, double ca, double cb,
                                                        int reunit) {
-    // units = (logical block, direction), direction fastest: one thread per link, and the
-    // four units of a block, which read the same neighbour links, run close together
-    uint32_t lo, hi;
-    my_range(4u * total, chunk, lo, hi);
-    for (uint32_t lu = lo; lu < hi; ++lu) {
-        const uint32_t lb = lu >> 2;
-        const int mu = (int)(lu & 3u);
-        const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
-        const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
-        if (s < e.L.V) {
-            const FieldView<R, BUF> f{win + e.off, e.L.V};
-            int c[4];
-            site_coords(e.L, s, c);
-            flow_link(e.L, f, wout + e.off, acc + e.acc_off, s, c, mu, eps, ca, cb, reunit);
-        }
-    }
+    const uint32_t lu = xcd_block(blockIdx.x, gridDim.x), lb = lu >> 2;
+    const int mu = (int)(lu & 3u);
+    const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
+    const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
+    if (s >= e.L.V) return;
+    const FieldView<R, BUF> f{win + e.off, e.L.V};
+    int c[4];
+    site_coords(e.L, s, c);
+    flow_link(e.L, f, wout + e.off, acc + e.acc_off, s, c, mu, eps, ca, cb, reunit);
 }
 
 // Plaquette-first stencil over the ensemble: the six plaquette parts of every site of every
 // field (48 reals per site, config c's block at 2/3 of its field offset), then the links, the
 // four waves of a workgroup on the four directions of 64 sites.
 template <typename R, bool BUF>
-__global__ void __launch_bounds__(kBS) ens_plaq_ta_kernel(const EnsEntry* __restrict__ tab, int n, uint32_t total,
-                                                          uint32_t chunk, const R* __restrict__ win, R* __restrict__ T) {
-    uint32_t lo, hi;
-    my_range(total, chunk, lo, hi);
-    for (uint32_t lb = lo; lb < hi; ++lb) {
-        const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
-        const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
-        if (s < e.L.V) {
-            const FieldView<R, BUF> f{win + e.off, e.L.V};
-            int c[4];
-            site_coords(e.L, s, c);
-            plaquette_ta_site<true>(e.L, f, s, c, T + e.off / 72 * 48);
-        }
-    }
+__global__ void __launch_bounds__(kBS) ens_plaq_ta_kernel(const EnsEntry* __restrict__ tab, int n,
+                                                          const R* __restrict__ win, R* __restrict__ T) {
+    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
+    const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
+    const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
+    if (s >= e.L.V) return;
+    const FieldView<R, BUF> f{win + e.off, e.L.V};
+    int c[4];
+    site_coords(e.L, s, c);
+    plaquette_ta_site<true>(e.L, f, s, c, T + e.off / 72 * 48);
 }
 
 template <typename R, bool BUF>
-__global__ void __launch_bounds__(kBS) ens_flow_pf_kernel(const EnsEntry* __restrict__ tab, int n, uint32_t total,
-                                                          uint32_t chunk, const R* __restrict__ win,
-                                                          const R* __restrict__ T, R* __restrict__ wout,
-                                                          R* __restrict__ acc, double eps, double ca, double cb,
-                                                          int reunit) {
+__global__ void __launch_bounds__(kBS) ens_flow_pf_kernel(const EnsEntry* __restrict__ tab, int n,
+                                                          const R* __restrict__ win, const R* __restrict__ T,
+                                                          R* __restrict__ wout, R* __restrict__ acc, double eps, double ca,
+                                                          double cb, int reunit) {
     const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    uint32_t lo, hi;
-    my_range(4u * total, chunk, lo, hi);
-    for (uint32_t lu = lo; lu < hi; ++lu) {
-        const uint32_t lb = lu >> 2;
-        const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
-        const uint32_t s = (lb - e.blk0) * kBS + (lu & 3u) * 64u + (threadIdx.x & 63u);
-        if (s < e.L.V) {
-            const FieldView<R, BUF> f{win + e.off, e.L.V};
-            int c[4];
-            site_coords(e.L, s, c);
-            flow_link_pf(e.L, f, T + e.off / 72 * 48, wout + e.off, acc + e.acc_off, s, c, mu, eps, ca, cb, reunit);
-        }
-    }
+    const uint32_t lu = xcd_block(blockIdx.x, gridDim.x), lb = lu >> 2;
+    const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
+    const uint32_t s = (lb - e.blk0) * kBS + (lu & 3u) * 64u + (threadIdx.x & 63u);
+    if (s >= e.L.V) return;
+    const FieldView<R, BUF> f{win + e.off, e.L.V};
+    int c[4];
+    site_coords(e.L, s, c);
+    flow_link_pf(e.L, f, T + e.off / 72 * 48, wout + e.off, acc + e.acc_off, s, c, mu, eps, ca, cb, reunit);
 }
 
 // OBS = 0: sum of ReTr over all 6V plaquettes; OBS = 1: sum of -ReTr F_i^2 (magnetic)
 template <typename R, bool BUF, int OBS>
-__global__ void __launch_bounds__(kBS) ens_sum_kernel(const EnsEntry* __restrict__ tab, int n, uint32_t total,
-                                                      uint32_t chunk, const R* __restrict__ fld, double* __restrict__ partials) {
-    uint32_t lo, hi;
-    my_range(total, chunk, lo, hi);
-    for (uint32_t lb = lo; lb < hi; ++lb) {
-        const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
-        const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
-        double v = 0.0;
-        if (s < e.L.V) {
-            const FieldView<R, BUF> f{fld + e.off, e.L.V};
-            v = OBS == 0 ? plaquette_site(e.L, f, s, 0, 3, 3) : magnetic_site(e.L, f, s);
-        }
-        const DD r = block_sum<kBS>(DD{v, 0.0});
-        if (threadIdx.x == 0) {
-            partials[2 * lb] = r.hi;
-            partials[2 * lb + 1] = r.lo;
-        }
-        __syncthreads();  // block_sum's shared slots are reused by the next logical block
+__global__ void __launch_bounds__(kBS) ens_sum_kernel(const EnsEntry* __restrict__ tab, int n,
+                                                      const R* __restrict__ fld, double* __restrict__ partials) {
+    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
+    const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
+    const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
+    double v = 0.0;
+    if (s < e.L.V) {
+        const FieldView<R, BUF> f{fld + e.off, e.L.V};
+        v = OBS == 0 ? plaquette_site(e.L, f, s, 0, 3, 3) : magnetic_site(e.L, f, s);
+    }
+    const DD r = block_sum<kBS>(DD{v, 0.0});
+    if (threadIdx.x == 0) {
+        partials[2 * lb] = r.hi;
+        partials[2 * lb + 1] = r.lo;
     }
 }
 
@@ -183,33 +156,31 @@ void with_real(int is_f32, bool buf, Fn&& fn) {
 
 hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* win,
                                  int is_f32, void* wout, void* acc, double eps, double ca, double cb, int reunit,
-                                 uint32_t grid, void* T, hipStream_t st) {
+                                 void* T, hipStream_t st) {
     with_real(is_f32, fits_buffer(maxV, is_f32), [&](auto r, auto buf) {
         using R = decltype(r);
         constexpr bool B = decltype(buf)::value;
-        const uint32_t chunk4 = (4u * total + grid - 1) / grid;
         if (T) {
-            ens_plaq_ta_kernel<R, B><<<grid, kBS, 0, st>>>(tab, n, total, (total + grid - 1) / grid, (const R*)win, (R*)T);
-            ens_flow_pf_kernel<R, B><<<grid, kBS, 0, st>>>(tab, n, total, chunk4, (const R*)win, (const R*)T, (R*)wout,
-                                                           (R*)acc, eps, ca, cb, reunit);
+            ens_plaq_ta_kernel<R, B><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T);
+            ens_flow_pf_kernel<R, B><<<4 * total, kBS, 0, st>>>(tab, n, (const R*)win, (const R*)T, (R*)wout, (R*)acc, eps,
+                                                                ca, cb, reunit);
         } else {
-            ens_flow_kernel<R, B><<<grid, kBS, 0, st>>>(tab, n, total, chunk4, (const R*)win, (R*)wout, (R*)acc, eps,
-                                                        ca, cb, reunit);
+            ens_flow_kernel<R, B><<<4 * total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)wout, (R*)acc, eps, ca, cb,
+                                                             reunit);
         }
     });
     return hipGetLastError();
 }
 
 hipError_t launch_ens_sum(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* fld, int is_f32,
-                          int obs, double* partials, uint32_t grid, hipStream_t st) {
-    const uint32_t chunk = (total + grid - 1) / grid;
+                          int obs, double* partials, hipStream_t st) {
     with_real(is_f32, fits_buffer(maxV, is_f32), [&](auto r, auto buf) {
         using R = decltype(r);
         constexpr bool B = decltype(buf)::value;
         if (obs == 0)
-            ens_sum_kernel<R, B, 0><<<grid, kBS, 0, st>>>(tab, n, total, chunk, (const R*)fld, partials);
+            ens_sum_kernel<R, B, 0><<<total, kBS, 0, st>>>(tab, n, (const R*)fld, partials);
         else
-            ens_sum_kernel<R, B, 1><<<grid, kBS, 0, st>>>(tab, n, total, chunk, (const R*)fld, partials);
+            ens_sum_kernel<R, B, 1><<<total, kBS, 0, st>>>(tab, n, (const R*)fld, partials);
     });
     return hipGetLastError();
 }

@@ -670,6 +670,9 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
     return hipGetLastError();
 }
 
+// (FP32: each of enough sites that the forms' B differ by 6e-10 at most)
+constexpr uint32_t kEnsRectSitesF32 = 49152;
+
 // Every configuration has to suit the tiles (extents as in rect_fits) and its footprints to fit the
 // plaquette parts' 48 reals a site; the sites are counted over the ensemble, since it runs as one launch,
 // and the tiles are those that cost least on a full chip.  A measurement (B and the plaquettes), ms by
@@ -687,7 +690,7 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
         if (relayout_edge(tab[c].L, 3) == 8) g->copy_edge = 8;
     for (int c = 0; c < n; ++c) {
         const Lat& L = tab[c].L;
-        if (std::min({L.n[1], L.n[2], L.n[3]}) < 12) return false;
+        if (std::min({L.n[1], L.n[2], L.n[3]}) < 12 || (is_f32 && L.V < kEnsRectSitesF32)) return false;
         EnsRect& r = rect[c];
         r.rt = rect_split(L, is_f32 ? kMaxCells<float> : kMaxCells<double>, 1);
         if (rect_cells(r.rt) * 9 > (uint64_t)48 * L.V) return false;
@@ -702,7 +705,7 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
     }
     g->tiles = (uint32_t)tiles;
     g->copies = (uint32_t)copies;
-    return sites >= (is_f32 ? kRectSitesF32 : kRectSites) && tiles < 0x80000000ull && copies < 0x80000000ull;
+    return sites >= kRectSites && tiles < 0x80000000ull && copies < 0x80000000ull;
 }
 
 hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, const EnsRectGrid& g, const void* fld,

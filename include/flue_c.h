@@ -401,7 +401,7 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
 /* hipEvents on the caller's field; the fastest is remembered per (device, op, precision,  */
 /* extents) and used by every later call of that operation (and by the *_ex entries when  */
 /* their variant argument is 0).  The table persists through save/load.  Variants of one   */
-/* operation compute the same quantity: the flow orders and the ensemble grids give        */
+/* operation compute the same quantity: the flow orders and the ensemble's give            */
 /* bit-identical results, the others agree to rounding (their summation orders differ).    */
 /*   FLUE_OP_MAGNETIC       1..7  kernel form x waves per SIMD, or rectangle-first (7, timed  */
 /*                                only where it applies) (flue_magnetic_ex)                 */
@@ -415,9 +415,9 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
 /*                                in storage order (7), the largest boxes (8) or the five     */
 /*                                box orders (9..13), bit-identical; the two stencils agree   */
 /*                                to rounding                                                 */
-/*   FLUE_OP_ENSEMBLE_FLOW  1..8  persistent grid of 1, 2, 4, 8 workgroups per CU with the   */
-/*                                staple stencil (1..4) or the plaquette-first one (5..8)    */
-/*                                (flue_ensemble_flow; tuned by flue_ensemble_autotune)      */
+/*   FLUE_OP_ENSEMBLE_FLOW  1..8  the staple stencil (1..4, one form) or the plaquette-first  */
+/*                                one (5..8, one form) (flue_ensemble_flow; tuned by          */
+/*                                flue_ensemble_autotune)                                    */
 /* ------------------------------------------------------------------ */
 enum { FLUE_OP_MAGNETIC = 0, FLUE_OP_B2_GRAD = 1, FLUE_OP_PLAQUETTE = 2, FLUE_OP_FLOW = 3, FLUE_OP_ENSEMBLE_FLOW = 4 };
 /* device bytes flue_autotune needs as `ws` for op (0 for an invalid op) */
