@@ -279,11 +279,12 @@ double now_s() {
 }
 
 // host drop-in prologue: dims by reference, field copied to the device as FP64 SoA; one allocation for
-// the planes, the array as it came and a scalar result
+// the planes, the array as it came and a scalar result (two where the array is below 2 MiB: the runtime
+// serves those from a block it holds)
 struct HostField {
     int32_t dims[4];
     Lat L;
-    DevBuf mem;
+    DevBuf mem, arr;
     void* soa;
     double* scalar;
 };
@@ -313,10 +314,12 @@ int load_host_field(const int32_t* NT, const int32_t* NX, const int32_t* NY, con
     // each of another size, took 0.3 ms more.)
     const size_t n = (size_t)(hi - lo + 1), dir = (size_t)h.L.V * sizeof(flue_c128);
     const size_t soa = align256(flue_field_bytes(h.dims, FLUE_F64)), raw = align256(36 * dir);
-    FLUE_TRY(hipMalloc(&h.mem.p, soa + raw + 256));
+    const bool apart = raw < (size_t)2 << 20;
+    FLUE_TRY(hipMalloc(&h.mem.p, soa + (apart ? 0 : raw) + 256));
+    if (apart) FLUE_TRY(hipMalloc(&h.arr.p, raw));
     h.soa = h.mem.p;
-    char* array = (char*)h.mem.p + soa;
-    h.scalar = (double*)(array + raw);
+    char* array = apart ? (char*)h.arr.p : (char*)h.mem.p + soa;
+    h.scalar = (double*)((char*)h.mem.p + soa + (apart ? 0 : raw));
     if (n == 4)
         FLUE_TRY(hipMemcpy(array, data, 36 * dir, hipMemcpyHostToDevice));
     else
