@@ -164,7 +164,10 @@ __global__ void __launch_bounds__(256) tangent_kernel(Lat L, ArrayLayout l, cons
     }
 }
 
-// kArrayPlanes: a 32 x 32 tile of (f, x); blockIdx.y is the link direction
+// kArrayPlanes: a 32 x 32 tile of (f, x); blockIdx.y is a row of a link.  Bound by memory, and by the chain
+// of a block's planes where the lattice is small.  FP64 import with 9 / 3 / 1 planes a block: 9x6x9x6 8.7 /
+// 5.6 / 5.8 us, 16^4 19.0 / 17.3 / 21.1, 24^3x48 168 / 156 / 147, 48^3x96 2514 / 2468 / 2450; FP32 of
+// complex64 there 1387 / 1380 / 1509.
 template <bool IN, typename Ra, typename Rf>
 __global__ void __launch_bounds__(256) plane_tile_kernel(Lat L, ArrayLayout l, Pair<Ra>* __restrict__ arr,
                                                          Pair<Rf>* __restrict__ fld) {
@@ -175,7 +178,7 @@ __global__ void __launch_bounds__(256) plane_tile_kernel(Lat L, ArrayLayout l, P
     const int nx = L.n[1] - c0[1], nf = L.ext(l.f) - f0;
     const int j = (int)threadIdx.x & 31, i0 = (int)threadIdx.x >> 5;
 #pragma unroll 1
-    for (int e = (int)blockIdx.y * 9; e < (int)blockIdx.y * 9 + 9; ++e) {
+    for (int e = (int)blockIdx.y * 3; e < (int)blockIdx.y * 3 + 3; ++e) {
         Pair<Ra>* a = arr + element_offset(l, e);
         Pair<Rf>* p = fld + (size_t)e * L.V;
         // array side: f along the lanes; field side: x along the lanes
@@ -471,7 +474,7 @@ static hipError_t convert_layout(const Lat& L, int order, const ArrayLayout& l, 
         site_block_kernel<IN, Ra, Rf><<<g, 256, 0, st>>>(L, l, a, p);
     } else if (order == kArrayPlanes) {
         const uint32_t g = ((uint32_t)L.n[1] + 31) / 32 * (((uint32_t)L.ext(l.f) + 31) / 32) * rest;
-        plane_tile_kernel<IN, Ra, Rf><<<dim3(g, ndir), 256, 0, st>>>(L, l, a, p);
+        plane_tile_kernel<IN, Ra, Rf><<<dim3(g, 3 * ndir), 256, 0, st>>>(L, l, a, p);
     } else {
         row_kernel<IN, Ra, Rf><<<dim3(grid_for(L.V), ndir), 256, 0, st>>>(L, l, a, p);
     }
