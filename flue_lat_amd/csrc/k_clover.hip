@@ -121,25 +121,30 @@ magnetic_kernel(Lat L, FV f, PlaneOrder po, uint32_t nb, double* __restrict__ pa
 // planes (element e = a*3+b, re/im) in the field precision.
 template <typename FV, bool CLOVER>
 __global__ void __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(sizeof(typename FV::real) == 4 ? 2 : 1)))
-fmunu_kernel(Lat L, FV f, int mu, int nu, void* __restrict__ out, int layout, OutStrides os) {
+fmunu_kernel(Lat L, FV f, int mu, int nu, void* __restrict__ out, int layout, OutStrides os, uint32_t unit,
+             uint32_t tb) {
     using R = typename FV::real;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    // planes (x, z): each slice taken along z; planes containing time: along their spatial direction
+    const int d = mu == 0 || nu == 0 ? mu + nu : (mu + nu == 4 ? 3 : 1);
     uint32_t s;
-    if (mu == 0 || nu == 0) {
-        // the leaves reach 3 slices either way: blocks take the same sites of consecutive
-        // slices one after another, so the blocks running together share those slices in L2
-        const uint32_t NT = (uint32_t)L.n[0];
-        const uint32_t chunk = blk / NT, t = blk - chunk * NT;
-        const uint32_t idx = chunk * kBS + threadIdx.x;
+    if (tb) {
+        // blocks or waves (units of 256 or 64 sites) take the same sites of tb consecutive slices one after
+        // another, then the next sites
+        const uint32_t w = unit == kBS ? blk
+                                       : (uint32_t)__builtin_amdgcn_readfirstlane((int)(blk * (kBS / 64) + threadIdx.x / 64));
+        const uint32_t NT = (uint32_t)L.n[0], chunks = (L.Vs + unit - 1) / unit;
+        if (w >= NT * chunks) return;
+        const uint32_t t0 = w / (tb * chunks) * tb, r = w - t0 * chunks;
+        const uint32_t ext = min(tb, NT - t0), chunk = r / ext;
+        const uint32_t idx = chunk * unit + threadIdx.x % unit;
         if (idx >= L.Vs) return;
-        s = slice_site_along(L, idx, mu + nu) + L.Vs * t;  // mu + nu: the spatial direction
+        s = slice_site_along(L, idx, d) + L.Vs * (t0 + r - chunk * ext);
     } else {
         s = blk * kBS + threadIdx.x;
         if (s >= L.V) return;
-        if (mu + nu == 4) {  // plane (x, z): each slice taken along z
-            const uint32_t t = s / L.Vs;
-            s = slice_site_along(L, s - t * L.Vs, 3) + L.Vs * t;
-        }
+        const uint32_t t = s / L.Vs;
+        s = slice_site_along(L, s - t * L.Vs, d) + L.Vs * t;
     }
     int c[4];
     site_coords(L, s, c);
@@ -222,15 +227,27 @@ hipError_t launch_magnetic(const Lat& L, const void* U, int is_f32, int su3, dou
 
 hipError_t launch_fmunu(const Lat& L, const void* U, int is_f32, int mu, int nu, int clover_only, void* out,
                         int out_layout, const int64_t s6[6], hipStream_t st) {
-    // planes containing time: every slice's blocks, slice fastest
-    const uint32_t g = (mu == 0 || nu == 0) ? (uint32_t)L.n[0] * ((L.Vs + kBS - 1) / kBS) : (L.V + kBS - 1) / kBS;
+    // Order of the sites.  Planes containing time: the same sites of all slices one after another, as the
+    // leaves reach 3 slices either way and the blocks running together then share those slices in L2.
+    // Spatial planes: storage order, but where t is dense in the output and more than one wave per SIMD
+    // runs, 8 slices, whose elements fill a line of the output, one after another: in storage order a line is
+    // written 16 B at a time, long apart.  Clover sums, a third of the work, take it by waves.  48^3x96, FP32 /
+    // FP64, ms: clover (x, y) 4.63 / 4.94 -> 1.59 / 2.59, (x, t) 1.88 / 3.00 -> 1.64 / 2.55; five-loop F (FP32,
+    // blocks) (x, y) 4.99 -> 4.20.  Five-loop planes (y, z) lose 2% by it and those containing time 5% by
+    // waves; at 10^3x43, 672 waves, every plane loses 2 to 10%.
+    const bool time = mu == 0 || nu == 0;
+    const bool lines = out_layout == 0 && s6 && s6[0] < s6[1] && L.V >= 65536 && L.Vs >= 2048;
+    const uint32_t unit = lines && clover_only ? 64 : kBS;
+    const uint32_t tb = time ? (uint32_t)L.n[0] : (lines && (clover_only || mu + nu != 5) ? 8 : 0);
+    const uint32_t units = tb ? (uint32_t)L.n[0] * ((L.Vs + unit - 1) / unit) : (L.V + kBS - 1) / kBS;
+    const uint32_t g = unit == 64 ? (units + kBS / 64 - 1) / (kBS / 64) : units;
     OutStrides os{0, 0, 0, 0, 0, 0};
     if (s6) os = OutStrides{s6[0], s6[1], s6[2], s6[3], s6[4], s6[5]};
     with_view(L.V, U, is_f32, [&](auto f) {
         if (clover_only)
-            fmunu_kernel<decltype(f), true><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os);
+            fmunu_kernel<decltype(f), true><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb);
         else
-            fmunu_kernel<decltype(f), false><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os);
+            fmunu_kernel<decltype(f), false><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb);
     });
     return hipGetLastError();
 }

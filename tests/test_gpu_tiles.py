@@ -121,6 +121,30 @@ def test_fmunu_of_links_that_are_not_unitary(FL, mu, nu, d):
     assert torch.equal(g.fmunu(mu, nu), want)
 
 
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims", [(23, 13, 16, 17), (35, 11, 17, 11), (8, 32, 16, 16), (33, 8, 16, 16), (65, 3, 5, 71)])
+def test_fmunu_orders_of_the_output(FL, dims, prec, variant):
+    # an output whose t is dense takes the sites of large lattices in another order than one whose x comes
+    # before t: the same arithmetic for each site, so the same numbers
+    from flue_lat_amd import _lib
+    f = FL.GaugeField.random(dims, 21, 0.3, prec)
+    for mu in range(1, 5):
+        for nu in range(1, 5):
+            got = []
+            for order in ((5, 4, 3, 2, 1, 0), (0, 1, 2, 3, 4, 5)):
+                shape = dims + (3, 3)
+                out = torch.full([shape[k] for k in order], float("nan"), dtype=torch.complex128, device=f.device)
+                out = out.permute([order.index(k) for k in range(6)])
+                st = (ctypes.c_int64 * 6)(*out.stride())
+                assert out.shape == shape and _lib.lib().flue_fmunu(
+                    f._cdims, ctypes.c_void_p(f.data.data_ptr()), f.prec, mu, nu, variant,
+                    ctypes.c_void_p(out.data_ptr()), _lib.FLUE_OUT_STRIDED, st,
+                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+                got.append(out)
+            assert torch.equal(*got), (mu, nu)
+
+
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 1e-6)])
 @pytest.mark.parametrize("R,T", [(6, 6), (1, 3), (4, 5), (6, 2)])
 @pytest.mark.parametrize("dims", [(5, 16, 16, 3), (4, 33, 31, 2), (2, 300, 7, 3), (31, 8, 5, 4), (3, 2, 128, 2)])
