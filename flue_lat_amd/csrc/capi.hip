@@ -167,21 +167,22 @@ int b2_grad_run(const Lat& L, const void* U, int32_t prec, int variant, void* wo
 }
 
 // flow work buffer: the second link buffer, then the accumulator, then the plaquette
-// parts, then a third link buffer
+// parts, then a third link buffer, then the word of a step whose links are tested
 size_t flow_acc_offset(const Lat& L, int32_t prec) {
     return ((size_t)L.V * kPlanes * (prec == FLUE_F32 ? 4 : 8) + 255) & ~(size_t)255;
 }
 size_t flow_w3_offset(const Lat& L, int32_t prec) {
     return flow_acc_offset(L, prec) + (size_t)L.V * 32 * 8 + align256(plaq_ta_bytes(L, prec == FLUE_F32));
 }
+size_t flow_word_offset(const Lat& L, int32_t prec) { return flow_w3_offset(L, prec) + flow_acc_offset(L, prec); }
 
 // one RK3 stage (Luescher: acc <- ca acc + cb Z, (ca, cb) = (0, 1/4), (-17/9, 8/9), (-1, 3/4))
 int flow_stage_run(const Lat& L, const void* Win, int32_t prec, void* Wout, void* acc, double eps, int stage,
-                   int variant, void* T, hipStream_t st) {
+                   int variant, void* T, hipStream_t st, uint32_t* bad = nullptr) {
     static const double ca[3] = {0.0, -17.0 / 9.0, -1.0};
     static const double cb[3] = {0.25, 8.0 / 9.0, 0.75};
     return hip_status(launch_flow_stage(L, Win, prec == FLUE_F32, Wout, acc, eps, ca[stage], cb[stage], stage == 2, st,
-                                        variant, T));
+                                        variant, T, bad));
 }
 
 // largest accepted max|U U^+ - 1| and |det U - 1|: a few hundred FP32 roundings of a unit
@@ -846,8 +847,8 @@ size_t flue_flow_work_bytes(const int32_t dims[4], int32_t prec) {
     if (check_dims(dims) || check_prec(prec)) return 0;
     const Lat L = make_lat(dims);
     // a second link buffer, the RK3 accumulator (8 su(3) coordinates per link, room for FP64), the
-    // plaquette parts of the plaquette-first stencil and a third link buffer (an odd step)
-    return flow_w3_offset(L, prec) + flow_acc_offset(L, prec);
+    // plaquette parts of the plaquette-first stencil, a third link buffer (an odd step) and a word
+    return flow_word_offset(L, prec) + 256;
 }
 
 int flue_wilson_action(const int32_t dims[4], const void* U, int32_t prec, double beta, double* d_S, void* ws,
@@ -953,11 +954,15 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
     void* T = (char*)acc + (size_t)L.V * 32 * 8;
     const int variant = variant_or(FLUE_OP_FLOW, dims, prec, flow_default(L));
     hipStream_t st = S(stream);
+    // plain FP64 links may be anything until the first step has reunitarised them
+    uint32_t* word = (uint32_t*)((char*)w + flow_word_offset(L, prec));
+    uint32_t* first = prec == FLUE_F64 && flow_is_pf(variant) ? word : nullptr;
     // three stages per step alternate between U and W2, so two steps return the field to U
-    auto two_steps = [&]() -> int {
+    auto two_steps = [&](uint32_t* bad) -> int {
         void* bufs[2] = {U, W2};
         for (int k = 0; k < 6; ++k) {
-            int r = flow_stage_run(L, bufs[k & 1], prec, bufs[(k + 1) & 1], acc, eps, k % 3, variant, T, st);
+            int r = flow_stage_run(L, bufs[k & 1], prec, bufs[(k + 1) & 1], acc, eps, k % 3, variant, T, st,
+                                   k < 3 ? bad : nullptr);
             if (r) return r;
         }
         return FLUE_OK;
@@ -967,8 +972,11 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
         if (st == nullptr) return FLUE_EINVAL;  // capture needs a non-default stream
         hipGraph_t graph;
         hipGraphExec_t exec;
+        // the graph is replayed for every pair; a first pair whose links are tested, with more to come, runs
+        // by itself
+        uint32_t* alone = pairs > 1 ? first : nullptr;
         FLUE_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        int r = two_steps();
+        int r = two_steps(alone ? nullptr : first);
         hipGraph_t g2 = nullptr;
         hipError_t e = hipStreamEndCapture(st, &g2);
         if (r) {
@@ -982,21 +990,25 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
             (void)hipGraphDestroy(graph);
             return hip_status(e);
         }
-        for (int32_t i = 0; i < pairs && e == hipSuccess; ++i) e = hipGraphLaunch(exec, st);
+        if (alone) r = two_steps(alone);
+        for (int32_t i = alone ? 1 : 0; i < pairs && e == hipSuccess && !r; ++i) e = hipGraphLaunch(exec, st);
         hipError_t e2 = hipStreamSynchronize(st);
         (void)hipGraphExecDestroy(exec);
         (void)hipGraphDestroy(graph);
+        if (r) return r;
         FLUE_TRY(e);
         FLUE_TRY(e2);
     } else {
         for (int32_t i = 0; i < pairs; ++i)
-            if ((rc = two_steps())) return rc;
+            if ((rc = two_steps(i ? nullptr : first))) return rc;
     }
     if (nsteps % 2) {
         // last odd step: U -> W2 -> W3 -> U, so its last stage writes U (no copy back)
         void* bufs[4] = {U, W2, (char*)w + flow_w3_offset(L, prec), U};
         for (int k = 0; k < 3; ++k)
-            if ((rc = flow_stage_run(L, bufs[k], prec, bufs[k + 1], acc, eps, k, variant, T, st))) return rc;
+            if ((rc = flow_stage_run(L, bufs[k], prec, bufs[k + 1], acc, eps, k, variant, T, st,
+                                     pairs ? nullptr : first)))
+                return rc;
     }
     return FLUE_OK;
 }

@@ -411,6 +411,50 @@ __device__ __forceinline__ void fill_row2(Mat<R>& M) {
     }
 }
 
+// whether M M^+ = 1 to 1e-13, in the sum of the entries' deviations (rounded SU(3) links are at
+// some 1e-15, and a leaf moved along three links that pass is right to 1e-12; NaN does not pass)
+template <typename R>
+__device__ __forceinline__ bool unitary(const Mat<R>& M) {
+    R dev = R(0);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        R n = R(-1);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            n = fmad(M.r[a * 3 + k], M.r[a * 3 + k], n);
+            n = fmad(M.i[a * 3 + k], M.i[a * 3 + k], n);
+        }
+        dev += n < R(0) ? -n : n;
+#pragma unroll
+        for (int b = 0; b < a; ++b) {
+            R xr = R(0), xi = R(0);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                xr = fmad(M.r[a * 3 + k], M.r[b * 3 + k], xr);
+                xr = fmad(M.i[a * 3 + k], M.i[b * 3 + k], xr);
+                xi = fmad(M.i[a * 3 + k], M.r[b * 3 + k], xi);
+                xi = fmad(-M.r[a * 3 + k], M.i[b * 3 + k], xi);
+            }
+            dev += (xr < R(0) ? -xr : xr) + (xi < R(0) ? -xi : xi);
+        }
+    }
+    return dev <= R(1e-13);
+}
+
+// whether M is special unitary to the same bound: unitary, and row 2 the conjugate of row 0 x row 1
+template <typename R>
+__device__ __forceinline__ bool special_unitary(const Mat<R>& M) {
+    Mat<R> W = M;
+    fill_row2(W);
+    R dev = R(0);
+#pragma unroll
+    for (int e = 6; e < 9; ++e) {
+        const R r = W.r[e] - M.r[e], i = W.i[e] - M.i[e];
+        dev += (r < R(0) ? -r : r) + (i < R(0) ? -i : i);
+    }
+    return unitary(M) && dev <= R(1e-13);
+}
+
 // The first two rows of a link (row 2 left zero)
 template <typename R, bool BUF>
 __device__ __forceinline__ Mat<R> load_rows2(const FieldView<R, BUF>& f, int mu, uint32_t s) {

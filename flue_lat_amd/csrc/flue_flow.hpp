@@ -148,6 +148,11 @@ __device__ __forceinline__ void flow_link(const Lat& L, const FV& f, typename FV
 // step of 0.01, against 1.595e-16 and 2.42e-8 from whole links.  The gradient itself would lose
 // (FP32: 9.1e-8 against 7.2e-8 rms), so without ROWS2 links are read whole and multiplied as
 // full matrices.
+//
+// The links of a plain FP64 field may be anything.  The first stage of a flow tests them in its first
+// pass, and where one is not SU(3) the three stages of that step take the staple sums of whole links
+// (flow_link); the step's reunitarisation makes SU(3) links of them for the steps that follow.  The
+// test reads row 2 of every link once in a flow.
 
 // plane index of (a, b), a < b: (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
 __device__ __forceinline__ int plaq_index(int a, int b) { return a == 0 ? b - 1 : (a == 1 ? b + 1 : 5); }
@@ -170,17 +175,24 @@ __device__ __forceinline__ void store_plaq_ta(R* __restrict__ T, uint32_t V, int
     }
 }
 
-// T_ab(s) of the six planes of site s (coordinates c) into T[(p * 8 + k) * V + s]
-template <bool ROWS2, typename FV>
-__device__ __forceinline__ void plaquette_ta_site(const Lat& L, const FV& f, uint32_t s, const int c[4],
+// T_ab(s) of the six planes of site s (coordinates c) into T[(p * 8 + k) * V + s].  TEST (with
+// ROWS2): also reads row 2 of the site's own links and returns whether they are SU(3).
+template <bool ROWS2, bool TEST = false, typename FV>
+__device__ __forceinline__ bool plaquette_ta_site(const Lat& L, const FV& f, uint32_t s, const int c[4],
                                                   typename FV::real* __restrict__ T) {
     using R = typename FV::real;
     uint32_t sf[4];
     Mat<R> own[4];
+    bool ok = true;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         sf[d] = c[d] == L.n[d] - 1 ? s - (uint32_t)(L.n[d] - 1) * L.st[d] : s + L.st[d];
-        if constexpr (ROWS2) own[d] = load_rows2(f, d, s);
+        if constexpr (TEST) {
+            own[d] = load_link(f, d, s);
+            ok = ok && special_unitary(own[d]);
+        } else if constexpr (ROWS2) {
+            own[d] = load_rows2(f, d, s);
+        }
     }
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -201,6 +213,7 @@ __device__ __forceinline__ void plaquette_ta_site(const Lat& L, const FV& f, uin
             store_plaq_ta<FV::buffered>(T, L.V, plaq_index(a, b), s, A, B);
         }
     }
+    return ok;
 }
 
 // the stored parts of T_p(s) as AH parts (off-diagonal parts doubled: o_ab = 2 T_ab)

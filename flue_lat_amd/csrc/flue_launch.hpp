@@ -146,8 +146,11 @@ int grad_default(const Lat& L);
 size_t plaq_ta_bytes(const Lat& L, int is_f32);
 hipError_t launch_wilson_grad(const Lat& L, const void* U, int is_f32, double beta, void* grad, hipStream_t st,
                               int variant, void* T);
+// bad != nullptr (FP64, plaquette-first): a word on the device for the three stages of a step whose links
+// may not be SU(3).  The step's first stage (ca == 0) tests them, and all three take staple sums if one is not
 hipError_t launch_flow_stage(const Lat& L, const void* Win, int is_f32, void* Wout, void* acc, double eps,
-                             double ca, double cb, int reunit, hipStream_t st, int variant, void* T);
+                             double ca, double cb, int reunit, hipStream_t st, int variant, void* T,
+                             uint32_t* bad = nullptr);
 hipError_t launch_magnetic_ah(const Lat& L, const void* U, int is_f32, void* Abuf, hipStream_t st);
 hipError_t launch_b2_grad(const Lat& L, const void* U, int is_f32, const void* Abuf, void* grad, hipStream_t st);
 // reverse-mode B^2 adjoint: slab by slab of time slices, per-rectangle terms into `slots`

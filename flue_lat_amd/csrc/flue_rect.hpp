@@ -71,36 +71,6 @@ __device__ __forceinline__ void ah_add(AH<R>& h, const AH<R>& g) {
     }
 }
 
-// whether M M^+ = 1 to 1e-13, in the sum of the entries' deviations (rounded SU(3) links are at
-// some 1e-15, and a leaf moved along three links that pass is right to 1e-12; NaN does not pass)
-template <typename R>
-__device__ __forceinline__ bool unitary(const Mat<R>& M) {
-    R dev = R(0);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        R n = R(-1);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            n = fmad(M.r[a * 3 + k], M.r[a * 3 + k], n);
-            n = fmad(M.i[a * 3 + k], M.i[a * 3 + k], n);
-        }
-        dev += n < R(0) ? -n : n;
-#pragma unroll
-        for (int b = 0; b < a; ++b) {
-            R xr = R(0), xi = R(0);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                xr = fmad(M.r[a * 3 + k], M.r[b * 3 + k], xr);
-                xr = fmad(M.i[a * 3 + k], M.i[b * 3 + k], xr);
-                xi = fmad(M.i[a * 3 + k], M.r[b * 3 + k], xi);
-                xi = fmad(-M.r[a * 3 + k], M.i[b * 3 + k], xi);
-            }
-            dev += (xr < R(0) ? -xr : xr) + (xi < R(0) ? -xi : xi);
-        }
-    }
-    return dev <= R(1e-13);
-}
-
 // One rectangle closed at both ends of its diagonal: the weighted AH part of the leaf at x
 // (W = CA CB^+) goes to h0 and to the two groups it belongs to; the weighted leaf at the
 // opposite corner (CB^+ CA) is returned.

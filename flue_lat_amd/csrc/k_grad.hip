@@ -6,6 +6,8 @@
 // per link is G = sum_a T^a D^a f, traceless anti-Hermitian; D^a f = -2 Tr(T^a G).
 //   Wilson action S = beta sum_p (1 - ReTr P/3):   G = (beta/6) P_TA(U Sigma)
 // with Sigma the staple sum (U Sigma = the six plaquettes through U).
+#include <algorithm>
+
 #include "flue_flow.hpp"
 #include "flue_launch.hpp"
 
@@ -92,13 +94,18 @@ __global__ void __launch_bounds__(kBS) flow_stage_kernel(Lat L, FV f, BlockOrder
 // At 48^3x96 the first pass takes 1.15 ms (FP32) and 2.11 ms (FP64) with ROWS2, at 4.0 and 4.4
 // TB/s beyond L2; taking two of the six planes per wave instead, with 21 link reads a site
 // instead of 16, took 1.33 and 2.34 ms and gained nothing on a lattice of 162,000 sites.
-template <bool ROWS2, typename FV>
-__global__ void __launch_bounds__(kBS) plaq_ta_kernel(Lat L, FV f, BlockOrder bo, typename FV::real* __restrict__ T) {
+// TEST: sets *bad where a link is not SU(3).
+template <bool ROWS2, bool TEST, typename FV>
+__global__ void __launch_bounds__(kBS) plaq_ta_kernel(Lat L, FV f, BlockOrder bo, typename FV::real* __restrict__ T,
+                                                      uint32_t* __restrict__ bad) {
     uint32_t s;
     int c[4];
     if (!order_site(L, bo, xcd_block(blockIdx.x, gridDim.x), threadIdx.x, s, c)) return;
-    plaquette_ta_site<ROWS2>(L, f, s, c, T);
+    const bool ok = plaquette_ta_site<ROWS2, TEST>(L, f, s, c, T);
+    if (TEST && !ok) __hip_atomic_store(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+__global__ void clear_word_kernel(uint32_t* w) { *w = 0; }
 
 template <typename FV>
 __global__ void __launch_bounds__(kBS) wilson_grad_pf_kernel(Lat L, FV f, BlockOrder bo,
@@ -120,18 +127,40 @@ __global__ void __launch_bounds__(kBS) wilson_grad_pf_kernel(Lat L, FV f, BlockO
     store_link_stream(grad, L.V, mu, s, G);
 }
 
-template <typename FV>
+// TESTED: nothing where the flow's first pass found links that are not SU(3) (flow_general_kernel's work).
+// Both forms in this kernel would leave the plaquette-first one at the staple form's two waves per SIMD
+// instead of four: 3.30 ms for ten steps of 18x15x20x30 instead of 3.27, and 3.26 with no test at all.
+template <bool TESTED, typename FV>
 __global__ void __launch_bounds__(kBS) flow_stage_pf_kernel(Lat L, FV f, BlockOrder bo,
                                                             const typename FV::real* __restrict__ T,
                                                             typename FV::real* __restrict__ wout,
                                                             typename FV::real* __restrict__ acc, double eps, double ca,
-                                                            double cb, int reunit) {
+                                                            double cb, int reunit, const uint32_t* __restrict__ bad) {
+    if (TESTED && *bad) return;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     uint32_t s;
     int c[4];
     if (!order_site(L, bo, blk >> 2, (blk & 3u) * 64u + (threadIdx.x & 63u), s, c)) return;
     flow_link_pf(L, f, T, wout, acc, s, c, mu, eps, ca, cb, reunit);
+}
+
+// The stage by staple sums where the links turned out not SU(3): the 4 nb (direction, block) pairs of
+// flow_stage_kernel in storage order on as many workgroups as are resident at once, which look first
+// whether there is anything to do.
+constexpr uint32_t kGeneralGrid = 1024;
+template <typename FV>
+__global__ void __launch_bounds__(kBS) flow_general_kernel(Lat L, FV f, uint32_t nb, typename FV::real* __restrict__ wout,
+                                                           typename FV::real* __restrict__ acc, double eps, double ca,
+                                                           double cb, int reunit, const uint32_t* __restrict__ bad) {
+    if (!*bad) return;
+    for (uint32_t blk = blockIdx.x; blk < 4 * nb; blk += gridDim.x) {
+        const uint32_t s = (blk >> 2) * kBS + threadIdx.x;
+        if (s >= L.V) continue;
+        int c[4];
+        site_coords(L, s, c);
+        flow_link(L, f, wout, acc, s, c, (int)(blk & 3u), eps, ca, cb, reunit);
+    }
 }
 
 }  // namespace
@@ -196,7 +225,7 @@ hipError_t launch_wilson_grad(const Lat& L, const void* U, int is_f32, double be
         using F = decltype(f);
         using R = typename F::real;
         if (flow_is_pf(variant)) {
-            plaq_ta_kernel<false, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T);
+            plaq_ta_kernel<false, false, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T, nullptr);
             wilson_grad_pf_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (const R*)T, beta, (R*)grad);
         } else {
             wilson_grad_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, beta, (R*)grad);
@@ -206,7 +235,7 @@ hipError_t launch_wilson_grad(const Lat& L, const void* U, int is_f32, double be
 }
 
 hipError_t launch_flow_stage(const Lat& L, const void* Win, int is_f32, void* Wout, void* acc_, double eps,
-                             double ca, double cb, int reunit, hipStream_t st, int variant, void* T) {
+                             double ca, double cb, int reunit, hipStream_t st, int variant, void* T, uint32_t* bad) {
     if (flow_is_pf(variant) && !T) return hipErrorInvalidValue;
     const BlockOrder bo = block_order(L, variant);
     with_view(L.V, Win, is_f32, [&](auto f) {
@@ -214,8 +243,27 @@ hipError_t launch_flow_stage(const Lat& L, const void* Win, int is_f32, void* Wo
         using R = typename F::real;
         R* acc = (R*)acc_;
         if (flow_is_pf(variant)) {
-            plaq_ta_kernel<true, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T);
-            flow_stage_pf_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (const R*)T, (R*)Wout, acc, eps, ca, cb, reunit);
+            constexpr bool kF64 = sizeof(R) == 8;
+            auto links = [&](auto tested) {
+                flow_stage_pf_kernel<decltype(tested)::value, F>
+                    <<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (const R*)T, (R*)Wout, acc, eps, ca, cb, reunit, bad);
+            };
+            if (kF64 && bad && ca == 0.0) {  // the step's first stage
+                clear_word_kernel<<<1, 1, 0, st>>>(bad);
+                plaq_ta_kernel<true, kF64, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T, bad);
+            } else {
+                plaq_ta_kernel<true, false, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T, nullptr);
+            }
+            if constexpr (kF64) {
+                if (bad) {
+                    const uint32_t nb = (L.V + kBS - 1) / kBS;
+                    links(std::true_type());
+                    flow_general_kernel<F><<<std::min(kGeneralGrid, 4 * nb), kBS, 0, st>>>(
+                        L, f, nb, (R*)Wout, acc, eps, ca, cb, reunit, bad);
+                    return;
+                }
+            }
+            links(std::false_type());
         } else {
             flow_stage_kernel<F><<<4 * bo.nb, kBS, 0, st>>>(L, f, bo, (R*)Wout, acc, eps, ca, cb, reunit);
         }

@@ -387,12 +387,12 @@ int flue_flow_stage(const int32_t dims[4], const void* Win, int32_t prec, void* 
  * buffer, which must then exist before any capture): two more link buffers, the
  * accumulator and the plaquette parts.  The stages alternate between U and the second
  * buffer, and an odd last step passes through the third, so every step ends in U without
- * a copy.  The flow moves SU(3) links along the
- * group (exponential map, reunitarisation after every step), so it takes SU(3) links in
- * every precision: the tuned FLUE_OP_FLOW variant is used, or untuned the plaquette-first
- * stencil (7 or 11) on lattices of 32768 sites or more.  The plaquette-first variants 7..13
- * read rows 0 and 1 of every link and rebuild row 2 from them.  flue_flow_stage (no workspace) uses the staple sums in the tuned
- * variant's visit order. */
+ * a copy.  The tuned FLUE_OP_FLOW variant is used, or untuned the plaquette-first stencil (7 or
+ * 11) on lattices of 32768 sites or more.  The plaquette-first variants 7..13 read rows 0 and 1
+ * of every link and rebuild row 2 from them, so they take SU(3) links: those of a FLUE_F64 field
+ * are tested on the way, and if one is not SU(3) to 1e-13 the first step takes staple sums of
+ * whole links (the reunitarisation at its end leaves SU(3) links for the others).
+ * flue_flow_stage (no workspace) uses the staple sums in the tuned variant's visit order. */
 int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, int32_t nsteps, int32_t use_graph,
                      void* work, size_t work_bytes, void* stream);
 
