@@ -1208,8 +1208,8 @@ void ens_key(const EnsPlan& p, int32_t n, int32_t key[4]) {
     key[3] = 0;
 }
 
-// the ensemble work buffer: tables, second link buffer, accumulators (room for FP64), partial sums, and
-// the plaquette parts of the plaquette-first stencil
+// the ensemble work buffer: tables, second link buffer, accumulators (room for FP64), partial sums, the
+// plaquette parts of the plaquette-first stencil, and the words of a step whose links are tested
 struct EnsWork {
     EnsEntry* tab;
     EnsRect* rect;
@@ -1217,6 +1217,7 @@ struct EnsWork {
     double* acc;
     double* partials;
     void* T;
+    uint32_t* bad;
 };
 
 EnsWork ens_work(void* w, int32_t n, const EnsPlan& p, size_t sz) {
@@ -1233,6 +1234,8 @@ EnsWork ens_work(void* w, int32_t n, const EnsPlan& p, size_t sz) {
     r.partials = (double*)base;
     base += align256((size_t)p.total_blocks * 16);
     r.T = base;
+    base += align256((size_t)p.field_reals / 72 * 48 * sz);
+    r.bad = (uint32_t*)base;
     return r;
 }
 
@@ -1247,10 +1250,11 @@ size_t flue_ensemble_field_bytes(int32_t n, const int32_t* dims, int32_t prec) {
 size_t flue_ensemble_work_bytes(int32_t n, const int32_t* dims, int32_t prec) {
     EnsPlan p;
     if (ens_plan(n, dims, p) || check_prec(prec)) return 0;
-    // tables, second link buffer, accumulators (room for FP64), per-block partial sums, plaquette parts
+    // tables, second link buffer, accumulators (room for FP64), per-block partial sums, plaquette parts, words
     const size_t sz = prec == FLUE_F32 ? 4 : 8;
     return align256(sizeof(EnsEntry) * n) + align256(sizeof(EnsRect) * n) + align256((size_t)p.field_reals * sz) + align256((size_t)p.acc_doubles * 8) +
-           align256((size_t)p.total_blocks * 16) + align256((size_t)p.field_reals / 72 * 48 * sz);
+           align256((size_t)p.total_blocks * 16) + align256((size_t)p.field_reals / 72 * 48 * sz) +
+           align256(sizeof(uint32_t) * ((size_t)n + 1));
 }
 
 int flue_ensemble_random(int32_t n, const int32_t* dims, const uint64_t* seeds, double eps, void* fields, int32_t prec,
@@ -1298,6 +1302,7 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
     ens_key(p, n, key);
     const int variant = variant_or(FLUE_OP_ENSEMBLE_FLOW, key, prec, ensemble_default(p.field_reals / kPlanes));
     void* T = variant > 4 ? ew.T : nullptr;  // the plaquette-first variants
+    uint32_t* first = T && prec == FLUE_F64 ? ew.bad : nullptr;  // as in flue_wilson_flow
 
     static const double ca[3] = {0.0, -17.0 / 9.0, -1.0};
     static const double cb[3] = {0.25, 8.0 / 9.0, 0.75};
@@ -1327,7 +1332,7 @@ int flue_ensemble_flow(int32_t n, const int32_t* dims, void* fields, int32_t pre
             for (int k = 0; k < 3 && e == hipSuccess; ++k) {
                 const int q = 3 * j + k;
                 e = launch_ens_flow_stage(d_tab, n, p.total_blocks, p.maxV, bufs[q & 1], is_f32, bufs[(q + 1) & 1], acc,
-                                          eps, ca[k], cb[k], k == 2, T, st);
+                                          eps, ca[k], cb[k], k == 2, T, st, j == 0 ? first : nullptr);
             }
             if (e == hipSuccess && nmeas > 0 && (j + 1) % measure_every == 0)
                 e = measure((j + 1) & 1, (j + 1) / measure_every);

@@ -195,10 +195,11 @@ struct EnsRect {
     uint32_t tile0, tiles, copy0;
 };
 // T != nullptr: the plaquette-first stencil with the plaquette parts of every field in T
-// (48 reals per site, field c's at 2/3 of its field offset); T == nullptr: staple sums
+// (48 reals per site, field c's at 2/3 of its field offset); T == nullptr: staple sums.
+// bad as for launch_flow_stage: a word for each configuration and one more
 hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* win,
                                  int is_f32, void* wout, void* acc, double eps, double ca, double cb, int reunit,
-                                 void* T, hipStream_t st);
+                                 void* T, hipStream_t st, uint32_t* bad = nullptr);
 hipError_t launch_ens_sum(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* fld, int is_f32,
                           int obs, double* partials, hipStream_t st);
 // the partials of configuration c: its logical blocks', or its tiles' with rect

@@ -66,33 +66,72 @@ __global__ void __launch_bounds__(kBS) ens_flow_kernel(const EnsEntry* __restric
 // Plaquette-first stencil over the ensemble: the six plaquette parts of every site of every
 // field (48 reals per site, config c's block at 2/3 of its field offset), then the links, the
 // four waves of a workgroup on the four directions of 64 sites.
-template <typename R, bool BUF>
+// TEST: sets bad[c] and bad[n] where a link of configuration c is not SU(3).
+template <typename R, bool BUF, bool TEST>
 __global__ void __launch_bounds__(kBS) ens_plaq_ta_kernel(const EnsEntry* __restrict__ tab, int n,
-                                                          const R* __restrict__ win, R* __restrict__ T) {
+                                                          const R* __restrict__ win, R* __restrict__ T,
+                                                          uint32_t* __restrict__ bad) {
     const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
-    const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
+    const int cfg = find_cfg(tab, n, lb);
+    const EnsEntry& e = entry(tab, cfg);
     const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
     if (s >= e.L.V) return;
     const FieldView<R, BUF> f{win + e.off, e.L.V};
     int c[4];
     site_coords(e.L, s, c);
-    plaquette_ta_site<true>(e.L, f, s, c, T + e.off / 72 * 48);
+    const bool ok = plaquette_ta_site<true, TEST>(e.L, f, s, c, T + e.off / 72 * 48);
+    if (TEST && !ok) {
+        __hip_atomic_store(bad + cfg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(bad + n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
-template <typename R, bool BUF>
+// TESTED: nothing for a configuration with links that are not SU(3) (ens_general_flow_kernel's work)
+template <typename R, bool BUF, bool TESTED>
 __global__ void __launch_bounds__(kBS) ens_flow_pf_kernel(const EnsEntry* __restrict__ tab, int n,
                                                           const R* __restrict__ win, const R* __restrict__ T,
                                                           R* __restrict__ wout, R* __restrict__ acc, double eps, double ca,
-                                                          double cb, int reunit) {
+                                                          double cb, int reunit, const uint32_t* __restrict__ bad) {
     const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const uint32_t lu = xcd_block(blockIdx.x, gridDim.x), lb = lu >> 2;
-    const EnsEntry& e = entry(tab, find_cfg(tab, n, lb));
+    const int cfg = find_cfg(tab, n, lb);
+    if (TESTED && bad[cfg]) return;
+    const EnsEntry& e = entry(tab, cfg);
     const uint32_t s = (lb - e.blk0) * kBS + (lu & 3u) * 64u + (threadIdx.x & 63u);
     if (s >= e.L.V) return;
     const FieldView<R, BUF> f{win + e.off, e.L.V};
     int c[4];
     site_coords(e.L, s, c);
     flow_link_pf(e.L, f, T + e.off / 72 * 48, wout + e.off, acc + e.acc_off, s, c, mu, eps, ca, cb, reunit);
+}
+
+// The stage by staple sums for the configurations whose links turned out not SU(3), the (direction,
+// logical block) pairs of ens_flow_kernel on as many workgroups as are resident at once, which look first
+// whether there is anything to do.
+constexpr uint32_t kGeneralGrid = 1024;
+template <typename R, bool BUF>
+__global__ void __launch_bounds__(kBS) ens_general_flow_kernel(const EnsEntry* __restrict__ tab, int n, uint32_t total,
+                                                               const R* __restrict__ win, R* __restrict__ wout,
+                                                               R* __restrict__ acc, double eps, double ca, double cb,
+                                                               int reunit, const uint32_t* __restrict__ bad) {
+    if (!bad[n]) return;
+    for (uint64_t lu = blockIdx.x; lu < 4 * (uint64_t)total; lu += gridDim.x) {
+        const uint32_t lb = (uint32_t)(lu >> 2);
+        const int cfg = find_cfg(tab, n, lb);
+        if (!bad[cfg]) continue;
+        const EnsEntry& e = entry(tab, cfg);
+        const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
+        if (s >= e.L.V) continue;
+        const FieldView<R, BUF> f{win + e.off, e.L.V};
+        int c[4];
+        site_coords(e.L, s, c);
+        flow_link(e.L, f, wout + e.off, acc + e.acc_off, s, c, (int)(lu & 3u), eps, ca, cb, reunit);
+    }
+}
+
+__global__ void clear_words_kernel(uint32_t* w, int n) {
+    const int i = (int)(blockIdx.x * kBS + threadIdx.x);
+    if (i < n) w[i] = 0;
 }
 
 // OBS = 0: sum of ReTr over all 6V plaquettes; OBS = 1: sum of -ReTr F_i^2 (magnetic)
@@ -156,14 +195,30 @@ void with_real(int is_f32, bool buf, Fn&& fn) {
 
 hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uint32_t maxV, const void* win,
                                  int is_f32, void* wout, void* acc, double eps, double ca, double cb, int reunit,
-                                 void* T, hipStream_t st) {
+                                 void* T, hipStream_t st, uint32_t* bad) {
     with_real(is_f32, fits_buffer(maxV, is_f32), [&](auto r, auto buf) {
         using R = decltype(r);
         constexpr bool B = decltype(buf)::value;
         if (T) {
-            ens_plaq_ta_kernel<R, B><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T);
-            ens_flow_pf_kernel<R, B><<<4 * total, kBS, 0, st>>>(tab, n, (const R*)win, (const R*)T, (R*)wout, (R*)acc, eps,
-                                                                ca, cb, reunit);
+            constexpr bool kF64 = sizeof(R) == 8;
+            const bool test = kF64 && bad && ca == 0.0;  // the step's first stage
+            if (test) {
+                clear_words_kernel<<<n / kBS + 1, kBS, 0, st>>>(bad, n + 1);
+                ens_plaq_ta_kernel<R, B, kF64><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T, bad);
+            } else {
+                ens_plaq_ta_kernel<R, B, false><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T, nullptr);
+            }
+            if constexpr (kF64) {
+                if (bad) {
+                    ens_flow_pf_kernel<R, B, true><<<4 * total, kBS, 0, st>>>(
+                        tab, n, (const R*)win, (const R*)T, (R*)wout, (R*)acc, eps, ca, cb, reunit, bad);
+                    ens_general_flow_kernel<R, B><<<(uint32_t)std::min<uint64_t>(kGeneralGrid, 4 * (uint64_t)total), kBS, 0, st>>>(
+                        tab, n, total, (const R*)win, (R*)wout, (R*)acc, eps, ca, cb, reunit, bad);
+                    return;
+                }
+            }
+            ens_flow_pf_kernel<R, B, false><<<4 * total, kBS, 0, st>>>(tab, n, (const R*)win, (const R*)T, (R*)wout,
+                                                                       (R*)acc, eps, ca, cb, reunit, nullptr);
         } else {
             ens_flow_kernel<R, B><<<4 * total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)wout, (R*)acc, eps, ca, cb,
                                                              reunit);

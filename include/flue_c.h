@@ -444,7 +444,9 @@ size_t flue_ensemble_work_bytes(int32_t n, const int32_t* dims, int32_t prec);
 int flue_ensemble_random(int32_t n, const int32_t* dims, const uint64_t* seeds, double eps, void* fields,
                          int32_t prec, void* stream);
 
-/* nsteps RK3 Wilson-flow steps of every field in place.  With measure_every > 0 the
+/* nsteps RK3 Wilson-flow steps of every field in place, by staple sums or by the
+ * plaquette-first stencil, which untuned ensembles of 32768 sites or more take; fields whose
+ * links are not SU(3) as for flue_wilson_flow, each by itself.  With measure_every > 0 the
  * plaquette sum (sum of ReTr P over the 6V plaquettes, as genPlaquette(1,4,4)) and the
  * magnetic B are written to d_plaq[m*n + c] and d_B[m*n + c] at steps
  * m*measure_every, m = 0 .. nsteps/measure_every.  use_graph != 0 captures the whole run

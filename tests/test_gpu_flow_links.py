@@ -74,3 +74,30 @@ def test_flow_of_links_that_are_not_su3(FL, dims, kind):
     W = f.clone()
     W.wilson_flow(EPS, 2, use_graph=False)
     assert_same(W.data, by_stages(FL, f, 2))
+
+
+@pytest.mark.parametrize("kind", ["scaled", "phase", "row 2", "nan"])
+def test_ensemble_flow_of_links_that_are_not_su3(FL, kind):
+    # two of four configurations spoiled, the second of them the smallest; the others are not affected
+    from flue_lat_amd.ensemble import Ensemble
+    dims = [(9, 11, 12, 13), (17, 12, 9, 8), (3, 4, 5, 6), (14, 8, 10, 12)]
+    for nsteps, use_graph in ((1, False), (3, True)):
+        e = Ensemble.random(dims, [5, 6, 7, 8], 0.3, "fp64")
+        clean = e.data.clone()
+        e.flow(EPS, nsteps, measure_every=0, use_graph=use_graph)
+        flowed = e.data.clone()
+        e.data.copy_(clean)
+        want = []
+        for c in range(4):
+            g = e.field(c)
+            if c in (1, 2):
+                U = g.to_complex()
+                spoil(U, kind)
+                g.data.copy_(FL.GaugeField.from_complex(U).data)
+            want.append(by_stages(FL, g, nsteps))
+        e.flow(EPS, nsteps, measure_every=0, use_graph=use_graph)
+        for c in range(4):
+            assert_same(e.field(c).data, want[c])
+        for c in (0, 3):
+            lo, hi = int(e.offsets[c]), int(e.offsets[c + 1])
+            assert torch.equal(e.data[lo:hi], flowed[lo:hi])
