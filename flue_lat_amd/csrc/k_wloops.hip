@@ -41,6 +41,15 @@ __device__ __forceinline__ double quad_swap(double v) {
     return __hiloint2double(hi, lo);
 }
 
+// sum over the 16 lanes of a row
+__device__ __forceinline__ double row_sum(double v) {
+    v += quad_swap<0xB1>(v);
+    v += quad_swap<0x4E>(v);
+    v += quad_swap<0x141>(v);  // half row mirrored: the other four
+    v += quad_swap<0x140>(v);  // row mirrored: the other eight
+    return v;
+}
+
 // Grid: groups x nb logical blocks, one group per time slice for kEverySlice, else one.
 // With time in the plane the slice is the fastest block index (for the whole lattice, nb
 // counts the blocks of every slice, slice fastest); otherwise the block within the group is.
@@ -48,7 +57,8 @@ __device__ __forceinline__ double quad_swap(double v) {
 // TM = Tmax is a template argument, so a row of the table (one R) is straight code: each step's two
 // products, of CA and of CB(T, .), each start the load of the link that the next step puts in place of
 // the one they used.  Each four lanes write the
-// sum of their traces to LDS slots of their own; the block adds those at the end.
+// sum of their traces to LDS slots of their own; the block adds those at the end, compensated like the
+// final pass over the blocks.
 template <typename FV, int TM>
 __global__ void __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(sizeof(typename FV::real) == 4 ? 2 : 1)))
 wloop_table_kernel(Lat L, FV f, int mu, int nu, int Rmax, int tslice, uint32_t nb, uint32_t groups,
@@ -157,17 +167,17 @@ wloop_table_kernel(Lat L, FV f, int mu, int nu, int Rmax, int tslice, uint32_t n
         row(std::true_type(), ap, M, N);
     }
     __syncthreads();
-    // a wave per entry sums its 64 slots (plain adds; the per-block partials and the final pass are
-    // compensated)
+    // a wave per entry sums its 64 slots, the 16 of a wave plainly, the four waves compensated (all six steps
+    // compensated: 1% of a large table and 4% of a small one)
     const int lane = threadIdx.x & 63;
     for (int k = threadIdx.x >> 6; k < Rmax * TM; k += kBS / 64) {
-        double v = sh[k][lane];
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+        DD v = {row_sum(sh[k][lane]), 0.0};
+        v = dd_add(v, dd_shfl_xor(v, 16));
+        v = dd_add(v, dd_shfl_xor(v, 32));
         if (lane == 0) {
             double* p = partials + 2 * (((size_t)k * groups + grp) * nb + blk);
-            p[0] = v;
-            p[1] = 0.0;
+            p[0] = v.hi;
+            p[1] = v.lo;
         }
     }
 }
@@ -177,13 +187,15 @@ wloop_table_kernel(Lat L, FV f, int mu, int nu, int Rmax, int tslice, uint32_t n
 template <typename R>
 constexpr uint32_t kTileCells = sizeof(R) == 4 ? 536 : 552;
 
-// sum over the 16 lanes of a row
-__device__ __forceinline__ double row_sum(double v) {
+// row_sum, compensated from the four sums of four lanes on
+template <int CTRL>
+__device__ __forceinline__ DD dd_swap_add(DD v) {
+    return dd_add(v, DD{quad_swap<CTRL>(v.hi), quad_swap<CTRL>(v.lo)});
+}
+__device__ __forceinline__ DD row_dd_sum(double v) {
     v += quad_swap<0xB1>(v);
     v += quad_swap<0x4E>(v);
-    v += quad_swap<0x141>(v);  // half row mirrored: the other four
-    v += quad_swap<0x140>(v);  // row mirrored: the other eight
-    return v;
+    return dd_swap_add<0x140>(dd_swap_add<0x141>(DD{v, 0.0}));
 }
 
 // The table of a plane with x, tile by tile: direction 1 of the tiles is x, direction 2 the other one,
@@ -287,13 +299,13 @@ wloop_tile_kernel(Lat L, FV f, int mu, int nu, int Rmax, PlaneTiles g, int tslic
         row(std::true_type(), M, N);
     }
     __syncthreads();
-    // 16 lanes per entry (plain adds; the per-block partials and the final pass are compensated)
+    // 16 lanes per entry
     for (int k = threadIdx.x >> 4; k < Rmax * TM; k += kBS / 16) {
-        const double v = row_sum(sh[k][threadIdx.x & 15]);
+        const DD v = row_dd_sum(sh[k][threadIdx.x & 15]);
         if ((threadIdx.x & 15) == 0) {
             double* p = partials + 2 * (((size_t)k * groups + grp) * nb + blk);
-            p[0] = v;
-            p[1] = 0.0;
+            p[0] = v.hi;
+            p[1] = v.lo;
         }
     }
 }
