@@ -411,8 +411,11 @@ __device__ __forceinline__ void fill_row2(Mat<R>& M) {
     }
 }
 
-// whether M M^+ = 1 to 1e-13, in the sum of the entries' deviations (rounded SU(3) links are at
-// some 1e-15, and a leaf moved along three links that pass is right to 1e-12; NaN does not pass)
+// Whether M M^+ = 1 to kLinkTol, in the sum of the entries' deviations (NaN does not pass).  SU(3) links are
+// at 2e-15 (reunitarised) to 1e-14 (QR, small matrix exponentials).  A leaf moved along three links that
+// pass is right to 6e-14 of the field strength, which is what the rounding of its products leaves of one
+// of 0.1; links that drifted further take the general forms.
+constexpr double kLinkTol = 2e-14;
 template <typename R>
 __device__ __forceinline__ bool unitary(const Mat<R>& M) {
     R dev = R(0);
@@ -438,7 +441,7 @@ __device__ __forceinline__ bool unitary(const Mat<R>& M) {
             dev += (xr < R(0) ? -xr : xr) + (xi < R(0) ? -xi : xi);
         }
     }
-    return dev <= R(1e-13);
+    return dev <= R(kLinkTol);
 }
 
 // whether M is special unitary to the same bound: unitary, and row 2 the conjugate of row 0 x row 1
@@ -452,7 +455,7 @@ __device__ __forceinline__ bool special_unitary(const Mat<R>& M) {
         const R r = W.r[e] - M.r[e], i = W.i[e] - M.i[e];
         dev += (r < R(0) ? -r : r) + (i < R(0) ? -i : i);
     }
-    return unitary(M) && dev <= R(1e-13);
+    return unitary(M) && dev <= R(kLinkTol);
 }
 
 // The first two rows of a link (row 2 left zero)

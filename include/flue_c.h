@@ -293,7 +293,7 @@ int flue_magnetic(const int32_t dims[4], const void* U, int32_t prec, double* d_
  *   7     rectangle-first: each rectangle of the clover is formed once and its leaves at
  *         the other three corners follow by conjugation (plane (z,y) from a z-fastest copy
  *         of its links).  That holds for unitary links: those of a FLUE_F64 field are
- *         tested on the way, and B comes from the quadrants if one is not unitary to 1e-13.
+ *         tested on the way, and B comes from the quadrants if one is not unitary to 2e-14.
  *         It needs NX, NY, NZ divisible by 16, or of 12 or more on a
  *         lattice of 90,000 sites or more, and a workspace of
  *         flue_magnetic_work_bytes (about 300 bytes per site in FP32, 600 in FP64);
@@ -390,7 +390,7 @@ int flue_flow_stage(const int32_t dims[4], const void* Win, int32_t prec, void* 
  * a copy.  The tuned FLUE_OP_FLOW variant is used, or untuned the plaquette-first stencil (7 or
  * 11) on lattices of 32768 sites or more.  The plaquette-first variants 7..13 read rows 0 and 1
  * of every link and rebuild row 2 from them, so they take SU(3) links: those of a FLUE_F64 field
- * are tested on the way, and if one is not SU(3) to 1e-13 the first step takes staple sums of
+ * are tested on the way, and if one is not SU(3) to 2e-14 the first step takes staple sums of
  * whole links (the reunitarisation at its end leaves SU(3) links for the others).
  * flue_flow_stage (no workspace) uses the staple sums in the tuned variant's visit order. */
 int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, int32_t nsteps, int32_t use_graph,
