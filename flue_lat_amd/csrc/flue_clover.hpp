@@ -608,6 +608,37 @@ __device__ __forceinline__ void store_f(const AH<R>& h, const int c[4], double* 
         }
 }
 
+// site o of the visit order of magnetic plane pl (k_clover.hip), with its coordinates
+__device__ __forceinline__ uint32_t plane_site(const Lat& L, const PlaneOrder& po, int pl, uint32_t o, int c[4]) {
+    const uint32_t nx = (uint32_t)L.n[1], ny = (uint32_t)L.n[2], nz = (uint32_t)L.n[3];
+    uint32_t q;
+    if (pl == 0) {
+        site_coords(L, o, c);
+    } else if (pl == 1) {
+        c[1] = (int)(o % nx);
+        q = o / nx;
+        c[3] = (int)(q % nz);
+        q /= nz;
+        c[2] = (int)(q % ny);
+        c[0] = (int)(q / ny);
+    } else {
+        const uint32_t xi = o % po.xw;
+        q = o / po.xw;
+        c[2] = (int)(q % ny);
+        q /= ny;
+        c[3] = (int)(q % nz);
+        q /= nz;
+        const uint32_t nxc = nx / po.xw;
+        c[1] = (int)((q % nxc) * po.xw + xi);
+        c[0] = (int)(q / nxc);
+    }
+    return (uint32_t)c[1] + nx * ((uint32_t)c[2] + ny * ((uint32_t)c[3] + nz * (uint32_t)c[0]));
+}
+
+// (mu, nu) of magnetic plane pl: (y, x), (x, z), (z, y) in 0-based directions
+__device__ __forceinline__ int plane_mu(int pl) { return pl == 0 ? 2 : (pl == 1 ? 1 : 3); }
+__device__ __forceinline__ int plane_nu(int pl) { return pl == 0 ? 1 : (pl == 1 ? 3 : 2); }
+
 // sum_ab |F_ab|^2 = -ReTr(F F) for F = A^T/4 with A the accumulated anti-Hermitian part
 // (FP64): |F_aa|^2 = d_a^2/16 and |F_ab|^2 + |F_ba|^2 = |o_ab|^2/32
 template <typename R>

@@ -32,6 +32,12 @@ struct Lat {
     }
 };
 
+// the plane-major visit order of the magnetic plane (z, y) (k_clover.hip): x in chunks of xw sites, a
+// divisor of NX
+struct PlaneOrder {
+    uint32_t xw;
+};
+
 inline Lat make_lat(const int32_t dims_tx_yz[4]) {
     // dims are given in the reference order (NT, NX, NY, NZ)
     Lat L;

@@ -55,14 +55,16 @@ hipError_t launch_finalize(const double* partials, uint32_t n, double* out, doub
 // 5-loop (or 1x1 clover) field strength for one plane; out_layout 0 = complex128 with
 // strides (t, x, y, z, a, b) in complex elements, 1 = SoA planes (9 elem x re/im) in the
 // field precision
+// (bad != nullptr, FP64 5-loop: only where *bad)
 hipError_t launch_fmunu(const Lat& L, const void* U, int is_f32, int mu, int nu, int clover_only, void* out,
-                        int out_layout, const int64_t strides[6], hipStream_t st);
+                        int out_layout, const int64_t strides[6], hipStream_t st, const uint32_t* bad = nullptr);
 // the 5-loop F of a plane of an FP64 field on rectangle-first tiles (k_rect.hip), into an array with
 // stride 1 along t; fmunu_rect_bytes of workspace, 0 where the plane does not take them
 size_t fmunu_rect_bytes(const Lat& L, int mu, int nu);
 hipError_t launch_fmunu_rect(const Lat& L, const void* U, int mu, int nu, void* out, const int64_t strides[6], void* ws,
                              hipStream_t st);
 uint32_t magnetic_blocks(const Lat& L, int is_f32);
+PlaneOrder plane_order(const Lat& L, size_t real_bytes);
 int magnetic_default_variant(int is_f32);
 // rectangular Wilson-loop table (k_wloops.hip): R, T up to kMaxLoopRT
 constexpr int kMaxLoopRT = 6;
@@ -188,11 +190,13 @@ struct EnsEntry {
     uint32_t nblk;
 };
 // configuration c in the rectangle-first magnetic: its tiles [tile0, tile0 + tiles) (the three planes'
-// in turn) and the blocks from copy0 that make its z-fastest copy
+// in turn), the blocks from copy0 that make its z-fastest copy, and the groups of blocks from grp0 that form
+// its B by quadrants where links are not unitary
 struct EnsRect {
     RectTiles rt;
     Lat Lzy;
-    uint32_t tile0, tiles, copy0;
+    PlaneOrder po;
+    uint32_t tile0, tiles, copy0, grp0;
 };
 // T != nullptr: the plaquette-first stencil with the plaquette parts of every field in T
 // (48 reals per site, field c's at 2/3 of its field offset); T == nullptr: staple sums.
@@ -211,7 +215,7 @@ hipError_t launch_ens_finalize(const EnsEntry* tab, const EnsRect* rect, int n, 
 // that in `fp` (48 reals a site); one partial per tile (EnsRectGrid::tiles)
 // and the word behind them.
 struct EnsRectGrid {
-    uint32_t tiles, copies;
+    uint32_t tiles, copies, groups;
     int copy_edge;
     bool square;
 };

@@ -24,39 +24,6 @@ constexpr int kBS = 256;
 //   plane 2 (z,y), rho = x:  x mod xw, y, z, x / xw, t   (x in chunks of xw sites, at
 //                            least 128 bytes of one element plane, so loads coalesce)
 // This cuts the traffic behind L2 several-fold; it pays where occupancy is low (FP64).
-struct PlaneOrder {
-    uint32_t xw;   // x chunk width for plane 2 (divides NX)
-};
-
-__device__ __forceinline__ uint32_t plane_site(const Lat& L, const PlaneOrder& po, int pl, uint32_t o, int c[4]) {
-    const uint32_t nx = (uint32_t)L.n[1], ny = (uint32_t)L.n[2], nz = (uint32_t)L.n[3];
-    uint32_t q;
-    if (pl == 0) {
-        site_coords(L, o, c);
-    } else if (pl == 1) {
-        c[1] = (int)(o % nx);
-        q = o / nx;
-        c[3] = (int)(q % nz);
-        q /= nz;
-        c[2] = (int)(q % ny);
-        c[0] = (int)(q / ny);
-    } else {
-        const uint32_t xi = o % po.xw;
-        q = o / po.xw;
-        c[2] = (int)(q % ny);
-        q /= ny;
-        c[3] = (int)(q % nz);
-        q /= nz;
-        const uint32_t nxc = nx / po.xw;
-        c[1] = (int)((q % nxc) * po.xw + xi);
-        c[0] = (int)(q / nxc);
-    }
-    return (uint32_t)c[1] + nx * ((uint32_t)c[2] + ny * ((uint32_t)c[3] + nz * (uint32_t)c[0]));
-}
-
-// (mu, nu) of magnetic plane pl: (y, x), (x, z), (z, y) in 0-based directions
-__device__ __forceinline__ int plane_mu(int pl) { return pl == 0 ? 2 : (pl == 1 ? 1 : 3); }
-__device__ __forceinline__ int plane_nu(int pl) { return pl == 0 ? 1 : (pl == 1 ? 3 : 2); }
 
 // B = -(1/V) sum_x sum_i ReTr(F_i F_i) over the planes (y,x), (x,z), (z,y)
 // (src/wloops.F90:502-506, 530-543); each block writes one compensated partial sum.
@@ -118,12 +85,14 @@ magnetic_kernel(Lat L, FV f, PlaneOrder po, uint32_t nb, double* __restrict__ pa
 }
 
 // per-site F for one plane.  layout 0: complex128 at the given strides; layout 1: SoA
-// planes (element e = a*3+b, re/im) in the field precision.
-template <typename FV, bool CLOVER>
+// planes (element e = a*3+b, re/im) in the field precision.  TESTED: only where *bad (links of an FP64 field
+// that the tiles of k_rect.hip found not unitary).
+template <typename FV, bool CLOVER, bool TESTED = false>
 __global__ void __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(sizeof(typename FV::real) == 4 ? 2 : 1)))
 fmunu_kernel(Lat L, FV f, int mu, int nu, void* __restrict__ out, int layout, OutStrides os, uint32_t unit,
-             uint32_t tb) {
+             uint32_t tb, const uint32_t* __restrict__ bad) {
     using R = typename FV::real;
+    if (TESTED && !*bad) return;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     // planes (x, z): each slice taken along z; planes containing time: along their spatial direction
     const int d = mu == 0 || nu == 0 ? mu + nu : (mu + nu == 4 ? 3 : 1);
@@ -168,8 +137,8 @@ fmunu_kernel(Lat L, FV f, int mu, int nu, void* __restrict__ out, int layout, Ou
 
 uint32_t magnetic_blocks(const Lat& L, int) { return 3 * ((L.V + kBS - 1) / kBS); }
 
-// x chunk width of plane 2: the smallest divisor of NX spanning >= 128 bytes, else NX
-static PlaneOrder plane_order(const Lat& L, size_t real_bytes) {
+// the least divisor of NX that spans 128 bytes of one element plane, else whole rows
+PlaneOrder plane_order(const Lat& L, size_t real_bytes) {
     PlaneOrder po{(uint32_t)L.n[1]};
     for (int w = 1; w < L.n[1]; ++w)
         if (L.n[1] % w == 0 && (size_t)w * real_bytes >= 128) {
@@ -226,7 +195,7 @@ hipError_t launch_magnetic(const Lat& L, const void* U, int is_f32, int su3, dou
 }
 
 hipError_t launch_fmunu(const Lat& L, const void* U, int is_f32, int mu, int nu, int clover_only, void* out,
-                        int out_layout, const int64_t s6[6], hipStream_t st) {
+                        int out_layout, const int64_t s6[6], hipStream_t st, const uint32_t* bad) {
     // Order of the sites.  Planes containing time: the same sites of all slices one after another, as the
     // leaves reach 3 slices either way and the blocks running together then share those slices in L2.
     // Spatial planes: storage order, but where t is dense in the output and more than one wave per SIMD
@@ -244,10 +213,17 @@ hipError_t launch_fmunu(const Lat& L, const void* U, int is_f32, int mu, int nu,
     OutStrides os{0, 0, 0, 0, 0, 0};
     if (s6) os = OutStrides{s6[0], s6[1], s6[2], s6[3], s6[4], s6[5]};
     with_view(L.V, U, is_f32, [&](auto f) {
+        using F = decltype(f);
+        if constexpr (sizeof(typename F::real) == 8 && F::buffered) {
+            if (bad) {
+                fmunu_kernel<F, false, true><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb, bad);
+                return;
+            }
+        }
         if (clover_only)
-            fmunu_kernel<decltype(f), true><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb);
+            fmunu_kernel<F, true><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb, nullptr);
         else
-            fmunu_kernel<decltype(f), false><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb);
+            fmunu_kernel<F, false><<<g, kBS, 0, st>>>(L, f, mu, nu, out, out_layout, os, unit, tb, nullptr);
     });
     return hipGetLastError();
 }

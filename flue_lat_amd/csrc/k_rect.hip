@@ -205,7 +205,8 @@ struct Cover {
     }
 };
 
-// Per tile: its sites' clover AH parts from the four footprints that cover them.  One wavefront
+// Per tile (none where `bad` says that the links are not unitary): its sites' clover AH parts from the four
+// footprints that cover them.  One wavefront
 // (measured faster than a thread per site).  STORE = false: sum |F|^2 over the tile into one
 // compensated partial per tile.  Otherwise write each site's AH parts into Abuf, 9 planes of V
 // values per plane, d0 d1 d2, o01r o02r o12r, o01i o02i o12i, for a form of the B^2 adjoint:
@@ -216,10 +217,11 @@ struct Cover {
 enum class Store { kNone, kTiles, kSites };
 template <typename R, Store STORE, int W>
 __global__ void __launch_bounds__(kRW) rect_gather_kernel(Lat L0, Lat Lzy, RectTiles rt, const R* __restrict__ fpin,
-                                                         double* __restrict__ partials, R* __restrict__ Abuf) {
+                                                         double* __restrict__ partials, R* __restrict__ Abuf,
+                                                         const uint32_t* __restrict__ bad) {
     const bool zy = blockIdx.y == 2;
     const PlaneTiles g = plane_tiles(rt);
-    if (blockIdx.x >= g.tiles) return;
+    if (blockIdx.x >= g.tiles || (bad && *bad)) return;
     const Lat L = zy ? Lzy : L0;
     const int rp = zy ? 0 : (int)blockIdx.y;
     const uint32_t tile = xcd_block(blockIdx.x, g.tiles);
@@ -329,37 +331,55 @@ __global__ void __launch_bounds__(256) zy_relayout_kernel(Lat L, const R* __rest
     relayout<R, T>(L, 3, 3, 2, blockIdx.x, U, P);
 }
 
-// B of links that turned out not unitary: partials[i] of `tiles`, by quadrants, i the share of the
-// lattice's sites that starts at V i / tiles.  (Full products in the order of magnetic variant 4.)
-template <typename FV>
-__device__ __forceinline__ void general_share(const Lat& L, const FV& f, uint32_t i, uint32_t tiles,
-                                              double* __restrict__ partial) {
-    const uint32_t lo = (uint32_t)((uint64_t)L.V * i / tiles), hi = (uint32_t)((uint64_t)L.V * (i + 1) / tiles);
-    double acc = 0.0;
-    for (uint32_t s = lo + threadIdx.x; s < hi; s += kRW) {
-        int c[4];
-        site_coords(L, s, c);
-#pragma unroll 1
-        for (int p = 0; p < 3; ++p) {
-            const int mu = p == 0 ? 2 : (p == 1 ? 1 : 3), nu = p == 0 ? 1 : (p == 1 ? 3 : 2);
-            acc += f_norm2(plane_ah<false, true, false, true>(plane_geom(L, f, s, c[mu], c[nu], mu, nu)));
-        }
-    }
-    const DD r = block_sum<kRW>(DD{acc, 0.0});
-    if (threadIdx.x == 0) {
-        partial[0] = r.hi;
-        partial[1] = r.lo;
-    }
-    __syncthreads();  // block_sum's shared slots serve the next share
+// B of links that turned out not unitary, into the same `tiles` partials: the plane-major quadrants
+// (k_clover.hip, variant 4), so many of whose blocks of 256 sites to a partial that no more are needed; the
+// partials left over are 0.  With the tiles given up on the way (every link off) 24^3x48 takes 1.30 ms and
+// 18x20x22x26 0.48 where the quadrant form alone takes 1.15 and 0.38; one bad link in the last tile, 1.49 and
+// 0.53.  (64-site shares of the lattice in storage order: 3.39 and 0.93.)
+constexpr int kGW = 256;
+__host__ __device__ __forceinline__ uint32_t general_blocks(const Lat& L) { return 3 * ((L.V + kGW - 1) / kGW); }
+__host__ __device__ __forceinline__ uint32_t general_size(const Lat& L, uint32_t tiles) {
+    return (general_blocks(L) + tiles - 1) / tiles;
+}
+__host__ __device__ __forceinline__ uint32_t general_groups(const Lat& L, uint32_t tiles) {
+    const uint32_t n = general_size(L, tiles);
+    return (general_blocks(L) + n - 1) / n;
 }
 
-// workgroups that look whether there is anything to do: those resident at once
+template <typename FV>
+__device__ __forceinline__ void general_group(const Lat& L, const FV& f, const PlaneOrder& po, uint32_t grp, uint32_t tiles,
+                                              double* __restrict__ partials) {
+    const uint32_t n = general_size(L, tiles), nb = general_blocks(L) / 3, hi = min(3 * nb, (grp + 1) * n);
+    double acc = 0.0;
+#pragma unroll 1
+    for (uint32_t b = grp * n; b < hi; ++b) {
+        const int pl = __builtin_amdgcn_readfirstlane((int)(b / nb));  // (a division leaves the scalar registers)
+        const uint32_t o = (b - (uint32_t)pl * nb) * kGW + threadIdx.x;
+        if (o >= L.V) continue;
+        int c[4];
+        const uint32_t s = plane_site(L, po, pl, o, c);
+        const int mu = plane_mu(pl), nu = plane_nu(pl);
+        acc += f_norm2(plane_ah<false, true, false, true>(plane_geom(L, f, s, c[mu], c[nu], mu, nu)));
+    }
+    const DD r = block_sum<kGW>(DD{acc, 0.0});
+    if (threadIdx.x == 0) {
+        partials[2 * grp] = r.hi;
+        partials[2 * grp + 1] = r.lo;
+    }
+    if (grp == 0)
+        for (uint32_t i = 2 * general_groups(L, tiles) + threadIdx.x; i < 2 * tiles; i += kGW) partials[i] = 0.0;
+    __syncthreads();  // block_sum's shared slots serve the next group
+}
+
+// workgroups that look whether there is anything to do (256 are resident at once; a multiple of the XCDs)
 constexpr uint32_t kGeneralGrid = 1024;
 template <typename FV>
-__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
-general_kernel(Lat L, FV f, uint32_t tiles, const uint32_t* __restrict__ bad, double* __restrict__ partials) {
+__global__ void __launch_bounds__(kGW) __attribute__((amdgpu_waves_per_eu(1, 1)))
+general_kernel(Lat L, FV f, PlaneOrder po, uint32_t tiles, const uint32_t* __restrict__ bad, double* __restrict__ partials) {
     if (!*bad) return;
-    for (uint32_t i = blockIdx.x; i < tiles; i += gridDim.x) general_share(L, f, i, tiles, partials + 2 * i);
+    const uint32_t groups = general_groups(L, tiles);
+    for (uint32_t b = blockIdx.x; b < groups; b += gridDim.x)
+        general_group(L, f, po, xcd_block(b, groups), tiles, partials);
 }
 
 // the copy read as a field of Lzy whose directions 1 and 2 are its two blocks (the view's base is one
@@ -428,22 +448,26 @@ ens_rect_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ re
 }
 
 template <typename R>
-__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
-ens_general_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ rect, int n, uint32_t tiles,
+__global__ void __launch_bounds__(kGW) __attribute__((amdgpu_waves_per_eu(1, 1)))
+ens_general_kernel(const EnsEntry* __restrict__ tab, const EnsRect* __restrict__ rect, int n, uint32_t groups,
                    const R* __restrict__ U, const uint32_t* __restrict__ bad, double* __restrict__ partials) {
     if (!*bad) return;
-    for (uint32_t i = blockIdx.x; i < tiles; i += gridDim.x) {
-        const int c = rect_cfg<&EnsRect::tile0>(rect, n, i);
+    for (uint32_t b = blockIdx.x; b < groups; b += gridDim.x) {
+        const uint32_t grp = xcd_block(b, groups);
+        const int c = rect_cfg<&EnsRect::grp0>(rect, n, grp);
         const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
+        const EnsRect& r = *(const EnsRect*)((CEnsRect*)rect + c);
         const FieldView<R, true> f{U + e.off, e.L.V};
-        general_share(e.L, f, i - rect[c].tile0, rect[c].tiles, partials + 2 * i);
+        general_group(e.L, f, r.po, grp - r.grp0, r.tiles, partials + 2 * (size_t)r.tile0);
     }
 }
 
 template <typename R, int W>
 __global__ void __launch_bounds__(kRW) ens_gather_kernel(const EnsEntry* __restrict__ tab,
                                                          const EnsRect* __restrict__ rect, int n,
-                                                         const R* __restrict__ fpin, double* __restrict__ partials) {
+                                                         const R* __restrict__ fpin, double* __restrict__ partials,
+                                                         const uint32_t* __restrict__ bad) {
+    if (bad && *bad) return;
     const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
     const int c = rect_cfg<&EnsRect::tile0>(rect, n, b);
     const EnsEntry& e = *(const EnsEntry*)((CEnsEntry*)tab + c);
@@ -496,8 +520,10 @@ constexpr int kFT = 16;
 template <typename R, bool TIME>
 __global__ void __launch_bounds__(kFT * kFT) plane_gather_kernel(Lat L, int rp, PlaneTiles g,
                                                                const R* __restrict__ fpin, R sign,
-                                                               double* __restrict__ out, OutStrides os) {
+                                                               double* __restrict__ out, OutStrides os,
+                                                               const uint32_t* __restrict__ bad) {
     __shared__ R parts[9][kFT][kFT + 1];
+    if (*bad) return;
     const uint32_t nx = (uint32_t)L.n[1], nt = (uint32_t)L.n[0], ny = (uint32_t)L.n[2];
     const uint32_t bts = (nt + kFT - 1) / kFT, bxs = (nx + kFT - 1) / kFT;
     uint32_t q = xcd_block(blockIdx.x, gridDim.x);
@@ -537,19 +563,6 @@ __global__ void __launch_bounds__(kFT * kFT) plane_gather_kernel(Lat L, int rp, 
         }
         const int c[4] = {(int)(t0 + i), (int)(x0 + j), (int)y, (int)z};
         store_f(h, c, out, os);
-    }
-}
-
-// F by quadrants, where a link turned out not unitary
-template <typename FV>
-__global__ void __launch_bounds__(kRW) __attribute__((amdgpu_waves_per_eu(1, 1)))
-plane_general_kernel(Lat L, FV f, int mu, int nu, const uint32_t* __restrict__ bad, double* __restrict__ out,
-                     OutStrides os) {
-    if (!*bad) return;
-    for (uint32_t s = blockIdx.x * kRW + threadIdx.x; s < L.V; s += gridDim.x * kRW) {
-        int c[4];
-        site_coords(L, s, c);
-        store_f(plane_ah<false, true, false, true>(plane_geom(L, f, s, c[mu], c[nu], mu, nu)), c, out, os);
     }
 }
 
@@ -650,20 +663,22 @@ hipError_t launch_magnetic_rect(const Lat& L, const void* U, int is_f32, int su3
                         rect_kernel<F, false, 1, W, true><<<g, kRW, 0, st>>>(L, f, Lzy, fzy, rt, fp, bad);
                 }
                 if (Abuf && tiled)
-                    rect_gather_kernel<R, Store::kTiles, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
+                    rect_gather_kernel<R, Store::kTiles, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf, nullptr);
                 else if (Abuf)
-                    rect_gather_kernel<R, Store::kSites, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf);
+                    rect_gather_kernel<R, Store::kSites, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, nullptr, (R*)Abuf, nullptr);
                 else
-                    rect_gather_kernel<R, Store::kNone, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, partials, nullptr);
+                    rect_gather_kernel<R, Store::kNone, W><<<g, kRW, 0, st>>>(L, Lzy, rt, fp, partials, nullptr, check ? bad : nullptr);
             };
             if (rt.p[0].square() && rt.p[1].square() && rt.p[2].square())
                 rect(std::integral_constant<int, 16>());
             else
                 rect(std::integral_constant<int, 0>());
             if constexpr (sizeof(R) == 8)
-                if (check && !Abuf)
-                    general_kernel<<<std::min(kGeneralGrid, rect_partials(L, is_f32)), kRW, 0, st>>>(
-                        L, f, rect_partials(L, is_f32), bad, partials);
+                if (check && !Abuf) {
+                    const uint32_t tiles = rt.p[0].tiles + rt.p[1].tiles + rt.p[2].tiles;
+                    general_kernel<<<std::min(kGeneralGrid, general_groups(L, tiles)), kGW, 0, st>>>(
+                        L, f, plane_order(L, sizeof(R)), tiles, bad, partials);
+                }
         }
     });
     if (npart) *npart = rect_partials(L, is_f32);
@@ -683,7 +698,7 @@ constexpr uint32_t kEnsRectSitesF32 = 49152;
 //   8 x 16^4           524,288         0.665 -> 0.365   1.191 -> 0.677
 bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRect* rect, EnsRectGrid* g) {
     if (!fits_buffer(maxV, is_f32)) return false;
-    uint64_t sites = 0, tiles = 0, copies = 0;
+    uint64_t sites = 0, tiles = 0, copies = 0, groups = 0;
     g->square = true;
     g->copy_edge = 16;
     for (int c = 0; c < n; ++c)
@@ -695,9 +710,12 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
         r.rt = rect_split(L, is_f32 ? kMaxCells<float> : kMaxCells<double>, 1);
         if (rect_cells(r.rt) * 9 > (uint64_t)48 * L.V) return false;
         r.Lzy = zy_lattice(L);
+        r.po = plane_order(L, sizeof(double));
         r.tile0 = (uint32_t)tiles;
         r.tiles = r.rt.p[0].tiles + r.rt.p[1].tiles + r.rt.p[2].tiles;
         r.copy0 = (uint32_t)copies;
+        r.grp0 = (uint32_t)groups;
+        groups += general_groups(L, r.tiles);
         for (const PlaneTiles& p : r.rt.p) g->square = g->square && p.square();
         sites += L.V;
         tiles += r.tiles;
@@ -705,6 +723,7 @@ bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRec
     }
     g->tiles = (uint32_t)tiles;
     g->copies = (uint32_t)copies;
+    g->groups = (uint32_t)groups;
     return sites >= kRectSites && tiles < 0x80000000ull && copies < 0x80000000ull;
 }
 
@@ -721,10 +740,10 @@ hipError_t launch_ens_rect(const EnsEntry* tab, const EnsRect* rect, int n, cons
             ens_relayout_kernel<R, 16><<<g.copies, 256, 0, st>>>(tab, rect, n, (const R*)fld, (R*)copy, bad);
         ens_rect_kernel<R, F32, F32 ? 2 : 1, W, !F32>
             <<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fld, (const R*)copy, (R*)fp, bad);
-        ens_gather_kernel<R, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fp, partials);
+        ens_gather_kernel<R, W><<<g.tiles, kRW, 0, st>>>(tab, rect, n, (const R*)fp, partials, F32 ? nullptr : bad);
         if constexpr (!F32)  // links that are not unitary
-            ens_general_kernel<R><<<std::min(kGeneralGrid, g.tiles), kRW, 0, st>>>(tab, rect, n, g.tiles, (const R*)fld,
-                                                                                   bad, partials);
+            ens_general_kernel<R><<<std::min(kGeneralGrid, g.groups), kGW, 0, st>>>(tab, rect, n, g.groups,
+                                                                                    (const R*)fld, bad, partials);
     };
     auto sized = [&](auto real) {
         if (g.square)
@@ -808,14 +827,15 @@ hipError_t launch_fmunu_rect(const Lat& L, const void* U, int mu, int nu, void* 
         plane_kernel<F, TIME><<<p.g.tiles, kRW, 0, st>>>(p.L, fl, p.rp, p.g, fp, bad);
         const uint32_t nb = (uint32_t)((p.L.n[0] + kFT - 1) / kFT) * (uint32_t)((p.L.n[1] + kFT - 1) / kFT) *
                             (uint32_t)p.L.n[2] * (uint32_t)p.L.n[3];
-        plane_gather_kernel<double, TIME><<<nb, kFT * kFT, 0, st>>>(p.L, p.rp, p.g, fp, sign, (double*)out, osl);
+        plane_gather_kernel<double, TIME><<<nb, kFT * kFT, 0, st>>>(p.L, p.rp, p.g, fp, sign, (double*)out, osl,
+                                                                     bad);
     };
     if (p.rp == 2)
         run(std::true_type());
     else
         run(std::false_type());
-    plane_general_kernel<<<kGeneralGrid, kRW, 0, st>>>(L, f, mu, nu, bad, (double*)out, os);
-    return hipGetLastError();
+    // by quadrants, where a link turned out not unitary
+    return launch_fmunu(L, U, 0, mu, nu, 0, out, 0, s6, st, bad);
 }
 
 }  // namespace flue

@@ -39,3 +39,18 @@ def test_fmunu_of_drifted_links(FL, mu, nu):
                                      ctypes.c_void_p(want.data_ptr()), _lib.FLUE_OUT_STRIDED, st,
                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "flue_fmunu")
     assert torch.equal(f.fmunu(mu, nu), want)
+
+
+@pytest.mark.parametrize("dims", [(7, 24, 24, 23), (9, 20, 22, 24), (2, 34, 33, 47), (1, 400, 15, 16), (3, 16, 16, 16)])
+def test_magnetic_of_a_field_that_is_not_unitary(FL, dims):
+    # every link scaled: blocks of the quadrant form dealt to more partials than there are blocks, and to
+    # fewer.  Against the quadrant form: the same numbers in sums of another order; an ensemble likewise.
+    from flue_lat_amd.ensemble import Ensemble
+    e = Ensemble.random([dims, (13, 14, 17, 33), dims], [5, 6, 7], 0.3, "fp64")
+    e.data.mul_(1.01)
+    ref = [e.field(c).magnetic(variant=4) for c in range(3)]
+    for v in (0, 7):
+        assert abs(e.field(0).magnetic(variant=v) - ref[0]) < 1e-14 * ref[0]
+    _, B = e.flow(0.01, 0, measure_every=1)
+    for c in range(3):
+        assert abs(B[0, c] - ref[c]) < 1e-14 * ref[c]
