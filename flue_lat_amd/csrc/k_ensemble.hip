@@ -66,13 +66,15 @@ __global__ void __launch_bounds__(kBS) ens_flow_kernel(const EnsEntry* __restric
 // Plaquette-first stencil over the ensemble: the six plaquette parts of every site of every
 // field (48 reals per site, config c's block at 2/3 of its field offset), then the links, the
 // four waves of a workgroup on the four directions of 64 sites.
-// TEST: sets bad[c] and bad[n] where a link of configuration c is not SU(3).
+// TEST: sets bad[c] and bad[n] where a link of configuration c is not SU(3); else nothing for a configuration
+// of which that was found.
 template <typename R, bool BUF, bool TEST>
 __global__ void __launch_bounds__(kBS) ens_plaq_ta_kernel(const EnsEntry* __restrict__ tab, int n,
                                                           const R* __restrict__ win, R* __restrict__ T,
                                                           uint32_t* __restrict__ bad) {
     const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
     const int cfg = find_cfg(tab, n, lb);
+    if (!TEST && bad && bad[cfg]) return;
     const EnsEntry& e = entry(tab, cfg);
     const uint32_t s = (lb - e.blk0) * kBS + threadIdx.x;
     if (s >= e.L.V) return;
@@ -115,8 +117,8 @@ __global__ void __launch_bounds__(kBS) ens_general_flow_kernel(const EnsEntry* _
                                                                R* __restrict__ acc, double eps, double ca, double cb,
                                                                int reunit, const uint32_t* __restrict__ bad) {
     if (!bad[n]) return;
-    for (uint64_t lu = blockIdx.x; lu < 4 * (uint64_t)total; lu += gridDim.x) {
-        const uint32_t lb = (uint32_t)(lu >> 2);
+    for (uint32_t b = blockIdx.x; b < 4 * total; b += gridDim.x) {
+        const uint32_t lu = xcd_block(b, 4 * total), lb = lu >> 2;
         const int cfg = find_cfg(tab, n, lb);
         if (!bad[cfg]) continue;
         const EnsEntry& e = entry(tab, cfg);
@@ -206,13 +208,13 @@ hipError_t launch_ens_flow_stage(const EnsEntry* tab, int n, uint32_t total, uin
                 clear_words_kernel<<<n / kBS + 1, kBS, 0, st>>>(bad, n + 1);
                 ens_plaq_ta_kernel<R, B, kF64><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T, bad);
             } else {
-                ens_plaq_ta_kernel<R, B, false><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T, nullptr);
+                ens_plaq_ta_kernel<R, B, false><<<total, kBS, 0, st>>>(tab, n, (const R*)win, (R*)T, bad);
             }
             if constexpr (kF64) {
                 if (bad) {
                     ens_flow_pf_kernel<R, B, true><<<4 * total, kBS, 0, st>>>(
                         tab, n, (const R*)win, (const R*)T, (R*)wout, (R*)acc, eps, ca, cb, reunit, bad);
-                    ens_general_flow_kernel<R, B><<<(uint32_t)std::min<uint64_t>(kGeneralGrid, 4 * (uint64_t)total), kBS, 0, st>>>(
+                    ens_general_flow_kernel<R, B><<<std::min(kGeneralGrid, 4 * total), kBS, 0, st>>>(
                         tab, n, total, (const R*)win, (R*)wout, (R*)acc, eps, ca, cb, reunit, bad);
                     return;
                 }

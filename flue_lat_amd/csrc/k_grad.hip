@@ -94,10 +94,11 @@ __global__ void __launch_bounds__(kBS) flow_stage_kernel(Lat L, FV f, BlockOrder
 // At 48^3x96 the first pass takes 1.15 ms (FP32) and 2.11 ms (FP64) with ROWS2, at 4.0 and 4.4
 // TB/s beyond L2; taking two of the six planes per wave instead, with 21 link reads a site
 // instead of 16, took 1.33 and 2.34 ms and gained nothing on a lattice of 162,000 sites.
-// TEST: sets *bad where a link is not SU(3).
+// TEST: sets *bad where a link is not SU(3); else nothing where that was found.
 template <bool ROWS2, bool TEST, typename FV>
 __global__ void __launch_bounds__(kBS) plaq_ta_kernel(Lat L, FV f, BlockOrder bo, typename FV::real* __restrict__ T,
                                                       uint32_t* __restrict__ bad) {
+    if (!TEST && bad && *bad) return;
     uint32_t s;
     int c[4];
     if (!order_site(L, bo, xcd_block(blockIdx.x, gridDim.x), threadIdx.x, s, c)) return;
@@ -145,20 +146,19 @@ __global__ void __launch_bounds__(kBS) flow_stage_pf_kernel(Lat L, FV f, BlockOr
     flow_link_pf(L, f, T, wout, acc, s, c, mu, eps, ca, cb, reunit);
 }
 
-// The stage by staple sums where the links turned out not SU(3): the 4 nb (direction, block) pairs of
-// flow_stage_kernel in storage order on as many workgroups as are resident at once, which look first
-// whether there is anything to do.
+// The stage by staple sums where the links turned out not SU(3): the blocks of flow_stage_kernel on more
+// workgroups than are resident at once, which look first whether there is anything to do.
 constexpr uint32_t kGeneralGrid = 1024;
 template <typename FV>
-__global__ void __launch_bounds__(kBS) flow_general_kernel(Lat L, FV f, uint32_t nb, typename FV::real* __restrict__ wout,
+__global__ void __launch_bounds__(kBS) flow_general_kernel(Lat L, FV f, BlockOrder bo, typename FV::real* __restrict__ wout,
                                                            typename FV::real* __restrict__ acc, double eps, double ca,
                                                            double cb, int reunit, const uint32_t* __restrict__ bad) {
     if (!*bad) return;
-    for (uint32_t blk = blockIdx.x; blk < 4 * nb; blk += gridDim.x) {
-        const uint32_t s = (blk >> 2) * kBS + threadIdx.x;
-        if (s >= L.V) continue;
+    for (uint32_t b = blockIdx.x; b < 4 * bo.nb; b += gridDim.x) {
+        const uint32_t blk = xcd_block(b, 4 * bo.nb);
+        uint32_t s;
         int c[4];
-        site_coords(L, s, c);
+        if (!order_site(L, bo, blk >> 2, threadIdx.x, s, c)) continue;
         flow_link(L, f, wout, acc, s, c, (int)(blk & 3u), eps, ca, cb, reunit);
     }
 }
@@ -252,14 +252,13 @@ hipError_t launch_flow_stage(const Lat& L, const void* Win, int is_f32, void* Wo
                 clear_word_kernel<<<1, 1, 0, st>>>(bad);
                 plaq_ta_kernel<true, kF64, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T, bad);
             } else {
-                plaq_ta_kernel<true, false, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T, nullptr);
+                plaq_ta_kernel<true, false, F><<<bo.nb, kBS, 0, st>>>(L, f, bo, (R*)T, bad);
             }
             if constexpr (kF64) {
                 if (bad) {
-                    const uint32_t nb = (L.V + kBS - 1) / kBS;
                     links(std::true_type());
-                    flow_general_kernel<F><<<std::min(kGeneralGrid, 4 * nb), kBS, 0, st>>>(
-                        L, f, nb, (R*)Wout, acc, eps, ca, cb, reunit, bad);
+                    flow_general_kernel<F><<<std::min(kGeneralGrid, 4 * bo.nb), kBS, 0, st>>>(
+                        L, f, bo, (R*)Wout, acc, eps, ca, cb, reunit, bad);
                     return;
                 }
             }
