@@ -1060,6 +1060,11 @@ void remember(int op, const int32_t key[4], int prec, int v, double ms) {
     g_tune[tune_key(op, key, prec)] = TuneVal{v, ms};
 }
 
+void forget(int op, const int32_t key[4], int prec) {
+    std::lock_guard<std::mutex> lk(g_tune_mutex);
+    g_tune.erase(tune_key(op, key, prec));
+}
+
 }  // namespace
 
 extern "C" {
@@ -1119,7 +1124,18 @@ int flue_autotune(int32_t op, const int32_t dims[4], const void* U, int32_t prec
     // the rectangle-first magnetic form (the last variant) only where it applies
     const int nvar = op == FLUE_OP_MAGNETIC && !magnetic_rect_ok(L, prec) ? kMagneticRect - 1 : op_variants(op);
     if ((rc = time_variants(nvar, reps, st, launch, &bv, &bms))) return rc;
-    remember(op, dims, prec, bv, bms);
+    // the plaquette of small lattices has an untuned form without a number: left alone where it is faster
+    bool untuned = false;
+    if (op == FLUE_OP_PLAQUETTE && plaquette_default(L, is_f32) == kPlaquettePlanes) {
+        int only = 0;
+        double ms = 0.0;
+        if ((rc = time_variants(1, reps, st, [&](int) { return launch(kPlaquettePlanes); }, &only, &ms))) return rc;
+        untuned = ms <= bms;
+    }
+    if (untuned)
+        forget(op, dims, prec);
+    else
+        remember(op, dims, prec, bv, bms);
     if (best) *best = bv;
     if (best_ms) *best_ms = bms;
     return FLUE_OK;

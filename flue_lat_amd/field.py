@@ -325,7 +325,9 @@ class GaugeField:
         precision, extents); later calls of that operation use it.  op: "magnetic" (kernel
         form x waves per SIMD), "b2_grad" (gather or reverse-mode adjoint), "plaquette" (time
         slices per thread, also used by wilson_action), "flow" (stencil visit order, used by
-        wilson_flow and wilson_grad).  The field is only read.  Returns (variant, ms per call)."""
+        wilson_flow and wilson_grad).  The field is only read.  Returns (variant, ms per call) of the
+        fastest numbered variant (small lattices have untuned forms without a number: see
+        FLUE_OP_MAGNETIC and FLUE_OP_PLAQUETTE in flue_c.h)."""
         if op not in _lib.OPS or op == "ensemble_flow":
             raise ValueError(f"unknown operation {op!r}")
         code = _lib.OPS[op]

@@ -404,10 +404,15 @@ int flue_wilson_flow(const int32_t dims[4], void* U, int32_t prec, double eps, i
 /* operation compute the same quantity: the flow orders and the ensemble's give            */
 /* bit-identical results, the others agree to rounding (their summation orders differ).    */
 /*   FLUE_OP_MAGNETIC       1..7  kernel form x waves per SIMD, or rectangle-first (7, timed  */
-/*                                only where it applies) (flue_magnetic_ex)                 */
+/*                                only where it applies) (flue_magnetic_ex).  The untuned     */
+/*                                form of small FP64 lattices (up to 10,922 sites, or 16,384  */
+/*                                where 16 divides the spatial extents), a wave per quadrant, */
+/*                                has no number and is faster: leave those untuned            */
 /*   FLUE_OP_B2_GRAD        1..2  per-link gather / reverse mode (flue_b2_grad_ex)            */
 /*   FLUE_OP_PLAQUETTE      1..6  time slices per thread 2, 3, 4, 6, 8, 12 (flue_plaquette,   */
-/*                                flue_wilson_action)                                        */
+/*                                flue_wilson_action).  Where the untuned form of small       */
+/*                                lattices, a thread per site and plane, is faster than all   */
+/*                                of them nothing is remembered                               */
 /*   FLUE_OP_FLOW          1..13  stencil of the flow and the Wilson gradient: staple sums   */
 /*                                in storage order or in boxes of up to 1024, 2048, 3072,    */
 /*                                4096 or 6144 sites swept along t (1..6, bit-identical);     */
