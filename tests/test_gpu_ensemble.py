@@ -136,3 +136,28 @@ def test_ensemble_magnetic_tiles(FL, dims, prec, tol):
             if m < 3:
                 g.wilson_flow(0.01, 1, use_graph=False)
         assert torch.allclose(e.field(c).data, g.data, rtol=0, atol=1e-12 if prec == "fp64" else 2e-5)
+
+
+@pytest.mark.parametrize("dims", [
+    [(21, 14, 17, 13), (9, 17, 25, 16), (14, 12, 33, 19)],   # uneven tiles, copies in 8 x 8 pieces
+    [(16, 14, 16, 15), (12, 15, 30, 16)],                    # uneven tiles, copies in 16 x 16 pieces
+    [(12, 16, 16, 32), (13, 16, 16, 16)],                    # 16 x 16 tiles
+])
+def test_ensemble_magnetic_tiles_fp32(FL, dims):
+    # every field with the 49,152 sites from which FP32 ensembles take tiles.  Against the quadrant form of
+    # each field: products of a leaf rounded differently, 2^-24 each and averaged over the sites; 2e-7 is
+    # three roundings.  Against FP64 of the same links: the bound of FP32 links, 1e-6.
+    from flue_lat_amd.ensemble import Ensemble
+    e = Ensemble.random(dims, [60 + c for c in range(len(dims))], 0.3, "fp32")
+    singles = [e.field(c).clone() for c in range(len(dims))]
+    _, B = e.flow(0.01, 3, measure_every=1)
+    for c, g in enumerate(singles):
+        for m in range(4):
+            b = g.magnetic(variant=1)
+            assert B[m, c] != b or m > 0   # another form
+            assert abs(B[m, c] - b) < 2e-7 * b, (dims[c], m)
+            b64 = g.astype("fp64").magnetic(variant=1)
+            assert abs(B[m, c] - b64) < 1e-6 * b64, (dims[c], m)
+            if m < 3:
+                g.wilson_flow(0.01, 1, use_graph=False)
+        assert torch.allclose(e.field(c).data, g.data, rtol=0, atol=2e-5)

@@ -233,3 +233,19 @@ def test_flow_stage_entry_composes_to_one_step(FL):
     assert _lib.lib().flue_flow_stage(dims, ctypes.c_void_p(bufs[0].data_ptr()), _lib.FLUE_F64,
                                       ctypes.c_void_p(bufs[0].data_ptr()), ctypes.c_void_p(acc.data_ptr()),
                                       0.03, 0, stream) == 1
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5)])
+@pytest.mark.parametrize("dims", [(39, 13, 14, 15), (3, 16, 16, 16)])
+def test_autograd_magnetic_on_tiles(FL, dims, prec, tol):
+    # lattices whose B and adjoint run on tiles: value and gradient of autograd.magnetic against the oracle
+    from flue_lat_amd import autograd
+    Un = O.random_field(dims, 8300 + dims[1], 0.3)
+    U = torch.from_numpy(Un).cuda().requires_grad_()
+    B = autograd.magnetic(U, prec)
+    (3.0 * B).backward()
+    want = O.magnetic(Un)
+    assert abs(B.item() - want) < (1e-12 if prec == "fp64" else 1e-6) * want
+    E = 6.0 * torch.matmul(torch.from_numpy(O.b2_grad(Un)), torch.from_numpy(Un))
+    assert U.grad.dtype == torch.complex128 and U.grad.shape == U.shape
+    assert float((U.grad.cpu() - E).abs().max()) < tol * float(E.abs().max())

@@ -111,3 +111,22 @@ def test_host_functions_copy_what_they_read(FL, dims):
         assert np.array_equal(fc.loop5munucoord_c(U, mu, nu), f.fmunu(mu, nu).cpu().numpy())
         assert fc.wmunu_c(U, mu, nu, 2, 1) == f.wilson_loop(mu, nu, 2, 1)
         assert fc.wmunutau_c(U, 1, mu, nu, 1, 2) == f.wilson_loop(mu, nu, 1, 2, tau=1)
+
+
+def test_host_functions_copy_two_and_three_directions(FL):
+    # 18,018 sites: leaving out a single direction saves more than the 2 MB from which a part of the array is
+    # copied, so every call that reads two or three directions takes them out of the array by rows
+    dims = (14, 9, 11, 13)
+    fc = FL.compiled.flue_c
+    U = np.asfortranarray(FL.GaugeField.random(dims, 17, 0.4).to_complex().cpu().numpy())
+    f = FL.GaugeField.from_complex(U)
+    for args in ((1, 4, 4), (2, 4, 4), (1, 1, 4), (1, 3, 3), (2, 3, 3), (3, 3, 4), (1, 2, 2), (2, 2, 4)):
+        assert fc.plaquette_c(U, *args)[:2] == f.plaquette(*args), args
+        assert fc.genplaquette_c(U, *args)[:2] == f.plaquette(*args), args
+    assert fc.polyakov_c(U)[:2] == f.polyakov()
+    assert fc.magnetic_c(U) == f.magnetic()
+    for mu, nu in itertools.product(range(1, 5), range(1, 5)):
+        assert np.array_equal(fc.loop5munucoord_c(U, mu, nu), f.fmunu(mu, nu).cpu().numpy()), (mu, nu)
+        assert np.array_equal(fc.cloverloopmunucoord_c(U, mu, nu), f.fmunu(mu, nu, clover=True).cpu().numpy()), (mu, nu)
+        assert fc.wmunu_c(U, mu, nu, 2, 1) == f.wilson_loop(mu, nu, 2, 1), (mu, nu)
+        assert fc.wmunutau_c(U, 3, mu, nu, 1, 2) == f.wilson_loop(mu, nu, 1, 2, tau=3), (mu, nu)
