@@ -104,10 +104,14 @@ class GaugeField:
 
     def magnetic_workspace(self):
         """The workspace of magnetic(): every variant's, including the rectangle-first
-        form's footprints (flue_magnetic_work_bytes); kept with the field."""
+        form's footprints (flue_magnetic_work_bytes); kept with the field.  Where the card has
+        no room for those, workspace(), with which magnetic() takes the quadrant form."""
         if self._mws is None:
             n = _lib.lib().flue_magnetic_work_bytes(self._cdims, self.prec)
-            self._mws = torch.empty(n, dtype=torch.uint8, device=self.device)
+            try:
+                self._mws = torch.empty(n, dtype=torch.uint8, device=self.device)
+            except torch.cuda.OutOfMemoryError:
+                return self.workspace()
         return self._mws
 
     @classmethod
