@@ -329,11 +329,6 @@ b2_tile_kernel(Lat L0, FV f0, Lat Lzy, FV fzy, RectTiles rt, uint32_t t0, uint32
 
 // The 8 sums of the link of direction d1 (DIR = 0) or d2 (1) at local cell (cx, cy) of a tile: its
 // own footprint, then those of the tiles before it along d1, along d2 and diagonally.
-struct Cover {
-    const void* own;
-    int64_t left, below;  // offsets in cells to those tiles' footprints
-    int shift1, shift2;   // their extents
-};
 template <typename R>
 __device__ __forceinline__ void add_cover(double acc[8], const R* own, int64_t left, int64_t below, int fc, int f1,
                                           int dir, int cx, int cy, int shift1, int shift2) {
@@ -354,19 +349,13 @@ template <typename R>
 __device__ __forceinline__ void add_site(double acc[8], const PlaneTiles& g, uint64_t cell0, uint32_t ns,
                                          const R* __restrict__ fpin, int dir, uint32_t c1, uint32_t c2, uint32_t cs,
                                          uint32_t ct) {
-    auto find = [](uint32_t c, uint32_t q, uint32_t r, uint32_t& l) {
-        const uint32_t wide = r * (q + 1);
-        const uint32_t t = c < wide ? c / (q + 1) : r + (c - wide) / q;
-        l = c - (t * q + min(t, r));
-        return t;
-    };
-    uint32_t lx, ly;
-    const uint32_t t1 = find(c1, g.q1, g.r1, lx), t2 = find(c2, g.q2, g.r2, ly);
+    uint32_t o1, o2;
+    const uint32_t t1 = tile_of(c1, g.q1, g.r1, &o1), t2 = tile_of(c2, g.q2, g.r2, &o2);
     const uint32_t tl = t1 ? t1 - 1 : g.n1 - 1, tb = t2 ? t2 - 1 : g.n2 - 1;
     const uint64_t tile = (((uint64_t)ct * ns + cs) * g.n2 + t2) * g.n1 + t1;
     const R* own = fpin + 16 * (cell0 + tile * g.fc);
     add_cover(acc, own, ((int64_t)tl - t1) * (int64_t)g.fc, ((int64_t)tb - t2) * (int64_t)g.n1 * g.fc, (int)g.fc,
-              (int)g.f, dir, (int)lx, (int)ly, (int)(g.q1 + (tl < g.r1 ? 1u : 0u)), (int)(g.q2 + (tb < g.r2 ? 1u : 0u)));
+              (int)g.f, dir, (int)(c1 - o1), (int)(c2 - o2), (int)(g.q1 + (tl < g.r1 ? 1u : 0u)), (int)(g.q2 + (tb < g.r2 ? 1u : 0u)));
 }
 
 // Plane (z, y): the sums of the z and y links of the slab's sites, read z fastest and left x fastest
