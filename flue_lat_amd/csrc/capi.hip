@@ -92,6 +92,12 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // whether the rectangle-first magnetic form (variant 7) applies to the lattice
 bool magnetic_rect_ok(const Lat& L, int32_t prec) { return rect_fits(L) && fits_buffer(L.V, prec == FLUE_F32); }
 
+// the most blocks of any lattice sum but the Wilson-loop tables and the rectangle-first form
+uint32_t sum_blocks(const Lat& L) {
+    return std::max({plaquette_max_blocks(L), polyakov_blocks(L), path_blocks(L, -1, nullptr, 0), magnetic_blocks(L, 0),
+                     magnetic_blocks(L, 1), quad_fits(L, 0) ? quad_blocks(L) : 0u});
+}
+
 // magnetic workspace of a variant: the partials, and for variant 7 the footprints after them
 size_t magnetic_rect_partials(const Lat& L, int32_t prec) {
     return align256(partial_bytes(rect_partials(L, prec == FLUE_F32)));
@@ -281,12 +287,14 @@ double now_s() {
 
 // host drop-in prologue: dims by reference, field copied to the device as FP64 SoA; one allocation for
 // the planes, the array as it came and a scalar result (two where the array is below 2 MiB: the runtime
-// serves those from a block it holds)
+// serves those from a block it holds).  Once the planes are filled, the array's room is the call's
+// workspace: calls from several threads share nothing.
 struct HostField {
     int32_t dims[4];
     Lat L;
     DevBuf mem, arr;
-    void* soa;
+    void *soa, *ws;
+    size_t ws_bytes;
     double* scalar;
 };
 
@@ -314,12 +322,15 @@ int load_host_field(const int32_t* NT, const int32_t* NX, const int32_t* NY, con
     // runtime keeps a released allocation for the next of its size, and a program's calls on one lattice,
     // each of another size, took 0.3 ms more.)
     const size_t n = (size_t)(hi - lo + 1), dir = (size_t)h.L.V * sizeof(flue_c128);
-    const size_t soa = align256(flue_field_bytes(h.dims, FLUE_F64)), raw = align256(36 * dir);
+    const size_t soa = align256(flue_field_bytes(h.dims, FLUE_F64));
+    const size_t raw = align256(std::max({36 * dir, flue_magnetic_work_bytes(h.dims, FLUE_F64), partial_bytes(sum_blocks(h.L))}));
     const bool apart = raw < (size_t)2 << 20;
     FLUE_TRY(hipMalloc(&h.mem.p, soa + (apart ? 0 : raw) + 256));
     if (apart) FLUE_TRY(hipMalloc(&h.arr.p, raw));
     h.soa = h.mem.p;
     char* array = apart ? (char*)h.arr.p : (char*)h.mem.p + soa;
+    h.ws = array;
+    h.ws_bytes = raw;
     h.scalar = (double*)((char*)h.mem.p + soa + (apart ? 0 : raw));
     if (n == 4)
         FLUE_TRY(hipMemcpy(array, data, 36 * dir, hipMemcpyHostToDevice));
@@ -514,13 +525,7 @@ size_t flue_field_bytes(const int32_t dims[4], int32_t prec) {
 size_t flue_workspace_bytes(const int32_t dims[4]) {
     if (check_dims(dims)) return 0;
     const Lat L = make_lat(dims);
-    uint32_t nb = plaquette_max_blocks(L);
-    nb = std::max(nb, polyakov_blocks(L));
-    nb = std::max(nb, path_blocks(L, -1, nullptr, 0));
-    nb = std::max(nb, magnetic_blocks(L, 0));
-    nb = std::max(nb, magnetic_blocks(L, 1));
-    if (quad_fits(L, 0)) nb = std::max(nb, quad_blocks(L));
-    return std::max({partial_bytes(nb), wloop_partial_bytes(L, -1) + 256, wloop_partial_bytes(L, kEverySlice) + 256,
+    return std::max({partial_bytes(sum_blocks(L)), wloop_partial_bytes(L, -1) + 256, wloop_partial_bytes(L, kEverySlice) + 256,
                      check_bytes(L)});
 }
 
@@ -1445,7 +1450,7 @@ static int plaq_host(const int32_t* NT, const int32_t* NX, const int32_t* NY, co
                       : load_host_field(NT, NX, NY, NZ, data, h, lo, hi)))
         return rc;
     if ((rc = plaquette_count(h.dims, *muStart, *muEnd, *nuEnd, nP))) return rc;
-    if ((rc = flue_plaquette(h.dims, h.soa, FLUE_F64, *muStart, *muEnd, *nuEnd, h.scalar, nullptr, 0, nullptr)))
+    if ((rc = flue_plaquette(h.dims, h.soa, FLUE_F64, *muStart, *muEnd, *nuEnd, h.scalar, h.ws, h.ws_bytes, nullptr)))
         return rc;
     if ((rc = fetch_scalar(h.scalar, sumTrP))) return rc;
     *time = now_s() - t0;
@@ -1472,7 +1477,7 @@ int polyakov_c(const int32_t* NT, const int32_t* NX, const int32_t* NY, const in
     HostField h;
     int rc;
     if ((rc = load_host_field(NT, NX, NY, NZ, data, h, 0, 0))) return rc;  // time links
-    if ((rc = flue_polyakov(h.dims, h.soa, FLUE_F64, h.scalar, nullptr, 0, nullptr))) return rc;
+    if ((rc = flue_polyakov(h.dims, h.soa, FLUE_F64, h.scalar, h.ws, h.ws_bytes, nullptr))) return rc;
     if ((rc = fetch_scalar(h.scalar, sumTrP))) return rc;
     *nP = (int32_t)h.L.Vs;
     *time = now_s() - t0;
@@ -1513,7 +1518,7 @@ int magnetic_c(const int32_t* NT, const int32_t* NX, const int32_t* NY, const in
     HostField h;
     int rc;
     if ((rc = load_host_field(NT, NX, NY, NZ, data, h, 1, 3))) return rc;  // spatial links
-    if ((rc = flue_magnetic(h.dims, h.soa, FLUE_F64, h.scalar, nullptr, 0, nullptr))) return rc;
+    if ((rc = flue_magnetic(h.dims, h.soa, FLUE_F64, h.scalar, h.ws, h.ws_bytes, nullptr))) return rc;
     return fetch_scalar(h.scalar, B);
 }
 
@@ -1533,7 +1538,7 @@ static int rect_host(const int32_t* NT, const int32_t* NX, const int32_t* NY, co
     int rc;
     if ((rc = load_host_field(NT, NX, NY, NZ, data, h, std::min(*mu, *nu) - 1, std::max(*mu, *nu) - 1))) return rc;
     if (tau < 0 || tau > h.dims[0]) return FLUE_EINVAL;
-    if ((rc = flue_path_trace(h.dims, h.soa, FLUE_F64, path, n, tau, h.scalar, nullptr, 0, nullptr))) return rc;
+    if ((rc = flue_path_trace(h.dims, h.soa, FLUE_F64, path, n, tau, h.scalar, h.ws, h.ws_bytes, nullptr))) return rc;
     double s;
     if ((rc = fetch_scalar(h.scalar, &s))) return rc;
     *loopVal = s / (double)(tau > 0 ? h.L.Vs : h.L.V);
