@@ -691,10 +691,10 @@ constexpr uint32_t kEnsRectSitesF32 = 49152;
 // Every configuration has to suit the tiles (extents as in rect_fits) and its footprints to fit the
 // plaquette parts' 48 reals a site; the sites are counted over the ensemble, since it runs as one launch,
 // and the tiles are those that cost least on a full chip.  A measurement (B and the plaquettes), ms by
-// quadrants -> by tiles, FP32 and FP64:
+// quadrants -> by tiles, FP32 (of fields large enough) and FP64:
 //   2 x 16^3x12         98,304 sites   0.156 -> 0.115   0.272 -> 0.194
-//   5 x 12^3x13        112,320         0.167 -> 0.155   0.277 -> 0.241
-//   8 x 12x13x14x10    174,720         0.247 -> 0.166   0.392 -> 0.304
+//   5 x 12^3x13        112,320                          0.277 -> 0.241
+//   8 x 12x13x14x10    174,720                          0.392 -> 0.304
 //   8 x 16^4           524,288         0.665 -> 0.365   1.191 -> 0.677
 bool ens_rect_plan(const EnsEntry* tab, int n, int is_f32, uint32_t maxV, EnsRect* rect, EnsRectGrid* g) {
     if (!fits_buffer(maxV, is_f32)) return false;
